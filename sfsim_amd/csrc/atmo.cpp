@@ -243,7 +243,7 @@ int validate(sfsim_atmo_ctx* ctx, const sfsim_atmo_params* p) {
   if (count4(p->scatter_shape) > (1LL << 31) / 4 || count2(p->transmittance_shape) > (1LL << 30) ||
       count2(p->surface_radiance_shape) > (1LL << 30))
     return fail(ctx, SFSIM_ATMO_ERR_ARGUMENT, "table too large");
-  if ((long long)p->scatter_shape[2] * p->scatter_shape[3] > 1024)
+  if ((long long)p->scatter_shape[2] * p->scatter_shape[3] > kMaxSlab)
     return fail(ctx, SFSIM_ATMO_ERR_ARGUMENT, "sun-elevation x heading size must be <= 1024");
   if (p->ray_steps < 1 || p->ray_steps > kMaxSteps)
     return fail(ctx, SFSIM_ATMO_ERR_ARGUMENT, "ray_steps must be in [1, 256]");
@@ -342,6 +342,7 @@ DevParams make_dev_params(const sfsim_atmo_params* p) {
     P.nE[d] = p->surface_radiance_shape[d];
   }
   for (int d = 0; d < 4; ++d) P.nS[d] = p->scatter_shape[d];
+  rs_split(P);
   P.ray_steps = p->ray_steps;
   P.inv_steps = 1.0 / p->ray_steps;
   // SFSIM_ATMO_GRAZE_HEIGHT (metres, >= 0) overrides the altitude below which a segment's lowest
@@ -367,9 +368,7 @@ DevParams dev_params(const sfsim_atmo_ctx* ctx, const sfsim_atmo_params* p) {
   P.ray_geo = (char*)ctx->ray_geo.ptr;
   P.rmap = (char*)ctx->rmap.ptr;  // filled by launch_resample_map at the start of a pipeline
   if (ctx->sunmap.ptr) {          // filled with rmap
-    P.sun_ps = (float4*)ctx->sunmap.ptr;
-    P.sun_rs = P.sun_ps + count4(p->scatter_shape);
-    P.sun_ss = (double2*)(P.sun_rs + count4(p->scatter_shape));
+    sun_map_view(P, ctx->sunmap.ptr);
   }
   P.sgeo = (float4*)ctx->sgeo.ptr;  // filled by launch_surface_geometry before the surface-radiance stages
   P.ray_order = (const int*)ctx->ray_order.ptr;  // set by ensure_ray_order
@@ -419,9 +418,10 @@ int ensure_sun_depth(sfsim_atmo_ctx* ctx) {
 int ensure_scatter_buffers(sfsim_atmo_ctx* ctx, const sfsim_atmo_params* p) {
   TRY(ensure_sun_depth(ctx));
   TRY(ensure_ray_order(ctx, p));
-  TRY(ensure(ctx, ctx->rmap, resample_map_bytes(make_dev_params(p))));
-  TRY(ensure(ctx, ctx->sunmap, (2 * sizeof(float4) + sizeof(double2)) * (size_t)count4(p->scatter_shape)));
-  return ensure(ctx, ctx->ray_geo, ray_geometry_bytes(make_dev_params(p)));
+  const DevParams P = make_dev_params(p);
+  TRY(ensure(ctx, ctx->rmap, resample_map_bytes(P)));
+  TRY(ensure(ctx, ctx->sunmap, sun_map_bytes(P)));
+  return ensure(ctx, ctx->ray_geo, ray_geometry_bytes(P));
 }
 
 // sphere.clj:62-105 for the normal (1 0 0) of every grid point: rings theta_i = range (i + 1/2) / N,
@@ -561,11 +561,11 @@ int prepare_pipeline(sfsim_atmo_ctx* ctx, const sfsim_atmo_params* p) {
     TRY(ensure(ctx, ctx->dE[i], nE * sizeof(float4)));
     TRY(ensure(ctx, ctx->Eacc[i], nE * sizeof(float4)));
     TRY(ensure(ctx, ctx->dS[i], nS * sizeof(float4)));
-    TRY(ensure(ctx, ctx->Sacc[i], nS * sizeof(float4)));
   }
+  TRY(ensure(ctx, ctx->Sacc[0], nS * sizeof(float4)));
   TRY(ensure(ctx, ctx->R1, nS * sizeof(float4)));
   TRY(ensure(ctx, ctx->M1, nS * sizeof(float4)));
-  TRY(ensure(ctx, ctx->dJ, nS * sizeof(float4)));
+  TRY(ensure(ctx, ctx->dJ, nS * 3 * sizeof(float)));
   if (p->iterations > 0)
     for (int i = 0; i < 2; ++i) TRY(ensure(ctx, ctx->Ssum[i], nS * sizeof(float4)));
   const size_t outc[4] = {nT * 3, nE * 3, nS * 3, nS * 3};
@@ -605,7 +605,7 @@ int enqueue_prologue(sfsim_atmo_ctx* ctx, const sfsim_atmo_params* p, const DevP
     J.half_n = ctx->half_n;
     J.wc = wc;
     LAUNCH(timer, kRayGeometry, launch_prologue(P, J, ctx->stream));
-    LAUNCH(timer, kSingleScatter, launch_single_scatter(P, f4(ctx->R1), f4(ctx->M1), wc, ctx->stream, true));
+    LAUNCH(timer, kSingleScatter, launch_single_scatter(P, f4(ctx->R1), f4(ctx->M1), wc, ctx->stream, true, dirs));
     return 0;
   }
   LAUNCH(timer, kTransmittance, launch_transmittance(P, f4(ctx->T), wc, ctx->stream));
@@ -618,7 +618,7 @@ int enqueue_prologue(sfsim_atmo_ctx* ctx, const sfsim_atmo_params* p, const DevP
   }
   LAUNCH(timer, kRayGeometry, launch_ray_geometry(P, wc, ctx->stream));
   LAUNCH(timer, kAccumulate, launch_resample_map(P, ctx->stream));
-  LAUNCH(timer, kSingleScatter, launch_single_scatter(P, f4(ctx->R1), f4(ctx->M1), wc, ctx->stream));
+  LAUNCH(timer, kSingleScatter, launch_single_scatter(P, f4(ctx->R1), f4(ctx->M1), wc, ctx->stream, false, dirs));
   return 0;
 }
 
@@ -665,7 +665,7 @@ int enqueue_pipeline(sfsim_atmo_ctx* ctx, const sfsim_atmo_params* p, const DevP
     const SrJob sr{0, ctx->half_n, dS_tab, mie, f4(ctx->dE[dE_new])};
     LAUNCH(timer, kPointScatter,
            launch_point_scatter(P, sdirs, ctx->sphere_n, ctx->geom.ptr, dS_tab, mie, f4(ctx->dE[dE_cur]), f4(ctx->slab),
-                                f4(ctx->slab_mie), f4(ctx->dJ), wc, ctx->stream, sr_along ? &sr : nullptr));
+                                f4(ctx->slab_mie), (float*)ctx->dJ.ptr, wc, ctx->stream, sr_along ? &sr : nullptr));
     if (!sr_along)
       LAUNCH(timer, kSurfaceRadiance,
              launch_surface_radiance(P, ctx->half_n, dS_tab, mie, f4(ctx->dE[dE_new]), wc, ctx->stream));
@@ -677,7 +677,8 @@ int enqueue_pipeline(sfsim_atmo_ctx* ctx, const sfsim_atmo_params* p, const DevP
     acc.dE = f4(ctx->dE[dE_new]);
     acc.E_in = E_cur;
     acc.E_out = f4(ctx->Eacc[e_next]);
-    LAUNCH(timer, kRayScatter, launch_ray_scatter(P, f4(ctx->dJ), f4(ctx->dS[dS_new]), wc, ctx->stream, acc));
+    LAUNCH(timer, kRayScatter, launch_ray_scatter(P, (const float*)ctx->dJ.ptr, f4(ctx->dS[dS_new]), wc, ctx->stream, acc,
+                                                  capture != nullptr));
     dE_cur = dE_new;
     dS_cur = dS_new;
     E_cur = f4(ctx->Eacc[e_next]);
@@ -827,7 +828,7 @@ int prepare_seeded(sfsim_atmo_ctx* ctx, const sfsim_atmo_params* p, int m, const
   }
   TRY(ensure(ctx, ctx->R1, nS * sizeof(float4)));
   TRY(ensure(ctx, ctx->M1, nS * sizeof(float4)));
-  TRY(ensure(ctx, ctx->dJ, nS * sizeof(float4)));
+  TRY(ensure(ctx, ctx->dJ, nS * 3 * sizeof(float)));
   for (int i = 0; i < N; ++i) TRY(ensure(ctx, ctx->pred[i], nS * sizeof(float4)));
   TRY(ensure(ctx, ctx->resid, residual_scratch_floats((long long)nS) * sizeof(float)));
   if (host_sums) TRY(ensure(ctx, ctx->stage_rgb, nS * 3 * sizeof(float)));
@@ -897,8 +898,8 @@ int enqueue_seeded(sfsim_atmo_ctx* ctx, const sfsim_atmo_params* p, const DevPar
     const SrJob sr{0, ctx->half_n, A, f4(ctx->M1), f4(ctx->dE[1])};
     LAUNCH(timer, kPointScatter,
            launch_point_scatter(P, sdirs, ctx->sphere_n, ctx->geom.ptr, A, f4(ctx->M1), Esum, f4(ctx->slab),
-                                f4(ctx->slab_mie), f4(ctx->dJ), nullptr, ctx->stream, sr_along ? &sr : nullptr));
-    LAUNCH(timer, kRayScatter, launch_ray_scatter(P, f4(ctx->dJ), Pk, nullptr, ctx->stream));
+                                f4(ctx->slab_mie), (float*)ctx->dJ.ptr, nullptr, ctx->stream, sr_along ? &sr : nullptr));
+    LAUNCH(timer, kRayScatter, launch_ray_scatter(P, (const float*)ctx->dJ.ptr, Pk, nullptr, ctx->stream));
     if (!sr_along)
       LAUNCH(timer, kSurfaceRadiance,
              launch_surface_radiance(P, ctx->half_n, A, f4(ctx->M1), f4(ctx->dE[1]), nullptr, ctx->stream));
@@ -1058,7 +1059,7 @@ size_t layout_shared(sfsim_atmo_ctx* c, const sfsim_atmo_params* p, char* base) 
   const size_t nS = (size_t)count4(p->scatter_shape);
   k.take(c->ray_order, (size_t)p->scatter_shape[0] * p->scatter_shape[1] * sizeof(int));
   k.take(c->rmap, resample_map_bytes(P));
-  k.take(c->sunmap, (2 * sizeof(float4) + sizeof(double2)) * nS);
+  k.take(c->sunmap, sun_map_bytes(P));
   if (p->iterations > 0) {
     const int sn = sfsim_atmo_sphere_directions(0, p->sphere_steps), hn = sfsim_atmo_sphere_directions(1, p->ray_steps);
     k.take(c->sphere_dirs, (size_t)sn * sizeof(Dir));
@@ -1090,11 +1091,11 @@ size_t layout_atmosphere(sfsim_atmo_ctx* c, const sfsim_atmo_params* p, char* ba
     k.take(c->dE[i], nE * sizeof(float4));
     k.take(c->Eacc[i], nE * sizeof(float4));
     k.take(c->dS[i], nS * sizeof(float4));
-    k.take(c->Sacc[i], nS * sizeof(float4));
   }
+  k.take(c->Sacc[0], nS * sizeof(float4));
   k.take(c->R1, nS * sizeof(float4));
   k.take(c->M1, nS * sizeof(float4));
-  k.take(c->dJ, nS * sizeof(float4));
+  k.take(c->dJ, nS * 3 * sizeof(float));
   if (with_outputs) {
     const size_t outc[4] = {nT * 3, nE * 3, nS * 3, nS * 3};
     for (int i = 0; i < 4; ++i) k.take(c->out[i], outc[i] * sizeof(float));
@@ -1247,13 +1248,16 @@ int sfsim_atmo_point_scatter_table(sfsim_atmo_ctx* ctx, const sfsim_atmo_params*
   TRY(upload_table(ctx, 1, mie_strength, n, &dM));
   TRY(upload_table(ctx, 2, dE, ne, &ddE));
   int rc;
-  float4* o = stage_out(ctx, n, &rc);
+  float* o = (float*)stage_out(ctx, n, &rc);
   TRY(rc);
   TRY(prepare_point_scatter(ctx, P, dM != nullptr, nullptr));
   HIP_TRY(ctx, launch_resample_map(P, ctx->stream));  // with it the per-entry sun terms
   HIP_TRY(ctx, launch_point_scatter(P, (const Dir*)ctx->sphere_dirs.ptr, ctx->sphere_n, ctx->geom.ptr, ddS, dM, ddE,
                                     (float4*)ctx->slab.ptr, (float4*)ctx->slab_mie.ptr, o, nullptr, ctx->stream));
-  return download_table(ctx, o, out, n);
+  HIP_TRY(ctx, launch_transpose_rgb(o, (float*)ctx->stage_rgb.ptr, (long long)n, P.nS[3], P.nS[2], ctx->stream));
+  HIP_TRY(ctx, hipMemcpyAsync(out, ctx->stage_rgb.ptr, n * 3 * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
+  HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+  return 0;
 }
 
 int sfsim_atmo_ray_scatter_table(sfsim_atmo_ctx* ctx, const sfsim_atmo_params* p, const float* dJ, float* out) {
@@ -1263,13 +1267,19 @@ int sfsim_atmo_ray_scatter_table(sfsim_atmo_ctx* ctx, const sfsim_atmo_params* p
   TRY(ensure_scatter_buffers(ctx, p));
   DevParams P = dev_params(ctx, p);
   size_t n = (size_t)count4(p->scatter_shape);
-  const float4* ddJ;
-  TRY(upload_table(ctx, 0, dJ, n, &ddJ));
+  if (!finite_floats(dJ, n * 3)) return fail(ctx, SFSIM_ATMO_ERR_NONFINITE, "input table holds NaN/Inf");
+  TRY(ensure(ctx, ctx->stage_rgb, n * 3 * sizeof(float)));
+  TRY(ensure(ctx, ctx->stage_in[0], n * 3 * sizeof(float)));
+  float* ddJ = (float*)ctx->stage_in[0].ptr;
+  HIP_TRY(ctx, hipMemcpyAsync(ctx->stage_rgb.ptr, dJ, n * 3 * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
+  HIP_TRY(ctx, launch_transpose_rgb((const float*)ctx->stage_rgb.ptr, ddJ, (long long)n, P.nS[2], P.nS[3], ctx->stream));
+  HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
   int rc;
   float4* o = stage_out(ctx, n, &rc);
   TRY(rc);
   HIP_TRY(ctx, launch_ray_geometry(P, nullptr, ctx->stream));
   HIP_TRY(ctx, launch_resample_map(P, ctx->stream));  // with it the per-entry sun terms
+  HIP_TRY(ctx, launch_ray_items(P, ctx->stream));
   HIP_TRY(ctx, launch_ray_scatter(P, ddJ, o, nullptr, ctx->stream));
   return download_table(ctx, o, out, n);
 }

@@ -9,7 +9,19 @@
 namespace sfsim {
 
 constexpr int kMaxSteps = 256;   // ray_steps limit (LDS arrays of the per-ray kernels)
+constexpr int kMaxSlab = 1024;   // sun elevations x headings of a view ray
+constexpr int kMaxRsGroups = 8;  // column groups of the ray-scatter kernel
 constexpr int kMaxSphereDirs = 1000;  // 64 bytes of LDS per direction in the point-scatter kernel
+
+// One lookup per sample of the ray-scatter kernel: a sun direction (v . l and x . l rounded from FP64) and a column
+// of the slab; at: column << 16 | the entry's place in its ray's (sun elevation, heading) slab.
+struct RsItem {
+  float vl, xl;
+  unsigned at;
+};
+
+// Items of a group that ray_scatter_kernel looks up with TS texels per lane (64 per slot).
+__host__ __device__ constexpr int rs_items(int ts) { return ts == 1 ? 128 : ts == 2 ? 256 : ts == 4 ? 384 : 512; }
 
 struct DevParams {
   Geo g;
@@ -51,14 +63,20 @@ struct DevParams {
   // per-entry lookup of the 4D re-sampling (forward(backward(i))): NH x NE x NL x NA float4 weights
   // followed by as many ushort4 lower indices (resample_map_bytes); null: computed per launch
   char* rmap;
-  // per-entry sun terms, written with the re-sampling map (launch_resample_map) and read by every
-  // point- and ray-scatter launch: sun_ps = (l, the sun-elevation coordinate) for point scattering,
-  // sun_rs = (v . l, x . l, the heading coordinate, 0) for ray scattering, each rounded once from FP64
-  // (NH x NE x NL x NA float4 each); sun_ss = (v . l, x . l) in FP64 for single scattering's horizon
-  // tests (the table path)
+  // per-entry sun terms, written with the re-sampling map (launch_resample_map): sun_ps = (l, the sun-elevation
+  // coordinate) for point scattering, rounded once from FP64 (NH x NE x NL x NA float4); sun_ss = (v . l, x . l) in
+  // FP64 for single scattering's horizon tests (the table path) and the exact sun coordinate
   float4* sun_ps;
-  float4* sun_rs;
   double2* sun_ss;
+  // the split of a ray's (sun elevation, heading) slab in ray_scatter_kernel (rs_split): rs_groups groups of rs_cols
+  // columns (headings), rs_ts texels per lane, rs_slots items per group at most
+  int rs_cols, rs_groups, rs_ts, rs_slots;
+  // written by launch_ray_items (from sun_ss): the rays' items (2 NL NA places per ray, group after group), the place where
+  // each group's items start (rs_groups + 1 per ray), and for each entry the places of its two items (group x
+  // rs_slots + place in the group, low and high half) and the second one's weight
+  RsItem* rs_items;
+  int* rs_heads;
+  uint2* rs_entries;
   // per (surface-radiance height, half-sphere direction): omega.x, omega.y, elevation coordinate of
   // omega at the height's grid point, cosine-weighted quadrature weight (nE[0] x directions float4)
   float4* sgeo;
@@ -89,8 +107,10 @@ __device__ __forceinline__ decltype(auto) params_of(const DevParams& P0, const D
     P.ray_geo = P0.ray_geo ? P0.ray_geo + off : nullptr;
     P.rmap = P0.rmap;
     P.sun_ps = P0.sun_ps;
-    P.sun_rs = P0.sun_rs;
     P.sun_ss = P0.sun_ss;
+    P.rs_items = P0.rs_items;
+    P.rs_heads = P0.rs_heads;
+    P.rs_entries = P0.rs_entries;
     P.sgeo = P0.sgeo;
     P.ray_order = P0.ray_order;
     return P;
@@ -115,6 +135,37 @@ __device__ __forceinline__ T* atm_ptr(T* p, const DevParams& P) {
 
 __host__ __device__ inline size_t resample_map_bytes(const DevParams& P) {
   return (size_t)P.nS[0] * P.nS[1] * P.nS[2] * P.nS[3] * (sizeof(float4) + sizeof(ushort4));
+}
+
+// The split of a ray's slab: as many whole columns per group as 256 texels hold (4 per lane), evenly; a
+// column of more than 256 rows is a group of its own.  The texels per lane also set how many items a group may
+// have: per sun elevation one for each heading whose sun direction is not clamped and two for each of the
+// clamped directions (at most two), NL (NA + 2) in a slab of one group; of several groups, their share and a
+// quarter (rays with more take the sample-by-sample path).
+inline void rs_split(DevParams& P) {
+  const int NL = P.nS[2], NA = P.nS[3], most = NL > 256 ? 1 : 256 / NL;
+  const int want = (NA + most - 1) / most;
+  P.rs_cols = (NA + want - 1) / want;
+  P.rs_groups = (NA + P.rs_cols - 1) / P.rs_cols;
+  const int texels = P.rs_cols * NL;
+  const int items = P.rs_groups == 1 ? NL * (NA + 2) : (int)(1.25 * NL * (NA + 2) * P.rs_cols / NA);
+  for (P.rs_ts = 1; P.rs_ts < 8 && (texels > 64 * P.rs_ts || items > rs_items(P.rs_ts));) P.rs_ts *= 2;
+  P.rs_slots = rs_items(P.rs_ts);
+}
+
+// Bytes of the sun terms and the ray-scatter items (laid out by sun_map_view).
+__host__ __device__ inline size_t sun_map_bytes(const DevParams& P) {
+  const size_t rays = (size_t)P.nS[0] * P.nS[1], n = rays * P.nS[2] * P.nS[3];
+  return n * (sizeof(float4) + sizeof(double2) + sizeof(uint2) + 2 * sizeof(RsItem)) + rays * (P.rs_groups + 1) * sizeof(int);
+}
+
+inline void sun_map_view(DevParams& P, void* mem) {
+  const size_t rays = (size_t)P.nS[0] * P.nS[1], n = rays * P.nS[2] * P.nS[3];
+  P.sun_ps = (float4*)mem;
+  P.sun_ss = (double2*)(P.sun_ps + n);
+  P.rs_entries = (uint2*)(P.sun_ss + n);
+  P.rs_items = (RsItem*)(P.rs_entries + n);
+  P.rs_heads = (int*)(P.rs_items + 2 * n);
 }
 
 // Views of DevParams::ray_geo: m = NH x NE x ray_steps samples, sample i of view ray (ih, ie) at

@@ -22,7 +22,6 @@ namespace sfsim {
 namespace {
 
 constexpr int kBlock = 256;
-constexpr int kMaxRayChunk = 8;  // samples per slab chunk of the ray-scatter kernel
 
 __device__ __forceinline__ float fexp2(float x) { return __builtin_amdgcn_exp2f(x); }
 // min(floor(x), hi) for a coordinate already clamped to x >= 0, as one med3 (fminf would quiet a
@@ -627,6 +626,70 @@ __global__ void __launch_bounds__(kBlock) ray_geometry_kernel(const DevParams P,
   ray_geometry_body(P, wc, blockIdx.x);
 }
 
+// The ray-scatter items of one view ray (DevParams::rs_items), by one workgroup: one per entry whose heading
+// coordinate is integral, two (the columns beside it) otherwise, none for an entry with the sun direction of the
+// heading before it (clamped to the same one: the same FP64 v . l at the same sun elevation).  In (heading, sun
+// elevation) order, so that neighbouring lanes of ray_scatter_kernel read neighbouring rows of a column; with
+// several groups of columns counted first and then written group after group.  s_pos: NL x NA words of LDS.
+__device__ __forceinline__ void ray_items_body(const DevParams& P, int rayid, unsigned* s_pos) {
+  __shared__ int s_count[kMaxRsGroups], s_start[kMaxRsGroups + 1];
+  const int NL = P.nS[2], NA = P.nS[3], NLA = NL * NA, groups = P.rs_groups;
+  const long long base = (long long)rayid * NLA;
+  const double2* __restrict__ ss = P.sun_ss + base;
+  const int lane = threadIdx.x & 63;
+  if (threadIdx.x <= kMaxRsGroups) {
+    s_start[threadIdx.x] = 0;
+    if (threadIdx.x < kMaxRsGroups) s_count[threadIdx.x] = 0;
+  }
+  __syncthreads();
+  for (int pass = groups == 1 ? 1 : 0; pass < 2; ++pass) {
+    for (int b = threadIdx.x - lane; b < NLA; b += blockDim.x) {
+      const int q = min(b + lane, NLA - 1), a = q / NL, s = q - a * NL, k = s * NA + a;
+      const double2 d = ss[k];
+      const Lerp L = make_lerp((float)sun_angle_to_index(NA, d.x), NA);
+      const bool same = a > 0 && d.x == ss[max(k - 1, 0)].x, own = b + lane < NLA && !same;
+      unsigned pos[2] = {0, 0};
+      for (int g = 0; g < groups; ++g)
+        for (int j = 0; j < 2; ++j) {
+          const int col = j ? L.i1 : L.i0;
+          const bool want = own && (j == 0 || L.s != 0.0f) && (groups == 1 || col / P.rs_cols == g);
+          const unsigned long long mask = __ballot(want);
+          if (mask == 0) continue;
+          int first = 0;
+          if (lane == 0) first = atomicAdd(&s_count[g], __popcll(mask));
+          const int idx = __builtin_amdgcn_readfirstlane(first) + __popcll(mask & ((1ull << lane) - 1));
+          if (want && pass == 1) {
+            P.rs_items[2 * base + s_start[g] + idx] = RsItem{(float)d.x, (float)d.y, ((unsigned)col << 16) | (unsigned)k};
+            pos[j] = (unsigned)(g * P.rs_slots + idx);  // (read only where every group's items fit the slots)
+          }
+        }
+      if (b + lane < NLA && pass == 1) s_pos[k] = same ? 0xffffffffu : (pos[1] << 16) | (pos[0] & 0xffffu);
+    }
+    __syncthreads();
+    if (pass == 0) {
+      if (threadIdx.x == 0)
+        for (int g = 0; g < groups; ++g) {
+          s_start[g + 1] = s_start[g] + s_count[g];
+          s_count[g] = 0;
+        }
+      __syncthreads();
+    }
+  }
+  if ((int)threadIdx.x <= groups)
+    P.rs_heads[(long long)rayid * (groups + 1) + threadIdx.x] =
+        (int)threadIdx.x < groups ? s_start[threadIdx.x] : s_start[groups - 1] + s_count[groups - 1];
+  for (int k = threadIdx.x; k < NLA; k += blockDim.x) {
+    unsigned p = s_pos[k];
+    for (int q = k; p == 0xffffffffu;) p = s_pos[--q];
+    P.rs_entries[base + k] = make_uint2(p, __float_as_uint(make_lerp((float)sun_angle_to_index(NA, ss[k].x), NA).s));
+  }
+}
+
+__global__ void __launch_bounds__(kBlock) ray_items_kernel(const DevParams P) {
+  extern __shared__ unsigned s_pos[];
+  ray_items_body(P, (int)blockIdx.x, s_pos);
+}
+
 // Single scatter with the sun segments' optical depths read from the sun_depth table: one block per
 // view ray, one thread per (sun elevation, heading) entry, each adding its lit samples in sample order.
 // The ray's samples (t, h, T(x, p_i), sun-table terms) come from the per-build geometry through LDS.
@@ -636,8 +699,14 @@ template <bool kB>
 __global__ void __launch_bounds__(kSSTBlock) single_scatter_table_kernel(
     const DevParams P0, const DevParams* __restrict__ PB, const double2* __restrict__ geo_th,
     const float4* __restrict__ geo_T, const float4* __restrict__ geo_ss, const float2* __restrict__ geo_row,
-    float4* __restrict__ R1, float4* __restrict__ M1, WorkCounters* wc) {
+    float4* __restrict__ R1, float4* __restrict__ M1, int item_blocks, WorkCounters* wc) {
+  extern __shared__ unsigned char s_raw[];
   const DevParams& P = params_of<kB>(P0, PB);
+  // the rays' ray-scatter items (shared by the atmospheres of a batch) ride in the launch's first workgroups
+  if ((int)blockIdx.x < item_blocks) {
+    if (!kB || blockIdx.z == 0) ray_items_body(P, (int)blockIdx.x, (unsigned*)s_raw);
+    return;
+  }
   if constexpr (kB) {  // this atmosphere's tables and ray geometry (offsets of the restrict arguments, whose
                        // loads stay provably unclobbered and uniform: scalar loads)
     geo_th = atm_ptr<kB>(geo_th, P0);
@@ -650,12 +719,11 @@ __global__ void __launch_bounds__(kSSTBlock) single_scatter_table_kernel(
   const int NE = P.nS[1], NL = P.nS[2], NA = P.nS[3];
   const int NLA = NL * NA;
   const int n = P.ray_steps, cols = P.sun_cols;
-  const int rayid = xcd_ray(blockIdx.x, P.nS[0] * NE);
+  const int rayid = xcd_ray(blockIdx.x - item_blocks, P.nS[0] * NE);
   const int ih = rayid / NE, ie = rayid - ih * NE;
   const Ray ray = make_ray(P, ih, ie);
   const double dt = ray.D / n;
   // this ray's samples from the per-build geometry, staged in LDS
-  extern __shared__ unsigned char s_raw[];
   double2* s_th = (double2*)s_raw;      // [n] t_i, h_i
   float4* s_w = (float4*)(s_th + n);    // [n] T(x, p_i) rgb, w: exp(-h_i / H_mie)
   float4* s_g = s_w + n;                // [n] Rt^2 - r_i^2, D_min, (cols - 1) / (D_max - D_min), exp(-h_i / H_rayleigh)
@@ -715,18 +783,26 @@ __global__ void __launch_bounds__(kSSTBlock) single_scatter_table_kernel(
 }
 
 // dS' = ray-scatter of an interpolated dJ table (atmosphere_lut.clj:92,94; atmosphere.clj:192-200).
-// One workgroup per view ray; lanes over (sun elevation, heading) entries, up to EPT per lane.
-// At sample p_i the height and elevation coordinates of the dJ lookup are the same for every
-// entry of the ray, so the workgroup first folds those two dimensions into a (sun elevation,
-// heading) slab in LDS (coalesced reads of four dJ slabs), Q samples at a time; each lane then
-// interpolates its own sun-elevation / heading coordinates in that slab.
-// One entry's samples i0 .. i0 + qn - 1 of the folded slabs.  The sun-elevation coordinate of
-// sun-elevation-to-index (atmosphere.clj:322-326) at p_i, (NL - 1) max(0, (1 - exp(-3 s - 0.6)) / (1 - exp(-3.6)))
-// with s = dot(p_i, l) / |p_i| = (xl + t_i vl) / r_i, is A - A exp2(alpha_i xl + beta_i vl + c) with
-// A = (NL - 1) / (1 - exp(-3.6)), alpha_i = -3 log2(e) / r_i, beta_i = alpha_i t_i, c = -0.6 log2(e), clamped
-// to [0, NL - 1] (interpolate.clj:75-98 clips the coordinate); the lower row is min(floor, NL - 2), so
-// the upper row is always the next one (weight 1 on it at the clamped top).  LDS byte offsets are
-// formed in FP32 (exact below 2^24).
+//
+// dJ comes packed: 3 floats per entry, each ray's slab in (heading, sun elevation) order, a "column" being
+// the sun elevations of one heading.  At sample p_i the height and elevation coordinates of the lookup are the
+// same for every entry of the ray, so those two dimensions are folded once per sample, and each entry then
+// interpolates its own sun-elevation coordinate in the folded slab.  Its heading coordinate is constant along
+// the ray: the sum over the samples is taken per column and the two columns are mixed at the end, so that a
+// lookup needs one column only ("item": a column and a sun direction).  Entries whose sun direction
+// index-to-sun-direction clamps to the same one share their items.
+//
+// One workgroup per view ray.  A wavefront owns a group of columns (TS x 64 folded texels at most) and a
+// contiguous segment of the ray's samples: it folds its columns into a slab of its own in LDS and looks its
+// items up there, so no barrier separates the two.  What bounds it is VALU issue: per sample and wavefront
+// of the 32 x 64 x 32 x 8 grid 4 x 12 multiply-adds of the fold and 5 x 20 instructions of the lookups, with
+// the nodes' loads (L2) and the slab's LDS reads behind them.
+//
+// The sun-elevation coordinate of sun-elevation-to-index (atmosphere.clj:322-326) at p_i,
+// (NL - 1) max(0, (1 - exp(-3 s - 0.6)) / (1 - exp(-3.6))) with s = dot(p_i, l) / |p_i| = (xl + t_i vl) / r_i, is
+// A - A exp2(alpha_i xl + beta_i vl + c) with A = (NL - 1) / (1 - exp(-3.6)), alpha_i = -3 log2(e) / r_i,
+// beta_i = alpha_i t_i, c = -0.6 log2(e), clamped to [0, NL - 1] (interpolate.clj:75-98 clips the coordinate).
+// Each column of the slab ends in a zero texel, which only the coordinate NL - 1 reads, with weight zero.
 struct SunCoord {
   float A, c, top;  // A, c, NL - 1
 };
@@ -749,7 +825,7 @@ constexpr int kExactSunRows = 16;
 // its lower row and weight, the weight formed in FP64 before rounding (a coordinate just above a row, say
 // 1 + 5e-6, would lose 1% of its weight to the FP32 spacing at 1).  A64: (NL - 1) / (1 - e^-3.6).
 __device__ __forceinline__ void sun_coord_exact(const SunCoord& sc, double A64, double R, double2 th, double xl,
-                                                double vl, float& row, float& s) {
+                                                double vl, unsigned& row, float& s) {
   const double r = R + th.y;
   double inv = (double)__builtin_amdgcn_rcpf((float)r);
   inv = fma(inv, fma(-r, inv, 1.0), inv);
@@ -757,138 +833,12 @@ __device__ __forceinline__ void sun_coord_exact(const SunCoord& sc, double A64, 
   const double z = fma(a * th.x, vl, fma(a, xl, -0.6));
   const double c = fmin(fmax(-expm1(z) * A64, 0.0), (double)sc.top);
   const double r0 = fmin(floor(c), (double)sc.top - 1.0);
-  row = (float)r0;
+  row = (unsigned)r0;
   s = (float)(c - r0);
 }
 
 __device__ __forceinline__ float3 lerp3(float4 a, float4 b, float s) {
   return make_float3(fmaf(s, b.x - a.x, a.x), fmaf(s, b.y - a.y, a.y), fmaf(s, b.z - a.z, a.z));
-}
-
-__device__ __forceinline__ float4 lds4(const float4* base, unsigned byte_offset) {
-  return *(const float4*)((const char*)base + byte_offset);
-}
-
-// Samples whose per-sample terms (the lookups' T and sun-coordinate terms, the fold's steps) are requested
-// together, before the barrier that precedes their chunk: one wait per group instead of one per sample.
-constexpr int kStepGroup = 4;
-
-// Per-sample terms of kStepGroup consecutive samples for the lookups, in scalar registers: T(x, p_i) and
-// (alpha_i, beta_i), requested together (before the barrier that precedes their chunk).
-struct SampleGroup {
-  float4 T[kStepGroup];
-  float2 ab[kStepGroup];
-  double2 th[kStepGroup];  // t_i, h_i (the exact sun coordinate only)
-};
-
-template <bool kExact>
-__device__ __forceinline__ void load_sample_group(const float4* __restrict__ gT, const float4* __restrict__ gRS,
-                                                  const double2* __restrict__ gTH, int i, int n, SampleGroup& g) {
-#pragma unroll
-  for (int q = 0; q < kStepGroup; ++q) {
-    const int j = min(i + q, n - 1);  // in bounds
-    g.T[q] = gT[j];
-    const float4 r = gRS[j];
-    g.ab[q] = make_float2(r.z, r.w);
-    if (kExact) g.th[q] = gTH[j];
-  }
-}
-
-// The entry's sun-elevation coordinate terms: FP32 (xl, vl) and, for the exact form, FP64 ones, R and A64.
-struct SunTerms {
-  float xl, vl;
-  double xl64, vl64, R, A64;
-};
-
-// ray_scatter_samples over samples b .. min(b + kStepGroup, qn) - 1 of the chunk (b a multiple of
-// kStepGroup), their terms in g: the same operations in the same order.
-template <bool kColumn, bool kExact>
-__device__ __forceinline__ float3 ray_scatter_sample_group(const SunCoord& sc, const float4* s_slab,
-                                                           const SampleGroup& g, int b, int qn, float row_bytes,
-                                                           float col_bytes, int NLA, const SunTerms& st, Lerp La,
-                                                           float3 acc) {
-  const unsigned rb = (unsigned)row_bytes;
-  const float slab_bytes = (float)(NLA * (int)sizeof(float4));
-  float q_bytes = fmaf((float)b, slab_bytes, col_bytes);  // byte offset of the entry's column in slab b (exact)
-#pragma unroll
-  for (int q = 0; q < kStepGroup; ++q, q_bytes += slab_bytes) {
-    if (b + q < qn) {
-      const float4 w = g.T[q];
-      float row, s;
-      if (kExact) {
-        sun_coord_exact(sc, st.A64, st.R, g.th[q], st.xl64, st.vl64, row, s);
-      } else {
-        const float c = sun_coord(sc, g.ab[q], st.xl, st.vl);
-        row = lower_cell(c, sc.top - 1.0f);
-        s = c - row;
-      }
-      const unsigned off = (unsigned)fmaf(row, row_bytes, q_bytes);
-      float3 v;
-      if (kColumn) {
-        v = lerp3(lds4(s_slab, off), lds4(s_slab, off + rb), s);
-      } else {
-        const unsigned d = (unsigned)(La.i1 - La.i0) * (unsigned)sizeof(float4);
-        const float3 u = lerp3(lds4(s_slab, off), lds4(s_slab, off + d), La.s);
-        const float3 t = lerp3(lds4(s_slab, off + rb), lds4(s_slab, off + rb + d), La.s);
-        v = make_float3(fmaf(s, t.x - u.x, u.x), fmaf(s, t.y - u.y, u.y), fmaf(s, t.z - u.z, u.z));
-      }
-      acc.x = fmaf(w.x, v.x, acc.x);
-      acc.y = fmaf(w.y, v.y, acc.y);
-      acc.z = fmaf(w.z, v.z, acc.z);
-    }
-  }
-  return acc;
-}
-
-template <bool kColumn, bool kExact>
-__device__ __forceinline__ float3 ray_scatter_samples(const SunCoord& sc, const float4* s_slab,
-                                                      const float4* __restrict__ gT, const float4* __restrict__ gRS,
-                                                      const double2* __restrict__ gTH, int i0, int qn, float row_bytes,
-                                                      float col_bytes, int NLA, const SunTerms& st, Lerp La,
-                                                      float3 acc) {
-  const unsigned rb = (unsigned)row_bytes;
-  const float slab_bytes = (float)(NLA * (int)sizeof(float4));
-  float q_bytes = col_bytes;  // byte offset of the entry's column in slab q
-  for (int q = 0; q < qn; ++q, q_bytes += slab_bytes) {
-    const int i = i0 + q;
-    const float4 w = gT[i];  // workgroup-uniform: scalar loads
-    const float4 g = gRS[i];
-    float row, s;
-    if (kExact) {
-      sun_coord_exact(sc, st.A64, st.R, gTH[i], st.xl64, st.vl64, row, s);
-    } else {
-      const float c = sun_coord(sc, make_float2(g.z, g.w), st.xl, st.vl);
-      row = lower_cell(c, sc.top - 1.0f);
-      s = c - row;
-    }
-    const unsigned off = (unsigned)fmaf(row, row_bytes, q_bytes);
-    float3 v;
-    if (kColumn) {
-      v = lerp3(lds4(s_slab, off), lds4(s_slab, off + rb), s);
-    } else {
-      const unsigned d = (unsigned)(La.i1 - La.i0) * (unsigned)sizeof(float4);
-      const float3 u = lerp3(lds4(s_slab, off), lds4(s_slab, off + d), La.s);
-      const float3 t = lerp3(lds4(s_slab, off + rb), lds4(s_slab, off + rb + d), La.s);
-      v = make_float3(fmaf(s, t.x - u.x, u.x), fmaf(s, t.y - u.y, u.y), fmaf(s, t.z - u.z, u.z));
-    }
-    acc.x = fmaf(w.x, v.x, acc.x);
-    acc.y = fmaf(w.y, v.y, acc.y);
-    acc.z = fmaf(w.z, v.z, acc.z);
-  }
-  return acc;
-}
-
-// Register slots of the fold: slot ((h & 1) << 1) | (e & 1) holds dJ at node (h, e) for the folding
-// thread's entry.  The four corners of a cell have distinct parities, so every sample's corners occupy
-// the four slots, and a corner shared with the previous sample is already in its slot: a slot is
-// re-read only when its node changes (about 60 node reads per ray of 64 samples instead of four per
-// sample that changes cell).  The nodes and weights of every sample come from the per-build ray geometry.
-struct FoldSlots {
-  float4 v[4];
-};
-
-__device__ __forceinline__ void fold_slots_init(FoldSlots& f) {
-  for (int s = 0; s < 4; ++s) f.v[s] = make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
 // The per-build fold steps of one ray, read-only while a ray-scatter launch runs.  The single-atmosphere
@@ -906,109 +856,186 @@ __device__ __forceinline__ FoldStep fold_step(ConstFoldSteps fs, int i) {
   return st;
 }
 
-// The folded value of one entry: the weighted sum of its four slots.
-__device__ __forceinline__ float4 fold_value(const FoldSlots& f, const float4 w) {
-  const float4 a = f.v[0], b = f.v[1], c = f.v[2], d = f.v[3];
-  return make_float4(fmaf(w.w, d.x, fmaf(w.z, c.x, fmaf(w.y, b.x, w.x * a.x))),
-                     fmaf(w.w, d.y, fmaf(w.z, c.y, fmaf(w.y, b.y, w.x * a.y))),
-                     fmaf(w.w, d.z, fmaf(w.z, c.z, fmaf(w.y, b.z, w.x * a.z))), 0.f);
+// Orders LDS accesses of one wavefront's lanes (the hardware keeps a wavefront's LDS accesses in order; this
+// keeps the compiler from moving them across).
+__device__ __forceinline__ void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Fold steps of kStepGroup consecutive samples, held in scalar registers: requested together, one wait
-// for all of them instead of one per sample.
-struct StepGroup {
-  FoldStep s[kStepGroup];
+struct Rgb {
+  float x, y, z;
 };
 
-template <class Steps>
-__device__ __forceinline__ void load_step_group(const Steps fs, int i, int n, StepGroup& g) {
-#pragma unroll
-  for (int q = 0; q < kStepGroup; ++q) g.s[q] = fold_step(fs, min(i + q, n - 1));  // in bounds
+// Register slots of the fold: slot ((h & 1) << 1) | (e & 1) holds dJ at node (h, e) for the lane's texels.
+// The four corners of a cell have distinct parities, so every sample's corners occupy the four slots, and a
+// corner shared with the previous sample is already in its slot: a slot is re-read only when its node
+// changes (about 60 node reads per ray of 64 samples).
+template <int TS>
+struct FoldSlots {
+  Rgb v[4][TS];
+};
+
+// The group's texels of a node as a buffer of `bytes` bytes: lane l's texels lie at 12 (l + 64 j) from its start, and
+// those past the group's read as zero.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t node_buffer(const float* __restrict__ dJ, int off, int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)(dJ + 3LL * off), 0, bytes, 0x00020000);
 }
 
-// Fold of the chunk of samples i0 .. i0 + qn - 1 into `slab` by the nt folding threads (t = 0 .. nt - 1):
-// slab[q][kk] = sum over slots of weight x dJ[node][kk].  fs: the ray's per-build fold steps (node offsets
-// and weights by slot; workgroup-uniform, read with scalar loads, so are the branches).  KPT == 1 (the
-// kernel with one entry per lookup lane, NLA <= nt = 256): the slots (f, f2) carry over from one of the
-// thread's samples to the next and a slot is re-read only where its node changed; prev: the node offsets of
-// the thread's previous sample; sg holds the steps of the chunk's first kStepGroup samples on entry and
-// those of the next chunk's on return (n: samples of the ray).  KPT > 1: every sample reads its nodes.
-template <int KPT, class Steps>
-__device__ __forceinline__ void ray_scatter_fold(const float4* __restrict__ dJ, const Steps fs,
-                                                 float4* slab, int i0, int qn, int NLA, int t, int nt, FoldSlots& f,
-                                                 FoldSlots& f2, int4& prev, StepGroup& sg, int n) {
-  if (KPT == 1) {
-    // the four fold wavefronts split the ray's samples by parity, which halves the chain of dependent
-    // node loads that each of them walks: wavefronts 0-1 fold the even samples, 2-3 the odd ones, each lane
-    // two entries of its pair's 256 (f: the first, f2: the second), the slots carrying over from the
-    // wavefront's previous sample, two samples back.  Lanes past the table read the last entry and store
-    // the same bits as the last entry's lane to the same place (no branch around the store, which would
-    // give the loop a path that skips the wait for the slot loads).
-    const int w = t >> 6, lane = t & 63, par = w >> 1;
-    const int kl0 = min((w & 1) * 128 + lane, NLA - 1), kl1 = min((w & 1) * 128 + 64 + lane, NLA - 1);
-    // sg holds the steps of samples i0 .. i0 + 3 (requested before the barrier that precedes this chunk)
-    for (int b = 0; b < qn; b += kStepGroup) {
-      if (b > 0) load_step_group(fs, i0 + b, n, sg);
+// Re-reads the slots whose node differs between two samples (workgroup-uniform offsets and branches).
+template <int TS>
+__device__ __forceinline__ void fold_load(const float* __restrict__ dJ, const int4 was, const int4 now, int bytes,
+                                          int lane, FoldSlots<TS>& f) {
+  const int o[4] = {now.x, now.y, now.z, now.w}, p[4] = {was.x, was.y, was.z, was.w};
 #pragma unroll
-      for (int q = 0; q < kStepGroup; ++q) {
-        if (b + q < qn && ((i0 + b + q) & 1) == par) {
-          const FoldStep st = sg.s[q];
-          const int4 o = st.off;
-          if (o.x >= 0 && o.x != prev.x) {
-            f.v[0] = dJ[o.x + kl0];
-            f2.v[0] = dJ[o.x + kl1];
-          }
-          if (o.y >= 0 && o.y != prev.y) {
-            f.v[1] = dJ[o.y + kl0];
-            f2.v[1] = dJ[o.y + kl1];
-          }
-          if (o.z >= 0 && o.z != prev.z) {
-            f.v[2] = dJ[o.z + kl0];
-            f2.v[2] = dJ[o.z + kl1];
-          }
-          if (o.w >= 0 && o.w != prev.w) {
-            f.v[3] = dJ[o.w + kl0];
-            f2.v[3] = dJ[o.w + kl1];
-          }
-          prev = o;
-          slab[(b + q) * NLA + kl0] = fold_value(f, st.wt);
-          slab[(b + q) * NLA + kl1] = fold_value(f2, st.wt);
-        }
+  for (int c = 0; c < 4; ++c)
+    if (o[c] >= 0 && o[c] != p[c]) {
+      const __amdgpu_buffer_rsrc_t node = node_buffer(dJ, o[c], bytes);
+#pragma unroll
+      for (int j = 0; j < TS; ++j) {
+        const auto v = __builtin_amdgcn_raw_buffer_load_b96(node, lane * (int)sizeof(Rgb) + j * 64 * (int)sizeof(Rgb), 0, 0);
+        f.v[c][j] = Rgb{__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2])};
       }
     }
-    // the next chunk's first steps, in flight across the barrier
-    if (i0 + qn < n) load_step_group(fs, i0 + qn, n, sg);
-  } else {  // KPT (even) entries per thread, NLA <= KPT nt: every sample reads its four nodes
-    for (int q = 0; q < qn; ++q) {
-      const FoldStep st = fold_step(fs, i0 + q);
-      const int4 o = st.off;
-      const float4 w = st.wt;
-      // an unused slot (offset -1, weight 0) reads node 0, which adds zero
-      const float4* __restrict__ d0 = dJ + max(o.x, 0);
-      const float4* __restrict__ d1 = dJ + max(o.y, 0);
-      const float4* __restrict__ d2 = dJ + max(o.z, 0);
-      const float4* __restrict__ d3 = dJ + max(o.w, 0);
-      // two entries per round, eight loads in flight (entries past the table repeat the last one, which
-      // stores the same bits to the same place)
+}
+
+// Texels of a wavefront's slab for TS texels per lane, with the zero texel that ends each column (a group has at
+// most 64 TS / NL columns; NL >= 16 but for the exact form, which takes NL >= 2).
+template <int TS>
+__host__ __device__ constexpr int rs_texels(bool exact) {
+  return 64 * TS + (exact ? 32 * TS : 4 * TS);
+}
+
+// LDS of one workgroup: the wavefronts' slabs, whose place the item sums take later ([segs][3][groups x items]).
+template <int TS>
+__host__ __device__ inline size_t rs_shared_bytes(int groups, int segs, bool exact) {
+  const size_t slabs = (size_t)groups * segs * rs_texels<TS>(exact) * sizeof(float4);
+  const size_t sums = (size_t)segs * 3 * groups * rs_items(TS) * sizeof(float);
+  return slabs > sums ? slabs : sums;
+}
+
+// One wavefront's samples i0 .. i1 - 1 over NS lookup slots: acc[j] = sum over its samples of T(x, p_i) times
+// the folded slab interpolated for the lane's item of slot j.
+template <int TS, int NS, bool kExact, class Steps>
+__device__ __forceinline__ void rs_segment(const float* __restrict__ dJ, const Steps gF, const float4* __restrict__ gT,
+                                           const float4* __restrict__ gRS, const double2* __restrict__ gTH, int i0, int i1,
+                                           int bytes, float4* slab, const unsigned (&laddr)[TS],
+                                           const RsItem* __restrict__ items, int nitems, const double2* __restrict__ ss,
+                                           int col0, int pitch, const SunCoord& sc, double R, double A64, int lane,
+                                           float* s_out, int out_pitch) {
+  FoldSlots<TS> f;
 #pragma unroll
-      for (int e = 0; e < KPT; e += 2) {
-        const int k0 = min(t + e * nt, NLA - 1), k1 = min(t + (e + 1) * nt, NLA - 1);
-        const float4 a0 = d0[k0], b0 = d1[k0], c0 = d2[k0], e0 = d3[k0];
-        const float4 a1 = d0[k1], b1 = d1[k1], c1 = d2[k1], e1 = d3[k1];
-        FoldSlots f0, f1;
-        f0.v[0] = a0;
-        f0.v[1] = b0;
-        f0.v[2] = c0;
-        f0.v[3] = e0;
-        f1.v[0] = a1;
-        f1.v[1] = b1;
-        f1.v[2] = c1;
-        f1.v[3] = e1;
-        slab[q * NLA + k0] = fold_value(f0, w);
-        slab[q * NLA + k1] = fold_value(f1, w);
-      }
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int j = 0; j < TS; ++j) f.v[c][j] = Rgb{0.f, 0.f, 0.f};
+  FoldStep st = fold_step(gF, i0);
+  fold_load<TS>(dJ, make_int4(-1, -1, -1, -1), st.off, bytes, lane, f);
+  float xl[NS], vl[NS];
+  double xl64[kExact ? NS : 1], vl64[kExact ? NS : 1];
+  unsigned caddr[NS];
+  Rgb acc[NS];
+#pragma unroll
+  for (int j = 0; j < NS; ++j) {
+    const RsItem it = items[min(64 * j + lane, nitems - 1)];  // lanes past the last item repeat it
+    vl[j] = it.vl;
+    xl[j] = it.xl;
+    if (kExact) {
+      const double2 d = ss[it.at & 0xffff];
+      vl64[j] = d.x;
+      xl64[j] = d.y;
     }
+    caddr[j] = ((it.at >> 16) - col0) * pitch * (unsigned)sizeof(float4);
+    acc[j] = Rgb{0.f, 0.f, 0.f};
   }
+  for (int i = i0; i < i1; ++i) {
+    const float4 w = st.wt;
+#pragma unroll
+    for (int j = 0; j < TS; ++j) {
+      const Rgb a = f.v[0][j], b = f.v[1][j], c = f.v[2][j], d = f.v[3][j];
+      *(float4*)((char*)slab + laddr[j]) = make_float4(fmaf(w.w, d.x, fmaf(w.z, c.x, fmaf(w.y, b.x, w.x * a.x))),
+                                                       fmaf(w.w, d.y, fmaf(w.z, c.y, fmaf(w.y, b.y, w.x * a.y))),
+                                                       fmaf(w.w, d.z, fmaf(w.z, c.z, fmaf(w.y, b.z, w.x * a.z))), 0.f);
+    }
+    wave_fence();
+    // the next sample's nodes, in flight during this sample's lookups
+    const FoldStep nx = fold_step(gF, min(i + 1, i1 - 1));
+    fold_load<TS>(dJ, st.off, nx.off, bytes, lane, f);
+    st = nx;
+    const float4 T = gT[i], g = gRS[i];  // uniform: scalar loads
+#pragma unroll
+    for (int j = 0; j < NS; ++j) {
+      unsigned row;
+      float s;
+      if (kExact) {
+        sun_coord_exact(sc, A64, R, gTH[i], xl64[j], vl64[j], row, s);
+      } else {
+        const float c = sun_coord(sc, make_float2(g.z, g.w), xl[j], vl[j]);
+        row = (unsigned)c;
+        s = __builtin_amdgcn_fractf(c);
+      }
+      const float4* p = (const float4*)((const char*)slab + (caddr[j] + row * (unsigned)sizeof(float4)));
+      const float3 v = lerp3(p[0], p[1], s);
+      acc[j].x = fmaf(T.x, v.x, acc[j].x);
+      acc[j].y = fmaf(T.y, v.y, acc[j].y);
+      acc[j].z = fmaf(T.z, v.z, acc[j].z);
+    }
+    wave_fence();
+  }
+  __syncthreads();  // every wavefront has done with its slab: the sums take their place
+#pragma unroll
+  for (int j = 0; j < NS; ++j) {
+    s_out[64 * j + lane] = acc[j].x;
+    s_out[out_pitch + 64 * j + lane] = acc[j].y;
+    s_out[2 * out_pitch + 64 * j + lane] = acc[j].z;
+  }
+}
+
+// One entry sample by sample from dJ itself, both columns mixed at every sample and the samples added in
+// order (vl, xl: FP64): for rays whose items exceed the lookup slots, and for the order sums that training and
+// sfsim_atmo_order_sums read, whose rounding stays that of this plain order (a network's training amplifies the
+// last bit of its targets).
+template <bool kExact, class Steps>
+__device__ float3 rs_entry_sum(const float* __restrict__ dJ, const Steps gF, const float4* __restrict__ gT,
+                               const float4* __restrict__ gRS, const double2* __restrict__ gTH, int n, int NL, int NA,
+                               double vl, double xl, const SunCoord& sc, double R, double A64) {
+  const Lerp L = make_lerp((float)sun_angle_to_index(NA, vl), NA);
+  const int c0 = L.i0 * NL, c1 = L.i1 * NL;
+  float3 acc = make_float3(0.f, 0.f, 0.f);
+  for (int i = 0; i < n; ++i) {
+    const FoldStep st = fold_step(gF, i);
+    const float4 T = gT[i], g = gRS[i];
+    int row;
+    float s;
+    if (kExact) {
+      unsigned r;
+      sun_coord_exact(sc, A64, R, gTH[i], xl, vl, r, s);
+      row = (int)r;
+    } else {
+      const float c = sun_coord(sc, make_float2(g.z, g.w), (float)xl, (float)vl);
+      row = min((int)c, NL - 2);
+      s = c - (float)row;
+    }
+    const int o[4] = {st.off.x, st.off.y, st.off.z, st.off.w};
+    const float w[4] = {st.wt.x, st.wt.y, st.wt.z, st.wt.w};
+    float4 f[2][2] = {};  // [row][column]: the fold of the four nodes
+    for (int q = 0; q < 4; ++q)
+      if (o[q] >= 0) {
+        auto add = [&](float4& t, int k) {
+          const Rgb v = ((const Rgb*)dJ)[(long long)o[q] + k];
+          t = make_float4(fmaf(w[q], v.x, t.x), fmaf(w[q], v.y, t.y), fmaf(w[q], v.z, t.z), 0.f);
+        };
+        add(f[0][0], c0 + row);
+        add(f[0][1], c1 + row);
+        add(f[1][0], c0 + row + 1);
+        add(f[1][1], c1 + row + 1);
+      }
+    const float3 u = lerp3(f[0][0], f[0][1], L.s), t = lerp3(f[1][0], f[1][1], L.s);
+    acc.x = fmaf(T.x, fmaf(s, t.x - u.x, u.x), acc.x);
+    acc.y = fmaf(T.y, fmaf(s, t.y - u.y, u.y), acc.y);
+    acc.z = fmaf(T.z, fmaf(s, t.z - u.z, u.z), acc.z);
+  }
+  return acc;
 }
 
 __device__ float3 resample4_value(const DevParams& P, const float4* __restrict__ a, const float4* __restrict__ b,
@@ -1017,20 +1044,14 @@ __device__ float3 resample4_value_lean(const DevParams& P, const float4* __restr
 __device__ float3 resample2_value(const DevParams& P, int space, const float4* __restrict__ a,
                                  const float4* __restrict__ b, long long idx);
 
-// Warp-specialised: waves 0-3 fold, waves 4-7 look up.  The folded slabs are double-buffered: while the
-// lookup waves read chunk c from one half, the fold waves fill the other half with chunk c + 1, and one
-// barrier per chunk hands both halves over (chunk c + 1 overwrites the half that chunk c - 1's lookups
-// read, finished before the previous barrier).
-constexpr int kRSBlock = 512;
-constexpr int kRSHalf = kRSBlock / 2;
-
-// Eight waves per SIMD (four workgroups per CU, as the LDS allows): at most 64 VGPRs, the re-sampling
-// of the accumulations spilling a few registers outside the loops.
-template <int EPT, bool kB, bool kExact>
-__global__ void __launch_bounds__(kRSBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) ray_scatter_kernel(
-    const DevParams P0, const DevParams* __restrict__ PB, const float4* __restrict__ dJ,
+// segs: sample segments per group of columns (P.rs_groups x segs wavefronts, wavefront w working on group
+// w / segs and segment w % segs).
+template <int TS, bool kB, bool kExact>
+__global__ void __launch_bounds__(1024) ray_scatter_kernel(
+    const DevParams P0, const DevParams* __restrict__ PB, const float* __restrict__ dJ,
     const double2* __restrict__ geo_th, const float4* __restrict__ geo_T, const float4* __restrict__ geo_rs,
-    const FoldStep* __restrict__ geo_fold, float4* __restrict__ out, const RsAccum accum_arg, int Q,
+    const FoldStep* __restrict__ geo_fold, const RsItem* __restrict__ items, const uint2* __restrict__ entries,
+    const int* __restrict__ heads, float4* __restrict__ out, const RsAccum accum_arg, int segs, int by_sample,
     WorkCounters* wc) {
   const DevParams& P = params_of<kB>(P0, PB);
   if constexpr (kB) {  // this atmosphere's tables and ray geometry (the accumulation tables where they are used);
@@ -1038,13 +1059,11 @@ __global__ void __launch_bounds__(kRSBlock) __attribute__((amdgpu_waves_per_eu(8
     geo_th = atm_ptr<kB>(geo_th, P0);
     geo_T = atm_ptr<kB>(geo_T, P0);
     geo_rs = atm_ptr<kB>(geo_rs, P0);
-    // the fold steps depend only on the planet and the grid, which the atmospheres of a batch share: all
-    // read atmosphere 0's copy (one copy in the caches instead of one per atmosphere)
+    // the fold steps and the items depend only on the planet and the grid, which the atmospheres of a batch
+    // share: all read atmosphere 0's copy (one copy in the caches instead of one per atmosphere)
     dJ = atm_ptr<kB>(dJ, P);
     out = atm_ptr<kB>(out, P);
   }
-  // dynamic LDS: 2 x Q x (NL x NA) slab entries (chunk c in half c % 2)
-  extern __shared__ float4 s_slab[];
   const int NH = P.nS[0], NE = P.nS[1], NL = P.nS[2], NA = P.nS[3];
   const int NLA = NL * NA;
   const int n = P.ray_steps;
@@ -1059,150 +1078,100 @@ __global__ void __launch_bounds__(kRSBlock) __attribute__((amdgpu_waves_per_eu(8
     }
     return;
   }
+  extern __shared__ float4 s_mem[];
+  const int groups = P.rs_groups, pitch_out = groups * rs_items(TS);
   // XCD-aware, in ascending impact parameter: every sample of a straight ray has the same
   // |p| sqrt(1 - mu^2), so the (height, elevation) cells that a ray folds lie along one curve, and an XCD
   // given a contiguous range of impact parameters reads a band of the dJ table
   const int ord = xcd_ray(blockIdx.x, NH * NE);
   const int rayid = P.ray_order ? P.ray_order[ord] : ord;
-  const bool folder = threadIdx.x < kRSHalf;  // whole wavefronts
-  const int t = folder ? (int)threadIdx.x : (int)threadIdx.x - kRSHalf;
-  // this ray's samples in the per-build geometry: T(x, p_i) rgb and (height coordinate, elevation
-  // coordinate, alpha_i, beta_i)
-  const float4* __restrict__ gT = geo_T + (long long)rayid * n;
-  const float4* __restrict__ gRS = geo_rs + (long long)rayid * n;
-  const int chunks = (n + Q - 1) / Q;
-  // with one entry per lane the fold waves, idle during the last chunk, re-sample S for the epilogue
-  // (0.5% per launch); with several entries per lane it is slower there and stays with the lookup waves
-  constexpr bool kFoldResamples = EPT == 1;
-  if (folder) {
-    const FoldStep* __restrict__ gS = geo_fold + (long long)rayid * n;
-    const auto gF = [&] {
-      if constexpr (kB) return (ConstFoldSteps)gS;
-      else return gS;
-    }();
-    FoldSlots fs, fs2;
-    fold_slots_init(fs);
-    fold_slots_init(fs2);
-    int4 prev = make_int4(-1, -1, -1, -1);
-    StepGroup sg;
-    if constexpr (EPT == 1) load_step_group(gF, 0, n, sg);
-    ray_scatter_fold<EPT>(dJ, gF, s_slab, 0, min(Q, n), NLA, t, kRSHalf, fs, fs2, prev, sg, n);
-    __syncthreads();
-    for (int c = 0; c + 1 < chunks; ++c) {
-      ray_scatter_fold<EPT>(dJ, gF, s_slab + ((c + 1) & 1) * Q * NLA, (c + 1) * Q, min(Q, n - (c + 1) * Q), NLA,
-                            t, kRSHalf, fs, fs2, prev, sg, n);
-      __syncthreads();
+  const long long base = (long long)rayid * NLA, base_n = (long long)rayid * n;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int group = wave / segs, seg = wave - group * segs;
+  const double2* __restrict__ ss = P.sun_ss + base;
+  const FoldStep* __restrict__ gS = geo_fold + base_n;
+  const auto gF = [&] {
+    if constexpr (kB) return (ConstFoldSteps)gS;
+    else return gS;
+  }();
+  const SunCoord sc = {(float)((NL - 1) * (double)P.sun_inv_den), (float)(-0.6 * 1.4426950408889634), (float)(NL - 1)};
+  const double A64 = kExact ? (NL - 1) / (1.0 - exp(-3.6)) : 0.0;
+  const int* __restrict__ head = heads + (long long)rayid * (groups + 1);
+  bool fits = !by_sample;
+  for (int g = 0; g < groups; ++g) fits = fits && head[g + 1] - head[g] <= rs_items(TS);
+  if (fits) {
+    const int nitems = head[group + 1] - head[group];
+    // the lane's texels in the LDS slab; those past the group's texels write zeros to the last column's zero texel
+    const int col0 = group * P.rs_cols, ncols = min(P.rs_cols, NA - col0), pitch = NL + 1;
+    float4* slab = s_mem + wave * rs_texels<TS>(kExact);
+    unsigned laddr[TS];
+#pragma unroll
+    for (int j = 0; j < TS; ++j) {
+      const unsigned t = 64 * j + lane;
+      laddr[j] = (t < (unsigned)(ncols * NL) ? t + t / (unsigned)NL : (unsigned)(ncols * pitch - 1)) * (unsigned)sizeof(float4);
     }
-    if (kFoldResamples && accum_arg.S_out) {
-      // while the last chunk's lookups run: the running sum S of atmosphere_lut.clj:95-97 at this ray's grid
-      // points into the half that the lookups of the chunk before the last have finished with, for the
-      // lookup waves to add their dS to after the barrier (the fold slots are dead by now)
-      const float4* S_in = atm_ptr<kB>(accum_arg.S_in, P);
-      float4* su = s_slab + (chunks & 1) * Q * NLA;
-      const long long base = (long long)rayid * NLA;
-      for (int kk = t; kk < NLA; kk += kRSHalf) {
-        const float3 u = accum_arg.S_resample ? resample4_value_lean(P, S_in, base + kk) : ld3(S_in, base + kk);
-        su[kk] = make_float4(u.x, u.y, u.z, 0.f);
-      }
+    for (int i = lane; i < ncols; i += 64) slab[i * pitch + NL] = make_float4(0.f, 0.f, 0.f, 0.f);
+    const int i0 = (int)((long long)n * seg / segs), i1 = (int)((long long)n * (seg + 1) / segs);
+    const RsItem* __restrict__ it = items + 2 * base + head[group];
+    float* s_out = (float*)s_mem + (size_t)seg * 3 * pitch_out + group * rs_items(TS);
+#define SFSIM_RS_CASE(NS)                                                                                             \
+  case NS:                                                                                                            \
+    if constexpr (64 * NS <= rs_items(TS))                                                                            \
+      rs_segment<TS, NS, kExact>(dJ + 3 * col0 * NL, gF, geo_T + base_n, geo_rs + base_n, geo_th + base_n, i0, i1,     \
+                                 ncols * NL * (int)sizeof(Rgb), slab, laddr, it, nitems, ss, col0, pitch, sc, P.g.R,  \
+                                 A64, lane, s_out, pitch_out);                                                        \
+    break
+    switch ((nitems + 63) / 64) {
+      SFSIM_RS_CASE(1);
+      SFSIM_RS_CASE(2);
+      SFSIM_RS_CASE(3);
+      SFSIM_RS_CASE(4);
+      SFSIM_RS_CASE(5);
+      SFSIM_RS_CASE(6);
+      SFSIM_RS_CASE(7);
+      SFSIM_RS_CASE(8);
+      default:  // no item of this group
+        __syncthreads();
     }
+#undef SFSIM_RS_CASE
     __syncthreads();
-    return;
   }
   // the ray's step D / n: twice its first sample's t = 0.5 D / n (FP64, exact), from the per-build geometry
-  const double dt = 2.0 * geo_th[(long long)rayid * n].x;
-  const SunCoord sc = {(float)((NL - 1) * (double)P.sun_inv_den), (float)(-0.6 * 1.4426950408889634), (float)(NL - 1)};
-  const float row_bytes = (float)(NA * (int)sizeof(float4));
-  // per-entry constants: heading coordinate and the terms of dot(p_i, l)
-  SunTerms st[EPT];
-  Lerp La[EPT];
-  float3 acc[EPT];
-#pragma unroll
-  for (int q = 0; q < EPT; ++q) {
-    int k = t + q * kRSHalf;
-    acc[q] = make_float3(0.f, 0.f, 0.f);
-    st[q].vl = 0.f;
-    st[q].xl = 0.f;
-    st[q].vl64 = 0.0;
-    st[q].xl64 = 0.0;
-    st[q].R = P.g.R;
-    st[q].A64 = kExact ? (NL - 1) / (1.0 - exp(-3.6)) : 0.0;
-    La[q] = make_lerp(0.f, NA);
-    if (k < NLA) {
-      // the per-build sun terms (v . l, x . l, the heading coordinate, rounded once from FP64)
-      const float4 m = P.sun_rs[(long long)rayid * NLA + k];
-      st[q].vl = m.x;
-      st[q].xl = m.y;
-      La[q] = make_lerp(m.z, NA);
-      if (kExact) {  // the same dot products in FP64
-        const double2 d = P.sun_ss[(long long)rayid * NLA + k];
-        st[q].vl64 = d.x;
-        st[q].xl64 = d.y;
-      }
-    }
-  }
-  SampleGroup sgp;
-  if constexpr (EPT == 1) load_sample_group<kExact>(gT, gRS, geo_th + (long long)rayid * n, 0, n, sgp);
-  __syncthreads();  // chunk 0 folded
-  for (int c = 0; c < chunks; ++c) {
-    const int i0 = c * Q, qn = min(Q, n - i0);
-    const float4* slab = s_slab + (c & 1) * Q * NLA;
-    if constexpr (EPT == 1) {
-      for (int b = 0; b < qn; b += kStepGroup) {
-        if (b > 0) load_sample_group<kExact>(gT, gRS, geo_th + (long long)rayid * n, i0 + b, n, sgp);
-        if (t < NLA) {
-          const float col_bytes = (float)(La[0].i0 * (int)sizeof(float4));
-          // a heading coordinate with zero weight (every entry but the clamped ones) reads one column;
-          // the choice is made per wavefront so that a wavefront never runs both loops
-          if (__all(La[0].s == 0.0f))
-            acc[0] = ray_scatter_sample_group<true, kExact>(sc, slab, sgp, b, qn, row_bytes, col_bytes, NLA, st[0],
-                                                            La[0], acc[0]);
-          else
-            acc[0] = ray_scatter_sample_group<false, kExact>(sc, slab, sgp, b, qn, row_bytes, col_bytes, NLA, st[0],
-                                                             La[0], acc[0]);
+  const float dt = (float)(2.0 * geo_th[base_n].x);
+  for (int kk = threadIdx.x; kk < NLA; kk += blockDim.x) {
+    float3 v;
+    if (fits) {
+      const uint2 e = entries[base + kk];
+      auto total = [&](unsigned at) {
+        const float* q = (const float*)s_mem + at;
+        float3 t = make_float3(q[0], q[pitch_out], q[2 * pitch_out]);
+        for (int g = 1; g < segs; ++g) {
+          q += 3 * pitch_out;
+          t.x += q[0];
+          t.y += q[pitch_out];
+          t.z += q[2 * pitch_out];
         }
+        return t;
+      };
+      v = total(e.x & 0xffffu);
+      const float s = __uint_as_float(e.y);
+      if (s != 0.0f) {
+        const float3 u = total(e.x >> 16);
+        v = make_float3(fmaf(s, u.x - v.x, v.x), fmaf(s, u.y - v.y, v.y), fmaf(s, u.z - v.z, v.z));
       }
-      if (c + 1 < chunks)  // in flight across the barrier
-        load_sample_group<kExact>(gT, gRS, geo_th + (long long)rayid * n, i0 + qn, n, sgp);
-    } else {  // several entries per lane: the terms per sample (a group would spill)
-#pragma unroll
-      for (int e = 0; e < EPT; ++e) {
-        if (t + e * kRSHalf < NLA) {
-          const float col_bytes = (float)(La[e].i0 * (int)sizeof(float4));
-          if (__all(La[e].s == 0.0f))
-            acc[e] = ray_scatter_samples<true, kExact>(sc, slab, gT, gRS, geo_th + (long long)rayid * n, i0, qn,
-                                                       row_bytes, col_bytes, NLA, st[e], La[e], acc[e]);
-          else
-            acc[e] = ray_scatter_samples<false, kExact>(sc, slab, gT, gRS, geo_th + (long long)rayid * n, i0, qn,
-                                                        row_bytes, col_bytes, NLA, st[e], La[e], acc[e]);
-        }
-      }
+    } else {
+      const double2 d = ss[kk];
+      v = rs_entry_sum<kExact>(dJ, gF, geo_T + base_n, geo_rs + base_n, geo_th + base_n, n, NL, NA, d.x, d.y, sc, P.g.R, A64);
     }
-    __syncthreads();
-  }
-  const long long base = (long long)rayid * NLA;
-  const float a = (float)dt;
-  unsigned long long lookups = 0;
-#pragma unroll
-  for (int e = 0; e < EPT; ++e) {
-    const int k = t + e * kRSHalf;
-    if (k < NLA) {
-      const float4 d = make_float4(acc[e].x * a, acc[e].y * a, acc[e].z * a, 0.f);
-      out[base + k] = d;
-      if (accum_arg.S_out) {  // S + dS at this grid point
-        float3 u;
-        if (kFoldResamples) {
-          const float4 v = s_slab[(chunks & 1) * Q * NLA + k];
-          u = make_float3(v.x, v.y, v.z);
-        } else {
-          const float4* S_in = atm_ptr<kB>(accum_arg.S_in, P);
-          u = accum_arg.S_resample ? resample4_value_lean(P, S_in, base + k) : ld3(S_in, base + k);
-        }
-        atm_ptr<kB>(accum_arg.S_out, P)[base + k] = make_float4(u.x + d.x, u.y + d.y, u.z + d.z, 0.f);
-      }
-      lookups += n;
+    const float4 d = make_float4(v.x * dt, v.y * dt, v.z * dt, 0.f);
+    out[base + kk] = d;
+    if (accum_arg.S_out) {  // S + dS at this grid point (the running sum S of atmosphere_lut.clj:95-97)
+      const float4* S_in = atm_ptr<kB>(accum_arg.S_in, P);
+      const float3 u = accum_arg.S_resample ? resample4_value_lean(P, S_in, base + kk) : ld3(S_in, base + kk);
+      atm_ptr<kB>(accum_arg.S_out, P)[base + kk] = make_float4(u.x + d.x, u.y + d.y, u.z + d.z, 0.f);
     }
+    count(wc, 0, 0, (unsigned long long)n, 0);
   }
-  count(wc, 0, 0, lookups, 0);
 }
 
 // dJ = point-scatter over the sphere quadrature (atmosphere_lut.clj:88,91; atmosphere.clj:203-222).
@@ -1436,7 +1405,7 @@ __global__ void __launch_bounds__(kBlock) point_scatter_kernel(const DevParams P
                                                                const DirGeom* __restrict__ geom, int ndirs,
                                                                const float4* __restrict__ slab,
                                                                const float4* __restrict__ slab_mie,
-                                                               const float4* __restrict__ dE, float4* __restrict__ out,
+                                                               const float4* __restrict__ dE, float* __restrict__ out,
                                                                const SrJob sr, WorkCounters* wc) {
   extern __shared__ DirLds s_dir[];
   float4* s_dE = (float4*)(s_dir + ndirs);
@@ -1512,7 +1481,10 @@ __global__ void __launch_bounds__(kBlock) point_scatter_kernel(const DevParams P
     l4 += (unsigned long long)ndirs * (kMie ? 2 : 1);
     if (wc)
       for (int j = 0; j < ndirs; ++j) l2 += s_dir[j].omega.w != 0.f;
-    out[base + k] = make_float4(acc.x, acc.y, acc.z, 0.f);
+    float* o = out + 3 * (base + (k % NA) * NL + k / NA);  // packed, (heading, sun elevation) order
+    o[0] = acc.x;
+    o[1] = acc.y;
+    o[2] = acc.z;
   }
   count(wc, 0, 0, l4, l2);
 }
@@ -1628,11 +1600,10 @@ __global__ void __launch_bounds__(kBlock) surface_radiance_kernel(const DevParam
 
 // f(backward(i)) re-sampling of interpolated tables (interpolate.clj:54-72 with interpolation-table).
 // Lerps of forward(backward(i)) for 4D entry i = ((ih NE + ie) NL + is) NA + ia (atmosphere.clj:233-422).
-// With ps / rs (nullable) also the entry's sun terms that the point- and ray-scatter kernels use
-// (DevParams::sun_ps, sun_rs), from the same FP64 values.
+// With ps / ss (nullable) also the entry's sun terms that the scatter kernels use (DevParams::sun_ps, sun_ss),
+// from the same FP64 values.
 __device__ __forceinline__ void resample4_lerps(const DevParams& P, int ih, int ie, int is, int ia, Lerp& Lh, Lerp& Le,
-                                                Lerp& Ls, Lerp& La, float4* ps = nullptr, float4* rs = nullptr,
-                                                double2* ss = nullptr) {
+                                                Lerp& Ls, Lerp& La, float4* ps = nullptr, double2* ss = nullptr) {
   SFSIM_EXACT  // the reference's rounding (see geometry.hpp)
   const int NH = P.nS[0], NE = P.nS[1], NL = P.nS[2], NA = P.nS[3];
   double r0 = index_to_radius(P.g, NH, ih);
@@ -1649,7 +1620,6 @@ __device__ __forceinline__ void resample4_lerps(const DevParams& P, int ih, int 
   Ls = make_lerp((float)cs, NL);
   La = make_lerp((float)ca, NA);
   if (ps) *ps = make_float4((float)l0, (float)l1, (float)l2, (float)cs);
-  if (rs) *rs = make_float4((float)vl, (float)(r0 * l0), (float)ca, 0.f);
   if (ss) *ss = make_double2(vl, r0 * l0);
 }
 
@@ -1673,13 +1643,12 @@ __device__ __forceinline__ void resample_map_body(const DevParams& P, unsigned b
   q /= NL;
   const int ie = (int)(q % NE), ih = (int)(q / NE);
   Lerp Lh, Le, Ls, La;
-  float4 ps, rs;
+  float4 ps;
   double2 ss;
-  resample4_lerps(P, ih, ie, is, ia, Lh, Le, Ls, La, &ps, &rs, &ss);
+  resample4_lerps(P, ih, ie, is, ia, Lh, Le, Ls, La, &ps, &ss);
   ((float4*)P.rmap)[idx] = make_float4(Lh.s, Le.s, Ls.s, La.s);
   if (P.sun_ps) {
     P.sun_ps[idx] = ps;
-    P.sun_rs[idx] = rs;
     P.sun_ss[idx] = ss;
   }
   ((ushort4*)(P.rmap + n * sizeof(float4)))[idx] =
@@ -1910,6 +1879,18 @@ __global__ void unpack_rgb_kernel(const float* __restrict__ in, float4* __restri
   out[i] = make_float4(in[i * 3], in[i * 3 + 1], in[i * 3 + 2], 0.f);
 }
 
+// Packed RGB entries of [blocks][d0][d1] order in [blocks][d1][d0] order.
+__global__ void transpose_rgb_kernel(const float* __restrict__ in, float* __restrict__ out, long long count, int d0,
+                                     int d1) {
+  long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;  // output entry
+  if (i >= count) return;
+  const long long q = i / d0, b = q / d1;
+  const float* v = in + 3 * ((b * d0 + (i - q * d0)) * d1 + (q - b * d1));
+  out[i * 3] = v[0];
+  out[i * 3 + 1] = v[1];
+  out[i * 3 + 2] = v[2];
+}
+
 __global__ void add4_kernel(const float4* __restrict__ a, const float4* __restrict__ b, float4* __restrict__ c,
                             long long count) {
   long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -2012,8 +1993,16 @@ hipError_t launch_ray_geometry(const DevParams& P, WorkCounters* wc, hipStream_t
   return hipGetLastError();
 }
 
+hipError_t launch_ray_items(const DevParams& P, hipStream_t stream) {
+  if (P.batch > 0) return hipErrorInvalidValue;  // batches make them in launch_single_scatter
+  if (!P.rs_items || !P.sun_ss || P.rs_groups > kMaxRsGroups) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(ray_items_kernel, dim3((unsigned)(P.nS[0] * P.nS[1])), dim3(kBlock),
+                     sizeof(unsigned) * (size_t)P.nS[2] * P.nS[3], stream, P);
+  return hipGetLastError();
+}
+
 hipError_t launch_single_scatter(const DevParams& P, float4* rayleigh, float4* mie, WorkCounters* wc,
-                                 hipStream_t stream, bool sun_table_built) {
+                                 hipStream_t stream, bool sun_table_built, bool ray_items) {
   unsigned rays = (unsigned)(P.nS[0] * P.nS[1]);
   // a batch runs the table path with the tables built by its prologue
   if (P.batch > 0 && (P.sun_rows <= 0 || !sun_table_built)) return hipErrorInvalidValue;
@@ -2025,14 +2014,20 @@ hipError_t launch_single_scatter(const DevParams& P, float4* rayleigh, float4* m
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const RayGeoView V = ray_geo_view(P);
-    const size_t shmem = (size_t)P.ray_steps * (sizeof(double2) + 2 * sizeof(float4) + sizeof(float2));
+    const unsigned extra = ray_items ? rays : 0;
+    const size_t shmem = std::max((size_t)P.ray_steps * (sizeof(double2) + 2 * sizeof(float4) + sizeof(float2)),
+                                  ray_items ? (size_t)P.nS[2] * P.nS[3] * sizeof(unsigned) : 0);
     if (P.batch > 0)
-      hipLaunchKernelGGL(single_scatter_table_kernel<true>, dim3(rays, 1, P.batch), dim3(kSSTBlock), shmem, stream, P,
-                         P.batch_params, V.th, V.T, V.ss, V.row, rayleigh, mie, wc);
+      hipLaunchKernelGGL(single_scatter_table_kernel<true>, dim3(rays + extra, 1, P.batch), dim3(kSSTBlock), shmem, stream, P,
+                         P.batch_params, V.th, V.T, V.ss, V.row, rayleigh, mie, (int)extra, wc);
     else
-      hipLaunchKernelGGL(single_scatter_table_kernel<false>, dim3(rays), dim3(kSSTBlock), shmem, stream, P,
-                         P.batch_params, V.th, V.T, V.ss, V.row, rayleigh, mie, wc);
+      hipLaunchKernelGGL(single_scatter_table_kernel<false>, dim3(rays + extra), dim3(kSSTBlock), shmem, stream, P,
+                         P.batch_params, V.th, V.T, V.ss, V.row, rayleigh, mie, (int)extra, wc);
     return hipGetLastError();
+  }
+  if (ray_items) {
+    const hipError_t e = launch_ray_items(P, stream);
+    if (e != hipSuccess) return e;
   }
   unsigned groups = (unsigned)((P.nS[2] * P.nS[3] + kSSWave - 1) / kSSWave);
   int n = P.ray_steps;
@@ -2054,7 +2049,7 @@ hipError_t launch_direction_geometry(const DevParams& P, const Dir* dirs, int nd
 size_t direction_geometry_bytes(const DevParams& P, int ndirs) { return sizeof(DirGeom) * (size_t)P.nS[0] * ndirs; }
 
 hipError_t launch_point_scatter(const DevParams& P, const Dir* dirs, int ndirs, const void* geom, const float4* dS,
-                                const float4* mie, const float4* dE, float4* slab, float4* slab_mie, float4* out,
+                                const float4* mie, const float4* dE, float4* slab, float4* slab_mie, float* out,
                                 WorkCounters* wc, hipStream_t stream, const SrJob* sr) {
   if (!P.sun_ps) return hipErrorInvalidValue;
   unsigned combos = (unsigned)(P.nS[0] * ndirs);
@@ -2113,68 +2108,49 @@ hipError_t launch_point_scatter(const DevParams& P, const Dir* dirs, int ndirs, 
   return hipGetLastError();
 }
 
-// Samples per folded-slab chunk of the ray-scatter kernel: its two slab halves take 2 x Q x NL x NA float4
-// of LDS, about 2 x 1024 slab entries (32 KiB, plus 36 B per ray step of offsets, weights and masks), so
-// that four 512-thread workgroups fit a CU; SFSIM_ATMO_RAY_CHUNK (1..8, within the same LDS bound)
-// overrides it.
-int ray_scatter_chunk(const DevParams& P) {
-  int nla = P.nS[2] * P.nS[3];
-  int q = 1024 / nla;
-  if (const char* env = std::getenv("SFSIM_ATMO_RAY_CHUNK")) {
-    int v = std::atoi(env);
-    if (v >= 1) q = v;
-  }
-  const int qmax = std::min(kMaxRayChunk, 1024 / nla);
-  return q < 1 ? 1 : (q > qmax ? std::max(qmax, 1) : q);
-}
-
-// launch_ray_scatter with the sun-elevation coordinate's form chosen (kExact: sun_coord_exact)
-template <bool kExact>
-hipError_t launch_ray_scatter_as(const DevParams& P, const float4* dJ, float4* out, WorkCounters* wc,
-                                 hipStream_t stream, const RsAccum& acc, unsigned rays, int Q, size_t shmem,
-                                 const RayGeoView& V, const DevParams* PB) {
-  const int nla = P.nS[2] * P.nS[3];
-  if (P.batch > 0) {
-    const dim3 grid(rays, 1, (unsigned)P.batch);
-    if (nla <= kRSHalf)
-      hipLaunchKernelGGL((ray_scatter_kernel<1, true, kExact>), grid, dim3(kRSBlock), shmem, stream, P, PB, dJ,
-                         V.th, V.T, V.rs, V.fold, out, acc, Q, wc);
-    else if (nla <= 2 * kRSHalf)
-      hipLaunchKernelGGL((ray_scatter_kernel<2, true, kExact>), grid, dim3(kRSBlock), shmem, stream, P, PB, dJ,
-                         V.th, V.T, V.rs, V.fold, out, acc, Q, wc);
-    else
-      hipLaunchKernelGGL((ray_scatter_kernel<4, true, kExact>), grid, dim3(kRSBlock), shmem, stream, P, PB, dJ,
-                         V.th, V.T, V.rs, V.fold, out, acc, Q, wc);
-  } else {
-    if (nla <= kRSHalf)
-      hipLaunchKernelGGL((ray_scatter_kernel<1, false, kExact>), dim3(rays), dim3(kRSBlock), shmem, stream, P, PB, dJ,
-                         V.th, V.T, V.rs, V.fold, out, acc, Q, wc);
-    else if (nla <= 2 * kRSHalf)
-      hipLaunchKernelGGL((ray_scatter_kernel<2, false, kExact>), dim3(rays), dim3(kRSBlock), shmem, stream, P, PB, dJ,
-                         V.th, V.T, V.rs, V.fold, out, acc, Q, wc);
-    else
-      hipLaunchKernelGGL((ray_scatter_kernel<4, false, kExact>), dim3(rays), dim3(kRSBlock), shmem, stream, P, PB, dJ,
-                         V.th, V.T, V.rs, V.fold, out, acc, Q, wc);
-  }
+// Sample segments per ray and group of columns: as many as let the workgroups of all rays be resident at once (four
+// wavefronts per SIMD, 16 per CU of 256, which is what the kernel's registers allow), down to two samples each and
+// within 64 KiB of LDS.  The 32 x 64 x 32 x 8 grid at 64 steps: 59 us with 2 segments, 76 with 1, 60 with 4 (two
+// rounds); 19 x 45 x 20 x 7 at 51 steps: 24 us with 4, 38 with 5 (a second round of few), 30 with 2, 48 with 1.
+template <int TS, bool kExact>
+hipError_t launch_ray_scatter_as(const DevParams& P, const float* dJ, float4* out, WorkCounters* wc, hipStream_t stream,
+                                 const RsAccum& acc, bool by_sample) {
+  const int groups = P.rs_groups;
+  const long long rays = (long long)P.nS[0] * P.nS[1];
+  int segs = (int)(16 / ((rays + 255) / 256)) / groups;
+  segs = std::max(1, std::min(segs, P.ray_steps / 2));
+  while (segs > 1 && rs_shared_bytes<TS>(groups, segs, kExact) > 65536) --segs;
+  const size_t shmem = rs_shared_bytes<TS>(groups, segs, kExact);
+  const RayGeoView V = ray_geo_view(P);
+  const dim3 grid((unsigned)rays + (acc.E_out ? 1u : 0u), 1, P.batch > 0 ? (unsigned)P.batch : 1u), block(64u * groups * segs);
+  if (P.batch > 0)
+    hipLaunchKernelGGL((ray_scatter_kernel<TS, true, kExact>), grid, block, shmem, stream, P, P.batch_params, dJ, V.th, V.T,
+                       V.rs, V.fold, P.rs_items, P.rs_entries, P.rs_heads, out, acc, segs, (int)by_sample, wc);
+  else
+    hipLaunchKernelGGL((ray_scatter_kernel<TS, false, kExact>), grid, block, shmem, stream, P, P.batch_params, dJ, V.th, V.T,
+                       V.rs, V.fold, P.rs_items, P.rs_entries, P.rs_heads, out, acc, segs, (int)by_sample, wc);
   return hipGetLastError();
 }
 
-hipError_t launch_ray_scatter(const DevParams& P, const float4* dJ, float4* out, WorkCounters* wc,
-                              hipStream_t stream, const RsAccum& acc) {
+hipError_t launch_ray_scatter(const DevParams& P, const float* dJ, float4* out, WorkCounters* wc, hipStream_t stream,
+                              const RsAccum& acc, bool by_sample) {
   if ((acc.S_in == nullptr) != (acc.S_out == nullptr) || (acc.E_out && !acc.dE)) return hipErrorInvalidValue;
-  if (!P.ray_geo || !P.sun_rs) return hipErrorInvalidValue;
-  const unsigned rays = (unsigned)(P.nS[0] * P.nS[1]) + (acc.E_out ? 1u : 0u);
-  int nla = P.nS[2] * P.nS[3];
-  int Q = ray_scatter_chunk(P);
-  const size_t shmem = 2 * sizeof(float4) * (size_t)Q * nla;
-  const RayGeoView V = ray_geo_view(P);
-  const DevParams* PB = P.batch_params;
-  if (nla > 4 * kRSHalf) return hipErrorInvalidValue;
+  if (!P.ray_geo || !P.sun_ss || !P.rs_items || P.rs_groups < 1 || P.rs_groups > kMaxRsGroups) return hipErrorInvalidValue;
   if (P.nS[2] < kExactSunRows) {
-    if (!P.sun_ss) return hipErrorInvalidValue;
-    return launch_ray_scatter_as<true>(P, dJ, out, wc, stream, acc, rays, Q, shmem, V, PB);
+    switch (P.rs_ts) {
+      case 1: return launch_ray_scatter_as<1, true>(P, dJ, out, wc, stream, acc, by_sample);
+      case 2: return launch_ray_scatter_as<2, true>(P, dJ, out, wc, stream, acc, by_sample);
+      case 4: return launch_ray_scatter_as<4, true>(P, dJ, out, wc, stream, acc, by_sample);
+    }
+    return hipErrorInvalidValue;
   }
-  return launch_ray_scatter_as<false>(P, dJ, out, wc, stream, acc, rays, Q, shmem, V, PB);
+  switch (P.rs_ts) {
+    case 1: return launch_ray_scatter_as<1, false>(P, dJ, out, wc, stream, acc, by_sample);
+    case 2: return launch_ray_scatter_as<2, false>(P, dJ, out, wc, stream, acc, by_sample);
+    case 4: return launch_ray_scatter_as<4, false>(P, dJ, out, wc, stream, acc, by_sample);
+    case 8: return launch_ray_scatter_as<8, false>(P, dJ, out, wc, stream, acc, by_sample);
+  }
+  return hipErrorInvalidValue;
 }
 
 hipError_t launch_surface_geometry(const DevParams& P, const Dir* dirs, int ndirs, hipStream_t stream) {
@@ -2316,6 +2292,11 @@ hipError_t launch_fill_zero(float* p, long long n, hipStream_t stream) {
 
 hipError_t launch_pack_rgb(const float4* in, float* out, long long count, hipStream_t stream) {
   hipLaunchKernelGGL(pack_rgb_kernel, dim3(blocks_for(count)), dim3(kBlock), 0, stream, in, out, count);
+  return hipGetLastError();
+}
+
+hipError_t launch_transpose_rgb(const float* in, float* out, long long count, int d0, int d1, hipStream_t stream) {
+  hipLaunchKernelGGL(transpose_rgb_kernel, dim3(blocks_for(count)), dim3(kBlock), 0, stream, in, out, count, d0, d1);
   return hipGetLastError();
 }
 

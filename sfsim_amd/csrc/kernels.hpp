@@ -15,7 +15,10 @@ hipError_t launch_ray_geometry(const DevParams& P, WorkCounters* wc, hipStream_t
 // R1 and M1; with a sun table (P.sun_rows > 0) builds it first (unless sun_table_built: launch_prologue
 // did) and reads P.ray_geo and the per-build sun map P.sun_ss (launch_resample_map).
 hipError_t launch_single_scatter(const DevParams& P, float4* rayleigh, float4* mie, WorkCounters* wc,
-                                 hipStream_t stream, bool sun_table_built = false);
+                                 hipStream_t stream, bool sun_table_built = false, bool ray_items = false);
+// The rays' ray-scatter items (DevParams::rs_items) from the sun map, once per build before launch_ray_scatter
+// (launch_single_scatter takes them along with ray_items).
+hipError_t launch_ray_items(const DevParams& P, hipStream_t stream);
 // The per-build launches that read nothing of each other, in one launch: direction geometry of the
 // sphere quadrature (when sdirs, into geom), transmittance T, E0, the half-sphere geometry (when hdirs,
 // into P.sgeo), the sun table (P.sun_rows > 0), the ray geometry and the re-sampling map.
@@ -38,7 +41,8 @@ size_t direction_geometry_bytes(const DevParams& P, int ndirs);
 // dS: previous-order scatter table; mie (nullable): first-iteration Mie strength table, added with the
 // Mie phase of the quadrature direction; dE: previous-order surface-radiance table.  slab / slab_mie
 // are scratch tables of NH x ndirs x NL x NA float4 (slab_mie used only when mie is given).  Reads the
-// per-build sun map P.sun_ps (launch_resample_map or launch_prologue).
+// per-build sun map P.sun_ps (launch_resample_map or launch_prologue).  out: dJ as launch_ray_scatter reads it,
+// packed RGB with each ray's slab in (heading, sun elevation) order.
 // The surface radiance of the same dS and Mie strength (launch_surface_radiance) computed in the
 // point-scatter launch: ndirs half-sphere directions, output table out; count is set by the launcher.
 struct SrJob {
@@ -52,7 +56,7 @@ struct SrJob {
 bool sr_fits_point_scatter(const DevParams& P, bool mie);
 size_t sr_fold_bytes(const DevParams& P, bool mie);
 hipError_t launch_point_scatter(const DevParams& P, const Dir* dirs, int ndirs, const void* geom, const float4* dS,
-                                const float4* mie, const float4* dE, float4* slab, float4* slab_mie, float4* out,
+                                const float4* mie, const float4* dE, float4* slab, float4* slab_mie, float* out,
                                 WorkCounters* wc, hipStream_t stream, const SrJob* sr = nullptr);
 // The accumulations of atmosphere_lut.clj:95-97 that ride in a ray-scatter launch.  S_out (nullable,
 // with S_in): the running sum S + dS at every grid point, S = S_in, or tab(S_in) when S_resample (S_in
@@ -66,10 +70,12 @@ struct RsAccum {
   const float4* E_in = nullptr;
   float4* E_out = nullptr;
 };
-// Reads P.ray_geo (launch_ray_geometry) and the per-build sun map P.sun_rs (launch_resample_map or
-// launch_prologue).
-hipError_t launch_ray_scatter(const DevParams& P, const float4* dJ, float4* out, WorkCounters* wc,
-                              hipStream_t stream, const RsAccum& acc = RsAccum());
+// by_sample: every entry's samples added one by one in order, with both heading columns mixed at each (slower; the
+// rounding that the surrogate's training data keeps).
+// Reads P.ray_geo (launch_ray_geometry) and the per-build items P.rs_items (launch_ray_items or
+// launch_single_scatter).
+hipError_t launch_ray_scatter(const DevParams& P, const float* dJ, float4* out, WorkCounters* wc,
+                              hipStream_t stream, const RsAccum& acc = RsAccum(), bool by_sample = false);
 // Half-sphere direction geometry of every surface-radiance height into P.sgeo (once per build, before
 // launch_surface_radiance).
 hipError_t launch_surface_geometry(const DevParams& P, const Dir* dirs, int ndirs, hipStream_t stream);
@@ -108,6 +114,8 @@ hipError_t launch_residual(const float4* a, const float4* x, const float4* y, lo
 // p[0 .. n) = 0 (a kernel, so that graph captures hold no memset node).
 hipError_t launch_fill_zero(float* p, long long n, hipStream_t stream);
 hipError_t launch_pack_rgb(const float4* in, float* out, long long count, hipStream_t stream);
+// Packed RGB entries of [blocks][d0][d1] order (count in all) in [blocks][d1][d0] order.
+hipError_t launch_transpose_rgb(const float* in, float* out, long long count, int d0, int d1, hipStream_t stream);
 hipError_t launch_unpack_rgb(const float* in, float4* out, long long count, hipStream_t stream);
 
 }  // namespace sfsim
