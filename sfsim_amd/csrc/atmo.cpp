@@ -117,7 +117,7 @@ struct sfsim_atmo_ctx {
   DeviceBuffer stage_in[3], stage_out4, stage_rgb;
   // quadrature directions
   DeviceBuffer sphere_dirs, half_dirs;
-  DeviceBuffer geom, slab, slab_mie;  // point-scatter direction geometry and folded dS slabs
+  DeviceBuffer geom;  // point-scatter direction geometry
   int sphere_key = -1, half_key = -1, sphere_n = 0, half_n = 0;
   // single scatter's sun optical-depth table (rows x cols of log2 node sums; 0 x 0 sums every segment)
   int sun_rows = kSunRows, sun_cols = kSunCols;
@@ -446,7 +446,7 @@ std::vector<Dir> sphere_directions(int half, int steps) {
   for (int i = 0; i < theta_steps; ++i) {
     double theta = theta_range * ((0.5 + i) / theta_steps);
     double factor = std::cos(theta - delta2) - std::cos(theta + delta2);
-    int ringsteps = (int)std::ceil(std::sin(theta) * steps);
+    int ringsteps = sphere_ring_directions(half, steps, i);
     double weight = (2 * M_PI) / ringsteps;
     double ct = std::cos(theta), st = std::sin(theta);
     for (int j = 0; j < ringsteps; ++j) {
@@ -477,12 +477,9 @@ int ensure_dirs(sfsim_atmo_ctx* ctx, int half, int steps) {
   return 0;
 }
 
-// Direction geometry of the sphere quadrature and the slab scratch of the point-scatter kernels.
-int prepare_point_scatter(sfsim_atmo_ctx* ctx, const DevParams& P, bool with_mie, WorkCounters* wc) {
-  size_t slab = (size_t)P.nS[0] * ctx->sphere_n * P.nS[2] * P.nS[3] * sizeof(float4);
+// Direction geometry of the sphere quadrature.
+int prepare_point_scatter(sfsim_atmo_ctx* ctx, const DevParams& P, WorkCounters* wc) {
   TRY(ensure(ctx, ctx->geom, direction_geometry_bytes(P, ctx->sphere_n)));
-  TRY(ensure(ctx, ctx->slab, slab));
-  if (with_mie) TRY(ensure(ctx, ctx->slab_mie, slab));
   HIP_TRY(ctx, launch_direction_geometry(P, (const Dir*)ctx->sphere_dirs.ptr, ctx->sphere_n, ctx->geom.ptr, wc,
                                          ctx->stream));
   return 0;
@@ -573,12 +570,7 @@ int prepare_pipeline(sfsim_atmo_ctx* ctx, const sfsim_atmo_params* p) {
     TRY(ensure(ctx, ctx->out[i], outc[i] * sizeof(float)));
     ctx->out_count[i] = outc[i];
   }
-  if (p->iterations > 0) {
-    const size_t slab = nS / ((size_t)p->scatter_shape[1]) * ctx->sphere_n * sizeof(float4);  // NH x dirs x NL x NA
-    TRY(ensure(ctx, ctx->geom, direction_geometry_bytes(make_dev_params(p), ctx->sphere_n)));
-    TRY(ensure(ctx, ctx->slab, slab));
-    TRY(ensure(ctx, ctx->slab_mie, slab));
-  }
+  if (p->iterations > 0) TRY(ensure(ctx, ctx->geom, direction_geometry_bytes(make_dev_params(p), ctx->sphere_n)));
   ctx->built = false;
   return 0;
 }
@@ -664,8 +656,8 @@ int enqueue_pipeline(sfsim_atmo_ctx* ctx, const sfsim_atmo_params* p, const DevP
     const bool sr_along = sr_fits_point_scatter(P, mie != nullptr);
     const SrJob sr{0, ctx->half_n, dS_tab, mie, f4(ctx->dE[dE_new])};
     LAUNCH(timer, kPointScatter,
-           launch_point_scatter(P, sdirs, ctx->sphere_n, ctx->geom.ptr, dS_tab, mie, f4(ctx->dE[dE_cur]), f4(ctx->slab),
-                                f4(ctx->slab_mie), (float*)ctx->dJ.ptr, wc, ctx->stream, sr_along ? &sr : nullptr));
+           launch_point_scatter(P, sdirs, ctx->sphere_n, p->sphere_steps, ctx->geom.ptr, dS_tab, mie, f4(ctx->dE[dE_cur]),
+                                (float*)ctx->dJ.ptr, wc, ctx->stream, sr_along ? &sr : nullptr));
     if (!sr_along)
       LAUNCH(timer, kSurfaceRadiance,
              launch_surface_radiance(P, ctx->half_n, dS_tab, mie, f4(ctx->dE[dE_new]), wc, ctx->stream));
@@ -838,9 +830,6 @@ int prepare_seeded(sfsim_atmo_ctx* ctx, const sfsim_atmo_params* p, int m, const
     ctx->out_count[i] = outc[i];
   }
   TRY(ensure(ctx, ctx->geom, direction_geometry_bytes(P, ctx->sphere_n)));
-  const size_t slab = nS / (size_t)p->scatter_shape[1] * ctx->sphere_n * sizeof(float4);  // NH x dirs x NL x NA
-  TRY(ensure(ctx, ctx->slab, slab));
-  TRY(ensure(ctx, ctx->slab_mie, slab));
   if (!host_sums) HIP_TRY(ctx, surrogate_reserve_tables(ctx->sg, P));
   ctx->built = false;
   return 0;
@@ -897,8 +886,8 @@ int enqueue_seeded(sfsim_atmo_ctx* ctx, const sfsim_atmo_params* p, const DevPar
     const bool sr_along = sr_fits_point_scatter(P, true);
     const SrJob sr{0, ctx->half_n, A, f4(ctx->M1), f4(ctx->dE[1])};
     LAUNCH(timer, kPointScatter,
-           launch_point_scatter(P, sdirs, ctx->sphere_n, ctx->geom.ptr, A, f4(ctx->M1), Esum, f4(ctx->slab),
-                                f4(ctx->slab_mie), (float*)ctx->dJ.ptr, nullptr, ctx->stream, sr_along ? &sr : nullptr));
+           launch_point_scatter(P, sdirs, ctx->sphere_n, p->sphere_steps, ctx->geom.ptr, A, f4(ctx->M1), Esum,
+                                (float*)ctx->dJ.ptr, nullptr, ctx->stream, sr_along ? &sr : nullptr));
     LAUNCH(timer, kRayScatter, launch_ray_scatter(P, (const float*)ctx->dJ.ptr, Pk, nullptr, ctx->stream));
     if (!sr_along)
       LAUNCH(timer, kSurfaceRadiance,
@@ -1081,9 +1070,6 @@ size_t layout_atmosphere(sfsim_atmo_ctx* c, const sfsim_atmo_params* p, char* ba
   if (p->iterations > 0) {
     const int sn = sfsim_atmo_sphere_directions(0, p->sphere_steps);
     k.take(c->geom, direction_geometry_bytes(P, sn));
-    const size_t slab = nS / (size_t)p->scatter_shape[1] * sn * sizeof(float4);
-    k.take(c->slab, slab);
-    k.take(c->slab_mie, slab);
     for (int i = 0; i < 2; ++i) k.take(c->Ssum[i], nS * sizeof(float4));
   }
   k.take(c->T, nT * sizeof(float4));
@@ -1152,7 +1138,7 @@ int sfsim_atmo_destroy(sfsim_atmo_ctx* ctx) {
                           &ctx->Sacc[0], &ctx->Sacc[1], &ctx->out[0],     &ctx->out[1],      &ctx->out[2],
                           &ctx->out[3], &ctx->stage_in[0], &ctx->stage_in[1], &ctx->stage_in[2], &ctx->stage_out4,
                           &ctx->stage_rgb, &ctx->sphere_dirs, &ctx->half_dirs, &ctx->counters,
-                          &ctx->geom,   &ctx->slab,    &ctx->slab_mie};
+                          &ctx->geom};
   for (DeviceBuffer* b : bufs) release(*b);
   DeviceBuffer* more[] = {&ctx->codes,   &ctx->targets, &ctx->sumS,    &ctx->cap[0],  &ctx->cap[1],
                           &ctx->cap[2],  &ctx->cap[3],  &ctx->cap[4],  &ctx->resid,  &ctx->sun_depth, &ctx->ray_geo, &ctx->rmap, &ctx->sunmap, &ctx->sgeo, &ctx->ray_order, &ctx->Ssum[0], &ctx->Ssum[1],
@@ -1250,10 +1236,10 @@ int sfsim_atmo_point_scatter_table(sfsim_atmo_ctx* ctx, const sfsim_atmo_params*
   int rc;
   float* o = (float*)stage_out(ctx, n, &rc);
   TRY(rc);
-  TRY(prepare_point_scatter(ctx, P, dM != nullptr, nullptr));
+  TRY(prepare_point_scatter(ctx, P, nullptr));
   HIP_TRY(ctx, launch_resample_map(P, ctx->stream));  // with it the per-entry sun terms
-  HIP_TRY(ctx, launch_point_scatter(P, (const Dir*)ctx->sphere_dirs.ptr, ctx->sphere_n, ctx->geom.ptr, ddS, dM, ddE,
-                                    (float4*)ctx->slab.ptr, (float4*)ctx->slab_mie.ptr, o, nullptr, ctx->stream));
+  HIP_TRY(ctx, launch_point_scatter(P, (const Dir*)ctx->sphere_dirs.ptr, ctx->sphere_n, p->sphere_steps, ctx->geom.ptr, ddS, dM,
+                                    ddE, o, nullptr, ctx->stream));
   HIP_TRY(ctx, launch_transpose_rgb(o, (float*)ctx->stage_rgb.ptr, (long long)n, P.nS[3], P.nS[2], ctx->stream));
   HIP_TRY(ctx, hipMemcpyAsync(out, ctx->stage_rgb.ptr, n * 3 * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
   HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
@@ -1773,10 +1759,8 @@ double sfsim_atmo_speed_of_sound(double temperature) { return 331.3 * std::sqrt(
 int sfsim_atmo_sphere_directions(int half, int steps) {
   int theta_steps = half ? (steps >> 2) : (steps >> 1);
   if (theta_steps < 1) return 0;
-  double theta_range = half ? M_PI / 2 : M_PI;
   int total = 0;
-  for (int i = 0; i < theta_steps; ++i)
-    total += (int)std::ceil(std::sin(theta_range * ((0.5 + i) / theta_steps)) * steps);
+  for (int i = 0; i < theta_steps; ++i) total += sphere_ring_directions(half, steps, i);
   return total;
 }
 

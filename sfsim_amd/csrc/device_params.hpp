@@ -1,6 +1,7 @@
 // Parameters of one table build as the kernels see them (host fills, passed by value).
 #pragma once
 
+#include <cmath>
 #include <cstdint>
 #include <type_traits>
 
@@ -11,7 +12,8 @@ namespace sfsim {
 constexpr int kMaxSteps = 256;   // ray_steps limit (LDS arrays of the per-ray kernels)
 constexpr int kMaxSlab = 1024;   // sun elevations x headings of a view ray
 constexpr int kMaxRsGroups = 8;  // column groups of the ray-scatter kernel
-constexpr int kMaxSphereDirs = 1000;  // 64 bytes of LDS per direction in the point-scatter kernel
+constexpr int kMaxSphereDirs = 1000;  // 16 bytes of LDS per direction and ray in the point-scatter kernel
+constexpr int kMaxRings = 32;         // latitude rings of at most kMaxSphereDirs directions (27)
 
 // One lookup per sample of the ray-scatter kernel: a sun direction (v . l and x . l rounded from FP64) and a column
 // of the slab; at: column << 16 | the entry's place in its ray's (sun elevation, heading) slab.
@@ -64,7 +66,8 @@ struct DevParams {
   // followed by as many ushort4 lower indices (resample_map_bytes); null: computed per launch
   char* rmap;
   // per-entry sun terms, written with the re-sampling map (launch_resample_map): sun_ps = (l, the sun-elevation
-  // coordinate) for point scattering, rounded once from FP64 (NH x NE x NL x NA float4); sun_ss = (v . l, x . l) in
+  // coordinate) for point scattering, rounded once from FP64 (NH x NE x NA x NL float4, each ray's slab in
+  // (heading, sun elevation) order); sun_ss = (v . l, x . l) in
   // FP64 for single scattering's horizon tests (the table path) and the exact sun coordinate
   float4* sun_ps;
   double2* sun_ss;
@@ -211,6 +214,14 @@ __host__ __device__ inline RayGeoView ray_geo_view(const DevParams& P) {
   b += m * sizeof(FoldStep);
   v.row = (float2*)b;
   return v;
+}
+
+// Directions in latitude ring i of integral-sphere (half = 0) or integral-half-sphere (half = 1) with the given steps:
+// ceil(sin(theta_i) steps), theta_i = range (i + 1/2) / rings (sphere.clj:62-105).
+inline int sphere_ring_directions(int half, int steps, int i) {
+  const int rings = half ? (steps >> 2) : (steps >> 1);
+  const double range = half ? M_PI / 2 : M_PI;
+  return (int)std::ceil(std::sin(range * ((0.5 + i) / rings)) * steps);
 }
 
 // Quadrature direction (FP64 unit vector in the frame of a grid point on +x) and its weight.

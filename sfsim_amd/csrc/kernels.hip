@@ -1178,9 +1178,9 @@ __global__ void __launch_bounds__(1024) ray_scatter_kernel(
 // Every grid point of a height index shares its position and quadrature frame, so the per-direction
 // geometry (ray extremity P, surface flag, T(x, P), elevation coordinate of omega at x) depends only
 // on (height, direction) and is computed once per build (direction_geometry_kernel).  The dS lookup
-// at (x, omega, l) has height and elevation coordinates that depend only on (height, direction) as
-// well: point_scatter_combine_kernel folds them into a (sun elevation, heading) slab per
-// (height, direction) once per iteration, shared by every view ray of that height.
+// at (x, omega, l) has a height coordinate that depends only on the height and an elevation coordinate that
+// depends only on the height and the direction's latitude ring (sphere.clj:62-105: the directions of a ring share
+// dot(x, omega)): point_scatter_kernel folds those two dimensions ring by ring.
 struct DirGeom {
   float4 omega;   // direction xyz, w: elevation coordinate of omega at x (flag: not surface)
   float4 ground;  // T(x, P) * brightness / pi (0 for sky directions), w: 1 for surface directions
@@ -1228,53 +1228,6 @@ __global__ void __launch_bounds__(kBlock) direction_geometry_kernel(const DevPar
   direction_geometry_body(P, dirs, ndirs, geom, wc, blockIdx.x);
 }
 
-// slab[h][j][s][a] = dS at (height of x_h, elevation coordinate of omega_j) for every (s, a) grid
-// point; with mie != nullptr the Mie strength slab is folded the same way into slab_mie.
-template <bool kB>
-__global__ void __launch_bounds__(kBlock) point_scatter_combine_kernel(const DevParams P0, const DevParams* __restrict__ PB,
-                                                                       const DirGeom* __restrict__ geom, int ndirs,
-                                                                       const float4* __restrict__ dS,
-                                                                       const float4* __restrict__ mie,
-                                                                       float4* __restrict__ slab,
-                                                                       float4* __restrict__ slab_mie) {
-  const DevParams& P = params_of<kB>(P0, PB);
-  geom = atm_ptr<kB>(geom, P);
-  dS = atm_ptr<kB>(dS, P);
-  mie = atm_ptr<kB>(mie, P);
-  slab = atm_ptr<kB>(slab, P);
-  slab_mie = atm_ptr<kB>(slab_mie, P);
-  const int NH = P.nS[0], NE = P.nS[1], NL = P.nS[2], NA = P.nS[3];
-  const int NLA = NL * NA;
-  const int b = xcd_ray(blockIdx.x, NH * ndirs);  // the XCD that reads this height's slabs (same ranges)
-  const int ih = b / ndirs;
-  const double r0 = index_to_radius(P.g, NH, ih);
-  const Lerp Lh = make_lerp((float)height_to_index(P.g, NH, r0), NH);
-  const Lerp Le = make_lerp(geom[b].omega.w, NE);
-  const long long sh = (long long)NE * NLA;
-  const long long o00 = Lh.i0 * sh + (long long)Le.i0 * NLA, o01 = Lh.i0 * sh + (long long)Le.i1 * NLA;
-  const long long o10 = Lh.i1 * sh + (long long)Le.i0 * NLA, o11 = Lh.i1 * sh + (long long)Le.i1 * NLA;
-  float4* dst = slab + (long long)b * NLA;
-  float4* dstm = slab_mie ? slab_mie + (long long)b * NLA : nullptr;
-  for (int k = threadIdx.x; k < NLA; k += blockDim.x) {
-    float3 c = mix3(mix3(ld3(dS, o00 + k), ld3(dS, o01 + k), Le.s), mix3(ld3(dS, o10 + k), ld3(dS, o11 + k), Le.s), Lh.s);
-    dst[k] = make_float4(c.x, c.y, c.z, 0.f);
-    if (mie) {
-      float3 m = mix3(mix3(ld3(mie, o00 + k), ld3(mie, o01 + k), Le.s), mix3(ld3(mie, o10 + k), ld3(mie, o11 + k), Le.s),
-                      Lh.s);
-      dstm[k] = make_float4(m.x, m.y, m.z, 0.f);
-    }
-  }
-}
-
-// One workgroup per view ray (x, v): quadrature weights sum_c beta_c(h(x)) phase_c(v . omega) w_j
-// and the direction geometry in LDS, lanes over (sun elevation, heading).
-struct DirLds {
-  float4 omega;   // direction xyz, w: 1 for surface directions
-  float4 weight;  // rgb quadrature weight times in-scattering
-  float4 ground;  // T(x, P) brightness / pi
-  float4 phat;    // P / |P|
-};
-
 // Constants of the per-direction lookups of one point-scatter launch.
 struct PsConst {
   float hA;            // (NA - 1) / 2: heading coordinate (NA - 1) (1 + dot(omega, l)) / 2 = hA + hA dot(omega, l)
@@ -1283,209 +1236,295 @@ struct PsConst {
   float mie_k, mie_a, mie_b;  // Mie phase K (1 + mu^2) (a - b mu)^(-3/2): K = 3 (1 - g^2) / (8 pi (2 + g^2))
 };
 
+// Without contraction: the same values whatever surrounds the call (near g = 1, 1 + g^2 - 2 g mu amplifies the last
+// bit of its terms).
+__device__ __forceinline__ void mie_constants(float g, PsConst& pc) {
+#pragma clang fp contract(off)
+  const float g2 = g * g;
+  pc.mie_k = 3.0f * (1.0f - g2) / (8.0f * 3.14159265358979f * (2.0f + g2));
+  pc.mie_a = 1.0f + g2;
+  pc.mie_b = 2.0f * g;
+}
+
+// phase_f with its constants as in mie_constants: the weights of the launch that adds the Mie term (the other
+// launches take phase_f; each keeps the rounding that the surrogate's training data has been made with).
+__device__ __forceinline__ float weight_phase(float g, float mu) {
+  float a, k, d;
+  {
+#pragma clang fp contract(off)
+    const float g2 = g * g;
+    a = 1.0f + g2;
+    k = 3.0f * (1.0f - g2);
+    d = 8.0f * 3.14159265358979f * (2.0f + g2);
+  }
+  const float x = a - 2.0f * g * mu;
+  return (k * (1.0f + mu * mu)) / (d * (x * sqrtf(x)));
+}
+
 // phase of atmosphere.clj:56-61 with the hardware reciprocal square root (x^-3/2 = rsq(x)^3)
 __device__ __forceinline__ float mie_phase(const PsConst& pc, float mu) {
   const float y = __builtin_amdgcn_rsqf(fmaf(-pc.mie_b, mu, pc.mie_a));
   return pc.mie_k * fmaf(mu, mu, 1.0f) * (y * y * y);
 }
 
-// the texel at byte_offset and the next one (the pointer is formed once, so the second read takes the
-// first one's address register with an immediate offset)
-__device__ __forceinline__ void ld4b_pair(const float4* base, unsigned byte_offset, float4& c0, float4& c1) {
-  const float4* p = (const float4*)((const char*)base + byte_offset);
-  c0 = p[0];
-  c1 = p[1];
-}
-
-__device__ __forceinline__ float3 lerp_pair(const float4* base, unsigned byte_offset, float s) {
-  float4 c0, c1;
-  ld4b_pair(base, byte_offset, c0, c1);
-  return lerp3(c0, c1, s);
-}
-
-// Sum over the quadrature directions of one entry (sun direction l, sun-elevation lerp Ls; row_bytes:
-// byte offset of row Ls.i0 in a slab).  Heading lerp: lower column min(floor, NA - 2), so the upper
-// column is always the next one; the dE lookup likewise in both dimensions (nested as lookup2).
-// kRow: the entry's sun-elevation weight is zero (one slab row)
-template <bool kRow, bool kMie>
-__device__ __forceinline__ float3 point_scatter_dirs(const PsConst& pc, const DirLds* s_dir, int ndirs,
-                                                     const float4* __restrict__ sh, const float4* __restrict__ shm,
-                                                     const float4* __restrict__ dE, int NA, int NLA, Lerp Ls,
-                                                     float row_bytes, float lx, float ly, float lz) {
-  float3 acc = make_float3(0.f, 0.f, 0.f);
-  const unsigned d_row = (unsigned)(Ls.i1 - Ls.i0) * (unsigned)NA * (unsigned)sizeof(float4);
-  // direction j's heading coordinate: cosine ol, column weight sa, byte offset of the lower column
-  auto heading = [&](int j, float& ol, float& sa) {
-    const DirLds& dd = s_dir[j];
-    ol = fmaf(dd.omega.z, lz, fmaf(dd.omega.y, ly, dd.omega.x * lx));
-    const float hc = __builtin_amdgcn_fmed3f(fmaf(pc.hA, ol, pc.hA), 0.0f, pc.na_top);
-    const float col = lower_cell(hc, pc.na_top - 1.0f);
-    sa = hc - col;
-    return (unsigned)fmaf(col, (float)sizeof(float4), row_bytes);
-  };
-  // the rest of direction j's term given the two texels c0, c1 of its lower slab row
-  auto term = [&](int j, float ol, float sa, unsigned off, float4 c0, float4 c1) {
-    const DirLds& dd = s_dir[j];
-    const float4* row = sh + j * NLA;
-    float3 v = lerp3(c0, c1, sa);
-    if (!kRow) {
-      const float3 u = lerp_pair(row, off + d_row, sa);
-      v = make_float3(fmaf(Ls.s, u.x - v.x, v.x), fmaf(Ls.s, u.y - v.y, v.y), fmaf(Ls.s, u.z - v.z, v.z));
-    }
-    if (kMie) {
-      const float4* rowm = shm + j * NLA;
-      float3 m = lerp_pair(rowm, off, sa);
-      if (!kRow) {
-        const float3 u = lerp_pair(rowm, off + d_row, sa);
-        m = make_float3(fmaf(Ls.s, u.x - m.x, m.x), fmaf(Ls.s, u.y - m.y, m.y), fmaf(Ls.s, u.z - m.z, m.z));
-      }
-      const float ph = mie_phase(pc, ol);
-      v.x = fmaf(m.x, ph, v.x);
-      v.y = fmaf(m.y, ph, v.y);
-      v.z = fmaf(m.z, ph, v.z);
-    }
-    if (dd.omega.w != 0.f) {
-      const float spl = fmaf(dd.phat.z, lz, fmaf(dd.phat.y, ly, dd.phat.x * lx));
-      const float ce = __builtin_amdgcn_fmed3f(
-          fmaf(-pc.se.A, fexp2(fmaf(-3.0f * 1.4426950408889634f, spl, pc.se.c)), pc.se.A), 0.0f, pc.se.top);
-      const float ecol = lower_cell(ce, pc.se.top - 1.0f);
-      const float se = ce - ecol;
-      const unsigned eo = (unsigned)ecol * (unsigned)sizeof(float4);  // height row 0: P is on the ground
-      const float3 u = lerp_pair(dE, eo, se);
-      v.x = fmaf(dd.ground.x, u.x, v.x);
-      v.y = fmaf(dd.ground.y, u.y, v.y);
-      v.z = fmaf(dd.ground.z, u.z, v.z);
-    }
-    acc.x = fmaf(dd.weight.x, v.x, acc.x);
-    acc.y = fmaf(dd.weight.y, v.y, acc.y);
-    acc.z = fmaf(dd.weight.z, v.z, acc.z);
-  };
-  // four directions at a time: their eight slab reads are issued before any of their ground terms
-  constexpr int kB = 4;
-  int j = 0;
-  for (; j + kB <= ndirs; j += kB) {
-    float ol[kB], sa[kB];
-    unsigned off[kB];
-    float4 c0[kB], c1[kB];
-#pragma unroll
-    for (int d = 0; d < kB; ++d) {
-      off[d] = heading(j + d, ol[d], sa[d]);
-      const float4* row = sh + (j + d) * NLA;
-      ld4b_pair(row, off[d], c0[d], c1[d]);
-    }
-#pragma unroll
-    for (int d = 0; d < kB; ++d) term(j + d, ol[d], sa[d], off[d], c0[d], c1[d]);
-  }
-  for (; j < ndirs; ++j) {
-    float ol, sa;
-    const unsigned off = heading(j, ol, sa);
-    const float4* row = sh + j * NLA;
-    float4 c0, c1;
-    ld4b_pair(row, off, c0, c1);
-    term(j, ol, sa, off, c0, c1);
-  }
-  return acc;
-}
-
-// kELds: the previous order's dE at the ground (height row 0) is staged in LDS after the direction
-// table (when it fits 16 KiB).  P, the ground point of a surface direction, is the ray's intersection
-// with the planet's sphere (atmosphere.clj:80-85, 213-221), so its height is 0: its FP64 |P| - R is
-// rounding noise of ~1e-9 m, whose height coordinate (through the square root of the horizon distance,
-// ~1.5e-6 for 16 rows and 100 km) would weight height row 1 by as much.
 template <bool kFold>
 __device__ __forceinline__ void surface_radiance_entry(const DevParams& P, int ndirs, const float4* __restrict__ dS,
                                                        const float4* __restrict__ mie, float4* __restrict__ out,
                                                        WorkCounters* wc, int entry, float4* s_fold, float3* s_red);
 
-// The iteration's surface radiance (it reads the same dS and Mie strength) rides in the launch: the
-// sr.count workgroups after the rays' compute its entries with the LDS-folded kernel body.
-template <bool kMie, bool kELds, bool kB>
-__global__ void __launch_bounds__(kBlock) point_scatter_kernel(const DevParams P0, const DevParams* __restrict__ PB,
-                                                               const Dir* __restrict__ dirs,
-                                                               const DirGeom* __restrict__ geom, int ndirs,
-                                                               const float4* __restrict__ slab,
-                                                               const float4* __restrict__ slab_mie,
-                                                               const float4* __restrict__ dE, float* __restrict__ out,
-                                                               const SrJob sr, WorkCounters* wc) {
-  extern __shared__ DirLds s_dir[];
-  float4* s_dE = (float4*)(s_dir + ndirs);
+// The split of a point-scatter launch.  A workgroup takes `rays` view rays of one height and `rows` sun elevations,
+// `waves` wavefronts per ray (64 EPT entries each); eblocks x sblocks workgroups per height.  pitch: texels per
+// column of its slab; misc: bytes of the weights and dE in LDS (below the slabs, see ps_shared_bytes).
+struct PsPlan {
+  int rows, sblocks, rays, waves, eblocks, pitch;
+  unsigned misc;
+};
+
+// LDS of a workgroup: the folded slab of one latitude ring, double-buffered (and of the Mie strength in the first
+// iteration), a texel for each column and sun elevation: its colour and the difference to the next column's, six
+// floats in two planes: 16 bytes (colour, first difference) at byte address A, the other 8 at A / 2.  The last
+// column, which only the heading coordinate NA - 1 reads, holds the column before it plus its difference (what the
+// interpolation between the two gives at weight 1) and no difference, so a lookup needs no clamped lower column.
+// The 8-byte plane begins at `misc` (at least its own size) and the 16-byte plane at 2 misc; the weights, dE (laid
+// out alike) and the surface-radiance workgroups' partial sums take the bytes below.
+__host__ __device__ inline unsigned ps_texels(const PsPlan& p, int na, bool mie) {
+  return 2u * (mie ? 2u : 1u) * (unsigned)p.pitch * (unsigned)na;
+}
+__host__ __device__ inline size_t ps_shared_bytes(const PsPlan& p, int na, bool mie) {
+  return 2 * (size_t)p.misc + 16 * (size_t)ps_texels(p, na, mie);
+}
+
+// One texel: u and the difference to v; `last`: what interpolation at weight 1 gives, and no difference.
+__device__ __forceinline__ void ps_store(float4* a, float2* b, float3 u, float3 v, bool last) {
+  const float3 d = make_float3(v.x - u.x, v.y - u.y, v.z - u.z);
+  *a = last ? make_float4(u.x + d.x, u.y + d.y, u.z + d.z, 0.f) : make_float4(u.x, u.y, u.z, d.x);
+  *b = last ? make_float2(0.f, 0.f) : make_float2(d.y, d.z);
+}
+
+// Latitude rings of the sphere quadrature: ring i holds directions start[i] .. start[i + 1] - 1.
+struct PsRings {
+  int count;
+  unsigned short start[kMaxRings + 1];
+};
+
+// What bounds it is VALU issue: about 14 instruction slots per (entry, sky direction) and 34 per ground direction, beside
+// 24 bytes of LDS reads per lookup.  The slab of a ring is shared by the ring's directions and by the rays of a
+// height, so it is folded in the kernel itself (nine times fewer texels than one slab per direction, and no
+// launch, table or gather from L2 for them); lanes run over the sun elevations of a column, so that their reads of a
+// slab's columns are contiguous whatever columns they need.
+//
+// kELds: the previous order's dE at the ground (height row 0) is staged in LDS.  P, the ground point of a surface
+// direction, is the ray's intersection with the planet's sphere (atmosphere.clj:80-85, 213-221), so its height is
+// 0: its FP64 |P| - R is rounding noise of ~1e-9 m, whose height coordinate (through the square root of the
+// horizon distance, ~1.5e-6 for 16 rows and 100 km) would weight height row 1 by as much.
+//
+// The iteration's surface radiance (it reads the same dS and Mie strength) rides in the launch: the sr.count
+// workgroups after the rays' compute its entries with the LDS-folded kernel body.
+template <int EPT, bool kMie, bool kELds, bool kB>
+__global__ void __launch_bounds__(kBlock) point_scatter_kernel(
+    const DevParams P0, const DevParams* __restrict__ PB, const Dir* __restrict__ dirs, const DirGeom* __restrict__ geom,
+    int ndirs, const PsRings rings, const float4* __restrict__ dS, const float4* __restrict__ mie,
+    const float4* __restrict__ dE, float* __restrict__ out, const SrJob sr, const PsPlan plan, WorkCounters* wc) {
+  extern __shared__ float4 s_mem[];
+  char* const lds = (char*)s_mem;
   const DevParams& P = params_of<kB>(P0, PB);
   const int NH = P.nS[0], NE = P.nS[1], NL = P.nS[2], NA = P.nS[3];
-  const int NLA = NL * NA;
-  if ((int)blockIdx.x >= NH * NE) {
-    __shared__ float3 s_red[kBlock / 64];
+  const int NLA = NL * NA, blocks = NH * plan.eblocks * plan.sblocks;
+  if ((int)blockIdx.x >= blocks) {
+    float3* s_red = (float3*)s_mem;  // one per wavefront
     surface_radiance_entry<true>(P, sr.ndirs, atm_ptr<kB>(sr.dS, P), atm_ptr<kB>(sr.mie, P), atm_ptr<kB>(sr.out, P),
-                                 wc, (int)blockIdx.x - NH * NE, (float4*)s_dir, s_red);
+                                 wc, (int)blockIdx.x - blocks, s_mem + 4, s_red);
     return;
   }
   geom = atm_ptr<kB>(geom, P);
-  slab = atm_ptr<kB>(slab, P);
-  slab_mie = atm_ptr<kB>(slab_mie, P);
+  dS = atm_ptr<kB>(dS, P);
+  mie = atm_ptr<kB>(mie, P);
   dE = atm_ptr<kB>(dE, P);
   out = atm_ptr<kB>(out, P);
-  const int rayid = xcd_ray(blockIdx.x, NH * NE);
-  if (kELds)
-    for (int i = threadIdx.x; i < P.nE[1]; i += blockDim.x) s_dE[i] = dE[i];
-  const int ih = rayid / NE, ie = rayid - ih * NE;
-  const double r0 = index_to_radius(P.g, NH, ih), h0 = index_to_altitude(P.g, NH, ih);
-  double se, ce;
-  bool above_unused;
-  index_to_elevation(P.g, NE, r0, ie, se, ce, above_unused);
-  const float bm = (float)exp(-h0 * P.inv_scale_mie), br = (float)exp(-h0 * P.inv_scale_ray);
-  const DirGeom* gh = geom + (long long)ih * ndirs;
+  const int b = xcd_ray(blockIdx.x, blocks), hb = b / plan.sblocks, ih = hb / plan.eblocks;
+  const int s0 = (b - hb * plan.sblocks) * plan.rows, rows = min(plan.rows, NL - s0);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = wave / plan.waves, part = wave - r * plan.waves;
+  const int ie = (hb - ih * plan.eblocks) * plan.rays + r;
+  const bool active = r < plan.rays && ie < NE;  // whole wavefronts; the others help to fold
   const int nE1 = P.nE[1];
-  for (int j = threadIdx.x; j < ndirs; j += blockDim.x) {
-    Dir d = dirs[j];
-    DirGeom g = gh[j];
-    float vw = (float)(se * d.x + ce * d.y);
-    float pm = phase_f(P.g_mie, vw) * bm, pr = phase_f(P.g_ray, vw) * br;
-    float w = (float)d.w;
-    DirLds dl;
-    dl.omega = make_float4(g.omega.x, g.omega.y, g.omega.z, g.ground.w);
-    dl.weight = make_float4((P.sca_mie[0] * pm + P.sca_ray[0] * pr) * w, (P.sca_mie[1] * pm + P.sca_ray[1] * pr) * w,
-                            (P.sca_mie[2] * pm + P.sca_ray[2] * pr) * w, 0.f);
-    dl.ground = make_float4(g.ground.x, g.ground.y, g.ground.z, 0.f);
-    dl.phat = make_float4(g.phat.x, g.phat.y, g.phat.z, 0.f);
-    s_dir[j] = dl;
+  float4* s_w = s_mem;                                    // [rays][ndirs] rgb quadrature weight times in-scattering
+  float4* s_ea = s_w + plan.rays * ndirs;                 // dE at the ground and the differences to the next entry's,
+  float2* s_eb = (float2*)(s_ea + (kELds ? nE1 : 0));     // as the slabs' texels
+  const double r0 = index_to_radius(P.g, NH, ih), h0 = index_to_altitude(P.g, NH, ih);
+  const DirGeom* __restrict__ gh = geom + (long long)ih * ndirs;
+
+  // Slab of one ring, columns fastest (coalesced reads).
+  const int fold_rows = min(plan.pitch, NL - s0), fold_n = NA * fold_rows;
+  const unsigned half = plan.misc, slab_texels = (unsigned)(plan.pitch * NA);
+  const Lerp Lh = make_lerp((float)height_to_index(P.g, NH, r0), NH);
+  const long long sh = (long long)NE * NLA;
+  auto fold = [&](int ring, unsigned buffer) {
+    const Lerp Le = make_lerp(gh[rings.start[ring]].omega.w, NE);
+    auto texel = [&](const float4* __restrict__ t, long long k) {
+      const float3 u = mix3(ld3(t, Lh.i0 * sh + (long long)Le.i0 * NLA + k), ld3(t, Lh.i0 * sh + (long long)Le.i1 * NLA + k), Le.s);
+      if (Lh.s == 0.0f) return u;  // mix3(u, v, 0) is u exactly
+      return mix3(u, mix3(ld3(t, Lh.i1 * sh + (long long)Le.i0 * NLA + k), ld3(t, Lh.i1 * sh + (long long)Le.i1 * NLA + k), Le.s), Lh.s);
+    };
+    for (int i = threadIdx.x; i < fold_n; i += blockDim.x) {
+      const int row = i / NA, col = i - row * NA;
+      const bool last = col == NA - 1;
+      const long long k = (long long)(s0 + row) * NA + col - last;
+      const unsigned t = buffer * (kMie ? 2u : 1u) * slab_texels + (unsigned)(col * plan.pitch + row);
+#pragma unroll
+      for (int m = 0; m < (kMie ? 2 : 1); ++m) {
+        const float4* __restrict__ tab = m ? mie : dS;
+        const unsigned A = 2 * half + 16 * (t + m * slab_texels);
+        ps_store((float4*)(lds + A), (float2*)(lds + (A >> 1)), texel(tab, k), texel(tab, k + 1), last);
+      }
+    }
+  };
+
+  if (kELds)
+    for (int i = threadIdx.x; i < nE1; i += blockDim.x) {
+      const int k = min(i, nE1 - 2);
+      ps_store(s_ea + i, s_eb + i, ld3(dE, k), ld3(dE, k + 1), k != i);
+    }
+  if (active) {
+    double se, ce;
+    bool above_unused;
+    index_to_elevation(P.g, NE, r0, ie, se, ce, above_unused);
+    const float bm = (float)exp(-h0 * P.inv_scale_mie), br = (float)exp(-h0 * P.inv_scale_ray);
+    for (int j = part * 64 + lane; j < ndirs; j += 64 * plan.waves) {
+      const Dir d = dirs[j];
+      const float vw = (float)(se * d.x + ce * d.y);
+      const float pm = (kMie ? weight_phase(P.g_mie, vw) : phase_f(P.g_mie, vw)) * bm;
+      const float pr = (kMie ? weight_phase(P.g_ray, vw) : phase_f(P.g_ray, vw)) * br;
+      const float w = (float)d.w;
+      s_w[r * ndirs + j] = make_float4((P.sca_mie[0] * pm + P.sca_ray[0] * pr) * w, (P.sca_mie[1] * pm + P.sca_ray[1] * pr) * w,
+                                       (P.sca_mie[2] * pm + P.sca_ray[2] * pr) * w, 0.f);
+    }
   }
-  const float gm = P.g_mie;
   PsConst pc;
   pc.hA = 0.5f * (float)(NA - 1);
   pc.na_top = (float)(NA - 1);
   pc.se = SunCoord{(float)((nE1 - 1) * (double)P.sun_inv_den), (float)(-0.6 * 1.4426950408889634), (float)(nE1 - 1)};
-  pc.mie_k = 3.0f * (1.0f - gm * gm) / (8.0f * 3.14159265358979f * (2.0f + gm * gm));
-  pc.mie_a = 1.0f + gm * gm;
-  pc.mie_b = 2.0f * gm;
-  __syncthreads();
-  const float4* eTab = kELds ? s_dE : dE;
-  const float4* sh = slab + (long long)ih * ndirs * NLA;
-  const float4* shm = kMie ? slab_mie + (long long)ih * ndirs * NLA : nullptr;
-  const long long base = (long long)rayid * NLA;
-  unsigned long long l4 = 0, l2 = 0;
-  for (int k = threadIdx.x; k < NLA; k += blockDim.x) {
-    float lx, ly, lz;
-    Lerp Ls;
-    {  // the per-build sun terms (l and the sun-elevation coordinate, rounded once from FP64)
-      const float4 m = P.sun_ps[base + k];
-      lx = m.x;
-      ly = m.y;
-      lz = m.z;
-      Ls = make_lerp(m.w, NL);
-    }
-    const float row_bytes = (float)(Ls.i0 * NA * (int)sizeof(float4));
-    // a grid entry's own sun-elevation coordinate is an integer, so its weight is exactly zero and only
-    // one row of each slab is read; the general lookup stays for safety
-    const float3 acc = Ls.s == 0.0f
-                           ? point_scatter_dirs<true, kMie>(pc, s_dir, ndirs, sh, shm, eTab, NA, NLA, Ls, row_bytes, lx, ly, lz)
-                           : point_scatter_dirs<false, kMie>(pc, s_dir, ndirs, sh, shm, eTab, NA, NLA, Ls, row_bytes, lx, ly, lz);
-    l4 += (unsigned long long)ndirs * (kMie ? 2 : 1);
-    if (wc)
-      for (int j = 0; j < ndirs; ++j) l2 += s_dir[j].omega.w != 0.f;
-    float* o = out + 3 * (base + (k % NA) * NL + k / NA);  // packed, (heading, sun elevation) order
-    o[0] = acc.x;
-    o[1] = acc.y;
-    o[2] = acc.z;
+  mie_constants(P.g_mie, pc);
+
+  // The lane's entries, EPT slots of 64 in (heading, sun elevation) order.  A grid entry's own sun-elevation
+  // coordinate is its row: index-to-sin-sun-elevation and back in FP64 is off by ~1e-13, which the rounding to FP32
+  // takes away but at row 0, where it may leave a weight of that order on row 1.
+  const int count_e = rows * NA;
+  const long long base = ((long long)ih * NE + (active ? ie : 0)) * NLA;
+  int at[EPT];
+  float lx[EPT], ly[EPT], lz[EPT], s_up[EPT];
+  unsigned row_bytes[EPT];
+  float3 acc[EPT];
+  bool two = false;
+#pragma unroll
+  for (int e = 0; e < EPT; ++e) {
+    const int q = min((part * EPT + e) * 64 + lane, count_e - 1), a = q / rows, is = q - a * rows;
+    at[e] = a * NL + s0 + is;
+    const float4 m = P.sun_ps[base + at[e]];  // l and the sun-elevation coordinate, rounded once from FP64
+    lx[e] = m.x;
+    ly[e] = m.y;
+    lz[e] = m.z;
+    s_up[e] = s0 + is == 0 ? make_lerp(m.w, NL).s : 0.0f;
+    two = two || s_up[e] != 0.0f;
+    row_bytes[e] = 2 * half + 16 * is;
+    acc[e] = make_float3(0.f, 0.f, 0.f);
   }
+  two = __any(two);
+  fold(0, 0);
+  __syncthreads();
+  const unsigned pitch_bytes = 16 * plan.pitch;
+  for (int ring = 0; ring < rings.count; ++ring) {
+    if (ring + 1 < rings.count) fold(ring + 1, (ring + 1) & 1);
+    if (active) {
+      const int j0 = rings.start[ring], j1 = rings.start[ring + 1];
+      const bool to_ground = gh[j0].ground.w != 0.f;  // the ring's directions meet the ground
+      const unsigned buffer_bytes = (ring & 1) * (kMie ? 32u : 16u) * slab_texels;
+      // one lookup of the slab at byte address A: colour + s x difference
+      auto lerp_at = [&](unsigned A, float s) {
+        const float4 u = *(const float4*)(lds + A);
+        const float2 d = *(const float2*)(lds + (A >> 1));
+        return make_float3(fmaf(s, u.w, u.x), fmaf(s, d.x, u.y), fmaf(s, d.y, u.z));
+      };
+      auto lookup = [&](unsigned A, float sa, int e, bool second) {
+        float3 v = lerp_at(A, sa);
+        if (second) {
+          const float3 u = lerp_at(A + 16, sa);
+          const float s = s_up[e];
+          if (s != 0.0f) v = make_float3(fmaf(s, u.x - v.x, v.x), fmaf(s, u.y - v.y, v.y), fmaf(s, u.z - v.z, v.z));
+        }
+        return v;
+      };
+      auto directions = [&](auto ground_ring, bool second) {
+        // dot(x, omega) is the ring's
+        float x0[EPT];
+        unsigned rb[EPT];
+#pragma unroll
+        for (int e = 0; e < EPT; ++e) {
+          x0[e] = gh[j0].omega.x * lx[e];
+          rb[e] = row_bytes[e] + buffer_bytes;
+        }
+#pragma unroll 2
+        for (int j = j0; j < j1; ++j) {
+          const float4 om = gh[j].omega, w = s_w[r * ndirs + j];
+#pragma unroll
+          for (int e = 0; e < EPT; ++e) {
+            const float ol = fmaf(om.z, lz[e], fmaf(om.y, ly[e], x0[e]));
+            const float hc = __builtin_amdgcn_fmed3f(fmaf(pc.hA, ol, pc.hA), 0.0f, pc.na_top);
+            const float sa = __builtin_amdgcn_fractf(hc);
+            const unsigned A = __umul24((unsigned)hc, pitch_bytes) + rb[e];
+            float3 v = lookup(A, sa, e, second);
+            if (kMie) {
+              const float3 m = lookup(A + 16 * slab_texels, sa, e, second);
+              const float ph = mie_phase(pc, ol);
+              v.x = fmaf(m.x, ph, v.x);
+              v.y = fmaf(m.y, ph, v.y);
+              v.z = fmaf(m.z, ph, v.z);
+            }
+            if (ground_ring) {
+              const float4 ph = gh[j].phat, ground = gh[j].ground;  // ground: T(x, P) brightness / pi
+              const float spl = fmaf(ph.z, lz[e], fmaf(ph.y, ly[e], ph.x * lx[e]));
+              const float ce = __builtin_amdgcn_fmed3f(
+                  fmaf(-pc.se.A, fexp2(fmaf(-3.0f * 1.4426950408889634f, spl, pc.se.c)), pc.se.A), 0.0f, pc.se.top);
+              float3 u;  // of height row 0: P is on the ground
+              if (kELds) {
+                const unsigned i = (unsigned)ce;
+                const float s = __builtin_amdgcn_fractf(ce);
+                const float4 c = s_ea[i];
+                const float2 d = s_eb[i];
+                u = make_float3(fmaf(s, c.w, c.x), fmaf(s, d.x, c.y), fmaf(s, d.y, c.z));
+              } else {
+                const float ecol = lower_cell(ce, pc.se.top - 1.0f);
+                u = lerp3(dE[(int)ecol], dE[(int)ecol + 1], ce - ecol);
+              }
+              v.x = fmaf(ground.x, u.x, v.x);
+              v.y = fmaf(ground.y, u.y, v.y);
+              v.z = fmaf(ground.z, u.z, v.z);
+            }
+            acc[e].x = fmaf(w.x, v.x, acc[e].x);
+            acc[e].y = fmaf(w.y, v.y, acc[e].y);
+            acc[e].z = fmaf(w.z, v.z, acc[e].z);
+          }
+        }
+      };
+      if (two) {
+        if (to_ground) directions(std::true_type(), true);
+        else directions(std::false_type(), true);
+      } else {
+        if (to_ground) directions(std::true_type(), false);
+        else directions(std::false_type(), false);
+      }
+    }
+    __syncthreads();
+  }
+  unsigned long long l4 = 0, l2 = 0;
+#pragma unroll
+  for (int e = 0; e < EPT; ++e)
+    if (active && (part * EPT + e) * 64 + lane < count_e) {
+      *(Rgb*)(out + 3 * (base + at[e])) = Rgb{acc[e].x, acc[e].y, acc[e].z};  // packed, (heading, sun elevation) order
+      l4 += (unsigned long long)ndirs * (kMie ? 2 : 1);
+      if (wc)
+        for (int j = 0; j < ndirs; ++j) l2 += gh[j].ground.w != 0.f;
+    }
   count(wc, 0, 0, l4, l2);
 }
 
@@ -1648,7 +1687,7 @@ __device__ __forceinline__ void resample_map_body(const DevParams& P, unsigned b
   resample4_lerps(P, ih, ie, is, ia, Lh, Le, Ls, La, &ps, &ss);
   ((float4*)P.rmap)[idx] = make_float4(Lh.s, Le.s, Ls.s, La.s);
   if (P.sun_ps) {
-    P.sun_ps[idx] = ps;
+    P.sun_ps[idx - (is * NA + ia) + ia * NL + is] = ps;
     P.sun_ss[idx] = ss;
   }
   ((ushort4*)(P.rmap + n * sizeof(float4)))[idx] =
@@ -2048,64 +2087,84 @@ hipError_t launch_direction_geometry(const DevParams& P, const Dir* dirs, int nd
 
 size_t direction_geometry_bytes(const DevParams& P, int ndirs) { return sizeof(DirGeom) * (size_t)P.nS[0] * ndirs; }
 
-hipError_t launch_point_scatter(const DevParams& P, const Dir* dirs, int ndirs, const void* geom, const float4* dS,
-                                const float4* mie, const float4* dE, float4* slab, float4* slab_mie, float* out,
-                                WorkCounters* wc, hipStream_t stream, const SrJob* sr) {
-  if (!P.sun_ps) return hipErrorInvalidValue;
-  unsigned combos = (unsigned)(P.nS[0] * ndirs);
-  const unsigned nz = P.batch > 0 ? (unsigned)P.batch : 1u;
+// The split of a point-scatter launch.  Sun elevations in equal blocks of about 16 rows (a wavefront's 16-lane LDS
+// phases then stay within a column: blocks of 8 or 32 rows took 4-30% longer), of at most 512 texels per slab;
+// two entries per lane where that leaves 4 wavefronts per SIMD, one on smaller grids: 32 x 64 x 32 x 8 with 66
+// directions 39 us with two and 48 with one, 19 x 45 x 20 x 7 with 38 directions 19.6 us with one and 20.3 with two.
+template <bool kMie>
+static PsPlan point_scatter_plan(const DevParams& P, int ndirs, bool e_lds, int& ept) {
+  const int NL = P.nS[2], NA = P.nS[3], most = std::max(1, 512 / ((kMie ? 2 : 1) * NA));
+  PsPlan p;
+  p.sblocks = std::max({1, (NL + 8) / 16, (NL + most - 1) / most});
+  p.rows = (NL + p.sblocks - 1) / p.sblocks;
+  p.sblocks = (NL + p.rows - 1) / p.rows;
+  p.pitch = std::max(2, p.rows);
+  const int slots = (p.rows * NA + 63) / 64;  // at most 8
+  const long long tiles = (long long)P.nS[0] * P.nS[1] * std::max(1, P.batch) * p.sblocks;
+  ept = slots > 4 || (slots > 1 && tiles * ((slots + 1) / 2) >= 4096) ? 2 : 1;
+  p.waves = (slots + ept - 1) / ept;
+  p.rays = 4 / p.waves;
+  p.eblocks = (P.nS[1] + p.rays - 1) / p.rays;
+  const size_t misc = sizeof(float4) * (size_t)p.rays * ndirs + (e_lds ? 24 * (size_t)P.nE[1] : 0);
+  p.misc = (unsigned)(std::max<size_t>(misc, 8 * (size_t)ps_texels(p, NA, kMie)) + 15) & ~15u;
+  return p;
+}
+
+template <int EPT, bool kMie, bool kELds>
+static void point_scatter_as(const DevParams& P, const Dir* dirs, int ndirs, const PsRings& rings, const DirGeom* geom,
+                             const float4* dS, const float4* mie, const float4* dE, float* out, WorkCounters* wc,
+                             hipStream_t stream, const SrJob& sr, const PsPlan& plan) {
+  const unsigned blocks = (unsigned)(P.nS[0] * plan.eblocks * plan.sblocks + sr.count);
+  size_t shmem = ps_shared_bytes(plan, P.nS[3], kMie);
+  if (sr.count > 0) shmem = std::max(shmem, 4 * sizeof(float4) + sr_fold_bytes(P, sr.mie != nullptr));
   if (P.batch > 0)
-    hipLaunchKernelGGL(point_scatter_combine_kernel<true>, dim3(combos, 1, nz), dim3(kBlock), 0, stream, P,
-                       P.batch_params, (const DirGeom*)geom, ndirs, dS, mie, slab, mie ? slab_mie : nullptr);
+    hipLaunchKernelGGL((point_scatter_kernel<EPT, kMie, kELds, true>), dim3(blocks, 1, (unsigned)P.batch), dim3(kBlock),
+                       shmem, stream, P, P.batch_params, dirs, geom, ndirs, rings, dS, mie, dE, out, sr, plan, wc);
   else
-    hipLaunchKernelGGL(point_scatter_combine_kernel<false>, dim3(combos), dim3(kBlock), 0, stream, P, P.batch_params,
-                       (const DirGeom*)geom, ndirs, dS, mie, slab, mie ? slab_mie : nullptr);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  const size_t e_bytes = sizeof(float4) * (size_t)P.nE[1];  // dE height row 0, the ground
-  const bool e_lds = e_bytes <= 16384;
-  size_t shmem = sizeof(DirLds) * (size_t)ndirs + (e_lds ? e_bytes : 0);
+    hipLaunchKernelGGL((point_scatter_kernel<EPT, kMie, kELds, false>), dim3(blocks), dim3(kBlock), shmem, stream, P,
+                       P.batch_params, dirs, geom, ndirs, rings, dS, mie, dE, out, sr, plan, wc);
+}
+
+template <bool kMie>
+static hipError_t launch_point_scatter_as(const DevParams& P, const Dir* dirs, int ndirs, const PsRings& rings,
+                                          const DirGeom* geom, const float4* dS, const float4* mie, const float4* dE,
+                                          float* out, WorkCounters* wc, hipStream_t stream, const SrJob& sr) {
+  const bool e_lds = P.nE[1] <= 1024;
+  int ept = 1;
+  const PsPlan plan = point_scatter_plan<kMie>(P, ndirs, e_lds, ept);
+#define SFSIM_PS_CASE(EPT, E) \
+  point_scatter_as<EPT, kMie, E>(P, dirs, ndirs, rings, geom, dS, mie, dE, out, wc, stream, sr, plan)
+  if (e_lds) {
+    if (ept == 1) SFSIM_PS_CASE(1, true);
+    else SFSIM_PS_CASE(2, true);
+  } else {
+    if (ept == 1) SFSIM_PS_CASE(1, false);
+    else SFSIM_PS_CASE(2, false);
+  }
+#undef SFSIM_PS_CASE
+  return hipGetLastError();
+}
+
+hipError_t launch_point_scatter(const DevParams& P, const Dir* dirs, int ndirs, int sphere_steps, const void* geom,
+                                const float4* dS, const float4* mie, const float4* dE, float* out, WorkCounters* wc,
+                                hipStream_t stream, const SrJob* sr) {
+  if (!P.sun_ps) return hipErrorInvalidValue;
+  PsRings rings;
+  rings.count = sphere_steps >> 1;
+  if (rings.count < 1 || rings.count > kMaxRings) return hipErrorInvalidValue;
+  rings.start[0] = 0;
+  for (int i = 0; i < rings.count; ++i)
+    rings.start[i + 1] = (unsigned short)(rings.start[i] + sphere_ring_directions(0, sphere_steps, i));
+  if (rings.start[rings.count] != ndirs) return hipErrorInvalidValue;
   SrJob job{};
-  unsigned extra = 0;
   if (sr) {
     if (!P.sgeo || !sr->out || !sr_fits_point_scatter(P, sr->mie != nullptr)) return hipErrorInvalidValue;
     job = *sr;
     job.count = P.nE[0] * P.nE[1];
-    extra = (unsigned)job.count;
-    shmem = std::max(shmem, sr_fold_bytes(P, sr->mie != nullptr));
   }
-  const unsigned blocks = (unsigned)(P.nS[0] * P.nS[1]) + extra;
-  const DirGeom* g = (const DirGeom*)geom;
-  const dim3 grid(blocks, 1, nz);
-  const DevParams* PB = P.batch_params;
-  if (P.batch > 0) {
-    if (mie && e_lds)
-      hipLaunchKernelGGL((point_scatter_kernel<true, true, true>), grid, dim3(kBlock), shmem, stream, P, PB, dirs, g,
-                         ndirs, slab, slab_mie, dE, out, job, wc);
-    else if (mie)
-      hipLaunchKernelGGL((point_scatter_kernel<true, false, true>), grid, dim3(kBlock), shmem, stream, P, PB, dirs, g,
-                         ndirs, slab, slab_mie, dE, out, job, wc);
-    else if (e_lds)
-      hipLaunchKernelGGL((point_scatter_kernel<false, true, true>), grid, dim3(kBlock), shmem, stream, P, PB, dirs, g,
-                         ndirs, slab, nullptr, dE, out, job, wc);
-    else
-      hipLaunchKernelGGL((point_scatter_kernel<false, false, true>), grid, dim3(kBlock), shmem, stream, P, PB, dirs, g,
-                         ndirs, slab, nullptr, dE, out, job, wc);
-  } else {
-    if (mie && e_lds)
-      hipLaunchKernelGGL((point_scatter_kernel<true, true, false>), grid, dim3(kBlock), shmem, stream, P, PB, dirs, g,
-                         ndirs, slab, slab_mie, dE, out, job, wc);
-    else if (mie)
-      hipLaunchKernelGGL((point_scatter_kernel<true, false, false>), grid, dim3(kBlock), shmem, stream, P, PB, dirs, g,
-                         ndirs, slab, slab_mie, dE, out, job, wc);
-    else if (e_lds)
-      hipLaunchKernelGGL((point_scatter_kernel<false, true, false>), grid, dim3(kBlock), shmem, stream, P, PB, dirs, g,
-                         ndirs, slab, nullptr, dE, out, job, wc);
-    else
-      hipLaunchKernelGGL((point_scatter_kernel<false, false, false>), grid, dim3(kBlock), shmem, stream, P, PB, dirs,
-                         g, ndirs, slab, nullptr, dE, out, job, wc);
-  }
-  return hipGetLastError();
+  if (mie)
+    return launch_point_scatter_as<true>(P, dirs, ndirs, rings, (const DirGeom*)geom, dS, mie, dE, out, wc, stream, job);
+  return launch_point_scatter_as<false>(P, dirs, ndirs, rings, (const DirGeom*)geom, dS, mie, dE, out, wc, stream, job);
 }
 
 // Sample segments per ray and group of columns: as many as let the workgroups of all rays be resident at once (four
