@@ -1045,7 +1045,6 @@ struct Carver {
 size_t layout_shared(sfsim_atmo_ctx* c, const sfsim_atmo_params* p, char* base) {
   Carver k{base};
   const DevParams P = make_dev_params(p);
-  const size_t nS = (size_t)count4(p->scatter_shape);
   k.take(c->ray_order, (size_t)p->scatter_shape[0] * p->scatter_shape[1] * sizeof(int));
   k.take(c->rmap, resample_map_bytes(P));
   k.take(c->sunmap, sun_map_bytes(P));
@@ -1553,21 +1552,19 @@ int sfsim_atmo_surrogate_eval(sfsim_atmo_ctx* ctx, const float* inputs, const fl
   TRY(ensure(ctx, ctx->stage_rgb, (size_t)rows * kMlpIn * sizeof(float)));
   HIP_TRY(ctx, hipMemcpyAsync(ctx->stage_rgb.ptr, inputs, (size_t)rows * kMlpIn * sizeof(float),
                               hipMemcpyHostToDevice, ctx->stream));
-  HIP_TRY(ctx, surrogate_encode_rows(sg, (const float*)ctx->stage_rgb.ptr, rows, ctx->stream));
-  HIP_TRY(ctx, surrogate_forward(sg, rows, ctx->stream));
+  if (targets)
+    HIP_TRY(ctx, hipMemcpyAsync(sg.T, targets, (size_t)rows * kMlpOut * sizeof(float), hipMemcpyHostToDevice,
+                                ctx->stream));
+  HIP_TRY(ctx, surrogate_eval_rows(sg, (const float*)ctx->stage_rgb.ptr, rows, targets != nullptr, ctx->stream));
   if (outputs)
     HIP_TRY(ctx, hipMemcpyAsync(outputs, sg.Y, (size_t)rows * kMlpOut * sizeof(float), hipMemcpyDeviceToHost,
                                 ctx->stream));
   if (targets) {
-    HIP_TRY(ctx, hipMemcpyAsync(sg.T, targets, (size_t)rows * kMlpOut * sizeof(float), hipMemcpyHostToDevice,
-                                ctx->stream));
-    HIP_TRY(ctx, surrogate_backward(sg, rows, ctx->stream));
     if (grad)
       HIP_TRY(ctx, hipMemcpyAsync(grad, sg.grad, MlpLayout::total * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
     if (loss) {
-      int parts = (rows * kMlpOut + 255) / 256;
-      std::vector<float> h(parts);
-      HIP_TRY(ctx, hipMemcpyAsync(h.data(), sg.loss, parts * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
+      std::vector<float> h(surrogate_loss_parts(rows));
+      HIP_TRY(ctx, hipMemcpyAsync(h.data(), sg.loss, h.size() * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
       HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
       double t = 0;
       for (float v : h) t += v;
@@ -1617,23 +1614,25 @@ int sfsim_atmo_surrogate_train(sfsim_atmo_ctx* ctx, const sfsim_atmo_params* atm
     HIP_TRY(ctx, surrogate_init_output_bias(sg, (const float*)ctx->targets.ptr, (long long)count * (long long)nS,
                                             ctx->stream));
   const int rows = sg.batch_capacity;
-  const int parts = (rows * kMlpOut + 255) / 256;
-  std::vector<float> part(parts);
+  const int parts = surrogate_loss_parts(rows), slots = surrogate_loss_slots(rows);
+  std::vector<float> part((size_t)parts * slots);  // the loss partials of up to `slots` steps, read together
   const int warmup = steps / 20;  // linear warm-up over 5% of the steps, then cosine decay
   for (int step = 0; step < steps; ++step) {
     float lr_t = step < warmup ? (float)(lr * (step + 1) / warmup)
                                : (float)(lr * 0.5 * (1.0 + std::cos(M_PI * (step - warmup) / (steps - warmup))));
-    HIP_TRY(ctx, surrogate_gather_batch(sg, P, (const AtmosphereCode*)ctx->codes.ptr, count,
-                                        (const float*)ctx->targets.ptr, seed, step, rows, ctx->stream));
-    HIP_TRY(ctx, surrogate_forward(sg, rows, ctx->stream));
-    HIP_TRY(ctx, surrogate_backward(sg, rows, ctx->stream));
+    const int slot = step % slots;
+    HIP_TRY(ctx, surrogate_train_rows(sg, P, (const AtmosphereCode*)ctx->codes.ptr, count, (const float*)ctx->targets.ptr,
+                                      seed, step, rows, slot, ctx->stream));
     HIP_TRY(ctx, surrogate_adam(sg, lr_t, ctx->stream));
-    if (losses) {
-      HIP_TRY(ctx, hipMemcpyAsync(part.data(), sg.loss, parts * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
+    if (losses && (slot == slots - 1 || step == steps - 1)) {
+      HIP_TRY(ctx, hipMemcpyAsync(part.data(), sg.loss, (size_t)(slot + 1) * parts * sizeof(float), hipMemcpyDeviceToHost,
+                                  ctx->stream));
       HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-      double t = 0;
-      for (float v : part) t += v;
-      losses[step] = (float)t;
+      for (int q = 0; q <= slot; ++q) {
+        double t = 0;
+        for (int i = 0; i < parts; ++i) t += part[(size_t)q * parts + i];
+        losses[step - slot + q] = (float)t;
+      }
     }
   }
   HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));

@@ -1,7 +1,8 @@
-// MLP surrogate kernels: bf16 matrix-core products with FP32 accumulation, Fourier features, SiLU,
-// loss, bias gradients and Adam, plus the batch gather of training data and table prediction.
+// MLP surrogate kernels: a batch's forward and backward pass (bf16 matrix-core products with FP32 accumulation, Fourier
+// features, SiLU, loss), weight and bias gradients, Adam, and table prediction.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 
@@ -43,50 +44,6 @@ __host__ __device__ inline uint64_t splitmix64(uint64_t x) {
   return x ^ (x >> 31);
 }
 
-// One wavefront computes a 32 x 32 tile of C with v_mfma_f32_32x32x8bf16_1k.  Operand layout of that
-// instruction: lane l supplies A(l % 32, 4 (l / 32) + i) and B(4 (l / 32) + i, l % 32), i = 0..3;
-// accumulator element e of lane l is C(8 (e / 4) + 4 (l / 32) + e % 4, l % 32).
-// Split K: workgroup z covers k in [z kc, min(K, (z + 1) kc)) and writes its partial product to
-// C + z * split_stride (the caller sums the partials in a fixed order).
-__global__ void __launch_bounds__(64) gemm_kernel(const uint16_t* __restrict__ A, long long sam, long long sak,
-                                                  const uint16_t* __restrict__ B, long long sbk, long long sbn,
-                                                  float* __restrict__ C, int ldc, const float* __restrict__ bias,
-                                                  int act, uint16_t* __restrict__ outb, int M, int N, int K, int kc,
-                                                  long long split_stride) {
-  const int lane = threadIdx.x;
-  const int m0 = blockIdx.y * 32, n0 = blockIdx.x * 32;
-  const int r = lane & 31, kq = (lane >> 5) * 4;
-  const int am = m0 + r, bn = n0 + r;
-  const bool arow = am < M, bcol = bn < N;
-  const int kbeg = blockIdx.z * kc, kend = min(K, kbeg + kc);
-  C += blockIdx.z * split_stride;
-  float16_t acc;
-#pragma unroll
-  for (int e = 0; e < 16; ++e) acc[e] = 0.f;
-  for (int k0 = kbeg; k0 < kend; k0 += 8) {
-    short4_t va, vb;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      int k = k0 + kq + i;
-      bool kin = k < kend;
-      va[i] = (short)((arow && kin) ? A[am * sam + k * sak] : 0);
-      vb[i] = (short)((bcol && kin) ? B[k * sbk + bn * sbn] : 0);
-    }
-    acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(va, vb, acc, 0, 0, 0);
-  }
-  const int n = n0 + r;
-#pragma unroll
-  for (int e = 0; e < 16; ++e) {
-    int m = m0 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
-    if (m < M && n < N) {
-      float v = acc[e] + (bias ? bias[n] : 0.f);
-      long long o = (long long)m * ldc + n;
-      if (C) C[o] = v;
-      if (outb) outb[o] = f2bf(act == 1 ? silu(v) : v);
-    }
-  }
-}
-
 // The 17 Fourier features of one input x: x, then sin / cos (2^b pi x) for b = 0..7 (bf16).
 __device__ inline void encode_value(float v, uint16_t* out) {
   out[0] = f2bf(v);
@@ -100,19 +57,7 @@ __device__ inline void encode_value(float v, uint16_t* out) {
   }
 }
 
-// Features of one input row: the 17 features of each of the 10 inputs, zero padded to 192.
-__device__ inline void encode_row(const float* x, uint16_t* out) {
-  for (int i = 0; i < kMlpIn; ++i) encode_value(x[i], out + kMlpBands * i);
-  for (int f = kMlpBands * kMlpIn; f < kMlpFeat; ++f) out[f] = 0;
-}
-
-__global__ void encode_rows_kernel(const float* __restrict__ in, uint16_t* __restrict__ X, int rows) {
-  int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= rows) return;
-  encode_row(in + (long long)r * kMlpIn, X + (long long)r * kMlpFeat);
-}
-
-__device__ inline void entry_coords(const DevParams& P, long long entry, float* x) {
+__device__ inline void entry_coords(const GridShape& P, long long entry, float* x) {
   const int NH = P.nS[0], NE = P.nS[1], NL = P.nS[2], NA = P.nS[3];
   int ia = (int)(entry % NA);
   long long q = entry / NA;
@@ -124,23 +69,6 @@ __device__ inline void entry_coords(const DevParams& P, long long entry, float* 
   x[1] = (float)ie / (NE - 1);
   x[2] = (float)is / (NL - 1);
   x[3] = (float)ia / (NA - 1);
-}
-
-__global__ void gather_kernel(const DevParams P, const AtmosphereCode* __restrict__ codes, int natm,
-                              const float* __restrict__ targets, uint64_t seed, int step, int rows,
-                              uint16_t* __restrict__ X, float* __restrict__ T) {
-  int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= rows) return;
-  const long long entries = (long long)P.nS[0] * P.nS[1] * P.nS[2] * P.nS[3];
-  uint64_t h = splitmix64(seed ^ splitmix64(((uint64_t)step << 32) | (uint64_t)r));
-  int atm = (int)(h % (uint64_t)natm);
-  long long entry = (long long)((h >> 16) % (uint64_t)entries);
-  float x[kMlpIn];
-  entry_coords(P, entry, x);
-  for (int i = 0; i < 6; ++i) x[4 + i] = codes[atm].v[i];
-  encode_row(x, X + (long long)r * kMlpFeat);
-  const float* t = targets + ((long long)atm * entries + entry) * kMlpUsed;
-  for (int o = 0; o < kMlpOut; ++o) T[(long long)r * kMlpOut + o] = o < kMlpUsed ? t[o] : 0.f;
 }
 
 struct SumTables {
@@ -156,40 +84,6 @@ __global__ void targets_kernel(const SumTables sums, long long entries, float* _
     t[e * kMlpUsed + 3 * k + 1] = logf(fmaxf(v.y, 0.f) + kMlpEps) + kMlpShift;
     t[e * kMlpUsed + 3 * k + 2] = logf(fmaxf(v.z, 0.f) + kMlpEps) + kMlpShift;
   }
-}
-
-// dY = mask (Y - T) / rows (FP32 and bf16), loss partials 0.5 sum d^2 / rows per block.
-__global__ void __launch_bounds__(kEw) loss_kernel(const float* __restrict__ Y, const float* __restrict__ T, int rows,
-                                                   float* __restrict__ dYf, uint16_t* __restrict__ dY,
-                                                   float* __restrict__ partial) {
-  __shared__ float red[kEw / 64];
-  long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  float l = 0.f;
-  if (i < (long long)rows * kMlpOut) {
-    int o = (int)(i % kMlpOut);
-    float d = o < kMlpUsed ? (Y[i] - T[i]) : 0.f;
-    l = 0.5f * d * d / rows;
-    float g = d / rows;
-    dYf[i] = g;
-    dY[i] = f2bf(g);
-  }
-  for (int off = 32; off > 0; off >>= 1) l += __shfl_down(l, off, 64);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = l;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    float s = 0.f;
-    for (int w = 0; w < kEw / 64; ++w) s += red[w];
-    partial[blockIdx.x] = s;
-  }
-}
-
-__global__ void dsilu_kernel(const float* __restrict__ dA, const float* __restrict__ Z, long long n,
-                             float* __restrict__ dZf, uint16_t* __restrict__ dZ) {
-  long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  float g = dA[i] * dsilu(Z[i]);
-  dZf[i] = g;
-  dZ[i] = f2bf(g);
 }
 
 // out[c] = mean over rows of T[row][c] for the kMlpUsed target columns (row stride kMlpUsed), FP64
@@ -210,41 +104,354 @@ __global__ void __launch_bounds__(kEw) target_mean_kernel(const float* __restric
   }
 }
 
-// out[c] = sum over rows of G[row][c] (one workgroup per column, fixed summation order).
-__global__ void __launch_bounds__(kEw) colsum_kernel(const float* __restrict__ G, int rows, int cols,
-                                                     float* __restrict__ out) {
-  __shared__ float red[kEw / 64];
-  int c = blockIdx.x;
-  float s = 0.f;
-  for (int r = threadIdx.x; r < rows; r += blockDim.x) s += G[(long long)r * cols + c];
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    float t = 0.f;
-    for (int w = 0; w < kEw / 64; ++w) t += red[w];
-    out[c] = t;
-  }
+// ---- one pass over a batch: forward, loss and backward --------------------------------------------
+// Every product runs on v_mfma_f32_32x32x8bf16_1k, K in ascending steps of 8.  Operand layout of that instruction: lane l
+// supplies A(l % 32, 4 (l / 32) + i) and B(4 (l / 32) + i, l % 32), i = 0..3; accumulator element e of lane l is
+// C(8 (e / 4) + 4 (l / 32) + e % 4, l % 32).  Operands that come from memory lie there as "fragments": for each tile of 32
+// and step of 8 the 64 lanes' 4 values side by side (8 bytes per lane, one coalesced read per step).  What a
+// lane's accumulator holds of 32 rows, rows 8 g + 4 h + i of one column, is its fragment of the products that sum over
+// the rows (the weight gradients), for steps g = 0..3: it is written as it stands.
+constexpr int kRows = 32;  // rows of the batch per workgroup
+constexpr int kFragWaves = 4;
+
+// Weight fragments in units of one step of one tile (256 values): forward layers (B operand W(k, n)), then the backward
+// products dA = dZ W^T of layers 2, 3 and 4 (B operand W(n, k)).
+struct FragLayout {
+  static constexpr int f1 = 0, f2 = f1 + 4 * kMlpFeat / 8, f3 = f2 + 4 * kMlpHidden / 8, f4 = f3 + 4 * kMlpHidden / 8;
+  static constexpr int b2 = f4 + kMlpHidden / 8, b3 = b2 + 4 * kMlpHidden / 8, b4 = b3 + 4 * kMlpHidden / 8;
+  static constexpr int total = b4 + 4 * kMlpOut / 8;
+};
+static_assert(FragLayout::total * 256 == kMlpFragments, "size of the weight fragments");
+
+__device__ __forceinline__ int frag_index(int tile, int steps, int k, int n) {
+  return (tile * steps + k / 8) * 256 + ((n & 31) + 32 * ((k & 7) >> 2)) * 4 + (k & 3);
 }
 
-__global__ void adam_kernel(float* __restrict__ theta, const float* __restrict__ g, float* __restrict__ m,
-                            float* __restrict__ v, long long n, float lr, float b1, float b2, float eps, float c1,
-                            float c2, uint16_t* __restrict__ theta_bf) {
+// The bf16 copies of weight i (a row-major one and its fragments); biases have none.
+__device__ __forceinline__ void store_bf16(size_t i, uint16_t v, uint16_t* __restrict__ bf, uint16_t* __restrict__ frag) {
+  bf[i] = v;
+  const size_t off[4] = {MlpLayout::W1, MlpLayout::W2, MlpLayout::W3, MlpLayout::W4};
+  const int kin[4] = {kMlpFeat, kMlpHidden, kMlpHidden, kMlpHidden}, out[4] = {kMlpHidden, kMlpHidden, kMlpHidden, kMlpOut};
+  const int fwd[4] = {FragLayout::f1, FragLayout::f2, FragLayout::f3, FragLayout::f4};
+  const int bwd[4] = {-1, FragLayout::b2, FragLayout::b3, FragLayout::b4};
+#pragma unroll
+  for (int l = 0; l < 4; ++l)
+    if (i >= off[l] && i < off[l] + (size_t)kin[l] * out[l]) {
+      const int k = (int)(i - off[l]) / out[l], n = (int)(i - off[l]) % out[l];
+      frag[fwd[l] * 256 + frag_index(n / 32, kin[l] / 8, k, n)] = v;
+      if (bwd[l] >= 0) frag[bwd[l] * 256 + frag_index(k / 32, out[l] / 8, n, k)] = v;
+    }
+}
+
+// A tile's weight fragments in registers, and its product over STEPS steps with the rows' values in LDS (row pitch in
+// values).
+template <int STEPS>
+struct Frags {
+  short4_t v[STEPS];
+};
+
+template <int STEPS>
+__device__ __forceinline__ Frags<STEPS> load_frags(const uint16_t* __restrict__ frag, int lane) {
+  Frags<STEPS> f;
+#pragma unroll
+  for (int k = 0; k < STEPS; ++k) f.v[k] = *(const short4_t*)(frag + (k * 64 + lane) * 4);
+  return f;
+}
+
+template <int STEPS>
+__device__ __forceinline__ float16_t tile_product(const uint16_t* a, int pitch, const Frags<STEPS>& w, int lane) {
+  float16_t acc;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) acc[e] = 0.f;
+  const uint16_t* row = a + (lane & 31) * pitch + 4 * (lane >> 5);
+#pragma unroll
+  for (int k = 0; k < STEPS; ++k)
+    acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(*(const short4_t*)(row + 8 * k), w.v[k], acc, 0, 0, 0);
+  return acc;
+}
+
+// Four rows of a lane's column: into the LDS tile of the next product and the fragments of the weight gradient.
+__device__ __forceinline__ void store_rows(const float (&v)[4], uint16_t* lds, int pitch, uint16_t* __restrict__ frag) {
+  uint16_t b[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    b[i] = f2bf(v[i]);
+    if (lds) lds[i * pitch] = b[i];
+  }
+  *(uint2*)frag = make_uint2(b[0] | (uint32_t)b[1] << 16, b[2] | (uint32_t)b[3] << 16);
+}
+
+// Row pitches (values) of the LDS tiles: 2 dwords modulo the 32 banks, so that 16 rows' 8-byte reads do not collide.
+constexpr int kPitchX = kMlpFeat + 4, kPitchH = kMlpHidden + 4, kPitchY = kMlpOut + 4;
+
+// Forward, loss and backward of 32 rows by one workgroup of 4 wavefronts, wavefront w computing columns 32 w .. 32 w + 31 of
+// every hidden layer: activations stay in LDS (bf16, as the products take them) and pre-activations in
+// registers.  The rows are given (in, with targets T) or drawn from the training data.  One launch for what had
+// been gather, four products, loss, three products, three activation derivatives, each through memory.
+__global__ void __launch_bounds__(64 * kFragWaves) pass_kernel(const PassSource src, int rows, const uint16_t* __restrict__ wfrag,
+                                                               const float* __restrict__ theta, const PassOutputs out) {
+  __shared__ __align__(16) uint16_t s_x[kRows * kPitchX];
+  __shared__ __align__(16) uint16_t s_a[2][kRows * kPitchH];
+  __shared__ __align__(16) uint16_t s_dy[kRows * kPitchY];
+  __shared__ float s_y[kRows][kMlpOut], s_t[kRows][kMlpOut], s_in[kRows][kMlpIn];
+  __shared__ float s_red[kFragWaves];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int h = lane >> 5, col = 32 * wave + (lane & 31);
+  const int row0 = blockIdx.x * kRows, steps = gridDim.x * (kRows / 8), step0 = blockIdx.x * (kRows / 8);
+  // the weights of a layer are requested a layer (the first two: the whole input stage) before they are needed: a
+  // workgroup has its CU to itself, so nothing else hides their latency, and registers are free
+  const auto w1 = load_frags<kMlpFeat / 8>(wfrag + (FragLayout::f1 + wave * (kMlpFeat / 8)) * 256, lane);
+  const auto w2 = load_frags<kMlpHidden / 8>(wfrag + (FragLayout::f2 + wave * (kMlpHidden / 8)) * 256, lane);
+  const float bias1 = theta[MlpLayout::b1 + col], bias2 = theta[MlpLayout::b2 + col], bias3 = theta[MlpLayout::b3 + col];
+  // inputs and targets
+  if (tid < kRows) {
+    const int r = row0 + tid;
+    float x[kMlpIn] = {};
+    if (r < rows) {
+      if (src.in) {
+        for (int i = 0; i < kMlpIn; ++i) x[i] = src.in[(long long)r * kMlpIn + i];
+      } else {
+        const long long entries = (long long)src.P.nS[0] * src.P.nS[1] * src.P.nS[2] * src.P.nS[3];
+        const uint64_t hash = splitmix64(src.seed ^ splitmix64(((uint64_t)src.step << 32) | (uint64_t)r));
+        const int atm = (int)(hash % (uint64_t)src.natm);
+        const long long entry = (long long)((hash >> 16) % (uint64_t)entries);
+        entry_coords(src.P, entry, x);
+        for (int i = 0; i < 6; ++i) x[4 + i] = src.codes[atm].v[i];
+        const float* t = src.targets + ((long long)atm * entries + entry) * kMlpUsed;
+        for (int o = 0; o < kMlpOut; ++o) s_t[tid][o] = o < kMlpUsed ? t[o] : 0.f;
+      }
+    }
+    for (int i = 0; i < kMlpIn; ++i) s_in[tid][i] = x[i];
+  }
+  if (src.T)
+    for (int i = tid; i < kRows * kMlpOut; i += blockDim.x)
+      s_t[i / kMlpOut][i % kMlpOut] = row0 + i / kMlpOut < rows ? src.T[(long long)row0 * kMlpOut + i] : 0.f;
+  __syncthreads();
+  // features: x, then sin / cos of 2^b pi x, zero padded; rows past the batch are zero
+  for (int i = tid; i < kRows * kMlpIn * 8; i += blockDim.x) {
+    const int r = i / (kMlpIn * 8), q = i - r * (kMlpIn * 8), in = q >> 3, band = q & 7;
+    uint16_t* f = s_x + r * kPitchX + kMlpBands * in;
+    const float v = s_in[r][in];
+    float sn, cs;
+    sincosf(3.14159265358979f * v * (float)(1 << band), &sn, &cs);
+    const bool valid = row0 + r < rows;
+    if (band == 0) f[0] = valid ? f2bf(v) : 0;
+    f[1 + 2 * band] = valid ? f2bf(sn) : 0;
+    f[2 + 2 * band] = valid ? f2bf(cs) : 0;
+  }
+  for (int i = tid; i < kRows * (kMlpFeat - kMlpBands * kMlpIn); i += blockDim.x)
+    s_x[(i / (kMlpFeat - kMlpBands * kMlpIn)) * kPitchX + kMlpBands * kMlpIn + i % (kMlpFeat - kMlpBands * kMlpIn)] = 0;
+  __syncthreads();
+  if (out.dZ[0])  // the features' fragments for the first layer's weight gradient
+    for (int i = tid; i < (kMlpFeat / 32) * (kRows / 8) * 64; i += blockDim.x) {
+      const int tile = i / (4 * 64), g = (i / 64) & 3, l = i & 63;
+      const uint16_t* v = s_x + (8 * g + 4 * (l >> 5)) * kPitchX + 32 * tile + (l & 31);
+      *(uint2*)(out.X + ((size_t)(tile * steps + step0 + g) * 64 + l) * 4) =
+          make_uint2(v[0] | (uint32_t)v[kPitchX] << 16, v[2 * kPitchX] | (uint32_t)v[3 * kPitchX] << 16);
+    }
+  // hidden layers: Z = A W + b, A = SiLU(Z)
+  float z[3][16];
+  auto activate = [&](int l, const float16_t acc, float b) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      float a[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        z[l][4 * g + i] = acc[4 * g + i] + b;
+        a[i] = silu(z[l][4 * g + i]);
+      }
+      store_rows(a, s_a[l & 1] + (8 * g + 4 * h) * kPitchH + col, kPitchH,
+                 out.A[l] + ((size_t)(wave * steps + step0 + g) * 64 + lane) * 4);
+    }
+    __syncthreads();
+  };
+  activate(0, tile_product(s_x, kPitchX, w1, lane), bias1);
+  const auto w3 = load_frags<kMlpHidden / 8>(wfrag + (FragLayout::f3 + wave * (kMlpHidden / 8)) * 256, lane);
+  activate(1, tile_product(s_a[0], kPitchH, w2, lane), bias2);
+  const auto w4 = load_frags<kMlpHidden / 8>(wfrag + FragLayout::f4 * 256, lane);
+  activate(2, tile_product(s_a[1], kPitchH, w3, lane), bias3);
+  const auto v4 = load_frags<kMlpOut / 8>(wfrag + (FragLayout::b4 + wave * (kMlpOut / 8)) * 256, lane);
+  const auto v3 = load_frags<kMlpHidden / 8>(wfrag + (FragLayout::b3 + wave * (kMlpHidden / 8)) * 256, lane);
+  // outputs (one wavefront: 16 columns)
+  if (wave == 0) {
+    const float16_t acc = tile_product(s_a[0], kPitchH, w4, lane);
+    if (col < kMlpOut) {
+      const float b = theta[MlpLayout::b4 + col];
+#pragma unroll
+      for (int e = 0; e < 16; ++e) s_y[(e >> 2) * 8 + 4 * h + (e & 3)][col] = acc[e] + b;
+    }
+  }
+  __syncthreads();
+  if (out.Y)
+    for (int i = tid; i < kRows * kMlpOut; i += blockDim.x)
+      if (row0 + i / kMlpOut < rows) out.Y[(long long)row0 * kMlpOut + i] = s_y[i / kMlpOut][i % kMlpOut];
+  if (!out.dZ[0]) return;
+  // dY = mask (Y - T) / rows; loss partials 0.5 sum d^2 / rows per 256 values (16 rows)
+  for (int blk = 0; blk < kRows * kMlpOut / kEw; ++blk) {
+    const int i = blk * kEw + tid, r = i / kMlpOut, o = i % kMlpOut;
+    const bool valid = row0 + r < rows;
+    float l = 0.f, g = 0.f;
+    if (valid) {
+      const float d = o < kMlpUsed ? (s_y[r][o] - s_t[r][o]) : 0.f;
+      l = 0.5f * d * d / rows;
+      g = d / rows;
+      out.dYf[(size_t)o * (8 * steps) + row0 + r] = g;
+    }
+    s_dy[r * kPitchY + o] = f2bf(g);
+    for (int off = 32; off > 0; off >>= 1) l += __shfl_down(l, off, 64);
+    if (lane == 0) s_red[wave] = l;
+    __syncthreads();
+    if (tid == 0 && row0 + blk * (kEw / kMlpOut) < rows) {
+      float s = 0.f;
+      for (int w = 0; w < kEw / 64; ++w) s += s_red[w];
+      out.loss[row0 / (kEw / kMlpOut) + blk] = s;
+    }
+    __syncthreads();
+  }
+  {  // dY's fragments (columns 16..31 zero)
+    const int g = wave, l = lane;
+    const uint16_t* v = s_dy + (8 * g + 4 * (l >> 5)) * kPitchY + (l & 15);
+    *(uint2*)(out.dY + ((size_t)(step0 + g) * 64 + l) * 4) =
+        (l & 31) < kMlpOut ? make_uint2(v[0] | (uint32_t)v[kPitchY] << 16, v[2 * kPitchY] | (uint32_t)v[3 * kPitchY] << 16)
+                           : make_uint2(0, 0);
+  }
+  // hidden layers backward: dA = dZ_next W^T, dZ = dA SiLU'(Z)
+  auto backward = [&](int l, const float16_t acc) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      float d[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        d[i] = acc[4 * g + i] * dsilu(z[l][4 * g + i]);
+        if (row0 + 8 * g + 4 * h + i >= rows) d[i] = 0.f;
+      }
+      *(float4*)(out.dZf[l] + (size_t)col * (8 * steps) + row0 + 8 * g + 4 * h) = make_float4(d[0], d[1], d[2], d[3]);
+      store_rows(d, l > 0 ? s_a[l & 1] + (8 * g + 4 * h) * kPitchH + col : nullptr, kPitchH,
+                 out.dZ[l] + ((size_t)(wave * steps + step0 + g) * 64 + lane) * 4);
+    }
+    __syncthreads();
+  };
+  backward(2, tile_product(s_dy, kPitchY, v4, lane));
+  const auto v2 = load_frags<kMlpHidden / 8>(wfrag + (FragLayout::b2 + wave * (kMlpHidden / 8)) * 256, lane);
+  backward(1, tile_product(s_a[0], kPitchH, v3, lane));
+  backward(0, tile_product(s_a[1], kPitchH, v2, lane));
+}
+
+// Weight gradients: 60 tiles (24 of W1, 16 of W2 and of W3, 4 of W4) times the splits of the rows, one wavefront each:
+// split z sums rows [z kc, min(rows, (z + 1) kc)) into partial + z MlpLayout::total (the sum over the splits follows in a
+// fixed order).  The first workgroups sum the bias gradients, a column (of the transposed FP32 dZ and dY) each:
+// thread t adds rows t, t + 256, ..., then the wavefronts' lanes and the wavefronts in order.
+constexpr int kGradTiles = 60, kBiases = kMlpOut + 3 * kMlpHidden;
+
+__global__ void __launch_bounds__(256) weight_gradient_kernel(const PassOutputs in, int rows, int steps, int kc, int splits,
+                                                              float* __restrict__ partial, float* __restrict__ grad) {
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if ((int)blockIdx.x < kBiases) {
+    __shared__ float s_red[4];
+    const int b = (int)blockIdx.x - kMlpOut, l = b / kMlpHidden;
+    const float* G = b < 0 ? in.dYf + (size_t)blockIdx.x * (8 * steps) : in.dZf[l] + (size_t)(b % kMlpHidden) * (8 * steps);
+    float s = 0.f;
+#pragma unroll 8
+    for (int r = threadIdx.x; r < rows; r += 256) s += G[r];
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
+    if (lane == 0) s_red[wave] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      float t = 0.f;
+      for (int w = 0; w < 4; ++w) t += s_red[w];
+      const size_t bias = b < 0 ? MlpLayout::b4 + blockIdx.x
+                                : (l == 0 ? MlpLayout::b1 : l == 1 ? MlpLayout::b2 : MlpLayout::b3) + (size_t)(b % kMlpHidden);
+      grad[bias] = t;
+    }
+    return;
+  }
+  const int item = (blockIdx.x - kBiases) * 4 + wave;
+  if (item >= kGradTiles * splits) return;
+  const int z = item / kGradTiles;
+  int t = item - z * kGradTiles, l, mt, nt;
+  if (t < 24) {
+    l = 0;
+    mt = t / 4;
+    nt = t & 3;
+  } else if (t < 56) {
+    l = 1 + (t - 24) / 16;
+    mt = ((t - 24) & 15) / 4;
+    nt = t & 3;
+  } else {
+    l = 3;
+    mt = t - 56;
+    nt = 0;
+  }
+  const uint16_t* a = l == 0 ? in.X : in.A[l - 1];
+  const uint16_t* b = l == 3 ? in.dY : in.dZ[l];
+  const int N = l == 3 ? kMlpOut : kMlpHidden;
+  const size_t off = l == 0 ? MlpLayout::W1 : l == 1 ? MlpLayout::W2 : l == 2 ? MlpLayout::W3 : MlpLayout::W4;
+  const int k0 = z * kc / 8, k1 = (min(rows, (z + 1) * kc) + 7) / 8;
+  const short4_t* fa = (const short4_t*)a + ((size_t)mt * steps + k0) * 64 + lane;
+  const short4_t* fb = (const short4_t*)b + ((size_t)nt * steps + k0) * 64 + lane;
+  float16_t acc;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) acc[e] = 0.f;
+  int k = k0;
+  for (; k + 8 <= k1; k += 8, fa += 8 * 64, fb += 8 * 64) {
+    short4_t va[8], vb[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      va[q] = fa[q * 64];
+      vb[q] = fb[q * 64];
+    }
+#pragma unroll
+    for (int q = 0; q < 8; ++q) acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(va[q], vb[q], acc, 0, 0, 0);
+  }
+  for (; k < k1; ++k, fa += 64, fb += 64) acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(*fa, *fb, acc, 0, 0, 0);
+  const int n = 32 * nt + (lane & 31);
+  float* c = partial + (size_t)z * MlpLayout::total + off + (size_t)(32 * mt + 4 * (lane >> 5)) * N + n;
+  if (n < N)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) c[(size_t)((e >> 2) * 8 + (e & 3)) * N] = acc[e];
+}
+
+__device__ __forceinline__ bool is_bias(long long i) {
+  return (i >= (long long)MlpLayout::b1 && i < (long long)MlpLayout::W2) ||
+         (i >= (long long)MlpLayout::b2 && i < (long long)MlpLayout::W3) ||
+         (i >= (long long)MlpLayout::b3 && i < (long long)MlpLayout::W4) || i >= (long long)MlpLayout::b4;
+}
+
+// The gradient of parameter i: a bias's own, a weight's sum over the splits in order.
+__device__ __forceinline__ float gradient(const float* __restrict__ partial, int splits, const float* __restrict__ grad,
+                                          long long i) {
+  if (is_bias(i)) return grad[i];
+  float s = 0.f;
+#pragma unroll 8
+  for (int z = 0; z < splits; ++z) s += partial[(size_t)z * MlpLayout::total + i];
+  return s;
+}
+
+__global__ void gradient_kernel(const float* __restrict__ partial, int splits, float* __restrict__ grad, long long n) {
+  long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n && !is_bias(i)) grad[i] = gradient(partial, splits, grad, i);
+}
+
+__global__ void adam_kernel(float* __restrict__ theta, const float* __restrict__ partial, int splits,
+                            const float* __restrict__ g, float* __restrict__ m, float* __restrict__ v, long long n, float lr,
+                            float b1, float b2, float eps, float c1, float c2, uint16_t* __restrict__ theta_bf,
+                            uint16_t* __restrict__ wfrag) {
   long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  float gi = g[i];
+  float gi = gradient(partial, splits, g, i);
   float mi = b1 * m[i] + (1.f - b1) * gi;
   float vi = b2 * v[i] + (1.f - b2) * gi * gi;
   m[i] = mi;
   v[i] = vi;
   float t = theta[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
   theta[i] = t;
-  theta_bf[i] = f2bf(t);
+  store_bf16((size_t)i, f2bf(t), theta_bf, wfrag);
 }
 
-__global__ void to_bf16_kernel(const float* __restrict__ in, uint16_t* __restrict__ out, long long n) {
+__global__ void to_bf16_kernel(const float* __restrict__ in, uint16_t* __restrict__ out, uint16_t* __restrict__ wfrag,
+                               long long n) {
   long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) out[i] = f2bf(in[i]);
+  if (i < n) store_bf16((size_t)i, f2bf(in[i]), out, wfrag);
 }
 
 // ---- fused inference over a scatter grid ---------------------------------------------------------
@@ -454,15 +661,6 @@ __global__ void __launch_bounds__(64 * kFusedWaves, 2) fused_predict_kernel(
   }
 }
 
-// C[i] = sum over z of partial[z][i], z in order.
-__global__ void split_sum_kernel(const float* __restrict__ partial, int splits, long long n, float* __restrict__ C) {
-  long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  float s = 0.f;
-  for (int z = 0; z < splits; ++z) s += partial[z * n + i];
-  C[i] = s;
-}
-
 inline unsigned ew_blocks(long long n) { return (unsigned)((n + kEw - 1) / kEw); }
 
 template <typename T>
@@ -471,34 +669,6 @@ hipError_t dalloc(T** p, size_t count) {
 }
 
 }  // namespace
-
-hipError_t mfma_gemm(const uint16_t* A, long long sam, long long sak, const uint16_t* B, long long sbk,
-                     long long sbn, float* C, int ldc, const float* bias, int act, uint16_t* out_bf16, int M, int N,
-                     int K, hipStream_t stream) {
-  dim3 grid((unsigned)((N + 31) / 32), (unsigned)((M + 31) / 32));
-  hipLaunchKernelGGL(gemm_kernel, grid, dim3(64), 0, stream, A, sam, sak, B, sbk, sbn, C, ldc, bias, act, out_bf16, M,
-                     N, K, K, 0LL);
-  return hipGetLastError();
-}
-
-// Weight gradients (M x N small, K = rows large): K split over kMaxSplits workgroups per tile, partial
-// products in `partial` (kMaxSplits x M x N floats), then summed in split order: deterministic.
-hipError_t mfma_gemm_split_k(const uint16_t* A, long long sam, long long sak, const uint16_t* B, long long sbk,
-                             long long sbn, float* C, int M, int N, int K, float* partial, hipStream_t stream) {
-  int kc = (K + kMaxSplits - 1) / kMaxSplits;
-  kc = (kc + 7) / 8 * 8;
-  if (kc < 64) kc = 64;
-  const int splits = (K + kc - 1) / kc;
-  dim3 grid((unsigned)((N + 31) / 32), (unsigned)((M + 31) / 32), (unsigned)splits);
-  hipLaunchKernelGGL(gemm_kernel, grid, dim3(64), 0, stream, A, sam, sak, B, sbk, sbn, partial, N, nullptr, 0,
-                     nullptr, M, N, K, kc, (long long)M * N);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  const long long n = (long long)M * N;
-  hipLaunchKernelGGL(split_sum_kernel, dim3((unsigned)((n + kEw - 1) / kEw)), dim3(kEw), 0, stream, partial, splits, n,
-                     C);
-  return hipGetLastError();
-}
 
 #define SG_TRY(expr)                         \
   do {                                       \
@@ -514,26 +684,28 @@ hipError_t surrogate_alloc(Surrogate& s, int batch) {
   SG_TRY(dalloc(&s.adam_m, n));
   SG_TRY(dalloc(&s.adam_v, n));
   SG_TRY(dalloc(&s.grad, n));
-  SG_TRY(dalloc(&s.X, (size_t)batch * kMlpFeat));
+  SG_TRY(dalloc(&s.wfrag, (size_t)kMlpFragments));
+  const size_t padded = (size_t)(batch + kRows - 1) / kRows * kRows;
+  SG_TRY(dalloc(&s.X, padded * kMlpFeat));
   for (int l = 0; l < 3; ++l) {
-    SG_TRY(dalloc(&s.Z[l], (size_t)batch * kMlpHidden));
-    SG_TRY(dalloc(&s.A[l], (size_t)batch * kMlpHidden));
+    SG_TRY(dalloc(&s.A[l], padded * kMlpHidden));
+    SG_TRY(dalloc(&s.dZ[l], padded * kMlpHidden));
+    SG_TRY(dalloc(&s.dZf[l], padded * kMlpHidden));
   }
   SG_TRY(dalloc(&s.Y, (size_t)batch * kMlpOut));
   SG_TRY(dalloc(&s.T, (size_t)batch * kMlpOut));
-  SG_TRY(dalloc(&s.dY, (size_t)batch * kMlpOut));
-  SG_TRY(dalloc(&s.dA, (size_t)batch * kMlpHidden));
-  SG_TRY(dalloc(&s.dZf, (size_t)batch * kMlpHidden));
-  SG_TRY(dalloc(&s.dZ, (size_t)batch * kMlpHidden));
-  SG_TRY(dalloc(&s.loss, (size_t)(batch * kMlpOut) / kEw + 2));
-  SG_TRY(dalloc(&s.partial, (size_t)kMaxSplits * kMlpFeat * kMlpHidden));
+  SG_TRY(dalloc(&s.dY, padded * 32));
+  SG_TRY(dalloc(&s.dYf, padded * kMlpOut));
+  SG_TRY(dalloc(&s.loss, (size_t)surrogate_loss_parts(batch) * surrogate_loss_slots(batch)));
+  SG_TRY(dalloc(&s.partial, (size_t)kMaxSplits * MlpLayout::total));
   s.batch_capacity = batch;
   return hipSuccess;
 }
 
 void surrogate_free(Surrogate& s) {
-  void* ptrs[] = {s.theta, s.theta_bf, s.adam_m, s.adam_v, s.grad, s.X,  s.Z[0], s.Z[1], s.Z[2], s.A[0], s.A[1],
-                  s.A[2],  s.Y,        s.T,      s.dY,     s.dA,   s.dZf, s.dZ,   s.loss, s.ztab, s.partial};
+  void* ptrs[] = {s.theta, s.theta_bf, s.wfrag, s.adam_m, s.adam_v, s.grad,   s.X,      s.A[0],   s.A[1], s.A[2], s.dZ[0],
+                  s.dZ[1], s.dZ[2],    s.dZf[0], s.dZf[1], s.dZf[2], s.Y,    s.T,      s.dY,     s.dYf,  s.loss, s.ztab,
+                  s.partial};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   s = Surrogate();
@@ -557,6 +729,7 @@ hipError_t surrogate_init(Surrogate& s, uint64_t seed, hipStream_t stream) {
   SG_TRY(hipMemcpyAsync(s.theta, h.data(), h.size() * sizeof(float), hipMemcpyHostToDevice, stream));
   SG_TRY(hipMemsetAsync(s.adam_m, 0, h.size() * sizeof(float), stream));
   SG_TRY(hipMemsetAsync(s.adam_v, 0, h.size() * sizeof(float), stream));
+  SG_TRY(hipMemsetAsync(s.wfrag, 0, kMlpFragments * sizeof(uint16_t), stream));  // columns past the outputs stay zero
   s.adam_step = 0;
   s.trained = false;
   SG_TRY(surrogate_sync_bf16(s, stream));
@@ -565,63 +738,62 @@ hipError_t surrogate_init(Surrogate& s, uint64_t seed, hipStream_t stream) {
 
 hipError_t surrogate_sync_bf16(Surrogate& s, hipStream_t stream) {
   long long n = (long long)MlpLayout::total;
-  hipLaunchKernelGGL(to_bf16_kernel, dim3(ew_blocks(n)), dim3(kEw), 0, stream, s.theta, s.theta_bf, n);
+  hipLaunchKernelGGL(to_bf16_kernel, dim3(ew_blocks(n)), dim3(kEw), 0, stream, s.theta, s.theta_bf, s.wfrag, n);
   return hipGetLastError();
 }
 
-hipError_t surrogate_encode_rows(Surrogate& s, const float* inputs_dev, int rows, hipStream_t stream) {
-  hipLaunchKernelGGL(encode_rows_kernel, dim3(ew_blocks(rows)), dim3(kEw), 0, stream, inputs_dev, s.X, rows);
-  return hipGetLastError();
-}
+int surrogate_loss_parts(int rows) { return (rows * kMlpOut + kEw - 1) / kEw; }
 
-hipError_t surrogate_forward(Surrogate& s, int rows, hipStream_t stream) {
-  const uint16_t* W[4] = {s.theta_bf + MlpLayout::W1, s.theta_bf + MlpLayout::W2, s.theta_bf + MlpLayout::W3,
-                          s.theta_bf + MlpLayout::W4};
-  const float* b[4] = {s.theta + MlpLayout::b1, s.theta + MlpLayout::b2, s.theta + MlpLayout::b3,
-                       s.theta + MlpLayout::b4};
-  // hidden layers: Z = A_prev W + b, A = SiLU(Z)
-  SG_TRY(mfma_gemm(s.X, kMlpFeat, 1, W[0], kMlpHidden, 1, s.Z[0], kMlpHidden, b[0], 1, s.A[0], rows, kMlpHidden,
-                   kMlpFeat, stream));
-  SG_TRY(mfma_gemm(s.A[0], kMlpHidden, 1, W[1], kMlpHidden, 1, s.Z[1], kMlpHidden, b[1], 1, s.A[1], rows, kMlpHidden,
-                   kMlpHidden, stream));
-  SG_TRY(mfma_gemm(s.A[1], kMlpHidden, 1, W[2], kMlpHidden, 1, s.Z[2], kMlpHidden, b[2], 1, s.A[2], rows, kMlpHidden,
-                   kMlpHidden, stream));
-  SG_TRY(mfma_gemm(s.A[2], kMlpHidden, 1, W[3], kMlpOut, 1, s.Y, kMlpOut, b[3], 0, nullptr, rows, kMlpOut, kMlpHidden,
-                   stream));
-  return hipSuccess;
-}
+int surrogate_loss_slots(int rows) { return std::max(1, std::min(256, (1 << 20) / surrogate_loss_parts(rows))); }
 
-hipError_t surrogate_backward(Surrogate& s, int rows, hipStream_t stream) {
-  const long long nout = (long long)rows * kMlpOut, nh = (long long)rows * kMlpHidden;
-  // dY = mask (Y - T) / rows; dYf reuses dZf's storage (rows x 16 <= rows x 128)
-  float* dYf = s.dZf;
-  hipLaunchKernelGGL(loss_kernel, dim3(ew_blocks(nout)), dim3(kEw), 0, stream, s.Y, s.T, rows, dYf, s.dY, s.loss);
-  SG_TRY(hipGetLastError());
-  // layer 4: gW4 = A3^T dY, gb4 = colsum(dY), dA3 = dY W4^T
-  SG_TRY(mfma_gemm_split_k(s.A[2], 1, kMlpHidden, s.dY, kMlpOut, 1, s.grad + MlpLayout::W4, kMlpHidden, kMlpOut,
-                           rows, s.partial, stream));
-  hipLaunchKernelGGL(colsum_kernel, dim3(kMlpOut), dim3(kEw), 0, stream, dYf, rows, kMlpOut, s.grad + MlpLayout::b4);
-  SG_TRY(hipGetLastError());
-  SG_TRY(mfma_gemm(s.dY, kMlpOut, 1, s.theta_bf + MlpLayout::W4, 1, kMlpOut, s.dA, kMlpHidden, nullptr, 0, nullptr,
-                   rows, kMlpHidden, kMlpOut, stream));
-  // hidden layers 3, 2, 1
-  const size_t Woff[3] = {MlpLayout::W1, MlpLayout::W2, MlpLayout::W3};
-  const size_t boff[3] = {MlpLayout::b1, MlpLayout::b2, MlpLayout::b3};
-  for (int l = 2; l >= 0; --l) {
-    hipLaunchKernelGGL(dsilu_kernel, dim3(ew_blocks(nh)), dim3(kEw), 0, stream, s.dA, s.Z[l], nh, s.dZf, s.dZ);
-    SG_TRY(hipGetLastError());
-    const uint16_t* prev = l == 0 ? s.X : s.A[l - 1];
-    const int kin = l == 0 ? kMlpFeat : kMlpHidden;
-    SG_TRY(mfma_gemm_split_k(prev, 1, kin, s.dZ, kMlpHidden, 1, s.grad + Woff[l], kin, kMlpHidden, rows, s.partial,
-                             stream));
-    hipLaunchKernelGGL(colsum_kernel, dim3(kMlpHidden), dim3(kEw), 0, stream, s.dZf, rows, kMlpHidden,
-                       s.grad + boff[l]);
-    SG_TRY(hipGetLastError());
-    if (l > 0)
-      SG_TRY(mfma_gemm(s.dZ, kMlpHidden, 1, s.theta_bf + Woff[l], 1, kMlpHidden, s.dA, kMlpHidden, nullptr, 0,
-                       nullptr, rows, kMlpHidden, kMlpHidden, stream));
+static hipError_t launch_pass(Surrogate& s, const PassSource& src, int rows, bool backward, int loss_slot, hipStream_t stream) {
+  PassOutputs o;
+  std::memset(&o, 0, sizeof(o));
+  o.X = s.X;
+  o.dY = s.dY;
+  o.dYf = s.dYf;
+  o.Y = src.in ? s.Y : nullptr;
+  o.loss = s.loss + (size_t)loss_slot * surrogate_loss_parts(rows);
+  for (int l = 0; l < 3; ++l) {
+    o.A[l] = s.A[l];
+    o.dZ[l] = backward ? s.dZ[l] : nullptr;
+    o.dZf[l] = s.dZf[l];
   }
-  return hipSuccess;
+  const unsigned blocks = (unsigned)((rows + kRows - 1) / kRows);
+  hipLaunchKernelGGL(pass_kernel, dim3(blocks), dim3(64 * kFragWaves), 0, stream, src, rows, s.wfrag, s.theta, o);
+  SG_TRY(hipGetLastError());
+  if (!backward) return hipSuccess;
+  int kc = (rows + kMaxSplits - 1) / kMaxSplits;
+  kc = std::max((kc + 7) / 8 * 8, 64);
+  s.splits = (rows + kc - 1) / kc;
+  hipLaunchKernelGGL(weight_gradient_kernel, dim3((unsigned)(kBiases + (kGradTiles * s.splits + 3) / 4)), dim3(256), 0,
+                     stream, o, rows, (int)blocks * (kRows / 8), kc, s.splits, s.partial, s.grad);
+  return hipGetLastError();
+}
+
+hipError_t surrogate_eval_rows(Surrogate& s, const float* inputs_dev, int rows, bool backward, hipStream_t stream) {
+  PassSource src;
+  std::memset(&src, 0, sizeof(src));
+  src.in = inputs_dev;
+  src.T = backward ? s.T : nullptr;
+  SG_TRY(launch_pass(s, src, rows, backward, 0, stream));
+  if (!backward) return hipSuccess;
+  const long long n = (long long)MlpLayout::total;
+  hipLaunchKernelGGL(gradient_kernel, dim3(ew_blocks(n)), dim3(kEw), 0, stream, s.partial, s.splits, s.grad, n);
+  return hipGetLastError();
+}
+
+hipError_t surrogate_train_rows(Surrogate& s, const DevParams& P, const AtmosphereCode* codes_dev, int natm,
+                                const float* targets_dev, uint64_t seed, int step, int rows, int loss_slot, hipStream_t stream) {
+  PassSource src;
+  std::memset(&src, 0, sizeof(src));
+  for (int d = 0; d < 4; ++d) src.P.nS[d] = P.nS[d];
+  src.codes = codes_dev;
+  src.natm = natm;
+  src.targets = targets_dev;
+  src.seed = seed;
+  src.step = step;
+  return launch_pass(s, src, rows, true, loss_slot, stream);
 }
 
 hipError_t surrogate_adam(Surrogate& s, float lr, hipStream_t stream) {
@@ -629,15 +801,8 @@ hipError_t surrogate_adam(Surrogate& s, float lr, hipStream_t stream) {
   s.adam_step += 1;
   float c1 = 1.f - std::pow(b1, (float)s.adam_step), c2 = 1.f - std::pow(b2, (float)s.adam_step);
   long long n = (long long)MlpLayout::total;
-  hipLaunchKernelGGL(adam_kernel, dim3(ew_blocks(n)), dim3(kEw), 0, stream, s.theta, s.grad, s.adam_m, s.adam_v, n, lr,
-                     b1, b2, eps, c1, c2, s.theta_bf);
-  return hipGetLastError();
-}
-
-hipError_t surrogate_gather_batch(Surrogate& s, const DevParams& P, const AtmosphereCode* codes_dev, int natm,
-                                  const float* targets_dev, uint64_t seed, int step, int rows, hipStream_t stream) {
-  hipLaunchKernelGGL(gather_kernel, dim3(ew_blocks(rows)), dim3(kEw), 0, stream, P, codes_dev, natm, targets_dev, seed,
-                     step, rows, s.X, s.T);
+  hipLaunchKernelGGL(adam_kernel, dim3(ew_blocks(n)), dim3(kEw), 0, stream, s.theta, s.partial, s.splits, s.grad, s.adam_m,
+                     s.adam_v, n, lr, b1, b2, eps, c1, c2, s.theta_bf, s.wfrag);
   return hipGetLastError();
 }
 

@@ -50,27 +50,62 @@ struct AtmosphereCode {
   float v[6];
 };
 
+// Weights of the matrix products as operand fragments (values): the four layers (outputs padded to a tile of 32 columns)
+// and the three backward products.
+constexpr size_t kMlpFragments = (4 * kMlpFeat / 8 + 8 * kMlpHidden / 8 + kMlpHidden / 8 + 8 * kMlpHidden / 8 + 4 * kMlpOut / 8) * 256;
+
+struct GridShape {
+  int nS[4];
+};
+
+// Where a pass takes its rows from: explicit inputs (in: rows x 10 values in [0, 1]; T: rows x 16 targets), or
+// entries drawn with a counter-based generator from `natm` atmospheres (targets[atm][entry][15]).
+struct PassSource {
+  const float* in;
+  const float* T;
+  GridShape P;
+  const AtmosphereCode* codes;
+  int natm;
+  const float* targets;
+  uint64_t seed;
+  int step;
+};
+
+// What a pass leaves: bf16 operand fragments of the weight gradients (features X, activations A, dZ of the hidden layers, dY),
+// FP32 dZ and dY by column for the bias gradients, outputs Y (nullable), loss partials.  dZ[0] null: forward only.
+struct PassOutputs {
+  uint16_t* X;
+  uint16_t* A[3];
+  uint16_t* dZ[3];
+  uint16_t* dY;
+  float* dZf[3];
+  float* dYf;
+  float* Y;
+  float* loss;
+};
+
 struct Surrogate {
   int batch_capacity = 0;
   bool trained = false;
   // device buffers
   float* theta = nullptr;      // FP32 master weights (MlpLayout::total)
   uint16_t* theta_bf = nullptr;  // bf16 copies of W1..W4 (same offsets)
+  uint16_t* wfrag = nullptr;     // the same as operand fragments (kMlpFragments)
   float* adam_m = nullptr;
   float* adam_v = nullptr;
   float* grad = nullptr;
-  // activations for one batch
-  uint16_t* X = nullptr;       // [B][192] bf16 features
-  float* Z[3] = {nullptr, nullptr, nullptr};      // [B][128] FP32 pre-activations
-  uint16_t* A[3] = {nullptr, nullptr, nullptr};   // [B][128] bf16 activations
+  // one batch of B rows (PassOutputs); fragments padded to 32 rows
+  uint16_t* X = nullptr;
+  uint16_t* A[3] = {nullptr, nullptr, nullptr};
+  uint16_t* dZ[3] = {nullptr, nullptr, nullptr};
+  float* dZf[3] = {nullptr, nullptr, nullptr}; // [128][B]
   float* Y = nullptr;          // [B][16] outputs
   float* T = nullptr;          // [B][16] targets
-  uint16_t* dY = nullptr;      // [B][16] bf16
-  float* dA = nullptr;         // [B][128] FP32 upstream gradient
-  float* dZf = nullptr;        // [B][128] FP32 gradient before the activation (bias gradients)
-  uint16_t* dZ = nullptr;      // [B][128] bf16
-  float* loss = nullptr;       // [1 + B / 256] partial sums
-  float* partial = nullptr;    // [kMaxSplits][192][128] split-K partial products
+  uint16_t* dY = nullptr;
+  float* dYf = nullptr;        // [16][B]
+  float* loss = nullptr;       // [surrogate_loss_slots][surrogate_loss_parts] partial sums
+  float* partial = nullptr;    // [kMaxSplits][MlpLayout::total] weight gradients by split of the rows
+  int splits = 0;              // splits of the last backward pass
   float* ztab = nullptr;       // layer-1 tables of the fused prediction
   size_t ztab_capacity = 0;
   int adam_step = 0;
@@ -84,19 +119,20 @@ hipError_t surrogate_init(Surrogate& s, uint64_t seed, hipStream_t stream);
 // Refresh the bf16 weight copies from the FP32 master weights.
 hipError_t surrogate_sync_bf16(Surrogate& s, hipStream_t stream);
 
-// Features of `rows` explicit input rows (host layout [rows][10], values in [0, 1]) -> s.X.
-hipError_t surrogate_encode_rows(Surrogate& s, const float* inputs_dev, int rows, hipStream_t stream);
-// Forward pass over s.X (rows <= capacity) -> s.Y.
-hipError_t surrogate_forward(Surrogate& s, int rows, hipStream_t stream);
-// Loss and gradient for targets s.T with output mask (first kMlpUsed outputs) -> s.grad, s.loss.
-hipError_t surrogate_backward(Surrogate& s, int rows, hipStream_t stream);
-// One Adam step on s.grad.
+// Loss partials of a pass over `rows` rows (256 values each, to be added in order), and how many passes' partials s.loss
+// holds.
+int surrogate_loss_parts(int rows);
+int surrogate_loss_slots(int rows);
+// Forward pass over explicit input rows (device, [rows][10], values in [0, 1]; rows <= capacity) -> s.Y; with backward also
+// the loss (slot 0 of s.loss) and the gradient (s.grad) for targets s.T, first kMlpUsed outputs.
+hipError_t surrogate_eval_rows(Surrogate& s, const float* inputs_dev, int rows, bool backward, hipStream_t stream);
+// Loss (slot loss_slot of s.loss) and gradient of `rows` entries drawn with a counter-based generator from `natm`
+// atmospheres of `entries` scatter-grid entries each; targets[atm][entry][15] hold log(P + eps) + shift.  The gradient
+// stays split by rows for surrogate_adam.
+hipError_t surrogate_train_rows(Surrogate& s, const DevParams& P, const AtmosphereCode* codes_dev, int natm,
+                                const float* targets_dev, uint64_t seed, int step, int rows, int loss_slot, hipStream_t stream);
+// One Adam step on the gradient of the last pass.
 hipError_t surrogate_adam(Surrogate& s, float lr, hipStream_t stream);
-
-// Training batch: `rows` entries drawn with a counter-based generator from `natm` atmospheres of
-// `entries` scatter-grid entries each; targets[atm][entry][9] hold log(P + eps) + shift.
-hipError_t surrogate_gather_batch(Surrogate& s, const DevParams& P, const AtmosphereCode* codes_dev, int natm,
-                                  const float* targets_dev, uint64_t seed, int step, int rows, hipStream_t stream);
 // Output biases b4[0 .. kMlpUsed) = mean of each target column over `rows` target rows.
 hipError_t surrogate_init_output_bias(Surrogate& s, const float* targets_dev, long long rows, hipStream_t stream);
 // Targets of one atmosphere from its order sums P_1..P_5 (float4 tables).
@@ -108,17 +144,6 @@ hipError_t surrogate_reserve_tables(Surrogate& s, const DevParams& P);
 // and the decoding.
 hipError_t surrogate_predict_tables(Surrogate& s, const DevParams& P, const AtmosphereCode& code, float4* const* out,
                                     hipStream_t stream);
-
-// Matrix product on the matrix cores: C[m][n] = sum_k A(m, k) B(k, n) (+ bias[n]), A(m, k) at
-// A[m * sam + k * sak], B(k, n) at B[k * sbk + n * sbn] (bf16), C row-major FP32 with leading dim ldc.
-// act: 0 none, 1 SiLU; out_bf16 (nullable) receives act(C) as bf16 with leading dimension ldc.
-hipError_t mfma_gemm(const uint16_t* A, long long sam, long long sak, const uint16_t* B, long long sbk,
-                     long long sbn, float* C, int ldc, const float* bias, int act, uint16_t* out_bf16, int M, int N,
-                     int K, hipStream_t stream);
-// The same product with K split over up to kMaxSplits workgroups per tile (C row-major, ldc = N);
-// partial holds kMaxSplits x M x N floats.
-hipError_t mfma_gemm_split_k(const uint16_t* A, long long sam, long long sak, const uint16_t* B, long long sbk,
-                             long long sbn, float* C, int M, int N, int K, float* partial, hipStream_t stream);
 
 AtmosphereCode atmosphere_code(const double* rayleigh_base, double rayleigh_scale, double mie_base, double mie_scale,
                                double mie_g, double albedo);
