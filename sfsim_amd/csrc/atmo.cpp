@@ -581,7 +581,8 @@ int prepare_pipeline(sfsim_atmo_ctx* ctx, const sfsim_atmo_params* p) {
 // (float4 tables, k = 1..min(iterations, 5)), the training targets of the surrogate.
 // The per-build launches before the iterations: T, E0 and (with iterations) the quadrature directions'
 // geometry, the ray geometry, the re-sampling map, the sun table, then R1/M1.  merged: the independent
-// ones in one launch (graph capture; the timed and counted builds launch them one by one).
+// ones in one launch, which the timed and counted builds take apart (64x64 / 32x16x32x16, 7 launches and 77 us of
+// kernels against 1 of 42 us: the short jobs fill each other's last workgroups).
 int enqueue_prologue(sfsim_atmo_ctx* ctx, const sfsim_atmo_params* p, const DevParams& P, WorkCounters* wc,
                      Timer& timer, bool merged) {
   auto f4 = [](DeviceBuffer& b) { return (float4*)b.ptr; };
@@ -724,7 +725,7 @@ int run_pipeline(sfsim_atmo_ctx* ctx, const sfsim_atmo_params* p, WorkCounters* 
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
     ctx->notes.clear();
   }
-  TRY(enqueue_pipeline(ctx, p, P, wc, timer, capture));
+  TRY(enqueue_pipeline(ctx, p, P, wc, timer, capture, !timed && !wc));
   HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
   TRY(timer.collect());
   ctx->built = true;
