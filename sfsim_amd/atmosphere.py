@@ -280,19 +280,19 @@ class Atmosphere:
 
     # ---------------------------------------------------------------- tables
     def transmittance_table(self, P):
-        out = np.zeros(tuple(P.transmittance_shape) + (3,), np.float32)
+        out = np.empty(tuple(P.transmittance_shape) + (3,), np.float32)
         self._check(lib().sfsim_atmo_transmittance_table(self._ctx, ctypes.byref(P), _fp(out)))
         return out
 
     def surface_radiance_base_table(self, P):
-        out = np.zeros(tuple(P.surface_radiance_shape) + (3,), np.float32)
+        out = np.empty(tuple(P.surface_radiance_shape) + (3,), np.float32)
         self._check(lib().sfsim_atmo_surface_radiance_base_table(self._ctx, ctypes.byref(P), _fp(out)))
         return out
 
     def single_scatter_tables(self, P):
         """(Rayleigh single scatter R1, Mie strength M1)."""
         shape = tuple(P.scatter_shape) + (3,)
-        r1, m1 = np.zeros(shape, np.float32), np.zeros(shape, np.float32)
+        r1, m1 = np.empty(shape, np.float32), np.empty(shape, np.float32)
         self._check(lib().sfsim_atmo_single_scatter_tables(self._ctx, ctypes.byref(P), _fp(r1), _fp(m1)))
         return r1, m1
 
@@ -300,21 +300,21 @@ class Atmosphere:
         n = int(np.prod(P.scatter_shape))
         ne = P.surface_radiance_shape[0] * P.surface_radiance_shape[1]
         a, m, e = _f32(dS, n), _f32(mie_strength, n), _f32(dE, ne)
-        out = np.zeros(tuple(P.scatter_shape) + (3,), np.float32)
+        out = np.empty(tuple(P.scatter_shape) + (3,), np.float32)
         self._check(lib().sfsim_atmo_point_scatter_table(self._ctx, ctypes.byref(P), _fp(a), _fp(m), _fp(e), _fp(out)))
         return out
 
     def ray_scatter_table(self, P, dJ):
         n = int(np.prod(P.scatter_shape))
         j = _f32(dJ, n)
-        out = np.zeros(tuple(P.scatter_shape) + (3,), np.float32)
+        out = np.empty(tuple(P.scatter_shape) + (3,), np.float32)
         self._check(lib().sfsim_atmo_ray_scatter_table(self._ctx, ctypes.byref(P), _fp(j), _fp(out)))
         return out
 
     def surface_radiance_table(self, P, dS, mie_strength=None):
         n = int(np.prod(P.scatter_shape))
         a, m = _f32(dS, n), _f32(mie_strength, n)
-        out = np.zeros(tuple(P.surface_radiance_shape) + (3,), np.float32)
+        out = np.empty(tuple(P.surface_radiance_shape) + (3,), np.float32)
         self._check(lib().sfsim_atmo_surface_radiance_table(self._ctx, ctypes.byref(P), _fp(a), _fp(m), _fp(out)))
         return out
 
@@ -324,7 +324,7 @@ class Atmosphere:
             raise AtmoError(ERR_ARGUMENT, f"unknown space {space}")
         n = int(np.prod(shape))
         aa, bb = _f32(a, n), _f32(b, n)
-        out = np.zeros(tuple(shape) + (3,), np.float32)
+        out = np.empty(tuple(shape) + (3,), np.float32)
         self._check(lib().sfsim_atmo_resample_table(self._ctx, ctypes.byref(P), space, _fp(aa), _fp(bb), _fp(out)))
         return out
 
@@ -332,11 +332,11 @@ class Atmosphere:
     def generate_atmosphere_luts(self, P):
         """atmosphere_lut.clj:43-105: the four tables in .scatter file layout, as float32 arrays
         shaped like the 2D images the files hold."""
-        T = np.zeros((P.transmittance_shape[0], P.transmittance_shape[1], 3), np.float32)
-        E = np.zeros((P.surface_radiance_shape[0], P.surface_radiance_shape[1], 3), np.float32)
+        T = np.empty((P.transmittance_shape[0], P.transmittance_shape[1], 3), np.float32)
+        E = np.empty((P.surface_radiance_shape[0], P.surface_radiance_shape[1], 3), np.float32)
         s = P.scatter_shape
-        S = np.zeros((s[0] * s[2], s[1] * s[3], 3), np.float32)
-        M = np.zeros_like(S)
+        S = np.empty((s[0] * s[2], s[1] * s[3], 3), np.float32)
+        M = np.empty_like(S)
         self._check(lib().sfsim_atmo_generate_luts(self._ctx, ctypes.byref(P), _fp(T), _fp(E), _fp(S), _fp(M)))
         return {"transmittance": T, "surface-radiance": E, "ray-scatter": S, "mie-strength": M}
 
@@ -361,7 +361,7 @@ class Atmosphere:
         shapes = [(P.transmittance_shape[0], P.transmittance_shape[1], 3),
                   (P.surface_radiance_shape[0], P.surface_radiance_shape[1], 3),
                   (s[0] * s[2], s[1] * s[3], 3), (s[0] * s[2], s[1] * s[3], 3)]
-        out = np.zeros(shapes[which], np.float32)
+        out = np.empty(shapes[which], np.float32)
         self._check(lib().sfsim_atmo_fetch(self._ctx, which, _fp(out), out.size))
         return out
 
@@ -378,7 +378,7 @@ class Atmosphere:
         shapes = [(P.transmittance_shape[0], P.transmittance_shape[1], 3),
                   (P.surface_radiance_shape[0], P.surface_radiance_shape[1], 3),
                   (s[0] * s[2], s[1] * s[3], 3), (s[0] * s[2], s[1] * s[3], 3)]
-        out = np.zeros(shapes[which], np.float32)
+        out = np.empty(shapes[which], np.float32)
         self._check(lib().sfsim_atmo_fetch_batch(self._ctx, atmosphere, which, _fp(out), out.size))
         return out
 

@@ -3,13 +3,18 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
+#include <condition_variable>
+#include <cstdint>
 #include <cstring>
 #include <deque>
+#include <memory>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/sfsim_atmo.h"
@@ -85,6 +90,160 @@ hipError_t scratch_address(int device, void** out) {
 
 }  // namespace
 
+// One stretch of device memory to be copied to the caller's.
+struct CopyOut {
+  const void* src;
+  void* dst;
+  size_t bytes;
+};
+
+// Copies device memory out to pageable host memory through a small ring of pinned chunks, emptied by the calling
+// thread and a few of the copier's own while the next chunks are on their way.  A plain copy into pages that the caller
+// has just allocated spends most of its time in page faults and one thread's memcpy (12.6 MB: 0.72-0.89 ms, against
+// 0.23 ms on the link); so a stage call that returns 12.6 MB takes 0.61 ms instead of 0.91.  One copier per context, used by one call at a time.
+struct HostCopier {
+  static constexpr int kSlots = 8, kThreads = 3, kMaxList = 4;
+  static constexpr size_t kChunk = 512 << 10;
+  int device = 0;
+  char* pinned = nullptr;
+  hipEvent_t event[kSlots] = {};
+  // the job in hand: pieces of at most kChunk bytes, numbered through the list (first[i]: the i-th stretch's first)
+  hipStream_t stream = nullptr;
+  const CopyOut* list = nullptr;
+  int first[kMaxList + 1] = {}, stretches = 0;
+  std::atomic<int> held[kSlots];  // the piece last queued into each slot
+  std::atomic<int> next{0}, error{0};
+  // the threads and the job they are on
+  std::vector<std::thread> threads;
+  std::mutex mu;
+  std::condition_variable wake, idle;
+  unsigned long long job = 0;
+  int busy = 0;
+  bool stop = false;
+
+  ~HostCopier() {
+    {
+      std::lock_guard<std::mutex> lock(mu);
+      stop = true;
+    }
+    wake.notify_all();
+    for (std::thread& t : threads) t.join();
+    for (hipEvent_t e : event)
+      if (e) (void)hipEventDestroy(e);
+    if (pinned) (void)hipHostFree(pinned);
+  }
+
+  // The ring, made on first use; false (and nothing held but events) where it cannot be had.
+  bool ready(int dev) {
+    if (pinned) return true;
+    device = dev;
+    for (hipEvent_t& e : event)
+      if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+        e = nullptr;
+        (void)hipGetLastError();
+        return false;
+      }
+    if (hipHostMalloc((void**)&pinned, kSlots * kChunk, hipHostMallocDefault) != hipSuccess) {
+      pinned = nullptr;
+      (void)hipGetLastError();
+    }
+    return pinned != nullptr;
+  }
+
+  CopyOut piece(int c) const {
+    int i = 0;
+    while (c >= first[i + 1]) ++i;
+    const size_t at = (size_t)(c - first[i]) * kChunk;
+    return CopyOut{(const char*)list[i].src + at, (char*)list[i].dst + at, std::min(kChunk, list[i].bytes - at)};
+  }
+
+  void queue(int c) {
+    const int slot = c % kSlots;
+    if (!error.load()) {
+      const CopyOut p = piece(c);
+      hipError_t e = hipMemcpyAsync(pinned + slot * kChunk, p.src, p.bytes, hipMemcpyDeviceToHost, stream);
+      if (e == hipSuccess) e = hipEventRecord(event[slot], stream);
+      if (e != hipSuccess) error.store((int)e);
+    }
+    held[slot].store(c, std::memory_order_release);
+  }
+
+  // Takes pieces until none is left; whoever has emptied a slot queues the slot's next piece.
+  void work() {
+    const int n = first[stretches];
+    for (int c; (c = next.fetch_add(1)) < n;) {
+      const int slot = c % kSlots;
+      while (held[slot].load(std::memory_order_acquire) != c) std::this_thread::yield();
+      if (!error.load()) {
+        const hipError_t e = hipEventSynchronize(event[slot]);
+        if (e != hipSuccess) error.store((int)e);
+        const CopyOut p = piece(c);
+        if (e == hipSuccess) std::memcpy(p.dst, pinned + slot * kChunk, p.bytes);
+      }
+      if (c + kSlots < n) queue(c + kSlots);
+    }
+  }
+
+  void serve(unsigned long long seen) {
+    (void)hipSetDevice(device);
+    std::unique_lock<std::mutex> lock(mu);
+    for (;;) {
+      wake.wait(lock, [&] { return stop || job != seen; });
+      if (stop) return;
+      seen = job;
+      lock.unlock();
+      work();
+      lock.lock();
+      if (--busy == 0) idle.notify_all();
+    }
+  }
+
+  // Copies the list (at most kMaxList stretches) behind what is on the stream; returns when it has arrived.
+  hipError_t run(hipStream_t on, const CopyOut* what, int count) {
+    stream = on;
+    list = what;
+    stretches = count;
+    for (int i = 0; i < count; ++i) first[i + 1] = first[i] + (int)((what[i].bytes + kChunk - 1) / kChunk);
+    const int n = first[count];
+    next.store(0);
+    error.store(0);
+    for (int c = 0; c < kSlots; ++c) held[c].store(-1);
+    for (int c = 0; c < std::min(n, kSlots); ++c) queue(c);
+    const bool help = n > 2;  // one or two chunks are copied sooner than threads wake
+    if (help) {
+      std::lock_guard<std::mutex> lock(mu);
+      const int most = std::max(0, std::min(kThreads, (int)std::thread::hardware_concurrency() - 1));
+      try {
+        while ((int)threads.size() < most) {
+          const unsigned long long seen = job;
+          threads.emplace_back([this, seen] { serve(seen); });
+        }
+      } catch (...) {  // as many threads as there are
+      }
+      ++job;
+      busy = (int)threads.size();
+    }
+    if (help) wake.notify_all();
+    work();
+    if (help) {
+      std::unique_lock<std::mutex> lock(mu);
+      idle.wait(lock, [&] { return busy == 0; });
+    }
+    return (hipError_t)error.load();
+  }
+};
+
+// The host-made tables of a build that depend on the planet and the grid: quadrature directions and the ray order,
+// made when their keys change.  Contexts upload them to buffers of their own; builds into memory that other calls may
+// have used since (sfsim_atmo_generate_luts_noalloc, batches) upload them every time, side by side in one copy.
+struct HostPlan {
+  double order_key[4] = {-1.0, -1.0, -1.0, -1.0};  // (R, H, NH, NE)
+  int sphere_key = -1, half_key = -1;
+  std::vector<int> order;
+  std::vector<Dir> sphere, half;
+  std::vector<char> image;
+};
+
 // One progress report queued on the stream (sfsim_atmo_set_progress); the runtime calls the host function
 // with its address once the stream reaches it.
 struct ProgressNote {
@@ -107,6 +266,8 @@ struct sfsim_atmo_ctx {
   // pre-assigned (in the batch's memory or the scratch array), and a request that does not fit is an error
   // instead of a hipMalloc
   bool no_alloc = false;
+  HostCopier copier;
+  HostPlan plan;
   // tables (float4 per entry)
   DeviceBuffer T, dE[2], Eacc[2], R1, M1, dJ, dS[2], Sacc[2];
   // packed outputs (RGB floats): 0 transmittance, 1 surface radiance, 2 ray scatter (tiled), 3 mie (tiled)
@@ -263,18 +424,31 @@ int validate_half_sphere(sfsim_atmo_ctx* ctx, int steps) {
   return 0;
 }
 
+// In blocks without a branch per value, which the compiler vectorises: a float is not finite where all its exponent
+// bits are set.
 bool finite_floats(const float* v, size_t n) {
-  for (size_t i = 0; i < n; ++i)
-    if (!std::isfinite(v[i])) return false;
+  constexpr size_t kBlock = 4096;
+  for (size_t o = 0; o < n; o += kBlock) {
+    const size_t m = std::min(kBlock, n - o);
+    uint32_t bad = 0;
+    for (size_t i = 0; i < m; ++i) {
+      uint32_t u;
+      std::memcpy(&u, v + o + i, sizeof(u));
+      bad |= (uint32_t)((u & 0x7f800000u) == 0x7f800000u);
+    }
+    if (bad) return false;
+  }
   return true;
 }
 
 // Polynomial of degree `deg` (2 or 3) through the deg + 1 Chebyshev nodes of [0, xh],
 // xh = (Rt^2 - R^2) / R^2, of f(x) = k (R / 2) p(x), p(x) = 2 (sqrt(1 + x) - 1) / x = 2 / (1 + sqrt(1 + x)),
-// so that k h = x f(x) for the altitude h = sqrt(R^2 + x R^2) - R.  Returns the largest relative error of
-// the fit over 2001 points of [0, xh].  Cubic: 4e-10 for a 100 km atmosphere on Earth, 4e-8 at the
+// so that k h = x f(x) for the altitude h = sqrt(R^2 + x R^2) - R.  Returns whether the relative error of the fit is at
+// most `bound` on 2001 points of [0, xh] (always for bound 0, unchecked): every 50th point first, which settles it
+// unless the largest error lies within a tenth of the bound (the error oscillates a few times over the
+// interval, so 41 points come within a percent of its maximum).  Cubic: 4e-10 for a 100 km atmosphere on Earth, 4e-8 at the
 // largest xh = 0.1 the parameters may have; quadratic: 7e-8 for 100 km.
-double altitude_fit(double R, double Rt, double k, int deg, double out[4]) {
+bool altitude_fit(double R, double Rt, double k, int deg, double bound, double out[4]) {
   const double xh = (Rt * Rt - R * R) / (R * R);
   const int m = deg + 1;
   auto f = [&](double x) { return k * 0.5 * R * 2.0 / (1.0 + std::sqrt(1.0 + x)); };
@@ -297,13 +471,19 @@ double altitude_fit(double R, double Rt, double k, int deg, double out[4]) {
     }
   }
   for (int j = 0; j < 4; ++j) out[j] = j < m ? A[j][4] / A[j][j] : 0.0;
-  double worst = 0.0;
-  for (int i = 0; i <= 2000; ++i) {
-    const double x = xh * i / 2000.0;
-    const double y = out[0] + x * (out[1] + x * (out[2] + x * out[3]));
-    worst = std::fmax(worst, std::fabs(y / f(x) - 1.0));
-  }
-  return worst;
+  if (bound == 0.0) return true;
+  auto worst = [&](int step) {
+    double w = 0.0;
+    for (int i = 0; i <= 2000; i += step) {
+      const double x = xh * i / 2000.0;
+      const double y = out[0] + x * (out[1] + x * (out[2] + x * out[3]));
+      w = std::fmax(w, std::fabs(y / f(x) - 1.0));
+    }
+    return w;
+  };
+  const double coarse = worst(50);
+  if (coarse > bound) return false;
+  return coarse <= 0.9 * bound || worst(1) <= bound;
 }
 
 DevParams make_dev_params(const sfsim_atmo_params* p) {
@@ -328,9 +508,9 @@ DevParams make_dev_params(const sfsim_atmo_params* p) {
   P.k_ray = (float)(-log2e / p->rayleigh.scatter_scale);
   P.inv_R = 1.0 / P.g.R;
   P.ray_over_mie = (float)(p->mie.scatter_scale / p->rayleigh.scatter_scale);
-  altitude_fit(P.g.R, P.g.Rt, -log2e / p->mie.scatter_scale, 3, P.alt_poly_d);
+  altitude_fit(P.g.R, P.g.Rt, -log2e / p->mie.scatter_scale, 3, 0.0, P.alt_poly_d);
   double quad[4];
-  P.alt_deg = altitude_fit(P.g.R, P.g.Rt, -log2e / p->mie.scatter_scale, 2, quad) <= 1e-7 ? 2 : 3;
+  P.alt_deg = altitude_fit(P.g.R, P.g.Rt, -log2e / p->mie.scatter_scale, 2, 1e-7, quad) ? 2 : 3;
   for (int j = 0; j < 4; ++j) P.alt_poly[j] = (float)(P.alt_deg == 2 ? quad[j] : P.alt_poly_d[j]);
   P.inv_scale_mie = 1.0 / p->mie.scatter_scale;
   P.inv_scale_ray = 1.0 / p->rayleigh.scatter_scale;
@@ -376,11 +556,11 @@ DevParams dev_params(const sfsim_atmo_ctx* ctx, const sfsim_atmo_params* p) {
 }
 
 // The view rays of the scatter grid in ascending impact parameter r0 sqrt(1 - mu0^2) (ties in grid
-// order), uploaded when the planet or the grid changes.
-int ensure_ray_order(sfsim_atmo_ctx* ctx, const sfsim_atmo_params* p) {
+// order), made when the planet or the grid changes.
+const std::vector<int>& host_ray_order(HostPlan& plan, const sfsim_atmo_params* p) {
   const double key[4] = {p->planet.radius, p->planet.height, (double)p->scatter_shape[0],
                          (double)p->scatter_shape[1]};
-  if (ctx->ray_order.ptr && std::memcmp(key, ctx->ray_order_key, sizeof(key)) == 0) return 0;
+  if (std::memcmp(key, plan.order_key, sizeof(key)) == 0) return plan.order;
   const DevParams P = make_dev_params(p);
   const int NH = p->scatter_shape[0], NE = p->scatter_shape[1];
   std::vector<double> b((size_t)NH * NE);
@@ -393,9 +573,18 @@ int ensure_ray_order(sfsim_atmo_ctx* ctx, const sfsim_atmo_params* p) {
       b[(size_t)ih * NE + ie] = r0 * std::fabs(ce);
     }
   }
-  std::vector<int> order(b.size());
-  for (size_t i = 0; i < order.size(); ++i) order[i] = (int)i;
-  std::stable_sort(order.begin(), order.end(), [&](int u, int v) { return b[u] < b[v]; });
+  plan.order.resize(b.size());
+  for (size_t i = 0; i < plan.order.size(); ++i) plan.order[i] = (int)i;
+  std::stable_sort(plan.order.begin(), plan.order.end(), [&](int u, int v) { return b[u] < b[v]; });
+  std::memcpy(plan.order_key, key, sizeof(key));
+  return plan.order;
+}
+
+int ensure_ray_order(sfsim_atmo_ctx* ctx, const sfsim_atmo_params* p) {
+  const double key[4] = {p->planet.radius, p->planet.height, (double)p->scatter_shape[0],
+                         (double)p->scatter_shape[1]};
+  if (ctx->ray_order.ptr && std::memcmp(key, ctx->ray_order_key, sizeof(key)) == 0) return 0;
+  const std::vector<int>& order = host_ray_order(ctx->plan, p);
   TRY(ensure(ctx, ctx->ray_order, order.size() * sizeof(int)));
   HIP_TRY(ctx, hipMemcpyAsync(ctx->ray_order.ptr, order.data(), order.size() * sizeof(int), hipMemcpyHostToDevice,
                               ctx->stream));
@@ -463,12 +652,22 @@ std::vector<Dir> sphere_directions(int half, int steps) {
   return dirs;
 }
 
+const std::vector<Dir>& host_directions(HostPlan& plan, int half, int steps) {
+  int& key = half ? plan.half_key : plan.sphere_key;
+  std::vector<Dir>& d = half ? plan.half : plan.sphere;
+  if (key != steps) {
+    d = sphere_directions(half, steps);
+    key = steps;
+  }
+  return d;
+}
+
 int ensure_dirs(sfsim_atmo_ctx* ctx, int half, int steps) {
   int& key = half ? ctx->half_key : ctx->sphere_key;
   int& count = half ? ctx->half_n : ctx->sphere_n;
   DeviceBuffer& buf = half ? ctx->half_dirs : ctx->sphere_dirs;
   if (key == steps) return 0;
-  std::vector<Dir> d = sphere_directions(half, steps);
+  const std::vector<Dir>& d = host_directions(ctx->plan, half, steps);
   TRY(ensure(ctx, buf, d.size() * sizeof(Dir)));
   HIP_TRY(ctx, hipMemcpyAsync(buf.ptr, d.data(), d.size() * sizeof(Dir), hipMemcpyHostToDevice, ctx->stream));
   HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
@@ -715,9 +914,10 @@ int enqueue_pipeline(sfsim_atmo_ctx* ctx, const sfsim_atmo_params* p, const DevP
   return 0;
 }
 
-// The whole driver, launched eagerly (timed: per-kernel events; wc: work counters).
+// The whole driver, launched eagerly (timed: per-kernel events; wc: work counters; wait: until the stream is idle,
+// or the caller's copies wait).
 int run_pipeline(sfsim_atmo_ctx* ctx, const sfsim_atmo_params* p, WorkCounters* wc, bool timed,
-                 float4* const* capture = nullptr) {
+                 float4* const* capture = nullptr, bool wait = true) {
   TRY(prepare_pipeline(ctx, p));
   const DevParams P = dev_params(ctx, p);
   Timer timer{ctx, timed};
@@ -726,7 +926,7 @@ int run_pipeline(sfsim_atmo_ctx* ctx, const sfsim_atmo_params* p, WorkCounters* 
     ctx->notes.clear();
   }
   TRY(enqueue_pipeline(ctx, p, P, wc, timer, capture, !timed && !wc));
-  HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+  if (wait) HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
   TRY(timer.collect());
   ctx->built = true;
   return 0;
@@ -1012,13 +1212,45 @@ int upload_table(sfsim_atmo_ctx* ctx, int slot, const float* host, size_t entrie
   return 0;
 }
 
+// The list's device memory to the caller's, behind what is on the stream; returns when all has arrived.  Up to one
+// chunk goes to the pinned ring in one go.
+int copy_out(sfsim_atmo_ctx* ctx, const CopyOut* list, int count) {
+  HostCopier& h = ctx->copier;
+  size_t total = 0;
+  for (int i = 0; i < count; ++i) total += list[i].bytes;
+  if (!h.ready(ctx->device)) {
+    for (int i = 0; i < count; ++i)
+      HIP_TRY(ctx, hipMemcpyAsync(list[i].dst, list[i].src, list[i].bytes, hipMemcpyDeviceToHost, ctx->stream));
+    HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    return 0;
+  }
+  if (total <= HostCopier::kChunk) {
+    size_t at = 0;
+    for (int i = 0; i < count; at += list[i++].bytes)
+      HIP_TRY(ctx, hipMemcpyAsync(h.pinned + at, list[i].src, list[i].bytes, hipMemcpyDeviceToHost, ctx->stream));
+    HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    at = 0;
+    for (int i = 0; i < count; at += list[i++].bytes) std::memcpy(list[i].dst, h.pinned + at, list[i].bytes);
+    return 0;
+  }
+  HIP_TRY(ctx, h.run(ctx->stream, list, count));
+  return 0;
+}
+
+// A float4 table to a packed RGB one of the caller's: small ones packed straight into pinned memory.
 int download_table(sfsim_atmo_ctx* ctx, const float4* dev, float* host, size_t entries) {
   if (!host) return 0;
-  TRY(ensure(ctx, ctx->stage_rgb, entries * 3 * sizeof(float)));
+  const size_t bytes = entries * 3 * sizeof(float);
+  if (bytes <= HostCopier::kChunk && ctx->copier.ready(ctx->device)) {
+    HIP_TRY(ctx, launch_pack_rgb(dev, (float*)ctx->copier.pinned, (long long)entries, ctx->stream));
+    HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    std::memcpy(host, ctx->copier.pinned, bytes);
+    return 0;
+  }
+  TRY(ensure(ctx, ctx->stage_rgb, bytes));
   HIP_TRY(ctx, launch_pack_rgb(dev, (float*)ctx->stage_rgb.ptr, (long long)entries, ctx->stream));
-  HIP_TRY(ctx, hipMemcpyAsync(host, ctx->stage_rgb.ptr, entries * 3 * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
-  HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-  return 0;
+  const CopyOut c{ctx->stage_rgb.ptr, host, bytes};
+  return copy_out(ctx, &c, 1);
 }
 
 float4* stage_out(sfsim_atmo_ctx* ctx, size_t entries, int* rc) {
@@ -1047,15 +1279,45 @@ size_t layout_shared(sfsim_atmo_ctx* c, const sfsim_atmo_params* p, char* base) 
   Carver k{base};
   const DevParams P = make_dev_params(p);
   k.take(c->ray_order, (size_t)p->scatter_shape[0] * p->scatter_shape[1] * sizeof(int));
-  k.take(c->rmap, resample_map_bytes(P));
-  k.take(c->sunmap, sun_map_bytes(P));
-  if (p->iterations > 0) {
+  if (p->iterations > 0) {  // beside the ray order: upload_plan copies the three together
     const int sn = sfsim_atmo_sphere_directions(0, p->sphere_steps), hn = sfsim_atmo_sphere_directions(1, p->ray_steps);
     k.take(c->sphere_dirs, (size_t)sn * sizeof(Dir));
     k.take(c->half_dirs, (size_t)hn * sizeof(Dir));
     k.take(c->sgeo, (size_t)p->surface_radiance_shape[0] * hn * sizeof(float4));
   }
+  k.take(c->rmap, resample_map_bytes(P));
+  k.take(c->sunmap, sun_map_bytes(P));
   return k.off;
+}
+
+// The host-made tables (owner's plan) into the buffers that layout_shared gave c, as prepare_pipeline would make them
+// one by one, in one copy that is not waited for: the call that uses them waits for the stream, also where it fails.
+// Made and uploaded by each call, with a wait per table, they kept the GPU idle for most of the 0.26 ms that a call of
+// 0.87 ms at 64x64 / 32x16x32x16 has lost since.
+int upload_plan(sfsim_atmo_ctx* owner, sfsim_atmo_ctx* c, const sfsim_atmo_params* p) {
+  HostPlan& plan = owner->plan;
+  const bool dirs = p->iterations > 0;
+  const std::vector<int>& order = host_ray_order(plan, p);
+  if (dirs) {
+    host_directions(plan, 0, p->sphere_steps);
+    host_directions(plan, 1, p->ray_steps);
+  }
+  char* base = (char*)c->ray_order.ptr;
+  const size_t end = dirs ? (size_t)((char*)c->half_dirs.ptr - base) + plan.half.size() * sizeof(Dir) : order.size() * sizeof(int);
+  plan.image.resize(end);
+  std::memcpy(plan.image.data(), order.data(), order.size() * sizeof(int));
+  if (dirs) {
+    std::memcpy(plan.image.data() + ((char*)c->sphere_dirs.ptr - base), plan.sphere.data(), plan.sphere.size() * sizeof(Dir));
+    std::memcpy(plan.image.data() + ((char*)c->half_dirs.ptr - base), plan.half.data(), plan.half.size() * sizeof(Dir));
+    c->sphere_key = p->sphere_steps;
+    c->half_key = p->ray_steps;
+    c->sphere_n = (int)plan.sphere.size();
+    c->half_n = (int)plan.half.size();
+  }
+  HIP_TRY(owner, hipMemcpyAsync(base, plan.image.data(), end, hipMemcpyHostToDevice, c->stream));
+  const double key[4] = {p->planet.radius, p->planet.height, (double)p->scatter_shape[0], (double)p->scatter_shape[1]};
+  std::memcpy(c->ray_order_key, key, sizeof(key));
+  return 0;
 }
 
 // The buffers of one atmosphere's build that prepare_pipeline asks for (with_outputs: also the four packed
@@ -1241,9 +1503,8 @@ int sfsim_atmo_point_scatter_table(sfsim_atmo_ctx* ctx, const sfsim_atmo_params*
   HIP_TRY(ctx, launch_point_scatter(P, (const Dir*)ctx->sphere_dirs.ptr, ctx->sphere_n, p->sphere_steps, ctx->geom.ptr, ddS, dM,
                                     ddE, o, nullptr, ctx->stream));
   HIP_TRY(ctx, launch_transpose_rgb(o, (float*)ctx->stage_rgb.ptr, (long long)n, P.nS[3], P.nS[2], ctx->stream));
-  HIP_TRY(ctx, hipMemcpyAsync(out, ctx->stage_rgb.ptr, n * 3 * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
-  HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-  return 0;
+  const CopyOut c{ctx->stage_rgb.ptr, out, n * 3 * sizeof(float)};
+  return copy_out(ctx, &c, 1);
 }
 
 int sfsim_atmo_ray_scatter_table(sfsim_atmo_ctx* ctx, const sfsim_atmo_params* p, const float* dJ, float* out) {
@@ -1335,19 +1596,23 @@ int sfsim_atmo_fetch(sfsim_atmo_ctx* ctx, int which, float* out, size_t count) {
   if (which < 0 || which > 3 || !out) return fail(ctx, SFSIM_ATMO_ERR_ARGUMENT, "which must be 0..3 and out non-NULL");
   if (!ctx->built) return fail(ctx, SFSIM_ATMO_ERR_ARGUMENT, "no completed build on this context");
   if (count != ctx->out_count[which]) return fail(ctx, SFSIM_ATMO_ERR_ARGUMENT, "count does not match the table size");
-  HIP_TRY(ctx, hipMemcpyAsync(out, ctx->out[which].ptr, count * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
-  HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-  return 0;
+  const CopyOut c{ctx->out[which].ptr, out, count * sizeof(float)};
+  return copy_out(ctx, &c, 1);
 }
 
 int sfsim_atmo_generate_luts(sfsim_atmo_ctx* ctx, const sfsim_atmo_params* p, float* transmittance,
                              float* surface_radiance, float* ray_scatter, float* mie_strength) {
   TRY(activate(ctx));
-  TRY(run_pipeline(ctx, p, nullptr, false));
   float* outs[4] = {transmittance, surface_radiance, ray_scatter, mie_strength};
+  CopyOut list[4];
+  int n = 0;
+  TRY(run_pipeline(ctx, p, nullptr, false, nullptr, false));
   for (int i = 0; i < 4; ++i)
-    if (outs[i]) TRY(sfsim_atmo_fetch(ctx, i, outs[i], ctx->out_count[i]));
-  return 0;
+    if (outs[i]) list[n++] = CopyOut{ctx->out[i].ptr, outs[i], ctx->out_count[i] * sizeof(float)};
+  const int rc = copy_out(ctx, list, n);
+  if (rc || n == 0) HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+  if (rc) ctx->built = false;
+  return rc;
 }
 
 int sfsim_atmo_generate_luts_noalloc(sfsim_atmo_ctx* ctx, const sfsim_atmo_params* p, float* transmittance,
@@ -1386,8 +1651,12 @@ int sfsim_atmo_generate_luts_noalloc(sfsim_atmo_ctx* ctx, const sfsim_atmo_param
     sh.out[i].ptr = outs[i];
     sh.out[i].bytes = outc[i] * sizeof(float);
   }
+  TRY(upload_plan(ctx, &sh, p));
   const int rc = run_pipeline(&sh, p, nullptr, false);
-  if (rc) ctx->error = sh.error;
+  if (rc) {
+    ctx->error = sh.error;
+    (void)hipStreamSynchronize(ctx->stream);  // the plan's upload
+  }
   return rc;
 }
 
@@ -1435,8 +1704,12 @@ int sfsim_atmo_build_batch(sfsim_atmo_ctx* ctx, const sfsim_atmo_params* ps, int
     ctx->error = sh.error;
     return rc;
   };
+  TRY(upload_plan(ctx, &sh, p0));
   int rc = prepare_pipeline(&sh, p0);
-  if (rc) return fail_sh(rc);
+  if (rc) {
+    (void)hipStreamSynchronize(ctx->stream);  // the plan's upload
+    return fail_sh(rc);
+  }
   // per-atmosphere parameters: each atmosphere's own ray geometry and sun table, the shared maps
   const DevParams* dparams = (const DevParams*)ctx->batch_params.ptr;
   std::vector<DevParams> host(count);
@@ -1449,8 +1722,12 @@ int sfsim_atmo_build_batch(sfsim_atmo_ctx* ctx, const sfsim_atmo_params* ps, int
     Pa.batch_params = dparams;
     host[a] = Pa;
   }
-  HIP_TRY(ctx, hipMemcpyAsync(ctx->batch_params.ptr, host.data(), (size_t)count * sizeof(DevParams),
-                              hipMemcpyHostToDevice, ctx->stream));
+  const hipError_t ep = hipMemcpyAsync(ctx->batch_params.ptr, host.data(), (size_t)count * sizeof(DevParams),
+                                       hipMemcpyHostToDevice, ctx->stream);
+  if (ep != hipSuccess) {
+    (void)hipStreamSynchronize(ctx->stream);  // the plan's upload
+    HIP_TRY(ctx, ep);
+  }
   Timer timer{&sh, false};
   rc = enqueue_pipeline(&sh, p0, host[0], nullptr, timer, nullptr, true);
   // the progress reports queued so far point into sh: wait for them on the failure path as well
@@ -1475,9 +1752,8 @@ int sfsim_atmo_fetch_batch(sfsim_atmo_ctx* ctx, int atmosphere, int which, float
   if (count != ctx->batch_out_count[which])
     return fail(ctx, SFSIM_ATMO_ERR_ARGUMENT, "count does not match the table size");
   const char* src = (const char*)ctx->batch_out[which] + (size_t)atmosphere * ctx->batch_stride;
-  HIP_TRY(ctx, hipMemcpyAsync(out, src, count * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
-  HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-  return 0;
+  const CopyOut c{src, out, count * sizeof(float)};
+  return copy_out(ctx, &c, 1);
 }
 
 int sfsim_atmo_stage_timings(const sfsim_atmo_ctx* ctx, double* ms, int* launches, int n) {
