@@ -86,6 +86,13 @@ __device__ __forceinline__ Segment make_segment(const DevParams& P, double h0, d
   return g;
 }
 
+// A uniform value held in a vector register.  A multiply-add of vector registers alone issues every 2 clocks
+// beside another wavefront's instruction, one that reads a scalar register every 4.
+__device__ __forceinline__ float in_vgpr(float x) {
+  asm("" : "+v"(x));
+  return x;
+}
+
 // Sums over the n midpoint nodes of exp(-h / H_mie) and exp(-h / H_rayleigh) with FP32 altitudes;
 // 8-node partial sums, Kahan-compensated across them.  Node j sits at s_j = s0 + j dt (units of R,
 // measured from the segment's lowest point), x_j = c0 + s_j (b + s_j) = (r_j^2 - R^2) / R^2, and the
@@ -94,8 +101,8 @@ __device__ __forceinline__ Segment make_segment(const DevParams& P, double h0, d
 // exponentials.
 template <int DEG>
 __device__ float2 density_sums_f32_deg(const DevParams& P, const Segment& g, int n) {
-  const float a0 = P.alt_poly[0], a1 = P.alt_poly[1], a2 = P.alt_poly[2], a3 = P.alt_poly[3];
-  const float rho = P.ray_over_mie;
+  const float a0 = in_vgpr(P.alt_poly[0]), a1 = in_vgpr(P.alt_poly[1]), a2 = in_vgpr(P.alt_poly[2]), a3 = in_vgpr(P.alt_poly[3]);
+  const float rho = in_vgpr(P.ray_over_mie);
   auto exponent = [&](float x) {
     const float p = DEG == 3 ? fmaf(fmaf(fmaf(a3, x, a2), x, a1), x, a0) : fmaf(fmaf(a2, x, a1), x, a0);
     return x * p;
@@ -104,19 +111,25 @@ __device__ float2 density_sums_f32_deg(const DevParams& P, const Segment& g, int
   int j = 0;
   for (; j + 8 <= n; j += 8) {
     const float base = fmaf((float)j, g.dt, g.s0);
-    float pm = 0.f, pr = 0.f;
+    float m[8], r[8];
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
       const float s = fmaf((float)q, g.dt, base);
-      const float em = exponent(fmaf(s, s + g.b, g.c0));
-      const float m = fexp2(em), r = fexp2(em * rho);
-      if (q == 0) {
-        pm = m;
-        pr = r;
-      } else {
-        pm += m;
-        pr += r;
-      }
+      m[q] = exponent(fmaf(s, s + g.b, g.c0));
+      r[q] = m[q] * rho;
+    }
+    __builtin_amdgcn_sched_barrier(0);  // 16 exponentials in a row: between them the additions would not issue in pairs
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      m[q] = fexp2(m[q]);
+      r[q] = fexp2(r[q]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    float pm = m[0], pr = r[0];
+#pragma unroll
+    for (int q = 1; q < 8; ++q) {
+      pm += m[q];
+      pr += r[q];
     }
     kahan_add(sm, cm, pm);
     kahan_add(sr, cr, pr);
@@ -370,14 +383,28 @@ __device__ __forceinline__ Ray make_ray(const DevParams& P, int ih, int ie) {
 }
 
 // R1 (Rayleigh with phase) and M1 (Mie strength) in one pass: atmosphere_lut.clj:70-78,
-// atmosphere.clj:154-200.  One wavefront per (view ray, group of 64 (sun elevation, heading)
-// entries); groups of high sun elevation (most samples lit) are launched first so that the light
-// groups fill the end of the grid.  The ray's samples are processed in chunks of kSSChunk: each lane
-// marks the samples where its sun is above the horizon, the wavefront compacts the lit
-// (entry, sample) pairs into an LDS list and all 64 lanes take items from it, so lanes never idle on
-// unlit samples; each entry then adds its results in sample order (deterministic sums).
-constexpr int kSSWave = 64;
-constexpr int kSSChunk = 8;
+// atmosphere.clj:154-200.  One workgroup per (view ray, group of 64 (sun elevation, heading) entries); groups of high
+// sun elevation (most samples lit) are launched first so that the light groups fill the end of the grid.  The ray's
+// samples are processed in chunks of kSSChunk: each thread marks the samples of its quarter of the chunk where its
+// entry's sun is above the horizon, the workgroup compacts the lit (entry, sample) pairs into an LDS list, and its
+// wavefronts take 64 items of it at a time, the FP64 ones first, so lanes never idle on unlit samples; each entry then
+// adds its results in sample order (deterministic sums).
+//
+// VALU issue bounds it: per item ray_steps nodes of two exponentials (8 clocks each) and ten further instructions, at
+// 60 clocks a node.  With one wavefront per group (32 x 64 x 32 x 8 entries: 32 per CU) the whole grid was resident at
+// once, and the CUs idled for 35% of the launch while the ones that held the most lit groups finished; four wavefronts
+// per group leave a quarter of the groups resident and the rest to whichever CU is free: 1080 us -> 798, and 760 with the
+// node loop's coefficients in vector registers and its exponentials in a row.
+constexpr int kSSEntries = 64;
+constexpr int kSSWaves = 4;
+constexpr int kSSChunk = 16;
+
+// LDS of a workgroup for n samples.
+inline size_t single_scatter_shared_bytes(int n) {
+  return (size_t)n * (2 * sizeof(double) + sizeof(float4)) + sizeof(float) * (size_t)((n + 3) & ~3) +
+         (3 * sizeof(float) + sizeof(unsigned short)) * kSSEntries * kSSChunk + 2 * sizeof(double) * kSSEntries +
+         kSSWaves * kSSEntries * sizeof(unsigned) + (2 * kSSWaves + 1) * sizeof(int);
+}
 
 __device__ __forceinline__ int wave_exclusive_scan(int v, int lane) {
   int x = v;
@@ -389,30 +416,35 @@ __device__ __forceinline__ int wave_exclusive_scan(int v, int lane) {
   return x - v;
 }
 
-__global__ void __launch_bounds__(kSSWave) single_scatter_kernel(const DevParams P, float4* __restrict__ R1,
-                                                                 float4* __restrict__ M1, WorkCounters* wc) {
+__global__ void __launch_bounds__(kSSEntries* kSSWaves) single_scatter_kernel(const DevParams P, float4* __restrict__ R1,
+                                                                              float4* __restrict__ M1, WorkCounters* wc) {
   extern __shared__ unsigned char s_raw[];
   const int NH = P.nS[0], NE = P.nS[1], NL = P.nS[2], NA = P.nS[3];
   const int NLA = NL * NA;
   const int n = P.ray_steps;
-  double* s_t = (double*)s_raw;                  // [n] sample distance along the ray
-  double* s_h = s_t + n;                         // [n] sample altitude
-  float4* s_w = (float4*)(s_h + n);              // [n] T(x, p_i) rgb, w: exp(-h_i / H_mie)
-  float* s_bray = (float*)(s_w + n);             // [n] exp(-h_i / H_rayleigh)
-  float* s_res = s_bray + ((n + 3) & ~3);  // [3][64 * kSSChunk] sun transmittance per item (r, g, b planes)
-  double* s_xl = (double*)(s_res + 3 * kSSWave * kSSChunk);  // [64] dot(x, l) of each lane's entry
-  double* s_vl = s_xl + kSSWave;                          // [64] dot(v, l)
-  unsigned short* s_item = (unsigned short*)(s_vl + kSSWave);  // lane << 8 | chunk sample
+  constexpr int kItems = kSSEntries * kSSChunk, kQuarter = kSSChunk / kSSWaves;
+  double* s_t = (double*)s_raw;                            // [n] sample distance along the ray
+  double* s_h = s_t + n;                                   // [n] sample altitude
+  double* s_xl = s_h + n;                                  // [64] dot(x, l) of each entry
+  double* s_vl = s_xl + kSSEntries;                        // [64] dot(v, l)
+  float4* s_w = (float4*)(s_vl + kSSEntries);              // [n] T(x, p_i) rgb, w: exp(-h_i / H_mie)
+  float* s_bray = (float*)(s_w + n);                       // [n] exp(-h_i / H_rayleigh)
+  float* s_res = s_bray + ((n + 3) & ~3);                  // [3][chunk sample][entry] sun transmittance (r, g, b planes)
+  unsigned* s_mask = (unsigned*)(s_res + 3 * kItems);      // [quarter][entry] lit samples of the chunk
+  int* s_total = (int*)(s_mask + kSSWaves * kSSEntries);   // [2][quarter] items listed, FP64 and FP32
+  int* s_next = s_total + 2 * kSSWaves;                    // the next 64 items
+  unsigned short* s_item = (unsigned short*)(s_next + 1);  // chunk sample * 64 + entry
 
   const int rays = NH * NE;
-  const int groups = (NLA + kSSWave - 1) / kSSWave;
+  const int groups = (NLA + kSSEntries - 1) / kSSEntries;
   const int group = groups - 1 - blockIdx.x / rays;
   const int rayid = blockIdx.x - (groups - 1 - group) * rays;
   const int ih = rayid / NE, ie = rayid - ih * NE;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const Ray ray = make_ray(P, ih, ie);
   const double dt = ray.D / n;
-  for (int i = lane; i < n; i += kSSWave) {
+  unsigned long long samples = 0, view = 0;
+  for (int i = threadIdx.x; i < n; i += kSSEntries * kSSWaves) {
     double t = (i + 0.5) * dt;
     double h = altitude_along(P.g, ray.h0, ray.pd0, t);
     s_t[i] = t;
@@ -420,8 +452,9 @@ __global__ void __launch_bounds__(kSSWave) single_scatter_kernel(const DevParams
     float3 T = segment_transmittance(P, ray.h0, ray.pd0, t, n);
     s_w[i] = make_float4(T.x, T.y, T.z, (float)exp(-h * P.inv_scale_mie));
     s_bray[i] = (float)exp(-h * P.inv_scale_ray);
+    view += n;
   }
-  const int k = group * kSSWave + lane;
+  const int k = group * kSSEntries + lane;
   const bool valid = k < NLA;
   double vl = 0.0, xl = 0.0;
   if (valid) {
@@ -432,11 +465,10 @@ __global__ void __launch_bounds__(kSSWave) single_scatter_kernel(const DevParams
     vl = ray.se * l0 + ray.ce * l1;
     xl = ray.r0 * l0;
   }
-  s_xl[lane] = xl;
+  s_xl[lane] = xl;  // every wavefront the same
   s_vl[lane] = vl;
   __syncthreads();
   float3 accR = make_float3(0.f, 0.f, 0.f), accM = make_float3(0.f, 0.f, 0.f);
-  unsigned long long samples = 0;
   for (int i0 = 0; i0 < n; i0 += kSSChunk) {
     const int cn = min(kSSChunk, n - i0);
     // lit samples (atmosphere.clj:154-160), split by the optical-depth path their sun segment takes:
@@ -444,7 +476,7 @@ __global__ void __launch_bounds__(kSSWave) single_scatter_kernel(const DevParams
     // graze_height, FP32 otherwise
     unsigned m32 = 0, m64 = 0;
     if (valid)
-      for (int c = 0; c < cn; ++c) {
+      for (int c = wave * kQuarter; c < min(cn, (wave + 1) * kQuarter); ++c) {
         const int i = i0 + c;
         const double h = s_h[i], pl = xl + s_t[i] * vl;
         if (is_above_horizon(P.g, h, pl)) {
@@ -455,57 +487,60 @@ __global__ void __launch_bounds__(kSSWave) single_scatter_kernel(const DevParams
         }
       }
     const int c32 = __popc(m32), c64 = __popc(m64);
-    const int o32 = wave_exclusive_scan(c32, lane), o64 = wave_exclusive_scan(c64, lane);
-    const int t32 = __shfl(o32 + c32, kSSWave - 1, 64), t64 = __shfl(o64 + c64, kSSWave - 1, 64);
-    {
-      unsigned m = m32;
-      for (int q = 0; q < c32; ++q) {
-        int c = __ffs(m) - 1;
-        m &= m - 1;
-        s_item[o32 + q] = (unsigned short)((lane << 8) | c);
-      }
-      m = m64;
-      for (int q = 0; q < c64; ++q) {
-        int c = __ffs(m) - 1;
-        m &= m - 1;
-        s_item[t32 + o64 + q] = (unsigned short)((lane << 8) | c);
-      }
+    int o32 = wave_exclusive_scan(c32, lane), o64 = wave_exclusive_scan(c64, lane);
+    s_mask[threadIdx.x] = m32 | m64;
+    if (lane == 63) {
+      s_total[wave] = o64 + c64;
+      s_total[kSSWaves + wave] = o32 + c32;
     }
+    if (threadIdx.x == 0) *s_next = 0;
     __syncthreads();
-    // sun transmittance T(p_i, l) of every listed item: the FP32 list, then the FP64 list, so the two
-    // loops never share a wavefront
-    for (int it = lane; it < t32; it += kSSWave) {
-      const unsigned item = s_item[it];
-      const int owner = item >> 8, i = i0 + (int)(item & 255);
-      const double h = s_h[i];
-      const double pl = s_xl[owner] + s_t[i] * s_vl[owner];  // dot(p_i, l)
-      const double Ds = sun_exit_distance(P.g, h, pl);
-      const float3 Ts = segment_transmittance_f32(P, make_segment(P, h, pl, Ds), Ds, n);
-      s_res[it] = Ts.x;
-      s_res[it + kSSWave * kSSChunk] = Ts.y;
-      s_res[it + 2 * kSSWave * kSSChunk] = Ts.z;
+    int t32 = 0, t64 = 0;
+#pragma unroll
+    for (int w = 0; w < kSSWaves; ++w) {
+      const int a = s_total[w], b = s_total[kSSWaves + w];
+      if (w < wave) {
+        o64 += a;
+        o32 += b;
+      }
+      t64 += a;
+      t32 += b;
     }
-    for (int it = t32 + lane; it < t32 + t64; it += kSSWave) {
-      const unsigned item = s_item[it];
-      const int owner = item >> 8, i = i0 + (int)(item & 255);
-      const double h = s_h[i];
-      const double pl = s_xl[owner] + s_t[i] * s_vl[owner];
-      const double Ds = sun_exit_distance(P.g, h, pl);
-      const float3 Ts = segment_transmittance_f64(P, make_segment(P, h, pl, Ds), Ds, n);
-      s_res[it] = Ts.x;
-      s_res[it + kSSWave * kSSChunk] = Ts.y;
-      s_res[it + 2 * kSSWave * kSSChunk] = Ts.z;
-    }
+    for (unsigned m = m64; m; m &= m - 1) s_item[o64++] = (unsigned short)((__ffs(m) - 1) * kSSEntries + lane);
+    for (unsigned m = m32; m; m &= m - 1) s_item[t64 + o32++] = (unsigned short)((__ffs(m) - 1) * kSSEntries + lane);
     __syncthreads();
-    {
+    // sun transmittance T(p_i, l) of every listed item; the two loops never share a wavefront
+    const int u64 = (t64 + 63) / 64, units = u64 + (t32 + 63) / 64;
+    for (;;) {
+      int u = 0;
+      if (lane == 0) u = atomicAdd(s_next, 1);
+      u = __builtin_amdgcn_readfirstlane(u);
+      if (u >= units) break;
+      const bool wide = u < u64;
+      const int it = wide ? u * 64 + lane : t64 + (u - u64) * 64 + lane;
+      if (it < (wide ? t64 : t64 + t32)) {
+        const unsigned item = s_item[it], owner = item & (kSSEntries - 1);
+        const int i = i0 + (int)(item / kSSEntries);
+        const double h = s_h[i];
+        const double pl = s_xl[owner] + s_t[i] * s_vl[owner];  // dot(p_i, l)
+        const double Ds = sun_exit_distance(P.g, h, pl);
+        const Segment g = make_segment(P, h, pl, Ds);
+        const float3 Ts = wide ? segment_transmittance_f64(P, g, Ds, n) : segment_transmittance_f32(P, g, Ds, n);
+        s_res[item] = Ts.x;
+        s_res[item + kItems] = Ts.y;
+        s_res[item + 2 * kItems] = Ts.z;
+      }
+    }
+    samples += (unsigned long long)(c32 + c64) * n;
+    __syncthreads();
+    if (wave == 0) {
       // each entry adds its lit samples in sample order (deterministic sums)
-      unsigned m = m32 | m64;
-      int r32 = o32, r64 = t32 + o64;
-      while (m) {
-        const int c = __ffs(m) - 1;
-        m &= m - 1;
-        const int idx = ((m32 >> c) & 1u) ? r32++ : r64++;
-        const float3 Ts = make_float3(s_res[idx], s_res[idx + kSSWave * kSSChunk], s_res[idx + 2 * kSSWave * kSSChunk]);
+      unsigned m = 0;
+#pragma unroll
+      for (int w = 0; w < kSSWaves; ++w) m |= s_mask[w * kSSEntries + lane];
+      for (; m; m &= m - 1) {
+        const int c = __ffs(m) - 1, idx = c * kSSEntries + lane;
+        const float3 Ts = make_float3(s_res[idx], s_res[idx + kItems], s_res[idx + 2 * kItems]);
         const float4 w = s_w[i0 + c];
         const float br = s_bray[i0 + c];
         const float3 t3 = make_float3(w.x * Ts.x, w.y * Ts.y, w.z * Ts.z);
@@ -513,10 +548,9 @@ __global__ void __launch_bounds__(kSSWave) single_scatter_kernel(const DevParams
         accM.x += t3.x * w.w; accM.y += t3.y * w.w; accM.z += t3.z * w.w;
       }
     }
-    samples += (unsigned long long)(c32 + c64) * n;
     __syncthreads();
   }
-  if (valid) {
+  if (valid && wave == 0) {
     const long long o = (long long)rayid * NLA + k;
     float a = (float)dt;
     float pr = phase_f(P.g_ray, (float)vl) * a;
@@ -525,7 +559,6 @@ __global__ void __launch_bounds__(kSSWave) single_scatter_kernel(const DevParams
     M1[o] = make_float4(accM.x * P.sca_mie[0] * P.intensity[0] * a, accM.y * P.sca_mie[1] * P.intensity[1] * a,
                         accM.z * P.sca_mie[2] * P.intensity[2] * a, 0.f);
   }
-  unsigned long long view = (lane < n) ? (unsigned long long)n * ((n - lane + kSSWave - 1) / kSSWave) : 0;
   count(wc, samples, samples + view, 0, 0);
 }
 
@@ -2068,11 +2101,9 @@ hipError_t launch_single_scatter(const DevParams& P, float4* rayleigh, float4* m
     const hipError_t e = launch_ray_items(P, stream);
     if (e != hipSuccess) return e;
   }
-  unsigned groups = (unsigned)((P.nS[2] * P.nS[3] + kSSWave - 1) / kSSWave);
-  int n = P.ray_steps;
-  size_t shmem = (size_t)n * (2 * sizeof(double) + sizeof(float4)) + sizeof(float) * (size_t)((n + 3) & ~3) +
-                 (3 * sizeof(float) + sizeof(unsigned short)) * kSSWave * kSSChunk + 2 * sizeof(double) * kSSWave;
-  hipLaunchKernelGGL(single_scatter_kernel, dim3(rays * groups), dim3(kSSWave), shmem, stream, P, rayleigh, mie, wc);
+  const unsigned groups = (unsigned)((P.nS[2] * P.nS[3] + kSSEntries - 1) / kSSEntries);
+  hipLaunchKernelGGL(single_scatter_kernel, dim3(rays * groups), dim3(kSSEntries * kSSWaves),
+                     single_scatter_shared_bytes(P.ray_steps), stream, P, rayleigh, mie, wc);
   return hipGetLastError();
 }
 
