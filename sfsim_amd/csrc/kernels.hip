@@ -1264,7 +1264,6 @@ __global__ void __launch_bounds__(kBlock) direction_geometry_kernel(const DevPar
 // Constants of the per-direction lookups of one point-scatter launch.
 struct PsConst {
   float hA;            // (NA - 1) / 2: heading coordinate (NA - 1) (1 + dot(omega, l)) / 2 = hA + hA dot(omega, l)
-  float na_top;        // NA - 1
   SunCoord se;         // sun-elevation coordinate of dE (size nE[1]): alpha = -3 log2(e), beta = 0
   float mie_k, mie_a, mie_b;  // Mie phase K (1 + mu^2) (a - b mu)^(-3/2): K = 3 (1 - g^2) / (8 pi (2 + g^2))
 };
@@ -1305,6 +1304,22 @@ __device__ __forceinline__ void surface_radiance_entry(const DevParams& P, int n
                                                        const float4* __restrict__ mie, float4* __restrict__ out,
                                                        WorkCounters* wc, int entry, float4* s_fold, float3* s_red);
 
+// A lookup's byte address base + column x pitch, formed as the bits of a denormal float: bases and pitches are below
+// 2^23, so the sum is exact and the column needs no conversion to an integer.  The multiply-add and the subtraction
+// that finds the column issue at twice the rate of a conversion, an integer multiply-add or a clamp.
+__device__ __forceinline__ unsigned lds_address(float column, unsigned pitch, unsigned base) {
+  return __float_as_uint(fmaf(column, __uint_as_float(pitch), __uint_as_float(base)));
+}
+
+// LDS by address, for a kernel without static LDS, whose dynamic LDS begins at 0.  (As an offset from the array it
+// would cost an addition of the array's place, 0, at each access.)
+typedef float Vec2 __attribute__((ext_vector_type(2)));
+typedef float Vec4 __attribute__((ext_vector_type(4)));
+template <class T>
+__device__ __forceinline__ T lds_read(unsigned address) {
+  return *(__attribute__((address_space(3))) const T*)(uintptr_t)address;
+}
+
 // The split of a point-scatter launch.  A workgroup takes `rays` view rays of one height and `rows` sun elevations,
 // `waves` wavefronts per ray (64 EPT entries each); eblocks x sblocks workgroups per height.  pitch: texels per
 // column of its slab; misc: bytes of the weights and dE in LDS (below the slabs, see ps_shared_bytes).
@@ -1315,13 +1330,20 @@ struct PsPlan {
 
 // LDS of a workgroup: the folded slab of one latitude ring, double-buffered (and of the Mie strength in the first
 // iteration), a texel for each column and sun elevation: its colour and the difference to the next column's, six
-// floats in two planes: 16 bytes (colour, first difference) at byte address A, the other 8 at A / 2.  The last
-// column, which only the heading coordinate NA - 1 reads, holds the column before it plus its difference (what the
-// interpolation between the two gives at weight 1) and no difference, so a lookup needs no clamped lower column.
+// floats in two planes: 16 bytes (colour, first difference) at byte address A, the other 8 at A / 2.  Column NA - 1
+// holds the column before it plus its difference (what the interpolation between the two gives at weight 1) and no
+// difference, and a column -1 column 0's colour and no difference: a heading coordinate that rounding has left just
+// outside 0 ... NA - 1 gives what the clamped one would, so a lookup clamps neither the coordinate nor the column.
 // The 8-byte plane begins at `misc` (at least its own size) and the 16-byte plane at 2 misc; the weights, dE (laid
 // out alike) and the surface-radiance workgroups' partial sums take the bytes below.
+// Where the directions' components are read: from LDS with one entry per lane, whose few lookups do not cover the
+// latency of scalar loads (19 x 45 x 20 x 7 entries, 38 directions: 17.4 us against 19.1); from scalar registers with
+// two entries per lane, which read more of the LDS per direction (1408 us against 1317 at 64 x 128 x 64 x 16 with 262
+// directions), and with the Mie strength (24 x 48 x 24 x 9, 134 directions: 69.2 us against 66.1).
+__host__ __device__ constexpr bool ps_omega_in_lds(int ept, bool mie) { return ept == 1 && !mie; }
+
 __host__ __device__ inline unsigned ps_texels(const PsPlan& p, int na, bool mie) {
-  return 2u * (mie ? 2u : 1u) * (unsigned)p.pitch * (unsigned)na;
+  return 2u * (mie ? 2u : 1u) * (unsigned)p.pitch * (unsigned)(na + 1);
 }
 __host__ __device__ inline size_t ps_shared_bytes(const PsPlan& p, int na, bool mie) {
   return 2 * (size_t)p.misc + 16 * (size_t)ps_texels(p, na, mie);
@@ -1340,9 +1362,12 @@ struct PsRings {
   unsigned short start[kMaxRings + 1];
 };
 
-// What bounds it is VALU issue: about 14 instruction slots per (entry, sky direction) and 34 per ground direction, beside
-// 24 bytes of LDS reads per lookup.  The slab of a ring is shared by the ring's directions and by the rays of a
-// height, so it is folded in the kernel itself (nine times fewer texels than one slab per direction, and no
+// What bounds it is VALU issue and, close behind, the LDS: 13 instructions per (entry, sky direction), 3 of them of the
+// kinds that issue at half rate, and some 32 per ground direction, beside 24 bytes of LDS reads per lookup (at
+// 64 x 128 x 64 x 16 and 262 directions the LDS is busy for 3/4 of the launch).  Lookup addresses formed as floats and
+// columns that need no clamp took that launch from 1370 to 1317 us, and 19 x 45 x 20 x 7 with 38 directions from 18.9 to
+// 17.4 us together with directions read from LDS.  The slab of a ring is shared by the ring's directions and by the
+// rays of a height, so it is folded in the kernel itself (nine times fewer texels than one slab per direction, and no
 // launch, table or gather from L2 for them); lanes run over the sun elevations of a column, so that their reads of a
 // slab's columns are contiguous whatever columns they need.
 //
@@ -1384,12 +1409,14 @@ __global__ void __launch_bounds__(kBlock) point_scatter_kernel(
   float4* s_w = s_mem;                                    // [rays][ndirs] rgb quadrature weight times in-scattering
   float4* s_ea = s_w + plan.rays * ndirs;                 // dE at the ground and the differences to the next entry's,
   float2* s_eb = (float2*)(s_ea + (kELds ? nE1 : 0));     // as the slabs' texels
+  float2* s_om = s_eb + (kELds ? nE1 : 0);                // [ndirs] omega's y and z
+  constexpr bool kOmLds = ps_omega_in_lds(EPT, kMie);
   const double r0 = index_to_radius(P.g, NH, ih), h0 = index_to_altitude(P.g, NH, ih);
   const DirGeom* __restrict__ gh = geom + (long long)ih * ndirs;
 
   // Slab of one ring, columns fastest (coalesced reads).
   const int fold_rows = min(plan.pitch, NL - s0), fold_n = NA * fold_rows;
-  const unsigned half = plan.misc, slab_texels = (unsigned)(plan.pitch * NA);
+  const unsigned half = plan.misc, slab_texels = (unsigned)(plan.pitch * (NA + 1));
   const Lerp Lh = make_lerp((float)height_to_index(P.g, NH, r0), NH);
   const long long sh = (long long)NE * NLA;
   auto fold = [&](int ring, unsigned buffer) {
@@ -1403,16 +1430,24 @@ __global__ void __launch_bounds__(kBlock) point_scatter_kernel(
       const int row = i / NA, col = i - row * NA;
       const bool last = col == NA - 1;
       const long long k = (long long)(s0 + row) * NA + col - last;
-      const unsigned t = buffer * (kMie ? 2u : 1u) * slab_texels + (unsigned)(col * plan.pitch + row);
+      const unsigned t = buffer * (kMie ? 2u : 1u) * slab_texels + (unsigned)((col + 1) * plan.pitch + row);
 #pragma unroll
       for (int m = 0; m < (kMie ? 2 : 1); ++m) {
         const float4* __restrict__ tab = m ? mie : dS;
         const unsigned A = 2 * half + 16 * (t + m * slab_texels);
-        ps_store((float4*)(lds + A), (float2*)(lds + (A >> 1)), texel(tab, k), texel(tab, k + 1), last);
+        const float3 u = texel(tab, k);
+        ps_store((float4*)(lds + A), (float2*)(lds + (A >> 1)), u, texel(tab, k + 1), last);
+        if (col == 0) {
+          const unsigned B = A - 16 * plan.pitch;
+          *(float4*)(lds + B) = make_float4(u.x, u.y, u.z, 0.f);
+          *(float2*)(lds + (B >> 1)) = make_float2(0.f, 0.f);
+        }
       }
     }
   };
 
+  if (kOmLds)
+    for (int j = threadIdx.x; j < ndirs; j += blockDim.x) s_om[j] = make_float2(gh[j].omega.y, gh[j].omega.z);
   if (kELds)
     for (int i = threadIdx.x; i < nE1; i += blockDim.x) {
       const int k = min(i, nE1 - 2);
@@ -1435,7 +1470,6 @@ __global__ void __launch_bounds__(kBlock) point_scatter_kernel(
   }
   PsConst pc;
   pc.hA = 0.5f * (float)(NA - 1);
-  pc.na_top = (float)(NA - 1);
   pc.se = SunCoord{(float)((nE1 - 1) * (double)P.sun_inv_den), (float)(-0.6 * 1.4426950408889634), (float)(nE1 - 1)};
   mie_constants(P.g_mie, pc);
 
@@ -1459,13 +1493,13 @@ __global__ void __launch_bounds__(kBlock) point_scatter_kernel(
     lz[e] = m.z;
     s_up[e] = s0 + is == 0 ? make_lerp(m.w, NL).s : 0.0f;
     two = two || s_up[e] != 0.0f;
-    row_bytes[e] = 2 * half + 16 * is;
+    row_bytes[e] = 2 * half + 16 * (plan.pitch + is);
     acc[e] = make_float3(0.f, 0.f, 0.f);
   }
   two = __any(two);
   fold(0, 0);
   __syncthreads();
-  const unsigned pitch_bytes = 16 * plan.pitch;
+  const unsigned pitch_bytes = 16 * plan.pitch, ea_bytes = (unsigned)((char*)s_ea - lds), eb_bytes = (unsigned)((char*)s_eb - lds);
   for (int ring = 0; ring < rings.count; ++ring) {
     if (ring + 1 < rings.count) fold(ring + 1, (ring + 1) & 1);
     if (active) {
@@ -1474,8 +1508,8 @@ __global__ void __launch_bounds__(kBlock) point_scatter_kernel(
       const unsigned buffer_bytes = (ring & 1) * (kMie ? 32u : 16u) * slab_texels;
       // one lookup of the slab at byte address A: colour + s x difference
       auto lerp_at = [&](unsigned A, float s) {
-        const float4 u = *(const float4*)(lds + A);
-        const float2 d = *(const float2*)(lds + (A >> 1));
+        const Vec4 u = lds_read<Vec4>(A);
+        const Vec2 d = lds_read<Vec2>(A >> 1);
         return make_float3(fmaf(s, u.w, u.x), fmaf(s, d.x, u.y), fmaf(s, d.y, u.z));
       };
       auto lookup = [&](unsigned A, float sa, int e, bool second) {
@@ -1498,13 +1532,13 @@ __global__ void __launch_bounds__(kBlock) point_scatter_kernel(
         }
 #pragma unroll 2
         for (int j = j0; j < j1; ++j) {
-          const float4 om = gh[j].omega, w = s_w[r * ndirs + j];
+          const float4 w = s_w[r * ndirs + j];
+          const float2 om = kOmLds ? s_om[j] : make_float2(gh[j].omega.y, gh[j].omega.z);
 #pragma unroll
           for (int e = 0; e < EPT; ++e) {
-            const float ol = fmaf(om.z, lz[e], fmaf(om.y, ly[e], x0[e]));
-            const float hc = __builtin_amdgcn_fmed3f(fmaf(pc.hA, ol, pc.hA), 0.0f, pc.na_top);
-            const float sa = __builtin_amdgcn_fractf(hc);
-            const unsigned A = __umul24((unsigned)hc, pitch_bytes) + rb[e];
+            const float ol = fmaf(om.y, lz[e], fmaf(om.x, ly[e], x0[e]));
+            const float hc = fmaf(pc.hA, ol, pc.hA), sa = __builtin_amdgcn_fractf(hc);
+            const unsigned A = lds_address(hc - sa, pitch_bytes, rb[e]);
             float3 v = lookup(A, sa, e, second);
             if (kMie) {
               const float3 m = lookup(A + 16 * slab_texels, sa, e, second);
@@ -1520,10 +1554,9 @@ __global__ void __launch_bounds__(kBlock) point_scatter_kernel(
                   fmaf(-pc.se.A, fexp2(fmaf(-3.0f * 1.4426950408889634f, spl, pc.se.c)), pc.se.A), 0.0f, pc.se.top);
               float3 u;  // of height row 0: P is on the ground
               if (kELds) {
-                const unsigned i = (unsigned)ce;
-                const float s = __builtin_amdgcn_fractf(ce);
-                const float4 c = s_ea[i];
-                const float2 d = s_eb[i];
+                const float s = __builtin_amdgcn_fractf(ce), i = ce - s;
+                const Vec4 c = lds_read<Vec4>(lds_address(i, 16, ea_bytes));
+                const Vec2 d = lds_read<Vec2>(lds_address(i, 8, eb_bytes));
                 u = make_float3(fmaf(s, c.w, c.x), fmaf(s, d.x, c.y), fmaf(s, d.y, c.z));
               } else {
                 const float ecol = lower_cell(ce, pc.se.top - 1.0f);
@@ -2136,7 +2169,7 @@ static PsPlan point_scatter_plan(const DevParams& P, int ndirs, bool e_lds, int&
   p.waves = (slots + ept - 1) / ept;
   p.rays = 4 / p.waves;
   p.eblocks = (P.nS[1] + p.rays - 1) / p.rays;
-  const size_t misc = sizeof(float4) * (size_t)p.rays * ndirs + (e_lds ? 24 * (size_t)P.nE[1] : 0);
+  const size_t misc = sizeof(float4) * (size_t)p.rays * ndirs + (ps_omega_in_lds(ept, kMie) ? 8 * (size_t)ndirs : 0) + (e_lds ? 24 * (size_t)P.nE[1] : 0);
   p.misc = (unsigned)(std::max<size_t>(misc, 8 * (size_t)ps_texels(p, NA, kMie)) + 15) & ~15u;
   return p;
 }
