@@ -178,10 +178,17 @@ SFSIM_HD double ground_distance(const Geo& g, double h, double pd) {
 }
 
 // atmosphere.clj:95-102 for a point of altitude h and dot(direction, point) = pd
-SFSIM_HD bool is_above_horizon(const Geo& g, double h, double pd) {
+SFSIM_HD double radius_excess(const Geo& g, double h) {
   SFSIM_EXACT
-  return (pd >= 0) || (sqr(pd) <= h * (2.0 * g.R + h));
+  return h * (2.0 * g.R + h);
 }
+
+SFSIM_HD bool is_above_horizon_at(double excess, double pd) {
+  SFSIM_EXACT
+  return (pd >= 0) || (sqr(pd) <= excess);
+}
+
+SFSIM_HD bool is_above_horizon(const Geo& g, double h, double pd) { return is_above_horizon_at(radius_excess(g, h), pd); }
 
 // Altitude after travelling t along a unit direction from altitude h0 with dot(point, direction) = pd0:
 // r(t)^2 - R^2 = h0 (2R + h0) + t (2 pd0 + t),  h = (r^2 - R^2) / (r + R).
