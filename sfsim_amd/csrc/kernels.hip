@@ -846,9 +846,13 @@ __global__ void __launch_bounds__(kSSTBlock) single_scatter_table_kernel(
 //
 // One workgroup per view ray.  A wavefront owns a group of columns (TS x 64 folded texels at most) and a
 // contiguous segment of the ray's samples: it folds its columns into a slab of its own in LDS and looks its
-// items up there, so no barrier separates the two.  What bounds it is VALU issue: per sample and wavefront
-// of the 32 x 64 x 32 x 8 grid 4 x 12 multiply-adds of the fold and 5 x 20 instructions of the lookups, with
-// the nodes' loads (L2) and the slab's LDS reads behind them.
+// items up there, so no barrier separates the two.  What bounds it is the LDS (busy for 2/3 to 3/4 of a launch) and the
+// latency between a sample's writes and reads, which 4 wavefronts per SIMD cover in part: per sample and wavefront of the
+// 32 x 64 x 32 x 8 grid 4 texels written and 5 lookups of two texels each, beside 4 x 12 multiply-adds of the fold and
+// 5 x 20 instructions of the lookups.  A slab therefore lies in two planes, red and green in 8 bytes at byte address A and
+// blue in 4 at A / 2: a 16-byte write takes 13.4 clocks where one of 8 and one of 4 take 10.7, and the rows of a column
+// then meet in a bank 32 (64) rows apart instead of 16.  57.4 -> 53.6 us; 64 x 128 x 64 x 16 with 128 samples 1385 -> 1235 us,
+// 32 x 127 x 32 x 8 with 100 samples 159 -> 143 us.
 //
 // The sun-elevation coordinate of sun-elevation-to-index (atmosphere.clj:322-326) at p_i,
 // (NL - 1) max(0, (1 - exp(-3 s - 0.6)) / (1 - exp(-3.6))) with s = dot(p_i, l) / |p_i| = (xl + t_i vl) / r_i, is
@@ -908,6 +912,30 @@ __device__ __forceinline__ FoldStep fold_step(ConstFoldSteps fs, int i) {
   return st;
 }
 
+// A lookup's byte address base + column x pitch, formed as the bits of a denormal float: bases and pitches are below
+// 2^23, so the sum is exact and the column needs no conversion to an integer.  The multiply-add and the subtraction
+// that finds the column issue at twice the rate of a conversion, an integer multiply-add or a clamp.
+__device__ __forceinline__ unsigned lds_address(float column, unsigned pitch, unsigned base) {
+  return __float_as_uint(fmaf(column, __uint_as_float(pitch), __uint_as_float(base)));
+}
+
+// LDS by address, for a kernel without static LDS, whose dynamic LDS begins at 0.  (As an offset from the array it
+// would cost an addition of the array's place, 0, at each access.)
+typedef float Vec2 __attribute__((ext_vector_type(2)));
+typedef float Vec4 __attribute__((ext_vector_type(4)));
+template <class T>
+__device__ __forceinline__ void lds_write(unsigned address, T v) {
+  *(__attribute__((address_space(3))) T*)(uintptr_t)address = v;
+}
+
+template <class T>
+__device__ __forceinline__ T lds_read(unsigned address) {
+  return *(__attribute__((address_space(3))) const T*)(uintptr_t)address;
+}
+
+// The split of a point-scatter launch.  A workgroup takes `rays` view rays of one height and `rows` sun elevations,
+// `waves` wavefronts per ray (64 EPT entries each); eblocks x sblocks workgroups per height.  pitch: texels per
+// column of its slab; misc: bytes of the weights and dE in LDS (below the slabs, see ps_shared_bytes).
 // Orders LDS accesses of one wavefront's lanes (the hardware keeps a wavefront's LDS accesses in order; this
 // keeps the compiler from moving them across).
 __device__ __forceinline__ void wave_fence() {
@@ -959,7 +987,9 @@ __host__ __device__ constexpr int rs_texels(bool exact) {
   return 64 * TS + (exact ? 32 * TS : 4 * TS);
 }
 
-// LDS of one workgroup: the wavefronts' slabs, whose place the item sums take later ([segs][3][groups x items]).
+// LDS of one workgroup: the wavefronts' slabs, whose place the item sums take later ([segs][3][groups x items]).  For W
+// wavefronts of N texels the 4-byte plane lies at 4 W N and the 8-byte plane at 8 W N: 16 bytes per texel, of which the
+// first 4 are not used, and no offset between an address and its half.
 template <int TS>
 __host__ __device__ inline size_t rs_shared_bytes(int groups, int segs, bool exact) {
   const size_t slabs = (size_t)groups * segs * rs_texels<TS>(exact) * sizeof(float4);
@@ -972,7 +1002,7 @@ __host__ __device__ inline size_t rs_shared_bytes(int groups, int segs, bool exa
 template <int TS, int NS, bool kExact, class Steps>
 __device__ __forceinline__ void rs_segment(const float* __restrict__ dJ, const Steps gF, const float4* __restrict__ gT,
                                            const float4* __restrict__ gRS, const double2* __restrict__ gTH, int i0, int i1,
-                                           int bytes, float4* slab, const unsigned (&laddr)[TS],
+                                           int bytes, unsigned slab, const unsigned (&laddr)[TS],
                                            const RsItem* __restrict__ items, int nitems, const double2* __restrict__ ss,
                                            int col0, int pitch, const SunCoord& sc, double R, double A64, int lane,
                                            float* s_out, int out_pitch) {
@@ -997,7 +1027,7 @@ __device__ __forceinline__ void rs_segment(const float* __restrict__ dJ, const S
       vl64[j] = d.x;
       xl64[j] = d.y;
     }
-    caddr[j] = ((it.at >> 16) - col0) * pitch * (unsigned)sizeof(float4);
+    caddr[j] = slab + ((it.at >> 16) - col0) * pitch * 8u;
     acc[j] = Rgb{0.f, 0.f, 0.f};
   }
   for (int i = i0; i < i1; ++i) {
@@ -1005,9 +1035,9 @@ __device__ __forceinline__ void rs_segment(const float* __restrict__ dJ, const S
 #pragma unroll
     for (int j = 0; j < TS; ++j) {
       const Rgb a = f.v[0][j], b = f.v[1][j], c = f.v[2][j], d = f.v[3][j];
-      *(float4*)((char*)slab + laddr[j]) = make_float4(fmaf(w.w, d.x, fmaf(w.z, c.x, fmaf(w.y, b.x, w.x * a.x))),
-                                                       fmaf(w.w, d.y, fmaf(w.z, c.y, fmaf(w.y, b.y, w.x * a.y))),
-                                                       fmaf(w.w, d.z, fmaf(w.z, c.z, fmaf(w.y, b.z, w.x * a.z))), 0.f);
+      lds_write(laddr[j], Vec2{fmaf(w.w, d.x, fmaf(w.z, c.x, fmaf(w.y, b.x, w.x * a.x))),
+                               fmaf(w.w, d.y, fmaf(w.z, c.y, fmaf(w.y, b.y, w.x * a.y)))});
+      lds_write(laddr[j] >> 1, fmaf(w.w, d.z, fmaf(w.z, c.z, fmaf(w.y, b.z, w.x * a.z))));
     }
     wave_fence();
     // the next sample's nodes, in flight during this sample's lookups
@@ -1017,17 +1047,21 @@ __device__ __forceinline__ void rs_segment(const float* __restrict__ dJ, const S
     const float4 T = gT[i], g = gRS[i];  // uniform: scalar loads
 #pragma unroll
     for (int j = 0; j < NS; ++j) {
-      unsigned row;
+      unsigned A;
       float s;
       if (kExact) {
+        unsigned row;
         sun_coord_exact(sc, A64, R, gTH[i], xl64[j], vl64[j], row, s);
+        A = caddr[j] + row * 8;
       } else {
         const float c = sun_coord(sc, make_float2(g.z, g.w), xl[j], vl[j]);
-        row = (unsigned)c;
         s = __builtin_amdgcn_fractf(c);
+        A = lds_address(c - s, 8, caddr[j]);
       }
-      const float4* p = (const float4*)((const char*)slab + (caddr[j] + row * (unsigned)sizeof(float4)));
-      const float3 v = lerp3(p[0], p[1], s);
+      const unsigned B = A >> 1;
+      const Vec2 u0 = lds_read<Vec2>(A), u1 = lds_read<Vec2>(A + 8);
+      const float b0 = lds_read<float>(B), b1 = lds_read<float>(B + 4);
+      const float3 v = make_float3(fmaf(s, u1[0] - u0[0], u0[0]), fmaf(s, u1[1] - u0[1], u0[1]), fmaf(s, b1 - b0, b0));
       acc[j].x = fmaf(T.x, v.x, acc[j].x);
       acc[j].y = fmaf(T.y, v.y, acc[j].y);
       acc[j].z = fmaf(T.z, v.z, acc[j].z);
@@ -1155,14 +1189,18 @@ __global__ void __launch_bounds__(1024) ray_scatter_kernel(
     const int nitems = head[group + 1] - head[group];
     // the lane's texels in the LDS slab; those past the group's texels write zeros to the last column's zero texel
     const int col0 = group * P.rs_cols, ncols = min(P.rs_cols, NA - col0), pitch = NL + 1;
-    float4* slab = s_mem + wave * rs_texels<TS>(kExact);
+    const unsigned texels = rs_texels<TS>(kExact), slab = 8 * (texels * (unsigned)(blockDim.x >> 6) + wave * texels);
     unsigned laddr[TS];
 #pragma unroll
     for (int j = 0; j < TS; ++j) {
       const unsigned t = 64 * j + lane;
-      laddr[j] = (t < (unsigned)(ncols * NL) ? t + t / (unsigned)NL : (unsigned)(ncols * pitch - 1)) * (unsigned)sizeof(float4);
+      laddr[j] = (t < (unsigned)(ncols * NL) ? t + t / (unsigned)NL : (unsigned)(ncols * pitch - 1)) * 8u + slab;
     }
-    for (int i = lane; i < ncols; i += 64) slab[i * pitch + NL] = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int i = lane; i < ncols; i += 64) {
+      const unsigned A = slab + (i * pitch + NL) * 8;
+      lds_write(A, Vec2{0.f, 0.f});
+      lds_write(A >> 1, 0.f);
+    }
     const int i0 = (int)((long long)n * seg / segs), i1 = (int)((long long)n * (seg + 1) / segs);
     const RsItem* __restrict__ it = items + 2 * base + head[group];
     float* s_out = (float*)s_mem + (size_t)seg * 3 * pitch_out + group * rs_items(TS);
@@ -1323,25 +1361,6 @@ __device__ __forceinline__ void surface_radiance_entry(const DevParams& P, int n
                                                        const float4* __restrict__ mie, float4* __restrict__ out,
                                                        WorkCounters* wc, int entry, float4* s_fold, float3* s_red);
 
-// A lookup's byte address base + column x pitch, formed as the bits of a denormal float: bases and pitches are below
-// 2^23, so the sum is exact and the column needs no conversion to an integer.  The multiply-add and the subtraction
-// that finds the column issue at twice the rate of a conversion, an integer multiply-add or a clamp.
-__device__ __forceinline__ unsigned lds_address(float column, unsigned pitch, unsigned base) {
-  return __float_as_uint(fmaf(column, __uint_as_float(pitch), __uint_as_float(base)));
-}
-
-// LDS by address, for a kernel without static LDS, whose dynamic LDS begins at 0.  (As an offset from the array it
-// would cost an addition of the array's place, 0, at each access.)
-typedef float Vec2 __attribute__((ext_vector_type(2)));
-typedef float Vec4 __attribute__((ext_vector_type(4)));
-template <class T>
-__device__ __forceinline__ T lds_read(unsigned address) {
-  return *(__attribute__((address_space(3))) const T*)(uintptr_t)address;
-}
-
-// The split of a point-scatter launch.  A workgroup takes `rays` view rays of one height and `rows` sun elevations,
-// `waves` wavefronts per ray (64 EPT entries each); eblocks x sblocks workgroups per height.  pitch: texels per
-// column of its slab; misc: bytes of the weights and dE in LDS (below the slabs, see ps_shared_bytes).
 struct PsPlan {
   int rows, sblocks, rays, waves, eblocks, pitch;
   unsigned misc;
