@@ -139,10 +139,20 @@ struct HostCopier {
     if (pinned) (void)hipHostFree(pinned);
   }
 
-  // The ring, made on first use; false (and no ring held) where it cannot be had.
+  // The pinned memory, made on first use; false where it cannot be had.
   bool ready(int dev) {
     if (pinned) return true;
     device = dev;
+    if (hipHostMalloc((void**)&pinned, kSlots * kChunk, hipHostMallocDefault) != hipSuccess) {
+      pinned = nullptr;
+      (void)hipGetLastError();
+    }
+    return pinned != nullptr;
+  }
+
+  // With it what more than one chunk needs (a first small copy does not wait for a stream to be made).
+  bool ring_ready(int dev) {
+    if (!ready(dev)) return false;
     auto made = [](hipEvent_t& e) {
       if (e || hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess) return true;
       e = nullptr;
@@ -151,9 +161,9 @@ struct HostCopier {
     bool ok = made(begin);
     for (hipEvent_t& e : event) ok = ok && made(e);
     if (ok && !side && hipStreamCreateWithFlags(&side, hipStreamNonBlocking) != hipSuccess) side = nullptr;
-    if (ok && side && hipHostMalloc((void**)&pinned, kSlots * kChunk, hipHostMallocDefault) != hipSuccess) pinned = nullptr;
-    if (!pinned) (void)hipGetLastError();
-    return pinned != nullptr;
+    if (ok && side) return true;
+    (void)hipGetLastError();
+    return false;
   }
 
   CopyOut piece(int c) const {
@@ -1229,13 +1239,14 @@ int copy_out(sfsim_atmo_ctx* ctx, const CopyOut* list, int count) {
   HostCopier& h = ctx->copier;
   size_t total = 0;
   for (int i = 0; i < count; ++i) total += list[i].bytes;
-  if (!h.ready(ctx->device)) {
+  const bool small = total <= HostCopier::kChunk;
+  if (small ? !h.ready(ctx->device) : !h.ring_ready(ctx->device)) {
     for (int i = 0; i < count; ++i)
       HIP_TRY(ctx, hipMemcpyAsync(list[i].dst, list[i].src, list[i].bytes, hipMemcpyDeviceToHost, ctx->stream));
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
     return 0;
   }
-  if (total <= HostCopier::kChunk) {
+  if (small) {
     size_t at = 0;
     for (int i = 0; i < count; at += list[i++].bytes)
       HIP_TRY(ctx, hipMemcpyAsync(h.pinned + at, list[i].src, list[i].bytes, hipMemcpyDeviceToHost, ctx->stream));
