@@ -312,7 +312,7 @@ __device__ __forceinline__ void count(WorkCounters* wc, unsigned long long singl
 // XCD-aware order of the view rays: workgroups are dispatched to the 8 XCDs round robin (workgroup b
 // to XCD b mod 8), each with its own L2.  Giving XCD x the contiguous range of rays
 // [x rays / 8, (x + 1) rays / 8) (4 of 32 heights at the full workload) keeps the tables that a height
-// range reads (dJ cells, point-scatter slabs, sun-table rows) in fewer L2s.  A bijection when rays is a
+// range reads (dJ cells, dS rows, sun-table rows) in fewer L2s.  A bijection when rays is a
 // multiple of 8; identity otherwise.
 constexpr int kXcds = 8;
 __device__ __forceinline__ int xcd_ray(int b, int rays) {
@@ -846,8 +846,9 @@ __global__ void __launch_bounds__(kSSTBlock) single_scatter_table_kernel(
 //
 // One workgroup per view ray.  A wavefront owns a group of columns (TS x 64 folded texels at most) and a
 // contiguous segment of the ray's samples: it folds its columns into a slab of its own in LDS and looks its
-// items up there, so no barrier separates the two.  What bounds it is the LDS (busy for 2/3 to 3/4 of a launch) and the
-// latency between a sample's writes and reads, which 4 wavefronts per SIMD cover in part: per sample and wavefront of the
+// items up there, so no barrier separates the two.  What bounds it is the LDS (busy for half of a
+// launch) and the latency between a sample's writes and reads, which 4 wavefronts per SIMD cover in part (they wait for
+// half of their time; a fifth wavefront spills registers, 60 us): per sample and wavefront of the
 // 32 x 64 x 32 x 8 grid 4 texels written and 5 lookups of two texels each, beside 4 x 12 multiply-adds of the fold and
 // 5 x 20 instructions of the lookups.  A slab therefore lies in two planes, red and green in 8 bytes at byte address A and
 // blue in 4 at A / 2: a 16-byte write takes 13.4 clocks where one of 8 and one of 4 take 10.7, and the rows of a column
