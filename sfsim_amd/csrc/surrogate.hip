@@ -45,16 +45,11 @@ __host__ __device__ inline uint64_t splitmix64(uint64_t x) {
 }
 
 // The 17 Fourier features of one input x: x, then sin / cos (2^b pi x) for b = 0..7 (bf16).
-__device__ inline void encode_value(float v, uint16_t* out) {
-  out[0] = f2bf(v);
-  float a = 3.14159265358979f * v;
-  for (int b = 0; b < 8; ++b) {
-    float sn, cs;
-    sincosf(a, &sn, &cs);
-    out[1 + 2 * b] = f2bf(sn);
-    out[2 + 2 * b] = f2bf(cs);
-    a *= 2.0f;  // exact
-  }
+__device__ inline uint16_t encode_feature(float v, int q) {
+  if (q == 0) return f2bf(v);
+  float sn, cs;
+  sincosf(ldexpf(3.14159265358979f * v, (q - 1) >> 1), &sn, &cs);
+  return f2bf(q & 1 ? sn : cs);
 }
 
 __device__ inline void entry_coords(const GridShape& P, long long entry, float* x) {
@@ -463,24 +458,25 @@ __global__ void to_bf16_kernel(const float* __restrict__ in, uint16_t* __restric
 __global__ void layer1_tables_kernel(const DevParams P, AtmosphereCode code, const uint16_t* __restrict__ wbf,
                                      const float* __restrict__ theta, float* __restrict__ ztab) {
   const int j = threadIdx.x;  // hidden unit (blockDim.x == kMlpHidden)
-  int row = blockIdx.x;
-  uint16_t f[kMlpBands];
-  const uint16_t* W1 = wbf + MlpLayout::W1;
-  float acc;
+  const int row = blockIdx.x;
+  // the row's features, each by one thread (every thread all of them: 8 sines and cosines in a row per input, 18 us)
+  __shared__ float f[6 * kMlpBands];
+  int first = 0, inputs = 1;  // coordinates row: input c of the four
+  float x = 0.f;
   if (row == 0) {
-    acc = theta[MlpLayout::b1 + j];
-    for (int i = 0; i < 6; ++i) {
-      encode_value(code.v[i], f);
-      for (int q = 0; q < kMlpBands; ++q)
-        acc += bf2f(W1[(size_t)(kMlpBands * (4 + i) + q) * kMlpHidden + j]) * bf2f(f[q]);
-    }
+    first = 4;
+    inputs = 6;
+    if (j < 6 * kMlpBands) x = code.v[j / kMlpBands];
   } else {
-    int v = row - 1, c = 0;
-    while (v >= P.nS[c]) v -= P.nS[c++];
-    encode_value((float)v / (float)(P.nS[c] - 1), f);
-    acc = 0.f;
-    for (int q = 0; q < kMlpBands; ++q) acc += bf2f(W1[(size_t)(kMlpBands * c + q) * kMlpHidden + j]) * bf2f(f[q]);
+    int v = row - 1;
+    while (v >= P.nS[first]) v -= P.nS[first++];
+    x = (float)v / (float)(P.nS[first] - 1);
   }
+  if (j < inputs * kMlpBands) f[j] = bf2f(encode_feature(x, j % kMlpBands));
+  __syncthreads();
+  const uint16_t* W1 = wbf + MlpLayout::W1 + (size_t)(kMlpBands * first) * kMlpHidden + j;
+  float acc = row == 0 ? theta[MlpLayout::b1 + j] : 0.f;
+  for (int q = 0; q < inputs * kMlpBands; ++q) acc += bf2f(W1[(size_t)q * kMlpHidden]) * f[q];
   ztab[(size_t)blockIdx.x * kMlpHidden + j] = acc;
 }
 
