@@ -231,6 +231,7 @@ struct HostCopier {
     for (int c = 0; c < std::min(n, kSlots); ++c) queue(c);
     const bool help = n > 2;  // one or two chunks are copied sooner than threads wake
     if (help) {
+      (void)hipEventSynchronize(begin);  // the threads sleep until there is something to copy; an error shows in work()
       std::lock_guard<std::mutex> lock(mu);
       const int most = std::max(0, std::min(kThreads, (int)std::thread::hardware_concurrency() - 1));
       try {
