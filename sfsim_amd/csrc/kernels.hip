@@ -1381,8 +1381,10 @@ struct PsPlan {
 // directions), and with the Mie strength (24 x 48 x 24 x 9, 134 directions: 69.2 us against 66.1).
 __host__ __device__ constexpr bool ps_omega_in_lds(int ept, bool mie) { return ept == 1 && !mie; }
 
+// One texel more than the slabs have: where a wavefront holds an entry with a weight on sun-elevation row 1, all its
+// lanes read the texel behind their own, also the one that ends the last slab (they do not use it).
 __host__ __device__ inline unsigned ps_texels(const PsPlan& p, int na, bool mie) {
-  return 2u * (mie ? 2u : 1u) * (unsigned)p.pitch * (unsigned)(na + 1);
+  return 2u * (mie ? 2u : 1u) * (unsigned)p.pitch * (unsigned)(na + 1) + 1u;
 }
 __host__ __device__ inline size_t ps_shared_bytes(const PsPlan& p, int na, bool mie) {
   return 2 * (size_t)p.misc + 16 * (size_t)ps_texels(p, na, mie);
@@ -2211,6 +2213,23 @@ static PsPlan point_scatter_plan(const DevParams& P, int ndirs, bool e_lds, int&
   const size_t misc = sizeof(float4) * (size_t)p.rays * ndirs + (ps_omega_in_lds(ept, kMie) ? 8 * (size_t)ndirs : 0) + (e_lds ? 24 * (size_t)P.nE[1] : 0);
   p.misc = (unsigned)(std::max<size_t>(misc, 8 * (size_t)ps_texels(p, NA, kMie)) + 15) & ~15u;
   return p;
+}
+
+PointScatterLds point_scatter_lds(const int* nS, int nE1, int sphere_steps, int batch, bool mie) {
+  DevParams P{};
+  for (int d = 0; d < 4; ++d) P.nS[d] = nS[d];
+  P.nE[1] = nE1;
+  P.batch = batch;
+  int ndirs = 0, ept = 1;
+  for (int i = 0; i < sphere_steps >> 1; ++i) ndirs += sphere_ring_directions(0, sphere_steps, i);
+  const bool e_lds = nE1 <= 1024;
+  const PsPlan p = mie ? point_scatter_plan<true>(P, ndirs, e_lds, ept) : point_scatter_plan<false>(P, ndirs, e_lds, ept);
+  PointScatterLds l;
+  l.bytes = (unsigned)ps_shared_bytes(p, nS[3], mie);
+  l.plane8 = p.misc;
+  l.plane16 = 2 * p.misc;
+  l.pitch = (unsigned)p.pitch;
+  return l;
 }
 
 template <int EPT, bool kMie, bool kELds>

@@ -55,6 +55,13 @@ struct SrJob {
 // Whether launch_point_scatter can take the surface radiance along (its LDS slab fits 16 KiB).
 bool sr_fits_point_scatter(const DevParams& P, bool mie);
 size_t sr_fold_bytes(const DevParams& P, bool mie);
+// Where the LDS of a point-scatter workgroup lies over a scatter grid nS, nE1 sun elevations of the surface-radiance table
+// and the directions of sphere_steps (checked on the host over all shapes): its bytes, where the two planes of its slabs
+// begin and the texels per column.
+struct PointScatterLds {
+  unsigned bytes, plane8, plane16, pitch;
+};
+PointScatterLds point_scatter_lds(const int* nS, int nE1, int sphere_steps, int batch, bool mie);
 hipError_t launch_point_scatter(const DevParams& P, const Dir* dirs, int ndirs, int sphere_steps, const void* geom,
                                 const float4* dS, const float4* mie, const float4* dE, float* out, WorkCounters* wc,
                                 hipStream_t stream, const SrJob* sr = nullptr);
