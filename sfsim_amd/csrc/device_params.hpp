@@ -12,7 +12,7 @@ namespace sfsim {
 constexpr int kMaxSteps = 256;   // ray_steps limit (LDS arrays of the per-ray kernels)
 constexpr int kMaxSlab = 1024;   // sun elevations x headings of a view ray
 constexpr int kMaxRsGroups = 8;  // column groups of the ray-scatter kernel
-constexpr int kMaxSphereDirs = 1000;  // 16 bytes of LDS per direction and ray in the point-scatter kernel
+constexpr int kMaxSphereDirs = 1000;  // directions of a sphere quadrature
 constexpr int kMaxRings = 32;         // latitude rings of at most kMaxSphereDirs directions (27)
 
 // One lookup per sample of the ray-scatter kernel: a sun direction (v . l and x . l rounded from FP64) and a column

@@ -93,6 +93,14 @@ __device__ __forceinline__ float in_vgpr(float x) {
   return x;
 }
 
+// A value that is the same in all lanes, in scalar registers.
+__device__ __forceinline__ float uniform(float x) {
+  return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x)));
+}
+__device__ __forceinline__ double uniform(double x) {
+  return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(x)), __builtin_amdgcn_readfirstlane(__double2loint(x)));
+}
+
 // Sums over the n midpoint nodes of exp(-h / H_mie) and exp(-h / H_rayleigh) with FP32 altitudes;
 // 8-node partial sums, Kahan-compensated across them.  Node j sits at s_j = s0 + j dt (units of R,
 // measured from the segment's lowest point), x_j = c0 + s_j (b + s_j) = (r_j^2 - R^2) / R^2, and the
@@ -934,9 +942,6 @@ __device__ __forceinline__ T lds_read(unsigned address) {
   return *(__attribute__((address_space(3))) const T*)(uintptr_t)address;
 }
 
-// The split of a point-scatter launch.  A workgroup takes `rays` view rays of one height and `rows` sun elevations,
-// `waves` wavefronts per ray (64 EPT entries each); eblocks x sblocks workgroups per height.  pitch: texels per
-// column of its slab; misc: bytes of the weights and dE in LDS (below the slabs, see ps_shared_bytes).
 // Orders LDS accesses of one wavefront's lanes (the hardware keeps a wavefront's LDS accesses in order; this
 // keeps the compiler from moving them across).
 __device__ __forceinline__ void wave_fence() {
@@ -1362,9 +1367,14 @@ __device__ __forceinline__ void surface_radiance_entry(const DevParams& P, int n
                                                        const float4* __restrict__ mie, float4* __restrict__ out,
                                                        WorkCounters* wc, int entry, float4* s_fold, float3* s_red);
 
+// The split of a point-scatter launch.  A workgroup takes `rays` view rays of one height and `rows` sun elevations,
+// `waves` wavefronts per ray (64 EPT entries each); eblocks x sblocks workgroups per height.  pitch: texels per
+// column of its slab.  dirs: directions whose weights are in LDS at a time.  e_lds: whether dE is.  The rest: byte
+// addresses of what the LDS holds (see ps_layout) and its size.
 struct PsPlan {
-  int rows, sblocks, rays, waves, eblocks, pitch;
-  unsigned misc;
+  int rows, sblocks, rays, waves, eblocks, pitch, dirs;
+  bool e_lds;
+  unsigned plane8, weights, dE16, dE8, omega, bytes;
 };
 
 // LDS of a workgroup: the folded slab of one latitude ring, double-buffered (and of the Mie strength in the first
@@ -1373,8 +1383,8 @@ struct PsPlan {
 // holds the column before it plus its difference (what the interpolation between the two gives at weight 1) and no
 // difference, and a column -1 column 0's colour and no difference: a heading coordinate that rounding has left just
 // outside 0 ... NA - 1 gives what the clamped one would, so a lookup clamps neither the coordinate nor the column.
-// The 8-byte plane begins at `misc` (at least its own size) and the 16-byte plane at 2 misc; the weights, dE (laid
-// out alike) and the surface-radiance workgroups' partial sums take the bytes below.
+// The 8-byte plane begins at its own size and the 16-byte plane at twice that (ps_layout); the weights, dE (laid
+// out alike) and the directions lie below the planes where they fit and else behind them.
 // Where the directions' components are read: from LDS with one entry per lane, whose few lookups do not cover the
 // latency of scalar loads (19 x 45 x 20 x 7 entries, 38 directions: 17.4 us against 19.1); from scalar registers with
 // two entries per lane, which read more of the LDS per direction (1408 us against 1317 at 64 x 128 x 64 x 16 with 262
@@ -1386,10 +1396,6 @@ __host__ __device__ constexpr bool ps_omega_in_lds(int ept, bool mie) { return e
 __host__ __device__ inline unsigned ps_texels(const PsPlan& p, int na, bool mie) {
   return 2u * (mie ? 2u : 1u) * (unsigned)p.pitch * (unsigned)(na + 1) + 1u;
 }
-__host__ __device__ inline size_t ps_shared_bytes(const PsPlan& p, int na, bool mie) {
-  return 2 * (size_t)p.misc + 16 * (size_t)ps_texels(p, na, mie);
-}
-
 // One texel: u and the difference to v; `last`: what interpolation at weight 1 gives, and no difference.
 __device__ __forceinline__ void ps_store(float4* a, float2* b, float3 u, float3 v, bool last) {
   const float3 d = make_float3(v.x - u.x, v.y - u.y, v.z - u.z);
@@ -1419,7 +1425,7 @@ struct PsRings {
 //
 // The iteration's surface radiance (it reads the same dS and Mie strength) rides in the launch: the sr.count
 // workgroups after the rays' compute its entries with the LDS-folded kernel body.
-template <int EPT, bool kMie, bool kELds, bool kB>
+template <int EPT, bool kMie, bool kELds, bool kB, bool kBatches>
 __global__ void __launch_bounds__(kBlock) point_scatter_kernel(
     const DevParams P0, const DevParams* __restrict__ PB, const Dir* __restrict__ dirs, const DirGeom* __restrict__ geom,
     int ndirs, const PsRings rings, const float4* __restrict__ dS, const float4* __restrict__ mie,
@@ -1447,17 +1453,17 @@ __global__ void __launch_bounds__(kBlock) point_scatter_kernel(
   const int ie = (hb - ih * plan.eblocks) * plan.rays + r;
   const bool active = r < plan.rays && ie < NE;  // whole wavefronts; the others help to fold
   const int nE1 = P.nE[1];
-  float4* s_w = s_mem;                                    // [rays][ndirs] rgb quadrature weight times in-scattering
-  float4* s_ea = s_w + plan.rays * ndirs;                 // dE at the ground and the differences to the next entry's,
-  float2* s_eb = (float2*)(s_ea + (kELds ? nE1 : 0));     // as the slabs' texels
-  float2* s_om = s_eb + (kELds ? nE1 : 0);                // [ndirs] omega's y and z
+  float4* s_w = (float4*)(lds + plan.weights) + r * plan.dirs;  // [rays][dirs] rgb quadrature weight times in-scattering
+  float4* s_ea = (float4*)(lds + plan.dE16);                    // dE at the ground and the differences to the next
+  float2* s_eb = (float2*)(lds + plan.dE8);                     // entry's, as the slabs' texels
+  float2* s_om = (float2*)(lds + plan.omega);                   // [dirs] omega's y and z
   constexpr bool kOmLds = ps_omega_in_lds(EPT, kMie);
   const double r0 = index_to_radius(P.g, NH, ih), h0 = index_to_altitude(P.g, NH, ih);
   const DirGeom* __restrict__ gh = geom + (long long)ih * ndirs;
 
   // Slab of one ring, columns fastest (coalesced reads).
   const int fold_rows = min(plan.pitch, NL - s0), fold_n = NA * fold_rows;
-  const unsigned half = plan.misc, slab_texels = (unsigned)(plan.pitch * (NA + 1));
+  const unsigned half = plan.plane8, slab_texels = (unsigned)(plan.pitch * (NA + 1));
   const Lerp Lh = make_lerp((float)height_to_index(P.g, NH, r0), NH);
   const long long sh = (long long)NE * NLA;
   auto fold = [&](int ring, unsigned buffer) {
@@ -1487,28 +1493,43 @@ __global__ void __launch_bounds__(kBlock) point_scatter_kernel(
     }
   };
 
-  if (kOmLds)
-    for (int j = threadIdx.x; j < ndirs; j += blockDim.x) s_om[j] = make_float2(gh[j].omega.y, gh[j].omega.z);
   if (kELds)
     for (int i = threadIdx.x; i < nE1; i += blockDim.x) {
       const int k = min(i, nE1 - 2);
       ps_store(s_ea + i, s_eb + i, ld3(dE, k), ld3(dE, k + 1), k != i);
     }
+  double se = 0.0, ce = 0.0;
+  float bm = 0.f, br = 0.f;
   if (active) {
-    double se, ce;
     bool above_unused;
     index_to_elevation(P.g, NE, r0, ie, se, ce, above_unused);
-    const float bm = (float)exp(-h0 * P.inv_scale_mie), br = (float)exp(-h0 * P.inv_scale_ray);
-    for (int j = part * 64 + lane; j < ndirs; j += 64 * plan.waves) {
+    bm = (float)exp(-h0 * P.inv_scale_mie);
+    br = (float)exp(-h0 * P.inv_scale_ray);
+  }
+  if (kBatches) {
+    se = uniform(se);
+    ce = uniform(ce);
+    bm = uniform(bm);
+    br = uniform(br);
+  }
+  // The weights of directions j0 .. j1 - 1.
+  auto weigh = [&](int j0, int j1) {
+    if (kOmLds)
+      for (int j = j0 + threadIdx.x; j < j1; j += blockDim.x) s_om[j - j0] = make_float2(gh[j].omega.y, gh[j].omega.z);
+    if (!active) return;
+    float g_mie = P.g_mie, g_ray = P.g_ray;
+    if (kBatches) asm volatile("" : "+s"(g_mie), "+s"(g_ray));  // the phases' terms are not kept in registers between batches
+    for (int j = j0 + part * 64 + lane; j < j1; j += 64 * plan.waves) {
       const Dir d = dirs[j];
       const float vw = (float)(se * d.x + ce * d.y);
-      const float pm = (kMie ? weight_phase(P.g_mie, vw) : phase_f(P.g_mie, vw)) * bm;
-      const float pr = (kMie ? weight_phase(P.g_ray, vw) : phase_f(P.g_ray, vw)) * br;
+      const float pm = (kMie ? weight_phase(g_mie, vw) : phase_f(g_mie, vw)) * bm;
+      const float pr = (kMie ? weight_phase(g_ray, vw) : phase_f(g_ray, vw)) * br;
       const float w = (float)d.w;
-      s_w[r * ndirs + j] = make_float4((P.sca_mie[0] * pm + P.sca_ray[0] * pr) * w, (P.sca_mie[1] * pm + P.sca_ray[1] * pr) * w,
-                                       (P.sca_mie[2] * pm + P.sca_ray[2] * pr) * w, 0.f);
+      s_w[j - j0] = make_float4((P.sca_mie[0] * pm + P.sca_ray[0] * pr) * w, (P.sca_mie[1] * pm + P.sca_ray[1] * pr) * w,
+                                (P.sca_mie[2] * pm + P.sca_ray[2] * pr) * w, 0.f);
     }
-  }
+  };
+  if (!kBatches) weigh(0, ndirs);
   PsConst pc;
   pc.hA = 0.5f * (float)(NA - 1);
   pc.se = SunCoord{(float)((nE1 - 1) * (double)P.sun_inv_den), (float)(-0.6 * 1.4426950408889634), (float)(nE1 - 1)};
@@ -1539,9 +1560,16 @@ __global__ void __launch_bounds__(kBlock) point_scatter_kernel(
   }
   two = __any(two);
   fold(0, 0);
-  __syncthreads();
-  const unsigned pitch_bytes = 16 * plan.pitch, ea_bytes = (unsigned)((char*)s_ea - lds), eb_bytes = (unsigned)((char*)s_eb - lds);
+  if (!kBatches) __syncthreads();
+  const unsigned pitch_bytes = 16 * plan.pitch, ea_bytes = plan.dE16, eb_bytes = plan.dE8;
+  int jb = 0, weighed = 0;  // the first direction of the weights in LDS, the first ring past them
   for (int ring = 0; ring < rings.count; ++ring) {
+    if (kBatches && ring == weighed) {  // as many rings as fit
+      jb = rings.start[ring];
+      for (weighed = ring + 1; weighed < rings.count && rings.start[weighed + 1] - jb <= plan.dirs;) ++weighed;
+      weigh(jb, rings.start[weighed]);
+      __syncthreads();
+    }
     if (ring + 1 < rings.count) fold(ring + 1, (ring + 1) & 1);
     if (active) {
       const int j0 = rings.start[ring], j1 = rings.start[ring + 1];
@@ -1573,8 +1601,8 @@ __global__ void __launch_bounds__(kBlock) point_scatter_kernel(
         }
 #pragma unroll 2
         for (int j = j0; j < j1; ++j) {
-          const float4 w = s_w[r * ndirs + j];
-          const float2 om = kOmLds ? s_om[j] : make_float2(gh[j].omega.y, gh[j].omega.z);
+          const float4 w = s_w[j - jb];
+          const float2 om = kOmLds ? s_om[j - jb] : make_float2(gh[j].omega.y, gh[j].omega.z);
 #pragma unroll
           for (int e = 0; e < EPT; ++e) {
             const float ol = fmaf(om.y, lz[e], fmaf(om.x, ly[e], x0[e]));
@@ -2196,8 +2224,37 @@ size_t direction_geometry_bytes(const DevParams& P, int ndirs) { return sizeof(D
 // phases then stay within a column: blocks of 8 or 32 rows took 4-30% longer), of at most 512 texels per slab;
 // two entries per lane where that leaves 4 wavefronts per SIMD, one on smaller grids: 32 x 64 x 32 x 8 with 66
 // directions 39 us with two and 48 with one, 19 x 45 x 20 x 7 with 38 directions 19.6 us with one and 20.3 with two.
+//
+// Weights and dE take LDS that the slabs leave of a quarter of a CU's 160 KiB (four wavefronts per SIMD).  dE stays in
+// memory where it and the fewest weights leave fewer than four workgroups per CU (64 x 128 x 64 x 16, 66 directions, mean
+// of the launches with and without the Mie strength: 768 columns, for which only the launch without it has room, 685 us,
+// 727 with dE in LDS in both; 1024 columns, in memory in both, 884 against 957).  The weights of all directions where they
+// fit, else those of as many latitude rings at a time as do, but at least of 64 directions and of the largest ring (a ring
+// never lies in two batches).  32 x 64 x 32 x 8 with 808 directions: 342 us; 996 with the weights of all of them in LDS.
+constexpr unsigned kCuLds = 163840;
+constexpr int kPsWorkgroups = 4;
+
+// The planes and, below or behind them, the other arrays: the weights of `dirs` directions, dE and omega.
+static void ps_layout(PsPlan& p, int na, bool mie, bool omega, int nE1, int dirs) {
+  const unsigned texels = ps_texels(p, na, mie);
+  p.dirs = dirs;
+  p.plane8 = (8 * texels + 15) & ~15u;
+  unsigned below = 0;
+  p.bytes = 2 * p.plane8 + 16 * texels;
+  auto place = [&](unsigned size) {
+    unsigned& at = below + size <= p.plane8 ? below : p.bytes;
+    const unsigned place = at;
+    at += (size + 15) & ~15u;
+    return place;
+  };
+  p.weights = place(16u * p.rays * dirs);
+  p.dE16 = place(p.e_lds ? 16u * nE1 : 0u);
+  p.dE8 = place(p.e_lds ? 8u * nE1 : 0u);
+  p.omega = place(omega ? 8u * dirs : 0u);
+}
+
 template <bool kMie>
-static PsPlan point_scatter_plan(const DevParams& P, int ndirs, bool e_lds, int& ept) {
+static PsPlan point_scatter_plan(const DevParams& P, int ndirs, int sphere_steps, int& ept) {
   const int NL = P.nS[2], NA = P.nS[3], most = std::max(1, 512 / ((kMie ? 2 : 1) * NA));
   PsPlan p;
   p.sblocks = std::max({1, (NL + 8) / 16, (NL + most - 1) / most});
@@ -2210,8 +2267,19 @@ static PsPlan point_scatter_plan(const DevParams& P, int ndirs, bool e_lds, int&
   p.waves = (slots + ept - 1) / ept;
   p.rays = 4 / p.waves;
   p.eblocks = (P.nS[1] + p.rays - 1) / p.rays;
-  const size_t misc = sizeof(float4) * (size_t)p.rays * ndirs + (ps_omega_in_lds(ept, kMie) ? 8 * (size_t)ndirs : 0) + (e_lds ? 24 * (size_t)P.nE[1] : 0);
-  p.misc = (unsigned)(std::max<size_t>(misc, 8 * (size_t)ps_texels(p, NA, kMie)) + 15) & ~15u;
+  const bool omega = ps_omega_in_lds(ept, kMie);
+  const int least = std::min(ndirs, std::max(64, sphere_steps));
+  auto fits = [&](int dirs, int workgroups) {
+    ps_layout(p, NA, kMie, omega, P.nE[1], dirs);
+    return p.bytes <= kCuLds / workgroups;
+  };
+  p.e_lds = true;
+  p.e_lds = P.nE[1] <= 1024 && fits(least, kPsWorkgroups);
+  int workgroups = kPsWorkgroups;
+  while (workgroups > 1 && !fits(least, workgroups)) --workgroups;
+  int dirs = ndirs;
+  while (dirs > least && !fits(dirs, workgroups)) dirs = std::max(dirs - 16, least);
+  ps_layout(p, NA, kMie, omega, P.nE[1], dirs);
   return p;
 }
 
@@ -2222,48 +2290,55 @@ PointScatterLds point_scatter_lds(const int* nS, int nE1, int sphere_steps, int 
   P.batch = batch;
   int ndirs = 0, ept = 1;
   for (int i = 0; i < sphere_steps >> 1; ++i) ndirs += sphere_ring_directions(0, sphere_steps, i);
-  const bool e_lds = nE1 <= 1024;
-  const PsPlan p = mie ? point_scatter_plan<true>(P, ndirs, e_lds, ept) : point_scatter_plan<false>(P, ndirs, e_lds, ept);
+  const PsPlan p = mie ? point_scatter_plan<true>(P, ndirs, sphere_steps, ept) : point_scatter_plan<false>(P, ndirs, sphere_steps, ept);
   PointScatterLds l;
-  l.bytes = (unsigned)ps_shared_bytes(p, nS[3], mie);
-  l.plane8 = p.misc;
-  l.plane16 = 2 * p.misc;
+  l.bytes = p.bytes;
+  l.plane8 = p.plane8;
+  l.plane16 = 2 * p.plane8;
   l.pitch = (unsigned)p.pitch;
+  l.dirs = (unsigned)p.dirs;
+  const unsigned at[4] = {p.weights, p.dE16, p.dE8, p.omega}, e = p.e_lds ? (unsigned)nE1 : 0u;
+  const unsigned size[4] = {16u * p.rays * p.dirs, 16 * e, 8 * e, ps_omega_in_lds(ept, mie) ? 8u * p.dirs : 0u};
+  for (int i = 0; i < 4; ++i) {
+    l.at[i] = at[i];
+    l.size[i] = size[i];
+  }
   return l;
 }
 
-template <int EPT, bool kMie, bool kELds>
+template <int EPT, bool kMie, bool kELds, bool kBatches>
 static void point_scatter_as(const DevParams& P, const Dir* dirs, int ndirs, const PsRings& rings, const DirGeom* geom,
                              const float4* dS, const float4* mie, const float4* dE, float* out, WorkCounters* wc,
                              hipStream_t stream, const SrJob& sr, const PsPlan& plan) {
   const unsigned blocks = (unsigned)(P.nS[0] * plan.eblocks * plan.sblocks + sr.count);
-  size_t shmem = ps_shared_bytes(plan, P.nS[3], kMie);
+  size_t shmem = plan.bytes;
   if (sr.count > 0) shmem = std::max(shmem, 4 * sizeof(float4) + sr_fold_bytes(P, sr.mie != nullptr));
   if (P.batch > 0)
-    hipLaunchKernelGGL((point_scatter_kernel<EPT, kMie, kELds, true>), dim3(blocks, 1, (unsigned)P.batch), dim3(kBlock),
+    hipLaunchKernelGGL((point_scatter_kernel<EPT, kMie, kELds, true, kBatches>), dim3(blocks, 1, (unsigned)P.batch), dim3(kBlock),
                        shmem, stream, P, P.batch_params, dirs, geom, ndirs, rings, dS, mie, dE, out, sr, plan, wc);
   else
-    hipLaunchKernelGGL((point_scatter_kernel<EPT, kMie, kELds, false>), dim3(blocks), dim3(kBlock), shmem, stream, P,
+    hipLaunchKernelGGL((point_scatter_kernel<EPT, kMie, kELds, false, kBatches>), dim3(blocks), dim3(kBlock), shmem, stream, P,
                        P.batch_params, dirs, geom, ndirs, rings, dS, mie, dE, out, sr, plan, wc);
 }
 
 template <bool kMie>
-static hipError_t launch_point_scatter_as(const DevParams& P, const Dir* dirs, int ndirs, const PsRings& rings,
+static hipError_t launch_point_scatter_as(const DevParams& P, const Dir* dirs, int ndirs, int sphere_steps, const PsRings& rings,
                                           const DirGeom* geom, const float4* dS, const float4* mie, const float4* dE,
                                           float* out, WorkCounters* wc, hipStream_t stream, const SrJob& sr) {
-  const bool e_lds = P.nE[1] <= 1024;
   int ept = 1;
-  const PsPlan plan = point_scatter_plan<kMie>(P, ndirs, e_lds, ept);
-#define SFSIM_PS_CASE(EPT, E) \
-  point_scatter_as<EPT, kMie, E>(P, dirs, ndirs, rings, geom, dS, mie, dE, out, wc, stream, sr, plan)
-  if (e_lds) {
-    if (ept == 1) SFSIM_PS_CASE(1, true);
-    else SFSIM_PS_CASE(2, true);
-  } else {
-    if (ept == 1) SFSIM_PS_CASE(1, false);
-    else SFSIM_PS_CASE(2, false);
-  }
-#undef SFSIM_PS_CASE
+  const PsPlan plan = point_scatter_plan<kMie>(P, ndirs, sphere_steps, ept);
+  if (plan.bytes > kCuLds) return hipErrorInvalidValue;  // (no accepted shape)
+  auto as = [&](auto entries, auto e_lds, auto batches) {
+    point_scatter_as<decltype(entries)::value, kMie, decltype(e_lds)::value, decltype(batches)::value>(
+        P, dirs, ndirs, rings, geom, dS, mie, dE, out, wc, stream, sr, plan);
+  };
+  auto with_dE = [&](auto entries, auto batches) {
+    plan.e_lds ? as(entries, std::true_type(), batches) : as(entries, std::false_type(), batches);
+  };
+  auto with_entries = [&](auto batches) {
+    ept == 1 ? with_dE(std::integral_constant<int, 1>(), batches) : with_dE(std::integral_constant<int, 2>(), batches);
+  };
+  plan.dirs < ndirs ? with_entries(std::true_type()) : with_entries(std::false_type());
   return hipGetLastError();
 }
 
@@ -2285,8 +2360,8 @@ hipError_t launch_point_scatter(const DevParams& P, const Dir* dirs, int ndirs, 
     job.count = P.nE[0] * P.nE[1];
   }
   if (mie)
-    return launch_point_scatter_as<true>(P, dirs, ndirs, rings, (const DirGeom*)geom, dS, mie, dE, out, wc, stream, job);
-  return launch_point_scatter_as<false>(P, dirs, ndirs, rings, (const DirGeom*)geom, dS, mie, dE, out, wc, stream, job);
+    return launch_point_scatter_as<true>(P, dirs, ndirs, sphere_steps, rings, (const DirGeom*)geom, dS, mie, dE, out, wc, stream, job);
+  return launch_point_scatter_as<false>(P, dirs, ndirs, sphere_steps, rings, (const DirGeom*)geom, dS, mie, dE, out, wc, stream, job);
 }
 
 // Sample segments per ray and group of columns: as many as let the workgroups of all rays be resident at once (four

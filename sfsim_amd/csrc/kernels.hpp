@@ -55,11 +55,12 @@ struct SrJob {
 // Whether launch_point_scatter can take the surface radiance along (its LDS slab fits 16 KiB).
 bool sr_fits_point_scatter(const DevParams& P, bool mie);
 size_t sr_fold_bytes(const DevParams& P, bool mie);
-// Where the LDS of a point-scatter workgroup lies over a scatter grid nS, nE1 sun elevations of the surface-radiance table
-// and the directions of sphere_steps (checked on the host over all shapes): its bytes, where the two planes of its slabs
-// begin and the texels per column.
+// How the LDS of a point-scatter workgroup is laid out over a scatter grid nS, nE1 sun elevations of the surface-radiance
+// table and the directions of sphere_steps (checked on the host over all shapes): its bytes, where the two planes of its
+// slabs begin, the texels per column, the directions whose weights it holds at a time, and the places and sizes of the
+// weights, of dE's two planes and of the directions.
 struct PointScatterLds {
-  unsigned bytes, plane8, plane16, pitch;
+  unsigned bytes, plane8, plane16, pitch, dirs, at[4], size[4];
 };
 PointScatterLds point_scatter_lds(const int* nS, int nE1, int sphere_steps, int batch, bool mie);
 hipError_t launch_point_scatter(const DevParams& P, const Dir* dirs, int ndirs, int sphere_steps, const void* geom,

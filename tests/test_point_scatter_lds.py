@@ -10,7 +10,8 @@ from sfsim_amd import atmosphere as atm
 
 
 class Lds(ctypes.Structure):
-    _fields_ = [(n, ctypes.c_uint) for n in ("bytes", "plane8", "plane16", "pitch")]
+    _fields_ = [(n, ctypes.c_uint) for n in ("bytes", "plane8", "plane16", "pitch", "dirs")] + [
+        ("at", ctypes.c_uint * 4), ("size", ctypes.c_uint * 4)]
 
 
 def lds_of(shape, ne1, steps, mie, batch=0):
@@ -35,3 +36,25 @@ def test_texel_behind_the_last_one_is_inside(rays, mie):
             assert p.plane16 == 2 * p.plane8 and p.plane16 % 16 == 0, where
             assert p.plane8 + 8 * texels <= p.plane16, where
             assert p.plane16 + 16 * texels <= p.bytes, where
+
+
+LDS_BYTES = 160 * 1024  # of a CU
+
+
+@pytest.mark.parametrize("mie", [False, True])
+@pytest.mark.parametrize("rays,batch", [((3, 5), 0), ((32, 64), 0), ((4, 2047), 16)])
+def test_every_accepted_shape_fits(rays, batch, mie):
+    """Within a CU's LDS whatever the number of directions and of surface-radiance columns, no array over another,
+    and the weights of at least the largest latitude ring (sphere_steps directions at most) at a time."""
+    for nl, na in SLABS:
+        for ne1 in (2, 512, 768, 1024, 1025):
+            for steps in (2, 3, 14, 28, 40, 50, 55):
+                p = lds_of((*rays, nl, na), ne1, steps, mie, batch)
+                where = (rays, nl, na, ne1, steps)
+                assert p.bytes <= LDS_BYTES, where
+                assert p.dirs >= min(steps, atm.sphere_directions(False, steps)), where
+                texels = (4 if mie else 2) * p.pitch * (na + 1) + 1
+                spans = sorted([(p.plane8, p.plane8 + 8 * texels), (p.plane16, p.plane16 + 16 * texels)] +
+                               [(a, a + n) for a, n in zip(p.at, p.size) if n])
+                assert all(a[1] <= b[0] for a, b in zip(spans, spans[1:])) and spans[-1][1] <= p.bytes, where
+                assert all(a % 16 == 0 for a in p.at), where
