@@ -22,8 +22,8 @@ struct RsItem {
   unsigned at;
 };
 
-// Items of a group that ray_scatter_kernel looks up with TS texels per lane (64 per slot).
-__host__ __device__ constexpr int rs_items(int ts) { return ts == 1 ? 128 : ts == 2 ? 256 : ts == 4 ? 384 : 512; }
+// Items that a wavefront of ray_scatter_kernel looks up at most with TS texels per lane (64 per slot).
+__host__ __device__ constexpr int rs_items(int ts) { return 128 * ts; }
 
 struct DevParams {
   Geo g;
@@ -72,7 +72,7 @@ struct DevParams {
   float4* sun_ps;
   double2* sun_ss;
   // the split of a ray's (sun elevation, heading) slab in ray_scatter_kernel (rs_split): rs_groups groups of rs_cols
-  // columns (headings), rs_ts texels per lane, rs_slots items per group at most
+  // columns (headings), rs_ts texels per lane, rs_slots items per group at most; rs_ts 0: ray_scatter_ordered_kernel
   int rs_cols, rs_groups, rs_ts, rs_slots;
   // written by launch_ray_items (from sun_ss): the rays' items (2 NL NA places per ray, group after group), the place where
   // each group's items start (rs_groups + 1 per ray), and for each entry the places of its two items (group x
@@ -140,20 +140,22 @@ __host__ __device__ inline size_t resample_map_bytes(const DevParams& P) {
   return (size_t)P.nS[0] * P.nS[1] * P.nS[2] * P.nS[3] * (sizeof(float4) + sizeof(ushort4));
 }
 
-// The split of a ray's slab: as many whole columns per group as 256 texels hold (4 per lane), evenly; a
-// column of more than 256 rows is a group of its own.  The texels per lane also set how many items a group may
-// have: per sun elevation one for each heading whose sun direction is not clamped and two for each of the
-// clamped directions (at most two), NL (NA + 2) in a slab of one group; of several groups, their share and a
-// quarter (rays with more take the sample-by-sample path).
+// The split of a ray's slab: as many whole columns per group as 256 texels hold (4 per lane), evenly.  Per sun elevation a
+// group of c columns has at most c + 2 items: one for each heading whose sun direction is not clamped, on its own column,
+// and two for each of the (at most two) clamped directions, of whose columns one has no item of its own (the same bound
+// holds where rounding has left the lowest heading's coordinate just above 0).  Where that is more than a wavefront
+// looks up (more than 170 sun elevations, where a group is one column) the slab is folded and looked up by the
+// whole workgroup (rs_ts 0): 32 x 64 x 200 x 5 at 32 samples 189 us, 261 with the items shared by two wavefronts; 32 x 64 x
+// 300 x 3 182 us against 820 with eight texels per lane, which spill.
 inline void rs_split(DevParams& P) {
   const int NL = P.nS[2], NA = P.nS[3], most = NL > 256 ? 1 : 256 / NL;
   const int want = (NA + most - 1) / most;
   P.rs_cols = (NA + want - 1) / want;
   P.rs_groups = (NA + P.rs_cols - 1) / P.rs_cols;
   const int texels = P.rs_cols * NL;
-  const int items = P.rs_groups == 1 ? NL * (NA + 2) : (int)(1.25 * NL * (NA + 2) * P.rs_cols / NA);
-  for (P.rs_ts = 1; P.rs_ts < 8 && (texels > 64 * P.rs_ts || items > rs_items(P.rs_ts));) P.rs_ts *= 2;
-  P.rs_slots = rs_items(P.rs_ts);
+  P.rs_ts = texels > 128 ? 4 : texels > 64 ? 2 : 1;
+  P.rs_slots = (NL * (P.rs_cols + 2) + 63) & ~63;
+  if (P.rs_slots > rs_items(P.rs_ts)) P.rs_ts = 0;
 }
 
 // Bytes of the sun terms and the ray-scatter items (laid out by sun_map_view).

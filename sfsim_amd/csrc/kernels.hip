@@ -675,6 +675,7 @@ __global__ void __launch_bounds__(kBlock) ray_geometry_kernel(const DevParams P,
 __device__ __forceinline__ void ray_items_body(const DevParams& P, int rayid, unsigned* s_pos) {
   __shared__ int s_count[kMaxRsGroups], s_start[kMaxRsGroups + 1];
   const int NL = P.nS[2], NA = P.nS[3], NLA = NL * NA, groups = P.rs_groups;
+  const int capacity = P.rs_slots;
   const long long base = (long long)rayid * NLA;
   const double2* __restrict__ ss = P.sun_ss + base;
   const int lane = threadIdx.x & 63;
@@ -701,7 +702,7 @@ __device__ __forceinline__ void ray_items_body(const DevParams& P, int rayid, un
           const int idx = __builtin_amdgcn_readfirstlane(first) + __popcll(mask & ((1ull << lane) - 1));
           if (want && pass == 1) {
             P.rs_items[2 * base + s_start[g] + idx] = RsItem{(float)d.x, (float)d.y, ((unsigned)col << 16) | (unsigned)k};
-            pos[j] = (unsigned)(g * P.rs_slots + idx);  // (read only where every group's items fit the slots)
+            pos[j] = (unsigned)(g * capacity + min(idx, capacity - 1));  // (rs_split: idx < capacity)
           }
         }
       if (b + lane < NLA && pass == 1) s_pos[k] = same ? 0xffffffffu : (pos[1] << 16) | (pos[0] & 0xffffu);
@@ -993,14 +994,12 @@ __host__ __device__ constexpr int rs_texels(bool exact) {
   return 64 * TS + (exact ? 32 * TS : 4 * TS);
 }
 
-// LDS of one workgroup: the wavefronts' slabs, whose place the item sums take later ([segs][3][groups x items]).  For W
+// LDS of one workgroup: the wavefronts' slabs, whose place the item sums take later ([segs][3][groups x slots]).  For W
 // wavefronts of N texels the 4-byte plane lies at 4 W N and the 8-byte plane at 8 W N: 16 bytes per texel, of which the
 // first 4 are not used, and no offset between an address and its half.
 template <int TS>
-__host__ __device__ inline size_t rs_shared_bytes(int groups, int segs, bool exact) {
-  const size_t slabs = (size_t)groups * segs * rs_texels<TS>(exact) * sizeof(float4);
-  const size_t sums = (size_t)segs * 3 * groups * rs_items(TS) * sizeof(float);
-  return slabs > sums ? slabs : sums;
+inline size_t rs_shared_bytes(int wavefronts, int slots, bool exact) {
+  return wavefronts * std::max(rs_texels<TS>(exact) * sizeof(float4), (size_t)slots * 3 * sizeof(float));
 }
 
 // One wavefront's samples i0 .. i1 - 1 over NS lookup slots: acc[j] = sum over its samples of T(x, p_i) times
@@ -1083,58 +1082,37 @@ __device__ __forceinline__ void rs_segment(const float* __restrict__ dJ, const S
   }
 }
 
-// One entry sample by sample from dJ itself, both columns mixed at every sample and the samples added in
-// order (vl, xl: FP64): for rays whose items exceed the lookup slots, and for the order sums that training and
-// sfsim_atmo_order_sums read, whose rounding stays that of this plain order (a network's training amplifies the
-// last bit of its targets).
-template <bool kExact, class Steps>
-__device__ float3 rs_entry_sum(const float* __restrict__ dJ, const Steps gF, const float4* __restrict__ gT,
-                               const float4* __restrict__ gRS, const double2* __restrict__ gTH, int n, int NL, int NA,
-                               double vl, double xl, const SunCoord& sc, double R, double A64) {
-  const Lerp L = make_lerp((float)sun_angle_to_index(NA, vl), NA);
-  const int c0 = L.i0 * NL, c1 = L.i1 * NL;
-  float3 acc = make_float3(0.f, 0.f, 0.f);
-  for (int i = 0; i < n; ++i) {
-    const FoldStep st = fold_step(gF, i);
-    const float4 T = gT[i], g = gRS[i];
-    int row;
-    float s;
-    if (kExact) {
-      unsigned r;
-      sun_coord_exact(sc, A64, R, gTH[i], xl, vl, r, s);
-      row = (int)r;
-    } else {
-      const float c = sun_coord(sc, make_float2(g.z, g.w), (float)xl, (float)vl);
-      row = min((int)c, NL - 2);
-      s = c - (float)row;
-    }
-    const int o[4] = {st.off.x, st.off.y, st.off.z, st.off.w};
-    const float w[4] = {st.wt.x, st.wt.y, st.wt.z, st.wt.w};
-    float4 f[2][2] = {};  // [row][column]: the fold of the four nodes
-    for (int q = 0; q < 4; ++q)
-      if (o[q] >= 0) {
-        auto add = [&](float4& t, int k) {
-          const Rgb v = ((const Rgb*)dJ)[(long long)o[q] + k];
-          t = make_float4(fmaf(w[q], v.x, t.x), fmaf(w[q], v.y, t.y), fmaf(w[q], v.z, t.z), 0.f);
-        };
-        add(f[0][0], c0 + row);
-        add(f[0][1], c1 + row);
-        add(f[1][0], c0 + row + 1);
-        add(f[1][1], c1 + row + 1);
-      }
-    const float3 u = lerp3(f[0][0], f[0][1], L.s), t = lerp3(f[1][0], f[1][1], L.s);
-    acc.x = fmaf(T.x, fmaf(s, t.x - u.x, u.x), acc.x);
-    acc.y = fmaf(T.y, fmaf(s, t.y - u.y, u.y), acc.y);
-    acc.z = fmaf(T.z, fmaf(s, t.z - u.z, u.z), acc.z);
-  }
-  return acc;
-}
-
 __device__ float3 resample4_value(const DevParams& P, const float4* __restrict__ a, const float4* __restrict__ b,
                                  long long idx, const float4* __restrict__ c = nullptr);
 __device__ float3 resample4_value_lean(const DevParams& P, const float4* __restrict__ a, long long idx);
 __device__ float3 resample2_value(const DevParams& P, int space, const float4* __restrict__ a,
                                  const float4* __restrict__ b, long long idx);
+
+// An entry's result of a ray-scatter launch, and S + dS at this grid point (the running sum S of atmosphere_lut.clj:95-97).
+template <bool kB>
+__device__ __forceinline__ void rs_store(const DevParams& P, const RsAccum& accum, float4* __restrict__ out, long long at,
+                                         float3 v, float dt) {
+  const float4 d = make_float4(v.x * dt, v.y * dt, v.z * dt, 0.f);
+  out[at] = d;
+  if (accum.S_out) {
+    const float4* S_in = atm_ptr<kB>(accum.S_in, P);
+    const float3 u = accum.S_resample ? resample4_value_lean(P, S_in, at) : ld3(S_in, at);
+    atm_ptr<kB>(accum.S_out, P)[at] = make_float4(u.x + d.x, u.y + d.y, u.z + d.z, 0.f);
+  }
+}
+
+// The extra workgroup: E <- tab(dE + E) (atmosphere_lut.clj:95-96).
+template <bool kB>
+__device__ __forceinline__ void rs_surface(const DevParams& P, const RsAccum& accum) {
+  const long long nE = (long long)P.nE[0] * P.nE[1];
+  const float4* dE = atm_ptr<kB>(accum.dE, P);
+  const float4* E_in = atm_ptr<kB>(accum.E_in, P);
+  float4* E_out = atm_ptr<kB>(accum.E_out, P);
+  for (long long i = threadIdx.x; i < nE; i += blockDim.x) {
+    const float3 v = resample2_value(P, 3, dE, E_in, i);
+    E_out[i] = make_float4(v.x, v.y, v.z, 0.f);
+  }
+}
 
 // segs: sample segments per group of columns (P.rs_groups x segs wavefronts, wavefront w working on group
 // w / segs and segment w % segs).
@@ -1143,8 +1121,7 @@ __global__ void __launch_bounds__(1024) ray_scatter_kernel(
     const DevParams P0, const DevParams* __restrict__ PB, const float* __restrict__ dJ,
     const double2* __restrict__ geo_th, const float4* __restrict__ geo_T, const float4* __restrict__ geo_rs,
     const FoldStep* __restrict__ geo_fold, const RsItem* __restrict__ items, const uint2* __restrict__ entries,
-    const int* __restrict__ heads, float4* __restrict__ out, const RsAccum accum_arg, int segs, int by_sample,
-    WorkCounters* wc) {
+    const int* __restrict__ heads, float4* __restrict__ out, const RsAccum accum, int segs, WorkCounters* wc) {
   const DevParams& P = params_of<kB>(P0, PB);
   if constexpr (kB) {  // this atmosphere's tables and ray geometry (the accumulation tables where they are used);
                        // offsets of the restrict arguments, whose loads stay provably unclobbered and uniform
@@ -1159,19 +1136,12 @@ __global__ void __launch_bounds__(1024) ray_scatter_kernel(
   const int NH = P.nS[0], NE = P.nS[1], NL = P.nS[2], NA = P.nS[3];
   const int NLA = NL * NA;
   const int n = P.ray_steps;
-  if ((int)blockIdx.x >= NH * NE) {  // the extra workgroup: E <- tab(dE + E) (atmosphere_lut.clj:95-96)
-    const long long nE = (long long)P.nE[0] * P.nE[1];
-    const float4* dE = atm_ptr<kB>(accum_arg.dE, P);
-    const float4* E_in = atm_ptr<kB>(accum_arg.E_in, P);
-    float4* E_out = atm_ptr<kB>(accum_arg.E_out, P);
-    for (long long i = threadIdx.x; i < nE; i += blockDim.x) {
-      const float3 v = resample2_value(P, 3, dE, E_in, i);
-      E_out[i] = make_float4(v.x, v.y, v.z, 0.f);
-    }
+  if ((int)blockIdx.x >= NH * NE) {
+    rs_surface<kB>(P, accum);
     return;
   }
   extern __shared__ float4 s_mem[];
-  const int groups = P.rs_groups, pitch_out = groups * rs_items(TS);
+  const int groups = P.rs_groups, slots = P.rs_slots, pitch_out = groups * slots;
   // XCD-aware, in ascending impact parameter: every sample of a straight ray has the same
   // |p| sqrt(1 - mu^2), so the (height, elevation) cells that a ray folds lie along one curve, and an XCD
   // given a contiguous range of impact parameters reads a band of the dJ table
@@ -1189,83 +1159,228 @@ __global__ void __launch_bounds__(1024) ray_scatter_kernel(
   const SunCoord sc = {(float)((NL - 1) * (double)P.sun_inv_den), (float)(-0.6 * 1.4426950408889634), (float)(NL - 1)};
   const double A64 = kExact ? (NL - 1) / (1.0 - exp(-3.6)) : 0.0;
   const int* __restrict__ head = heads + (long long)rayid * (groups + 1);
-  bool fits = !by_sample;
-  for (int g = 0; g < groups; ++g) fits = fits && head[g + 1] - head[g] <= rs_items(TS);
-  if (fits) {
-    const int nitems = head[group + 1] - head[group];
-    // the lane's texels in the LDS slab; those past the group's texels write zeros to the last column's zero texel
-    const int col0 = group * P.rs_cols, ncols = min(P.rs_cols, NA - col0), pitch = NL + 1;
-    const unsigned texels = rs_texels<TS>(kExact), slab = 8 * (texels * (unsigned)(blockDim.x >> 6) + wave * texels);
-    unsigned laddr[TS];
+  const int nitems = min(head[group + 1] - head[group], slots);
+  // the lane's texels in the LDS slab; those past the group's texels write zeros to the last column's zero texel
+  const int col0 = group * P.rs_cols, ncols = min(P.rs_cols, NA - col0), pitch = NL + 1;
+  const unsigned texels = rs_texels<TS>(kExact), slab = 8 * (texels * (unsigned)(blockDim.x >> 6) + wave * texels);
+  unsigned laddr[TS];
 #pragma unroll
-    for (int j = 0; j < TS; ++j) {
-      const unsigned t = 64 * j + lane;
-      laddr[j] = (t < (unsigned)(ncols * NL) ? t + t / (unsigned)NL : (unsigned)(ncols * pitch - 1)) * 8u + slab;
-    }
-    for (int i = lane; i < ncols; i += 64) {
-      const unsigned A = slab + (i * pitch + NL) * 8;
-      lds_write(A, Vec2{0.f, 0.f});
-      lds_write(A >> 1, 0.f);
-    }
-    const int i0 = (int)((long long)n * seg / segs), i1 = (int)((long long)n * (seg + 1) / segs);
-    const RsItem* __restrict__ it = items + 2 * base + head[group];
-    float* s_out = (float*)s_mem + (size_t)seg * 3 * pitch_out + group * rs_items(TS);
+  for (int j = 0; j < TS; ++j) {
+    const unsigned t = 64 * j + lane;
+    laddr[j] = (t < (unsigned)(ncols * NL) ? t + t / (unsigned)NL : (unsigned)(ncols * pitch - 1)) * 8u + slab;
+  }
+  for (int i = lane; i < ncols; i += 64) {
+    const unsigned A = slab + (i * pitch + NL) * 8;
+    lds_write(A, Vec2{0.f, 0.f});
+    lds_write(A >> 1, 0.f);
+  }
+  const int i0 = (int)((long long)n * seg / segs), i1 = (int)((long long)n * (seg + 1) / segs);
+  const RsItem* __restrict__ it = items + 2 * base + head[group];
+  float* s_out = (float*)s_mem + (size_t)seg * 3 * pitch_out + group * slots;
 #define SFSIM_RS_CASE(NS)                                                                                             \
   case NS:                                                                                                            \
-    if constexpr (64 * NS <= rs_items(TS))                                                                            \
+    if constexpr (64 * NS <= (kExact ? 64 * TS + 64 : rs_items(TS)))  /* exact: texels + 2 rows, of 15 at most */     \
       rs_segment<TS, NS, kExact>(dJ + 3 * col0 * NL, gF, geo_T + base_n, geo_rs + base_n, geo_th + base_n, i0, i1,     \
                                  ncols * NL * (int)sizeof(Rgb), slab, laddr, it, nitems, ss, col0, pitch, sc, P.g.R,  \
                                  A64, lane, s_out, pitch_out);                                                        \
     break
-    switch ((nitems + 63) / 64) {
-      SFSIM_RS_CASE(1);
-      SFSIM_RS_CASE(2);
-      SFSIM_RS_CASE(3);
-      SFSIM_RS_CASE(4);
-      SFSIM_RS_CASE(5);
-      SFSIM_RS_CASE(6);
-      SFSIM_RS_CASE(7);
-      SFSIM_RS_CASE(8);
-      default:  // no item of this group
-        __syncthreads();
-    }
-#undef SFSIM_RS_CASE
-    __syncthreads();
+  switch ((nitems + 63) / 64) {
+    SFSIM_RS_CASE(1);
+    SFSIM_RS_CASE(2);
+    SFSIM_RS_CASE(3);
+    SFSIM_RS_CASE(4);
+    SFSIM_RS_CASE(5);
+    SFSIM_RS_CASE(6);
+    SFSIM_RS_CASE(7);
+    SFSIM_RS_CASE(8);
+    default:  // no item of this group
+      __syncthreads();
   }
+#undef SFSIM_RS_CASE
+  __syncthreads();
   // the ray's step D / n: twice its first sample's t = 0.5 D / n (FP64, exact), from the per-build geometry
   const float dt = (float)(2.0 * geo_th[base_n].x);
   for (int kk = threadIdx.x; kk < NLA; kk += blockDim.x) {
-    float3 v;
-    if (fits) {
-      const uint2 e = entries[base + kk];
-      auto total = [&](unsigned at) {
-        const float* q = (const float*)s_mem + at;
-        float3 t = make_float3(q[0], q[pitch_out], q[2 * pitch_out]);
-        for (int g = 1; g < segs; ++g) {
-          q += 3 * pitch_out;
-          t.x += q[0];
-          t.y += q[pitch_out];
-          t.z += q[2 * pitch_out];
-        }
-        return t;
-      };
-      v = total(e.x & 0xffffu);
-      const float s = __uint_as_float(e.y);
-      if (s != 0.0f) {
-        const float3 u = total(e.x >> 16);
-        v = make_float3(fmaf(s, u.x - v.x, v.x), fmaf(s, u.y - v.y, v.y), fmaf(s, u.z - v.z, v.z));
+    const uint2 e = entries[base + kk];
+    auto total = [&](unsigned at) {
+      const float* q = (const float*)s_mem + at;
+      float3 t = make_float3(q[0], q[pitch_out], q[2 * pitch_out]);
+      for (int g = 1; g < segs; ++g) {
+        q += 3 * pitch_out;
+        t.x += q[0];
+        t.y += q[pitch_out];
+        t.z += q[2 * pitch_out];
       }
-    } else {
-      const double2 d = ss[kk];
-      v = rs_entry_sum<kExact>(dJ, gF, geo_T + base_n, geo_rs + base_n, geo_th + base_n, n, NL, NA, d.x, d.y, sc, P.g.R, A64);
+      return t;
+    };
+    float3 v = total(e.x & 0xffffu);
+    const float s = __uint_as_float(e.y);
+    if (s != 0.0f) {
+      const float3 u = total(e.x >> 16);
+      v = make_float3(fmaf(s, u.x - v.x, v.x), fmaf(s, u.y - v.y, v.y), fmaf(s, u.z - v.z, v.z));
     }
-    const float4 d = make_float4(v.x * dt, v.y * dt, v.z * dt, 0.f);
-    out[base + kk] = d;
-    if (accum_arg.S_out) {  // S + dS at this grid point (the running sum S of atmosphere_lut.clj:95-97)
-      const float4* S_in = atm_ptr<kB>(accum_arg.S_in, P);
-      const float3 u = accum_arg.S_resample ? resample4_value_lean(P, S_in, base + kk) : ld3(S_in, base + kk);
-      atm_ptr<kB>(accum_arg.S_out, P)[base + kk] = make_float4(u.x + d.x, u.y + d.y, u.z + d.z, 0.f);
+    rs_store<kB>(P, accum, out, base + kk, v, dt);
+    count(wc, 0, 0, (unsigned long long)n, 0);
+  }
+}
+
+// The same in plain order: both columns mixed at every sample and the samples added one by one.  The order sums that
+// training and sfsim_atmo_order_sums read come from it (a network's training amplifies the last bit of its targets, so
+// their rounding stays that of this plain order), and the results on grids whose columns have too many items (rs_split).
+//
+// One workgroup per view ray, TS texels and entries per lane.  The lanes' dJ values lie in registers as in
+// ray_scatter_kernel, the whole slab is folded into LDS, 16 bytes a texel.  With many rays (`samples` 1) all wavefronts fold
+// and look up each sample, in two slabs with one barrier per sample, and a lane adds its own entries.  A grid of few rays
+// waits for a sample's chain of loads and barriers: there `samples` samples are in work at once, each by wavefronts
+// of its own, and the values are added in their order from LDS (16 x 32 x 16 x 8 at 32 samples 18.5 us, 32 without).  Gathering
+// every lookup's 16 texels from dJ instead, sfsim_atmo_order_sums took 5.5 ms at 32 x 64 x 32 x 8 and 64 samples and 139 at
+// 64 x 128 x 64 x 16 and 128; now 2.5 and 35.5.
+template <int TS, bool kB, bool kExact>
+__global__ void __launch_bounds__(1024) ray_scatter_ordered_kernel(
+    const DevParams P0, const DevParams* __restrict__ PB, const float* __restrict__ dJ, const double2* __restrict__ geo_th, const float4* __restrict__ geo_T,
+    const float4* __restrict__ geo_rs, const FoldStep* __restrict__ geo_fold, float4* __restrict__ out, const RsAccum accum,
+    int samples, WorkCounters* wc) {
+  const DevParams& P = params_of<kB>(P0, PB);
+  if constexpr (kB) {  // as in ray_scatter_kernel
+    geo_th = atm_ptr<kB>(geo_th, P0);
+    geo_T = atm_ptr<kB>(geo_T, P0);
+    geo_rs = atm_ptr<kB>(geo_rs, P0);
+    dJ = atm_ptr<kB>(dJ, P);
+    out = atm_ptr<kB>(out, P);
+  }
+  const int NH = P.nS[0], NE = P.nS[1], NL = P.nS[2], NA = P.nS[3], NLA = NL * NA, n = P.ray_steps;
+  if ((int)blockIdx.x >= NH * NE) {
+    rs_surface<kB>(P, accum);
+    return;
+  }
+  extern __shared__ float4 s_mem[];
+  const int ord = xcd_ray(blockIdx.x, NH * NE);
+  const int rayid = P.ray_order ? P.ray_order[ord] : ord;
+  const long long base = (long long)rayid * NLA, base_n = (long long)rayid * n;
+  const double2* __restrict__ ss = P.sun_ss + base;
+  const FoldStep* __restrict__ gS = geo_fold + base_n;
+  const auto gF = [&] {
+    if constexpr (kB) return (ConstFoldSteps)gS;
+    else return gS;
+  }();
+  const SunCoord sc = {(float)((NL - 1) * (double)P.sun_inv_den), (float)(-0.6 * 1.4426950408889634), (float)(NL - 1)};
+  const double A64 = kExact ? (NL - 1) / (1.0 - exp(-3.6)) : 0.0;
+  const int lane = threadIdx.x & 63, all = (int)blockDim.x, threads = all / samples;  // threads: of a sample
+  const int mine = __builtin_amdgcn_readfirstlane((int)threadIdx.x / threads), tid = (int)threadIdx.x - mine * threads;
+  const int first = __builtin_amdgcn_readfirstlane(tid >> 6) * 64 * TS;
+  const int texels = max(0, min(64 * TS, NLA - first)), bytes = texels * (int)sizeof(Rgb);
+  const float* __restrict__ own = dJ + 3 * first;
+  float4* slabs = s_mem + mine * NLA;
+  float* terms = (float*)(s_mem + samples * NLA);  // [samples][3][NLA] (samples > 1)
+  int c0[TS], c1[TS];
+  float mix[TS], vl[TS], xl[TS];
+  Rgb acc[TS];
+  bool two = false;
+  // the lane's entries, in (heading, sun elevation) order: neighbouring lanes read neighbouring rows
+  auto entry = [&](int q) {
+    const int a = q / NL;
+    return (q - a * NL) * NA + a;
+  };
+#pragma unroll
+  for (int e = 0; e < TS; ++e) {
+    const double2 d = ss[entry(min(tid + e * threads, NLA - 1))];
+    const Lerp L = make_lerp((float)sun_angle_to_index(NA, d.x), NA);
+    c0[e] = L.i0 * NL;
+    c1[e] = L.i1 * NL;
+    mix[e] = L.s;
+    two = two || L.s != 0.0f;
+    vl[e] = (float)d.x;
+    xl[e] = (float)d.y;
+    acc[e] = Rgb{0.f, 0.f, 0.f};
+  }
+  two = __any(two);
+  FoldSlots<TS> f;
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int j = 0; j < TS; ++j) f.v[c][j] = Rgb{0.f, 0.f, 0.f};
+  FoldStep st = fold_step(gF, min(mine, n - 1));
+  fold_load<TS>(own, make_int4(-1, -1, -1, -1), st.off, bytes, lane, f);
+  for (int round = 0; round < n; round += samples) {
+    const int i = min(round + mine, n - 1);  // (past the last sample: the last again, not added)
+    float4* slab = samples == 1 ? slabs + (round & 1) * NLA : slabs;
+    const float4 w = st.wt;
+#pragma unroll
+    for (int j = 0; j < TS; ++j)
+      if (64 * j + lane < texels) {
+        const Rgb a = f.v[0][j], b = f.v[1][j], c = f.v[2][j], d = f.v[3][j];
+        slab[first + 64 * j + lane] = make_float4(fmaf(w.w, d.x, fmaf(w.z, c.x, fmaf(w.y, b.x, w.x * a.x))),
+                                                  fmaf(w.w, d.y, fmaf(w.z, c.y, fmaf(w.y, b.y, w.x * a.y))),
+                                                  fmaf(w.w, d.z, fmaf(w.z, c.z, fmaf(w.y, b.z, w.x * a.z))), 0.f);
+      }
+    const FoldStep nx = fold_step(gF, min(i + samples, n - 1));  // the next sample's nodes, in flight during the lookups
+    fold_load<TS>(own, st.off, nx.off, bytes, lane, f);
+    st = nx;
+    const float4 T = geo_T[base_n + i], g = geo_rs[base_n + i];
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < TS; ++e) {
+      unsigned row;
+      float s;
+      if (kExact) {
+        const double2 d = ss[entry(min(tid + e * threads, NLA - 1))];
+        sun_coord_exact(sc, A64, P.g.R, geo_th[base_n + i], d.y, d.x, row, s);
+      } else {
+        const float c = sun_coord(sc, make_float2(g.z, g.w), xl[e], vl[e]);
+        row = min((unsigned)c, (unsigned)NL - 2);
+        s = c - (float)row;
+      }
+      const float4 *p = slab + c0[e] + row, *q = slab + c1[e] + row;
+      const float4 p0 = p[0], p1 = p[1];
+      float3 u = make_float3(p0.x, p0.y, p0.z), v = make_float3(p1.x, p1.y, p1.z);
+      if (two) {
+        u = lerp3(p0, q[0], mix[e]);
+        v = lerp3(p1, q[1], mix[e]);
+      }
+      v = make_float3(fmaf(s, v.x - u.x, u.x), fmaf(s, v.y - u.y, u.y), fmaf(s, v.z - u.z, u.z));
+      if (samples == 1) {
+        acc[e].x = fmaf(T.x, v.x, acc[e].x);
+        acc[e].y = fmaf(T.y, v.y, acc[e].y);
+        acc[e].z = fmaf(T.z, v.z, acc[e].z);
+      } else if (tid + e * threads < NLA) {
+        float* t = terms + 3 * mine * NLA + tid + e * threads;
+        t[0] = v.x;
+        t[NLA] = v.y;
+        t[2 * NLA] = v.z;
+      }
     }
+    if (samples > 1) {
+      __syncthreads();
+#pragma unroll
+      for (int e = 0; e < TS; ++e) {
+        const int q = (int)threadIdx.x + e * all;
+        if (q < NLA)
+          for (int j = 0; j < min(samples, n - round); ++j) {
+            const float4 Tj = geo_T[base_n + round + j];
+            const float* t = terms + 3 * j * NLA + q;
+            acc[e].x = fmaf(Tj.x, t[0], acc[e].x);
+            acc[e].y = fmaf(Tj.y, t[NLA], acc[e].y);
+            acc[e].z = fmaf(Tj.z, t[2 * NLA], acc[e].z);
+          }
+      }
+    }
+  }
+  __syncthreads();
+  float* sums = (float*)s_mem;
+#pragma unroll
+  for (int e = 0; e < TS; ++e) {
+    const int q = (int)threadIdx.x + e * all;
+    if (q < NLA) {
+      const int k = entry(q);
+      sums[k] = acc[e].x;
+      sums[NLA + k] = acc[e].y;
+      sums[2 * NLA + k] = acc[e].z;
+    }
+  }
+  __syncthreads();
+  const float dt = (float)(2.0 * geo_th[base_n].x);  // as in ray_scatter_kernel
+  for (int k = threadIdx.x; k < NLA; k += all) {
+    rs_store<kB>(P, accum, out, base + k, make_float3(sums[k], sums[NLA + k], sums[2 * NLA + k]), dt);
     count(wc, 0, 0, (unsigned long long)n, 0);
   }
 }
@@ -2170,9 +2285,43 @@ hipError_t launch_ray_geometry(const DevParams& P, WorkCounters* wc, hipStream_t
 hipError_t launch_ray_items(const DevParams& P, hipStream_t stream) {
   if (P.batch > 0) return hipErrorInvalidValue;  // batches make them in launch_single_scatter
   if (!P.rs_items || !P.sun_ss || P.rs_groups > kMaxRsGroups) return hipErrorInvalidValue;
+  if (P.rs_ts == 0) return hipSuccess;  // ray_scatter_ordered_kernel reads none
   hipLaunchKernelGGL(ray_items_kernel, dim3((unsigned)(P.nS[0] * P.nS[1])), dim3(kBlock),
                      sizeof(unsigned) * (size_t)P.nS[2] * P.nS[3], stream, P);
   return hipGetLastError();
+}
+
+RayItems ray_items_most(const int* nS, double radius, double height) {
+  DevParams P{};
+  for (int d = 0; d < 4; ++d) P.nS[d] = nS[d];
+  P.g.R = radius;
+  P.g.H = height;
+  P.g.Rt = radius + height;
+  P.g.rho_max = std::sqrt(sqr(P.g.Rt) - sqr(P.g.R));
+  rs_split(P);
+  const int NL = nS[2], NA = nS[3];
+  RayItems r{0, P.rs_ts > 0 ? P.rs_slots : 0};
+  for (int ray = 0; ray < nS[0] * nS[1]; ++ray) {
+    double se, ce;
+    bool above;
+    index_to_elevation(P.g, nS[1], index_to_radius(P.g, nS[0], ray / nS[1]), ray % nS[1], se, ce, above);
+    int count[kMaxRsGroups] = {};
+    for (int is = 0; is < NL; ++is) {
+      double last = 2.0, l0, l1, l2;
+      for (int ia = 0; ia < NA; ++ia) {
+        index_to_sun_direction(NA, se, ce, index_to_sin_sun_elevation(NL, is), ia, l0, l1, l2);
+        const double vl = se * l0 + ce * l1;
+        if (vl != last) {
+          const float c = std::min(std::max((float)sun_angle_to_index(NA, vl), 0.0f), (float)(NA - 1));
+          ++count[(int)c / P.rs_cols];
+          if (c != (float)(int)c) ++count[((int)c + 1) / P.rs_cols];
+        }
+        last = vl;
+      }
+    }
+    for (int g = 0; g < P.rs_groups; ++g) r.most = std::max(r.most, count[g]);
+  }
+  return r;
 }
 
 hipError_t launch_single_scatter(const DevParams& P, float4* rayleigh, float4* mie, WorkCounters* wc,
@@ -2188,9 +2337,9 @@ hipError_t launch_single_scatter(const DevParams& P, float4* rayleigh, float4* m
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const RayGeoView V = ray_geo_view(P);
-    const unsigned extra = ray_items ? rays : 0;
+    const unsigned extra = ray_items && P.rs_ts > 0 ? rays : 0;
     const size_t shmem = std::max((size_t)P.ray_steps * (sizeof(double2) + 2 * sizeof(float4) + sizeof(float2)),
-                                  ray_items ? (size_t)P.nS[2] * P.nS[3] * sizeof(unsigned) : 0);
+                                  extra ? (size_t)P.nS[2] * P.nS[3] * sizeof(unsigned) : 0);
     if (P.batch > 0)
       hipLaunchKernelGGL(single_scatter_table_kernel<true>, dim3(rays + extra, 1, P.batch), dim3(kSSTBlock), shmem, stream, P,
                          P.batch_params, V.th, V.T, V.ss, V.row, rayleigh, mie, (int)extra, wc);
@@ -2369,42 +2518,69 @@ hipError_t launch_point_scatter(const DevParams& P, const Dir* dirs, int ndirs, 
 // within 64 KiB of LDS.  The 32 x 64 x 32 x 8 grid at 64 steps: 59 us with 2 segments, 76 with 1, 60 with 4 (two
 // rounds); 19 x 45 x 20 x 7 at 51 steps: 24 us with 4, 38 with 5 (a second round of few), 30 with 2, 48 with 1.
 template <int TS, bool kExact>
-hipError_t launch_ray_scatter_as(const DevParams& P, const float* dJ, float4* out, WorkCounters* wc, hipStream_t stream,
-                                 const RsAccum& acc, bool by_sample) {
+static hipError_t launch_ray_scatter_as(const DevParams& P, const float* dJ, float4* out, WorkCounters* wc, hipStream_t stream,
+                                        const RsAccum& acc) {
   const int groups = P.rs_groups;
   const long long rays = (long long)P.nS[0] * P.nS[1];
   int segs = (int)(16 / ((rays + 255) / 256)) / groups;
   segs = std::max(1, std::min(segs, P.ray_steps / 2));
-  while (segs > 1 && rs_shared_bytes<TS>(groups, segs, kExact) > 65536) --segs;
-  const size_t shmem = rs_shared_bytes<TS>(groups, segs, kExact);
+  while (segs > 1 && rs_shared_bytes<TS>(groups * segs, P.rs_slots, kExact) > 65536) --segs;
+  const size_t shmem = rs_shared_bytes<TS>(groups * segs, P.rs_slots, kExact);
   const RayGeoView V = ray_geo_view(P);
   const dim3 grid((unsigned)rays + (acc.E_out ? 1u : 0u), 1, P.batch > 0 ? (unsigned)P.batch : 1u), block(64u * groups * segs);
   if (P.batch > 0)
     hipLaunchKernelGGL((ray_scatter_kernel<TS, true, kExact>), grid, block, shmem, stream, P, P.batch_params, dJ, V.th, V.T,
-                       V.rs, V.fold, P.rs_items, P.rs_entries, P.rs_heads, out, acc, segs, (int)by_sample, wc);
+                       V.rs, V.fold, P.rs_items, P.rs_entries, P.rs_heads, out, acc, segs, wc);
   else
     hipLaunchKernelGGL((ray_scatter_kernel<TS, false, kExact>), grid, block, shmem, stream, P, P.batch_params, dJ, V.th, V.T,
-                       V.rs, V.fold, P.rs_items, P.rs_entries, P.rs_heads, out, acc, segs, (int)by_sample, wc);
+                       V.rs, V.fold, P.rs_items, P.rs_entries, P.rs_heads, out, acc, segs, wc);
+  return hipGetLastError();
+}
+
+// In plain order: the fewest texels per lane (1, 2 or 4) with which the workgroups of all rays are resident at once, and as
+// many samples at once as the wavefronts that are then left allow, within 64 KiB of LDS (28 bytes per texel and sample).
+template <bool kExact>
+static hipError_t launch_ray_scatter_ordered(const DevParams& P, const float* dJ, float4* out, WorkCounters* wc,
+                                             hipStream_t stream, const RsAccum& acc) {
+  const long long rays = (long long)P.nS[0] * P.nS[1];
+  const int NLA = P.nS[2] * P.nS[3], tiles = (NLA + 63) / 64, waves = std::max(1, (int)(16 / ((rays + 255) / 256)));
+  int ts = 1;
+  while (ts < 4 && (tiles + ts - 1) / ts > waves) ts *= 2;
+  const int own = (tiles + ts - 1) / ts;  // wavefronts per sample
+  const int samples = std::max(1, std::min({waves / own, (P.ray_steps + 1) / 2, 65536 / (28 * NLA)}));
+  const size_t shmem = samples == 1 ? 2 * sizeof(float4) * (size_t)NLA : 28 * (size_t)samples * NLA;
+  const RayGeoView V = ray_geo_view(P);
+  const dim3 grid((unsigned)rays + (acc.E_out ? 1u : 0u), 1, P.batch > 0 ? (unsigned)P.batch : 1u), block(64u * own * samples);
+  auto as = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, block, shmem, stream, P, P.batch_params, dJ, V.th, V.T, V.rs, V.fold, out, acc, samples, wc);
+  };
+  auto with = [&](auto kB) {
+    constexpr bool b = decltype(kB)::value;
+    if (ts == 1) as(ray_scatter_ordered_kernel<1, b, kExact>);
+    else if (ts == 2) as(ray_scatter_ordered_kernel<2, b, kExact>);
+    else as(ray_scatter_ordered_kernel<4, b, kExact>);
+  };
+  P.batch > 0 ? with(std::true_type()) : with(std::false_type());
   return hipGetLastError();
 }
 
 hipError_t launch_ray_scatter(const DevParams& P, const float* dJ, float4* out, WorkCounters* wc, hipStream_t stream,
-                              const RsAccum& acc, bool by_sample) {
+                              const RsAccum& acc, bool ordered) {
   if ((acc.S_in == nullptr) != (acc.S_out == nullptr) || (acc.E_out && !acc.dE)) return hipErrorInvalidValue;
   if (!P.ray_geo || !P.sun_ss || !P.rs_items || P.rs_groups < 1 || P.rs_groups > kMaxRsGroups) return hipErrorInvalidValue;
-  if (P.nS[2] < kExactSunRows) {
-    switch (P.rs_ts) {
-      case 1: return launch_ray_scatter_as<1, true>(P, dJ, out, wc, stream, acc, by_sample);
-      case 2: return launch_ray_scatter_as<2, true>(P, dJ, out, wc, stream, acc, by_sample);
-      case 4: return launch_ray_scatter_as<4, true>(P, dJ, out, wc, stream, acc, by_sample);
-    }
-    return hipErrorInvalidValue;
-  }
+  const bool exact = P.nS[2] < kExactSunRows;
+  if (ordered || P.rs_ts == 0)
+    return exact ? launch_ray_scatter_ordered<true>(P, dJ, out, wc, stream, acc)
+                 : launch_ray_scatter_ordered<false>(P, dJ, out, wc, stream, acc);
+  auto as = [&](auto ts) {
+    constexpr int TS = decltype(ts)::value;
+    return exact ? launch_ray_scatter_as<TS, true>(P, dJ, out, wc, stream, acc)
+                 : launch_ray_scatter_as<TS, false>(P, dJ, out, wc, stream, acc);
+  };
   switch (P.rs_ts) {
-    case 1: return launch_ray_scatter_as<1, false>(P, dJ, out, wc, stream, acc, by_sample);
-    case 2: return launch_ray_scatter_as<2, false>(P, dJ, out, wc, stream, acc, by_sample);
-    case 4: return launch_ray_scatter_as<4, false>(P, dJ, out, wc, stream, acc, by_sample);
-    case 8: return launch_ray_scatter_as<8, false>(P, dJ, out, wc, stream, acc, by_sample);
+    case 1: return as(std::integral_constant<int, 1>());
+    case 2: return as(std::integral_constant<int, 2>());
+    case 4: return as(std::integral_constant<int, 4>());
   }
   return hipErrorInvalidValue;
 }

@@ -19,6 +19,12 @@ hipError_t launch_single_scatter(const DevParams& P, float4* rayleigh, float4* m
 // The rays' ray-scatter items (DevParams::rs_items) from the sun map, once per build before launch_ray_scatter
 // (launch_single_scatter takes them along with ray_items).
 hipError_t launch_ray_items(const DevParams& P, hipStream_t stream);
+// The most items that a group of columns has on any ray of a scatter grid nS (counted on the host as the kernel lists
+// them), and how many its wavefronts look up (0: a grid that ray_scatter_ordered_kernel takes).
+struct RayItems {
+  int most, capacity;
+};
+RayItems ray_items_most(const int* nS, double radius, double height);
 // The per-build launches that read nothing of each other, in one launch: direction geometry of the
 // sphere quadrature (when sdirs, into geom), transmittance T, E0, the half-sphere geometry (when hdirs,
 // into P.sgeo), the sun table (P.sun_rows > 0), the ray geometry and the re-sampling map.
@@ -78,12 +84,12 @@ struct RsAccum {
   const float4* E_in = nullptr;
   float4* E_out = nullptr;
 };
-// by_sample: every entry's samples added one by one in order, with both heading columns mixed at each (slower; the
+// ordered: every entry's samples added one by one in order, with both heading columns mixed at each (the
 // rounding that the surrogate's training data keeps).
 // Reads P.ray_geo (launch_ray_geometry) and the per-build items P.rs_items (launch_ray_items or
 // launch_single_scatter).
 hipError_t launch_ray_scatter(const DevParams& P, const float* dJ, float4* out, WorkCounters* wc,
-                              hipStream_t stream, const RsAccum& acc = RsAccum(), bool by_sample = false);
+                              hipStream_t stream, const RsAccum& acc = RsAccum(), bool ordered = false);
 // Half-sphere direction geometry of every surface-radiance height into P.sgeo (once per build, before
 // launch_surface_radiance).
 hipError_t launch_surface_geometry(const DevParams& P, const Dir* dirs, int ndirs, hipStream_t stream);
