@@ -143,19 +143,20 @@ __host__ __device__ inline size_t resample_map_bytes(const DevParams& P) {
 // The split of a ray's slab: as many whole columns per group as 256 texels hold (4 per lane), evenly.  Per sun elevation a
 // group of c columns has at most c + 2 items: one for each heading whose sun direction is not clamped, on its own column,
 // and two for each of the (at most two) clamped directions, of whose columns one has no item of its own (the same bound
-// holds where rounding has left the lowest heading's coordinate just above 0).  Where that is more than a wavefront
-// looks up (more than 170 sun elevations, where a group is one column) the slab is folded and looked up by the
-// whole workgroup (rs_ts 0): 32 x 64 x 200 x 5 at 32 samples 189 us, 261 with the items shared by two wavefronts; 32 x 64 x
-// 300 x 3 182 us against 820 with eight texels per lane, which spill.
+// holds where rounding has left the lowest heading's coordinate just above 0); and on one column at most one per
+// heading.  The slab is folded and looked up by the whole workgroup (rs_ts 0) where that is more than a wavefront looks up,
+// with more than 170 sun elevations (32 x 64 x 200 x 5 at 32 samples 188 us, 261 with the items shared by two wavefronts; 32 x
+// 64 x 300 x 3 181 against 820 with eight texels per lane, which spill), and on grids of many rays whose groups are one
+// column of a large slab (40 x 100 x 150 x 6 351 us, 390 by items; 8 x 32 x 150 x 6 42 us, 34 by items).
 inline void rs_split(DevParams& P) {
   const int NL = P.nS[2], NA = P.nS[3], most = NL > 256 ? 1 : 256 / NL;
   const int want = (NA + most - 1) / most;
   P.rs_cols = (NA + want - 1) / want;
   P.rs_groups = (NA + P.rs_cols - 1) / P.rs_cols;
-  const int texels = P.rs_cols * NL;
+  const int texels = P.rs_cols * NL, c = P.rs_cols;
   P.rs_ts = texels > 128 ? 4 : texels > 64 ? 2 : 1;
-  P.rs_slots = (NL * (P.rs_cols + 2) + 63) & ~63;
-  if (P.rs_slots > rs_items(P.rs_ts)) P.rs_ts = 0;
+  P.rs_slots = (NL * (c == 1 ? (NA < 3 ? NA : 3) : c + 2) + 63) & ~63;
+  if (texels > 256 || P.rs_slots > rs_items(P.rs_ts) || (c == 1 && NL * NA >= 640 && P.nS[0] * P.nS[1] >= 2048)) P.rs_ts = 0;
 }
 
 // Bytes of the sun terms and the ray-scatter items (laid out by sun_map_view).

@@ -1271,7 +1271,10 @@ __global__ void __launch_bounds__(1024) ray_scatter_ordered_kernel(
   const int texels = max(0, min(64 * TS, NLA - first)), bytes = texels * (int)sizeof(Rgb);
   const float* __restrict__ own = dJ + 3 * first;
   float4* slabs = s_mem + mine * NLA;
-  float* terms = (float*)(s_mem + samples * NLA);  // [samples][3][NLA] (samples > 1)
+  float* terms = (float*)(s_mem + samples * NLA);  // [samples][3][NLA], and the samples' T (samples > 1)
+  float4* s_T = (float4*)(terms + (3 * samples * NLA + 3) / 4 * 4);
+  if (samples > 1)
+    for (int i = threadIdx.x; i < n; i += all) s_T[i] = geo_T[base_n + i];
   int c0[TS], c1[TS];
   float mix[TS], vl[TS], xl[TS];
   Rgb acc[TS];
@@ -1299,7 +1302,9 @@ __global__ void __launch_bounds__(1024) ray_scatter_ordered_kernel(
   for (int c = 0; c < 4; ++c)
 #pragma unroll
     for (int j = 0; j < TS; ++j) f.v[c][j] = Rgb{0.f, 0.f, 0.f};
-  FoldStep st = fold_step(gF, min(mine, n - 1));
+  // the next sample's nodes are in flight during a sample's lookups, and its step is read a sample before that
+  FoldStep st = fold_step(gF, min(mine, n - 1)), nx = fold_step(gF, min(mine + samples, n - 1));
+  float4 g = geo_rs[base_n + min(mine, n - 1)];
   fold_load<TS>(own, make_int4(-1, -1, -1, -1), st.off, bytes, lane, f);
   for (int round = 0; round < n; round += samples) {
     const int i = min(round + mine, n - 1);  // (past the last sample: the last again, not added)
@@ -1313,10 +1318,12 @@ __global__ void __launch_bounds__(1024) ray_scatter_ordered_kernel(
                                                   fmaf(w.w, d.y, fmaf(w.z, c.y, fmaf(w.y, b.y, w.x * a.y))),
                                                   fmaf(w.w, d.z, fmaf(w.z, c.z, fmaf(w.y, b.z, w.x * a.z))), 0.f);
       }
-    const FoldStep nx = fold_step(gF, min(i + samples, n - 1));  // the next sample's nodes, in flight during the lookups
     fold_load<TS>(own, st.off, nx.off, bytes, lane, f);
     st = nx;
-    const float4 T = geo_T[base_n + i], g = geo_rs[base_n + i];
+    nx = fold_step(gF, min(round + 2 * samples + mine, n - 1));
+    const float2 ab = make_float2(g.z, g.w);
+    g = geo_rs[base_n + min(round + samples + mine, n - 1)];
+    const float4 T = geo_T[base_n + i];
     __syncthreads();
 #pragma unroll
     for (int e = 0; e < TS; ++e) {
@@ -1326,7 +1333,7 @@ __global__ void __launch_bounds__(1024) ray_scatter_ordered_kernel(
         const double2 d = ss[entry(min(tid + e * threads, NLA - 1))];
         sun_coord_exact(sc, A64, P.g.R, geo_th[base_n + i], d.y, d.x, row, s);
       } else {
-        const float c = sun_coord(sc, make_float2(g.z, g.w), xl[e], vl[e]);
+        const float c = sun_coord(sc, ab, xl[e], vl[e]);
         row = min((unsigned)c, (unsigned)NL - 2);
         s = c - (float)row;
       }
@@ -1355,8 +1362,9 @@ __global__ void __launch_bounds__(1024) ray_scatter_ordered_kernel(
       for (int e = 0; e < TS; ++e) {
         const int q = (int)threadIdx.x + e * all;
         if (q < NLA)
+#pragma unroll 2
           for (int j = 0; j < min(samples, n - round); ++j) {
-            const float4 Tj = geo_T[base_n + round + j];
+            const float4 Tj = s_T[round + j];
             const float* t = terms + 3 * j * NLA + q;
             acc[e].x = fmaf(Tj.x, t[0], acc[e].x);
             acc[e].y = fmaf(Tj.y, t[NLA], acc[e].y);
@@ -2538,7 +2546,8 @@ static hipError_t launch_ray_scatter_as(const DevParams& P, const float* dJ, flo
 }
 
 // In plain order: the fewest texels per lane (1, 2 or 4) with which the workgroups of all rays are resident at once, and as
-// many samples at once as the wavefronts that are then left allow, within 64 KiB of LDS (28 bytes per texel and sample).
+// many samples at once as the wavefronts that are then left allow, within 64 KiB of LDS (28 bytes per texel and sample, and
+// the ray's T).
 template <bool kExact>
 static hipError_t launch_ray_scatter_ordered(const DevParams& P, const float* dJ, float4* out, WorkCounters* wc,
                                              hipStream_t stream, const RsAccum& acc) {
@@ -2547,8 +2556,9 @@ static hipError_t launch_ray_scatter_ordered(const DevParams& P, const float* dJ
   int ts = 1;
   while (ts < 4 && (tiles + ts - 1) / ts > waves) ts *= 2;
   const int own = (tiles + ts - 1) / ts;  // wavefronts per sample
-  const int samples = std::max(1, std::min({waves / own, (P.ray_steps + 1) / 2, 65536 / (28 * NLA)}));
-  const size_t shmem = samples == 1 ? 2 * sizeof(float4) * (size_t)NLA : 28 * (size_t)samples * NLA;
+  const int samples = std::max(1, std::min({waves / own, (P.ray_steps + 1) / 2, 61440 / (28 * NLA)}));
+  const size_t shmem = samples == 1 ? 2 * sizeof(float4) * (size_t)NLA
+                                    : ((28 * (size_t)samples * NLA + 15) & ~(size_t)15) + sizeof(float4) * P.ray_steps;
   const RayGeoView V = ray_geo_view(P);
   const dim3 grid((unsigned)rays + (acc.E_out ? 1u : 0u), 1, P.batch > 0 ? (unsigned)P.batch : 1u), block(64u * own * samples);
   auto as = [&](auto kernel) {
