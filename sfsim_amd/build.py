@@ -14,8 +14,9 @@ SOURCES = ["kernels.hip", "surrogate.hip", "atmo.cpp"]
 
 # -packed-fp32-ops: no v_pk_*_f32 generated for the device code (hipcc passes the flag to both
 # compilation passes; the host pass warns that it does not know the feature).
+# -fno-gpu-flush-denormals-to-zero: the kernels form LDS addresses as denormal floats.
 FLAGS = ["-O3", "-std=c++17", "-fPIC", "--offload-arch=gfx950", "-Xclang", "-target-feature", "-Xclang",
-         "-packed-fp32-ops", "-Wall", "-Wno-unused-function"]
+         "-packed-fp32-ops", "-fno-gpu-flush-denormals-to-zero", "-Wall", "-Wno-unused-function"]
 
 
 def hipcc():

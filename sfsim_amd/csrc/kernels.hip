@@ -13,6 +13,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstdlib>
 
 #include "kernels.hpp"
@@ -922,15 +923,15 @@ __device__ __forceinline__ FoldStep fold_step(ConstFoldSteps fs, int i) {
   return st;
 }
 
-// A lookup's byte address base + column x pitch, formed as the bits of a denormal float: bases and pitches are below
-// 2^23, so the sum is exact and the column needs no conversion to an integer.  The multiply-add and the subtraction
+// A lookup's byte address base + column x pitch, formed as the bits of a denormal float (build.py: denormals are kept):
+// bases and pitches are below 2^23, so the sum is exact and the column needs no conversion to an integer.  The multiply-add and the subtraction
 // that finds the column issue at twice the rate of a conversion, an integer multiply-add or a clamp.
 __device__ __forceinline__ unsigned lds_address(float column, unsigned pitch, unsigned base) {
   return __float_as_uint(fmaf(column, __uint_as_float(pitch), __uint_as_float(base)));
 }
 
-// LDS by address, for a kernel without static LDS, whose dynamic LDS begins at 0.  (As an offset from the array it
-// would cost an addition of the array's place, 0, at each access.)
+// LDS by address, for a kernel without static LDS, whose dynamic LDS begins at 0 (dynamic_lds_from_zero; as an offset
+// from the array it would cost an addition of the array's place, 0, at each access).
 typedef float Vec2 __attribute__((ext_vector_type(2)));
 typedef float Vec4 __attribute__((ext_vector_type(4)));
 template <class T>
@@ -2264,6 +2265,17 @@ __global__ void fill_zero_kernel(float* __restrict__ p, long long n) {
   if (i < n) p[i] = 0.f;
 }
 
+// Whether kernel K has no static LDS, so that its dynamic LDS begins at 0 as lds_read and lds_write take it; once per kernel.
+template <auto K>
+bool dynamic_lds_from_zero() {
+  static std::atomic<bool> seen{false};
+  if (seen.load()) return true;
+  hipFuncAttributes a;
+  if (hipFuncGetAttributes(&a, (const void*)K) != hipSuccess || a.sharedSizeBytes != 0) return false;
+  seen.store(true);
+  return true;
+}
+
 inline unsigned blocks_for(long long n) { return (unsigned)((n + kBlock - 1) / kBlock); }
 
 }  // namespace
@@ -2464,18 +2476,20 @@ PointScatterLds point_scatter_lds(const int* nS, int nE1, int sphere_steps, int 
 }
 
 template <int EPT, bool kMie, bool kELds, bool kBatches>
-static void point_scatter_as(const DevParams& P, const Dir* dirs, int ndirs, const PsRings& rings, const DirGeom* geom,
-                             const float4* dS, const float4* mie, const float4* dE, float* out, WorkCounters* wc,
-                             hipStream_t stream, const SrJob& sr, const PsPlan& plan) {
+static hipError_t point_scatter_as(const DevParams& P, const Dir* dirs, int ndirs, const PsRings& rings, const DirGeom* geom,
+                                   const float4* dS, const float4* mie, const float4* dE, float* out, WorkCounters* wc,
+                                   hipStream_t stream, const SrJob& sr, const PsPlan& plan) {
   const unsigned blocks = (unsigned)(P.nS[0] * plan.eblocks * plan.sblocks + sr.count);
   size_t shmem = plan.bytes;
   if (sr.count > 0) shmem = std::max(shmem, 4 * sizeof(float4) + sr_fold_bytes(P, sr.mie != nullptr));
-  if (P.batch > 0)
-    hipLaunchKernelGGL((point_scatter_kernel<EPT, kMie, kELds, true, kBatches>), dim3(blocks, 1, (unsigned)P.batch), dim3(kBlock),
-                       shmem, stream, P, P.batch_params, dirs, geom, ndirs, rings, dS, mie, dE, out, sr, plan, wc);
-  else
-    hipLaunchKernelGGL((point_scatter_kernel<EPT, kMie, kELds, false, kBatches>), dim3(blocks), dim3(kBlock), shmem, stream, P,
-                       P.batch_params, dirs, geom, ndirs, rings, dS, mie, dE, out, sr, plan, wc);
+  auto as = [&](auto kB) {
+    constexpr auto kernel = point_scatter_kernel<EPT, kMie, kELds, decltype(kB)::value, kBatches>;
+    if (!dynamic_lds_from_zero<kernel>()) return hipErrorInvalidKernelFile;
+    hipLaunchKernelGGL(kernel, dim3(blocks, 1, std::max(P.batch, 1)), dim3(kBlock), shmem, stream, P, P.batch_params, dirs, geom,
+                       ndirs, rings, dS, mie, dE, out, sr, plan, wc);
+    return hipGetLastError();
+  };
+  return P.batch > 0 ? as(std::true_type()) : as(std::false_type());
 }
 
 template <bool kMie>
@@ -2486,17 +2500,16 @@ static hipError_t launch_point_scatter_as(const DevParams& P, const Dir* dirs, i
   const PsPlan plan = point_scatter_plan<kMie>(P, ndirs, sphere_steps, ept);
   if (plan.bytes > kCuLds) return hipErrorInvalidValue;  // (no accepted shape)
   auto as = [&](auto entries, auto e_lds, auto batches) {
-    point_scatter_as<decltype(entries)::value, kMie, decltype(e_lds)::value, decltype(batches)::value>(
+    return point_scatter_as<decltype(entries)::value, kMie, decltype(e_lds)::value, decltype(batches)::value>(
         P, dirs, ndirs, rings, geom, dS, mie, dE, out, wc, stream, sr, plan);
   };
   auto with_dE = [&](auto entries, auto batches) {
-    plan.e_lds ? as(entries, std::true_type(), batches) : as(entries, std::false_type(), batches);
+    return plan.e_lds ? as(entries, std::true_type(), batches) : as(entries, std::false_type(), batches);
   };
   auto with_entries = [&](auto batches) {
-    ept == 1 ? with_dE(std::integral_constant<int, 1>(), batches) : with_dE(std::integral_constant<int, 2>(), batches);
+    return ept == 1 ? with_dE(std::integral_constant<int, 1>(), batches) : with_dE(std::integral_constant<int, 2>(), batches);
   };
-  plan.dirs < ndirs ? with_entries(std::true_type()) : with_entries(std::false_type());
-  return hipGetLastError();
+  return plan.dirs < ndirs ? with_entries(std::true_type()) : with_entries(std::false_type());
 }
 
 hipError_t launch_point_scatter(const DevParams& P, const Dir* dirs, int ndirs, int sphere_steps, const void* geom,
@@ -2536,13 +2549,14 @@ static hipError_t launch_ray_scatter_as(const DevParams& P, const float* dJ, flo
   const size_t shmem = rs_shared_bytes<TS>(groups * segs, P.rs_slots, kExact);
   const RayGeoView V = ray_geo_view(P);
   const dim3 grid((unsigned)rays + (acc.E_out ? 1u : 0u), 1, P.batch > 0 ? (unsigned)P.batch : 1u), block(64u * groups * segs);
-  if (P.batch > 0)
-    hipLaunchKernelGGL((ray_scatter_kernel<TS, true, kExact>), grid, block, shmem, stream, P, P.batch_params, dJ, V.th, V.T,
-                       V.rs, V.fold, P.rs_items, P.rs_entries, P.rs_heads, out, acc, segs, wc);
-  else
-    hipLaunchKernelGGL((ray_scatter_kernel<TS, false, kExact>), grid, block, shmem, stream, P, P.batch_params, dJ, V.th, V.T,
-                       V.rs, V.fold, P.rs_items, P.rs_entries, P.rs_heads, out, acc, segs, wc);
-  return hipGetLastError();
+  auto as = [&](auto kB) {
+    constexpr auto kernel = ray_scatter_kernel<TS, decltype(kB)::value, kExact>;
+    if (!dynamic_lds_from_zero<kernel>()) return hipErrorInvalidKernelFile;
+    hipLaunchKernelGGL(kernel, grid, block, shmem, stream, P, P.batch_params, dJ, V.th, V.T, V.rs, V.fold, P.rs_items, P.rs_entries,
+                       P.rs_heads, out, acc, segs, wc);
+    return hipGetLastError();
+  };
+  return P.batch > 0 ? as(std::true_type()) : as(std::false_type());
 }
 
 // In plain order: the fewest texels per lane (1, 2 or 4) with which the workgroups of all rays are resident at once, and as
