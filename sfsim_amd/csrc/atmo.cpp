@@ -1879,6 +1879,8 @@ int sfsim_atmo_surrogate_train(sfsim_atmo_ctx* ctx, const sfsim_atmo_params* atm
                                double lr, unsigned long long seed, float* losses) {
   TRY(activate(ctx));
   if (!atmospheres || count < 1 || steps < 0) return fail(ctx, SFSIM_ATMO_ERR_ARGUMENT, "need >= 1 atmosphere");
+  if (ctx->sg.batch_capacity < 0)
+    return fail(ctx, SFSIM_ATMO_ERR_ALLOC, "the surrogate's memory could not be had at its last reset");
   if (!ctx->sg.theta) TRY(sfsim_atmo_surrogate_reset(ctx, seed, 8192));
   const sfsim_atmo_params& p0 = atmospheres[0];
   for (int a = 0; a < count; ++a) {

@@ -672,8 +672,7 @@ hipError_t dalloc(T** p, size_t count) {
     if (e_ != hipSuccess) return e_;         \
   } while (0)
 
-hipError_t surrogate_alloc(Surrogate& s, int batch) {
-  surrogate_free(s);
+static hipError_t allocate(Surrogate& s, int batch) {
   const size_t n = MlpLayout::total;
   SG_TRY(dalloc(&s.theta, n));
   SG_TRY(dalloc(&s.theta_bf, n));
@@ -696,6 +695,16 @@ hipError_t surrogate_alloc(Surrogate& s, int batch) {
   SG_TRY(dalloc(&s.partial, (size_t)kMaxSplits * MlpLayout::total));
   s.batch_capacity = batch;
   return hipSuccess;
+}
+
+hipError_t surrogate_alloc(Surrogate& s, int batch) {
+  surrogate_free(s);
+  const hipError_t e = allocate(s, batch);
+  if (e != hipSuccess) {
+    surrogate_free(s);
+    s.batch_capacity = -1;
+  }
+  return e;
 }
 
 void surrogate_free(Surrogate& s) {
@@ -740,7 +749,7 @@ hipError_t surrogate_sync_bf16(Surrogate& s, hipStream_t stream) {
 
 int surrogate_loss_parts(int rows) { return (rows * kMlpOut + kEw - 1) / kEw; }
 
-int surrogate_loss_slots(int rows) { return std::max(1, std::min(256, (1 << 20) / surrogate_loss_parts(rows))); }
+int surrogate_loss_slots(int rows) { return std::max(1, std::min(256, (1 << 20) / std::max(1, surrogate_loss_parts(rows)))); }
 
 static hipError_t launch_pass(Surrogate& s, const PassSource& src, int rows, bool backward, int loss_slot, hipStream_t stream) {
   PassOutputs o;

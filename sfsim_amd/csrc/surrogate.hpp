@@ -85,7 +85,7 @@ struct PassOutputs {
 };
 
 struct Surrogate {
-  int batch_capacity = 0;
+  int batch_capacity = 0;  // -1: the last allocation failed (nothing is held)
   bool trained = false;
   // device buffers
   float* theta = nullptr;      // FP32 master weights (MlpLayout::total)
