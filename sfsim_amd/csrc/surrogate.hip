@@ -254,6 +254,7 @@ __global__ void __launch_bounds__(64 * kFragWaves) pass_kernel(const PassSource 
       for (int i = 0; i < 4; ++i) {
         z[l][4 * g + i] = acc[4 * g + i] + b;
         a[i] = silu(z[l][4 * g + i]);
+        if (row0 + 8 * g + 4 * h + i >= rows) a[i] = 0.f;  // (of the biases alone, not of a row: may be infinite)
       }
       store_rows(a, s_a[l & 1] + (8 * g + 4 * h) * kPitchH + col, kPitchH,
                  out.A[l] + ((size_t)(wave * steps + step0 + g) * 64 + lane) * 4);
