@@ -446,8 +446,10 @@ __global__ void __launch_bounds__(kSSEntries* kSSWaves) single_scatter_kernel(co
 
   const int rays = NH * NE;
   const int groups = (NLA + kSSEntries - 1) / kSSEntries;
-  const int group = groups - 1 - blockIdx.x / rays;
-  const int rayid = blockIdx.x - (groups - 1 - group) * rays;
+  const unsigned block = blockIdx.y * gridDim.x + blockIdx.x;  // (a launch's x holds less than 2^32 threads)
+  if (block >= (unsigned)groups * rays) return;
+  const int group = groups - 1 - (int)(block / rays);
+  const int rayid = (int)block - (groups - 1 - group) * rays;
   const int ih = rayid / NE, ie = rayid - ih * NE;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const Ray ray = make_ray(P, ih, ie);
@@ -2373,7 +2375,8 @@ hipError_t launch_single_scatter(const DevParams& P, float4* rayleigh, float4* m
     if (e != hipSuccess) return e;
   }
   const unsigned groups = (unsigned)((P.nS[2] * P.nS[3] + kSSEntries - 1) / kSSEntries);
-  hipLaunchKernelGGL(single_scatter_kernel, dim3(rays * groups), dim3(kSSEntries * kSSWaves),
+  const unsigned most = 1u << 22, blocks = rays * groups;
+  hipLaunchKernelGGL(single_scatter_kernel, dim3(std::min(blocks, most), (blocks + most - 1) / most), dim3(kSSEntries * kSSWaves),
                      single_scatter_shared_bytes(P.ray_steps), stream, P, rayleigh, mie, wc);
   return hipGetLastError();
 }
