@@ -32,6 +32,31 @@ def test_fetches_from_several_threads(built):
         np.testing.assert_array_equal(g.view(np.uint32), want[i].view(np.uint32))
 
 
+@pytest.mark.parametrize("rows", [682, 683, 1365, 1366, 2048, 5462])
+def test_sizes_around_one_copy_and_chunks(rows):
+    """768 bytes a row: 511.5 and 512.25 KiB, 1023.75 and 1024.5 KiB, exactly 3 chunks, 8 chunks and a little (one ring)."""
+    from sfsim_amd import atmosphere as atm
+    P = atm.make_params(planet={"height": 100000.0}, transmittance_shape=(rows, 64), surface_radiance_shape=(4, 9),
+                        scatter_shape=(2, 3, 2, 2), ray_steps=4, sphere_steps=4, iterations=0)
+    hip = ctypes.CDLL("libamdhip64.so.7")
+    hip.hipHostMalloc.argtypes = [ctypes.POINTER(ctypes.c_void_p), ctypes.c_size_t, ctypes.c_uint]
+    hip.hipHostFree.argtypes = [ctypes.c_void_p]
+    p, n = ctypes.c_void_p(), rows * 64 * 3
+    assert hip.hipHostMalloc(ctypes.byref(p), 4 * n, 0) == 0
+    try:
+        want = np.ctypeslib.as_array(ctypes.cast(p, ctypes.POINTER(ctypes.c_float)), (n,))
+        print("rows", rows, flush=True)
+        with atm.Atmosphere(0) as ctx:
+            ctx.build(P)
+            got = ctx.fetch(P, 0)
+            assert atm.lib().sfsim_atmo_fetch(ctx._ctx, 0, atm._fp(want), n) == 0
+            np.testing.assert_array_equal(got.ravel().view(np.uint32), want.view(np.uint32))
+            np.testing.assert_array_equal(ctx.generate_atmosphere_luts(P)["transmittance"].ravel().view(np.uint32),
+                                          want.view(np.uint32))
+    finally:
+        hip.hipHostFree(p)
+
+
 @pytest.mark.parametrize("which", range(4))
 def test_pinned_destination(built, which):
     atm, ctx, P, want = built
