@@ -1104,14 +1104,19 @@ __device__ __forceinline__ void rs_store(const DevParams& P, const RsAccum& accu
   }
 }
 
-// The extra workgroup: E <- tab(dE + E) (atmosphere_lut.clj:95-96).
+// The extra workgroups: E <- tab(dE + E) (atmosphere_lut.clj:95-96), an entry per thread.  (By one workgroup of the launch's
+// size, 128 threads at 32 x 64 x 32 x 8, a surface-radiance table of 16 x 1024 made a launch of 53 us 180.)
+inline unsigned rs_surface_blocks(const DevParams& P, const RsAccum& acc, unsigned threads) {
+  return acc.E_out ? (unsigned)(((long long)P.nE[0] * P.nE[1] + threads - 1) / threads) : 0;
+}
+
 template <bool kB>
-__device__ __forceinline__ void rs_surface(const DevParams& P, const RsAccum& accum) {
-  const long long nE = (long long)P.nE[0] * P.nE[1];
+__device__ __forceinline__ void rs_surface(const DevParams& P, const RsAccum& accum, int block) {
+  const long long nE = (long long)P.nE[0] * P.nE[1], i = (long long)block * blockDim.x + threadIdx.x;
   const float4* dE = atm_ptr<kB>(accum.dE, P);
   const float4* E_in = atm_ptr<kB>(accum.E_in, P);
   float4* E_out = atm_ptr<kB>(accum.E_out, P);
-  for (long long i = threadIdx.x; i < nE; i += blockDim.x) {
+  if (i < nE) {
     const float3 v = resample2_value(P, 3, dE, E_in, i);
     E_out[i] = make_float4(v.x, v.y, v.z, 0.f);
   }
@@ -1140,7 +1145,7 @@ __global__ void __launch_bounds__(1024) ray_scatter_kernel(
   const int NLA = NL * NA;
   const int n = P.ray_steps;
   if ((int)blockIdx.x >= NH * NE) {
-    rs_surface<kB>(P, accum);
+    rs_surface<kB>(P, accum, (int)blockIdx.x - NH * NE);
     return;
   }
   extern __shared__ float4 s_mem[];
@@ -1253,7 +1258,7 @@ __global__ void __launch_bounds__(1024) ray_scatter_ordered_kernel(
   }
   const int NH = P.nS[0], NE = P.nS[1], NL = P.nS[2], NA = P.nS[3], NLA = NL * NA, n = P.ray_steps;
   if ((int)blockIdx.x >= NH * NE) {
-    rs_surface<kB>(P, accum);
+    rs_surface<kB>(P, accum, (int)blockIdx.x - NH * NE);
     return;
   }
   extern __shared__ float4 s_mem[];
@@ -2551,7 +2556,8 @@ static hipError_t launch_ray_scatter_as(const DevParams& P, const float* dJ, flo
   while (segs > 1 && rs_shared_bytes<TS>(groups * segs, P.rs_slots, kExact) > 65536) --segs;
   const size_t shmem = rs_shared_bytes<TS>(groups * segs, P.rs_slots, kExact);
   const RayGeoView V = ray_geo_view(P);
-  const dim3 grid((unsigned)rays + (acc.E_out ? 1u : 0u), 1, P.batch > 0 ? (unsigned)P.batch : 1u), block(64u * groups * segs);
+  const dim3 block(64u * groups * segs);
+  const dim3 grid((unsigned)rays + rs_surface_blocks(P, acc, block.x), 1, P.batch > 0 ? (unsigned)P.batch : 1u);
   auto as = [&](auto kB) {
     constexpr auto kernel = ray_scatter_kernel<TS, decltype(kB)::value, kExact>;
     if (!dynamic_lds_from_zero<kernel>()) return hipErrorInvalidKernelFile;
@@ -2577,7 +2583,8 @@ static hipError_t launch_ray_scatter_ordered(const DevParams& P, const float* dJ
   const size_t shmem = samples == 1 ? 2 * sizeof(float4) * (size_t)NLA
                                     : ((28 * (size_t)samples * NLA + 15) & ~(size_t)15) + sizeof(float4) * P.ray_steps;
   const RayGeoView V = ray_geo_view(P);
-  const dim3 grid((unsigned)rays + (acc.E_out ? 1u : 0u), 1, P.batch > 0 ? (unsigned)P.batch : 1u), block(64u * own * samples);
+  const dim3 block(64u * own * samples);
+  const dim3 grid((unsigned)rays + rs_surface_blocks(P, acc, block.x), 1, P.batch > 0 ? (unsigned)P.batch : 1u);
   auto as = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, grid, block, shmem, stream, P, P.batch_params, dJ, V.th, V.T, V.rs, V.fold, out, acc, samples, wc);
   };
