@@ -2546,6 +2546,7 @@ hipError_t launch_point_scatter(const DevParams& P, const Dir* dirs, int ndirs, 
 // wavefronts per SIMD, 16 per CU of 256, which is what the kernel's registers allow), down to two samples each and
 // within 64 KiB of LDS.  The 32 x 64 x 32 x 8 grid at 64 steps: 59 us with 2 segments, 76 with 1, 60 with 4 (two
 // rounds); 19 x 45 x 20 x 7 at 51 steps: 24 us with 4, 38 with 5 (a second round of few), 30 with 2, 48 with 1.
+// Workgroups of five wavefronts do not share a CU's four SIMDs out (24 x 25 x 32 x 8 at 64 steps: 35 us with 5, 25 with 4).
 template <int TS, bool kExact>
 static hipError_t launch_ray_scatter_as(const DevParams& P, const float* dJ, float4* out, WorkCounters* wc, hipStream_t stream,
                                         const RsAccum& acc) {
@@ -2553,6 +2554,7 @@ static hipError_t launch_ray_scatter_as(const DevParams& P, const float* dJ, flo
   const long long rays = (long long)P.nS[0] * P.nS[1];
   int segs = (int)(16 / ((rays + 255) / 256)) / groups;
   segs = std::max(1, std::min(segs, P.ray_steps / 2));
+  if (groups * segs == 5) --segs;
   while (segs > 1 && rs_shared_bytes<TS>(groups * segs, P.rs_slots, kExact) > 65536) --segs;
   const size_t shmem = rs_shared_bytes<TS>(groups * segs, P.rs_slots, kExact);
   const RayGeoView V = ray_geo_view(P);
