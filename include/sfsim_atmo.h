@@ -5,7 +5,8 @@
  * returns 0 on success or a negative SFSIM_ATMO_ERR_* code; the message of the last failure on a
  * context is returned by sfsim_atmo_last_error.  No pointer passed in is kept after a call returns.
  * Calls on one context are serialised on that context's HIP stream and are synchronous for the
- * caller; different contexts may be used from different threads.
+ * caller; different contexts may be used from different threads.  Several threads may fetch tables of one
+ * context at once (sfsim_atmo_fetch, sfsim_atmo_fetch_batch).
  *
  * The reference builds these tables in Clojure with closures over sfsim.atmosphere functions
  * (src/clj/sfsim/atmosphere_lut.clj:43-105); closures cannot cross a C ABI, so the boundary is
@@ -233,7 +234,9 @@ int sfsim_atmo_build_seeded(sfsim_atmo_ctx* ctx, const sfsim_atmo_params* p, int
 int sfsim_atmo_build_from_sums(sfsim_atmo_ctx* ctx, const sfsim_atmo_params* p, int applications, const float* sums,
                                double tolerance, double* residual, int* fallback);
 /* The order sums P_1..P_5 of the plain iteration (iterations >= 5; only the first five orders run), and
- * the network's prediction of them: sums holds 5 scatter tables (RGB) one after the other. */
+ * the network's prediction of them: sums holds 5 scatter tables (RGB) one after the other.  The order sums (and
+ * the training targets) come from a kernel that adds each entry's samples one by one, the builds' tables from
+ * one that adds them by heading: the two differ by FP32 rounding, less than 2e-5 relative. */
 int sfsim_atmo_order_sums(sfsim_atmo_ctx* ctx, const sfsim_atmo_params* p, float* sums);
 int sfsim_atmo_surrogate_predict(sfsim_atmo_ctx* ctx, const sfsim_atmo_params* p, float* sums);
 

@@ -1337,8 +1337,7 @@ size_t layout_shared(sfsim_atmo_ctx* c, const sfsim_atmo_params* p, char* base) 
 
 // The host-made tables (owner's plan) into the buffers that layout_shared gave c, as prepare_pipeline would make them
 // one by one, in one copy that is not waited for: the call that uses them waits for the stream, also where it fails.
-// Made and uploaded by each call, with a wait per table, they kept the GPU idle for most of the 0.26 ms that a call of
-// 0.87 ms at 64x64 / 32x16x32x16 has lost since.
+// (Made and uploaded by each call, with a wait per table, a full-size no-alloc set of 32x64x32x8 took 0.87 ms; with this 0.61.)
 int upload_plan(sfsim_atmo_ctx* owner, sfsim_atmo_ctx* c, const sfsim_atmo_params* p) {
   HostPlan& plan = owner->plan;
   const bool dirs = p->iterations > 0;
